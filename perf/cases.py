@@ -2,7 +2,8 @@
 at `listed()`; `draw()` gives further cases of the same kinds over the same ranges of sizes, types and options.
 
 A case is a dict of plain values.  `prepare()` makes what the program holds before the call (tensors, handles, the
-workspace), `run()` makes the calls of one pass through the public entry points of `cubek_amd`.
+workspace), `run()` makes the calls of one pass through the public entry points of `cubek_amd`;
+`exact()` says in plain torch what the results stand for.
 """
 import math
 
@@ -289,3 +290,76 @@ def tolerance(case):
     if case["kind"] == "product":
         return {"rel": 0.007 if case["elem"] == "BF16" else 0.0009}
     return "exact"
+
+
+_RANGE = {"Q8S": (-127, 127), "Q8F": (-128, 127), "Q4S": (-7, 7), "Q4F": (-8, 7), "Q2S": (-1, 1), "Q2F": (-2, 1),
+          "E2M1": (-6, 6), "E4M3": (-448, 448), "E5M2": (-57344, 57344)}
+
+
+def _blocked(x, case):
+    """x with every block in one dimension, the last: [scales..., values of a block]."""
+    rows, cols = x.shape[-2:]
+    block, block_rows = case.get("block", 0), case.get("block_rows", 1)
+    if not block:
+        return x.reshape(1, -1)
+    lead = x.shape[:-2]
+    x = x.reshape(*lead, rows // block_rows, block_rows, cols // block, block)
+    return x.transpose(-2, -3).reshape(*lead, rows // block_rows, cols // block, block_rows * block)
+
+
+def _whole(v, shape, case):
+    """The reverse of _blocked."""
+    block, block_rows = case.get("block", 0), case.get("block_rows", 1)
+    if not block:
+        return v.reshape(shape)
+    rows, cols = shape[-2:]
+    v = v.reshape(*shape[:-2], rows // block_rows, cols // block, block_rows, block)
+    return v.transpose(-2, -3).reshape(shape)
+
+
+def _restored(x, case):
+    """The scales of a program's floats and the values its codes stand for, both in 64 bits.  The codes are whole numbers by
+    a rule in the float type itself (divide, round, clamp), which is followed here in that type."""
+    lo, hi = _RANGE[case["value"]]
+    param = _TORCH[case.get("param", "F32")]
+    v = _blocked(x, case)
+    scale = 2.0 * v.abs().amax(-1, keepdim=True).double() / (hi - lo)
+    stored = scale.float().to(x.dtype).to(param)
+    codes = (v / stored.to(x.dtype)).round_().clamp_(lo, hi).float().nan_to_num_(0.0)
+    if case.get("store") == "Native" and case["value"] in ("E4M3", "E5M2"):
+        codes = codes.to(torch.float8_e4m3fn if case["value"] == "E4M3" else torch.float8_e5m2).float()
+    elif case.get("store") == "Native" and case["value"] == "E2M1":
+        codes = torch.where(codes.abs() == 5.0, 4.0 * codes.sign(), codes)  # 5 lies between 4 and 6: to the even code
+    weights = codes.double() * stored.to(x.dtype).double()
+    return scale.squeeze(-1), _whole(weights, x.shape, case)
+
+
+def exact(case, seed):
+    """What run() returns, in 64 bits by plain torch; None for codes, which are words of bits."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    kind, dtype = case["kind"], _TORCH[case["elem"]]
+    if kind == "maxima":
+        x = _values(gen, (case["rows"], case["cols"]), "outliers", dtype)
+        return x.abs().amax(case["axis"], keepdim=True).double()
+    if kind == "cache":
+        x = _values(gen, (case["batch"], case["tokens"], case["heads"], case["head_dim"]), "normal1", dtype).permute(0, 2, 1, 3)
+    elif kind == "relayout":
+        x = _values(gen, (case["cols"], case["rows"]), "normal", dtype).t()
+    else:
+        x = _values(gen, (case["rows"], case["cols"]), "normal" if kind == "product" else case["dist"], dtype)
+    scale, restored = _restored(x, case)
+    if kind == "encode_tensor":
+        return None, scale.reshape(1)
+    if kind in ("round_trip", "cache"):
+        return None, scale, restored
+    if kind == "load":
+        return restored
+    if kind == "given":
+        return scale, None, scale, restored
+    if kind == "relayout":
+        return None, scale, None
+    v = case["vectors"]
+    weights = restored.to(dtype)  # a weight enters a product as the value that dequantize stores
+    x = _values(gen, (v, case["cols"]) if v > 1 else (case["cols"],), "normal1", dtype).double()
+    parts = [x @ weights[r:r + 4096].double().t() for r in range(0, case["rows"], 4096)]
+    return torch.cat(parts, dim=-1)
