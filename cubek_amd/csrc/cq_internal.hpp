@@ -279,10 +279,14 @@ bool gemv_streams(const GemvArgs& a);  // the launch takes the streaming kernel
 uint32_t gemv_vectors_per_launch(const GemvArgs& a, uint32_t remaining);
 hipError_t gemv_stream_f32_scales(hipStream_t s, const GemvArgs& a);    // the streaming kernels, by object
 hipError_t gemv_stream_16bit_scales(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_stream_batched(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_stream_wide(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_stream_f32_x(hipStream_t s, const GemvArgs& a);
-bool gemv_mfma_takes(const GemvArgs& a);  // ... on the matrix cores (4-bit fields, blocks of 32, f32 scales, 1 - 4 vectors)
-hipError_t gemv_mfma(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_bf16_f32(hipStream_t s, const GemvArgs& a);       // two to sixteen vectors, by type of x and of the scales
+hipError_t gemv_batch_bf16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a);
 hipError_t launch_gemv_quantized(hipStream_t s, const GemvArgs& a);
 
 }  // namespace cq

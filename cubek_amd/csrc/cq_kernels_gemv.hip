@@ -96,18 +96,14 @@ __device__ __forceinline__ void store_y(int dtype, void* y, uint64_t i, float v)
 // the same bits), or one of the native encodings below.
 constexpr int kCodeE4M3 = 100, kCodeE5M2 = 101, kCodeE2M1x2 = 102;
 
-// kVectors: 1, or room for that many right-hand vectors at once (x is then `vectors` <= kVectors rows of
-// x_stride elements, y as many rows of y_stride): every dequantized pair is used kVectors times out of its
-// registers, so a batch of vectors costs the weights' traffic and their dequantization once.
-// kSegment (several vectors, or rows too long for the LDS): strips of x staged at a time; the workgroup meets at a
+// kSegment (rows too long for the LDS): strips of x staged at a time; the workgroup meets at a
 // barrier and stages the next ones when its waves have worked through them (they all do the same work, so nobody
 // waits long).  0: all of x at once.
-template <dev::Float kF, class FS, int kCode, int kRows, int kWaves, int kDepth, int kVectors, int kSegment = 0>
+template <dev::Float kF, class FS, int kCode, int kRows, int kWaves, int kDepth, int kSegment = 0>
 __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
     const uint32_t* __restrict__ words, const FS* __restrict__ scales, const void* __restrict__ x, void* __restrict__ y,
     int y_dtype, uint32_t rows, uint32_t units_per_row, uint32_t units_per_block_log2, uint32_t block_rows,
-    uint64_t word_pitch, uint32_t scale_stride_row, uint32_t scale_stride_col, uint32_t vectors, uint32_t x_stride,
-    uint32_t y_stride) {
+    uint64_t word_pitch, uint32_t scale_stride_row, uint32_t scale_stride_col) {
     constexpr bool kPacked = kCode <= 8;
     constexpr int kBits = kPacked ? kCode : 8;      // (of the packed fields)
     constexpr uint32_t kVals = kPacked ? 128 / kBits : (kCode == kCodeE2M1x2 ? 32 : 16);  // values of a unit
@@ -115,28 +111,23 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
     constexpr uint32_t kPairs = kVals / 2;          // ... as packed pairs of x
     constexpr uint32_t kVecs = kWide32 ? kVals / 4 : kPairs / 4;  // ... as 16-byte pieces of x
     constexpr uint32_t kWordVals = kVals / 4;       // values out of one word
-    static_assert(!kWide32 || kVectors == 1, "several vectors at once: 16-bit float types");
     constexpr uint32_t kWordPairs = kVals / 8;      // pairs out of one word
     constexpr dev::Native kNative = kCode == kCodeE4M3 ? dev::Native::E4M3
                                     : kCode == kCodeE5M2 ? dev::Native::E5M2 : dev::Native::E2M1x2;
-    extern __shared__ u32x4 xs[];  // x, kVecs pieces per unit, whole strips; vector after vector
+    extern __shared__ u32x4 xs[];  // x, kVecs pieces per unit, whole strips
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t strips = (units_per_row + 63u) / 64u;
     constexpr bool kSegmented = kSegment > 0;
     constexpr uint32_t kSegmentOr1 = kSegment > 0 ? kSegment : 1;
-    static_assert(kVectors == 1 || kSegmented, "several vectors are staged in segments");
     static_assert(kSegment % kDepth == 0, "segments of whole rounds of the ring");
-    const uint32_t xs_vector = (kSegmented ? min(static_cast<uint32_t>(kSegment), strips) : strips) * 64u * kVecs;  // pieces of one staged vector
-    // strips [first, first + xs_vector / (64 * kVecs)) of every vector into LDS, zeros behind the end of x
+    const uint32_t xs_vector = (kSegmented ? min(static_cast<uint32_t>(kSegment), strips) : strips) * 64u * kVecs;  // pieces staged at once
+    // strips [first, first + xs_vector / (64 * kVecs)) into LDS, zeros behind the end of x
     const auto stage = [&](uint32_t first) {
-#pragma unroll
-        for (int v = 0; v < kVectors; v++) {
-            const u32x4* xv = reinterpret_cast<const u32x4*>(static_cast<const char*>(x) + static_cast<uint64_t>(v) * x_stride * (kWide32 ? 4u : 2u));
-            for (uint32_t i = threadIdx.x; i < xs_vector; i += blockDim.x) {
-                const uint32_t at = first * 64u * kVecs + i;
-                xs[v * xs_vector + i] = (static_cast<uint32_t>(v) < vectors && at < units_per_row * kVecs) ? xv[at] : u32x4{0, 0, 0, 0};
-            }
+        const u32x4* xv = static_cast<const u32x4*>(x);
+        for (uint32_t i = threadIdx.x; i < xs_vector; i += blockDim.x) {
+            const uint32_t at = first * 64u * kVecs + i;
+            xs[i] = at < units_per_row * kVecs ? xv[at] : u32x4{0, 0, 0, 0};
         }
     };
     if constexpr (!kSegmented) {
@@ -176,15 +167,15 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
     };
     // One row's share of this lane, the plain way (rolled loops, operands read again).  Only lanes whose scale
     // is not tame come here.
-    const auto plain_row = [&](const char* words_of_row, const char* scales_of_row, uint32_t strip, uint32_t v) {
+    const auto plain_row = [&](const char* words_of_row, const char* scales_of_row, uint32_t strip) {
         if constexpr (kWide32) {
             return 0.0f;  // (f32 x: the main path is the plain one)
         } else {
             const uint32_t u = strip * 64u + lane;
-            if (!kPacked || u >= units_per_row || v >= vectors) return 0.0f;
+            if (!kPacked || u >= units_per_row) return 0.0f;
             const uint32_t* wr = reinterpret_cast<const uint32_t*>(words_of_row) + u * 4u;
             const FS scale = *reinterpret_cast<const FS*>(scales_of_row + (u >> units_per_block_log2) * scale_step);
-            const typename Elem<kF>::T* xr = static_cast<const typename Elem<kF>::T*>(x) + static_cast<uint64_t>(v) * x_stride + u * kVals;
+            const typename Elem<kF>::T* xr = static_cast<const typename Elem<kF>::T*>(x) + u * kVals;
             float a = 0.0f;
     #pragma unroll 1
             for (int j = 0; j < 4; j++) {
@@ -201,72 +192,12 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
             return a;
         }
     };
-    float acc[kRows * kVectors];
+    float acc[kRows];
 #pragma unroll
-    for (int k = 0; k < kRows * kVectors; k++) acc[k] = 0.0f;
+    for (int k = 0; k < kRows; k++) acc[k] = 0.0f;
     // Lanes past the end of a row's last strip hold the row's last unit again (see `load`) against zeros of x: their
     // share is dropped, not added, because an infinite or NaN scale in that unit would turn the zeros into NaN.
     const auto lane_holds = [&](uint32_t strip) { return strip * 64u + lane < units_per_row; };
-    // several vectors: the pairs of the chunk's rows once, then vector after vector against them
-    const auto work_vectors = [&](const Chunk& c, uint32_t strip) {
-        if constexpr (kVectors > 1) {
-            uint32_t pairs[kRows][kPairs];
-            bool tame = true;
-    #pragma unroll
-            for (int k = 0; k < kRows; k++) {
-    #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if constexpr (kPacked)
-                        dev::dequantize_symmetric_packed_value_pairs_tame<kF, kBits>(c.w[k][j], c.s[k], &pairs[k][kWordPairs * j]);
-                    else
-                        dev::dequantize_symmetric_native_value_pairs<kF, kNative>(c.w[k][j], c.s[k], &pairs[k][kWordPairs * j]);
-                }
-                if constexpr (kPacked) tame = tame && dev::pairs_scale_is_tame<kF>(c.s[k]);
-            }
-            float part[kRows * kVectors];
-    #pragma unroll
-            for (int v = 0; v < kVectors; v++) {
-                uint32_t xp[kPairs];
-    #pragma unroll
-                for (uint32_t j = 0; j < kVecs; j++) {
-                    const u32x4 t = xs[v * xs_vector + ((strip % kSegmentOr1) * 64u + lane) * kVecs + j];
-                    xp[4 * j] = t[0], xp[4 * j + 1] = t[1], xp[4 * j + 2] = t[2], xp[4 * j + 3] = t[3];
-                }
-    #pragma unroll
-                for (int k = 0; k < kRows; k++) {
-                    float a = 0.0f;
-    #pragma unroll
-                    for (uint32_t i = 0; i < kPairs; i++) a = dot2<kF>(pairs[k][i], xp[i], a);
-                    part[k * kVectors + v] = a;
-                }
-            }
-            // lanes whose scale is not tame: the plain way, one (row, vector) at a time in a rolled loop (one copy of
-            // the code; unrolled, it took the compiler minutes)
-            if (kPacked && __builtin_amdgcn_ballot_w64(!tame) != 0) {
-                uint32_t plain_rows = 0;  // per lane: bit k set, row k's scale is not tame
-    #pragma unroll
-                for (int k = 0; k < kRows; k++) plain_rows |= dev::pairs_scale_is_tame<kF>(c.s[k]) ? 0u : 1u << k;
-    #pragma unroll 1
-                for (int kv = 0; kv < kRows * kVectors; kv++) {
-                    const int k = kv / kVectors;
-                    const char* wr = wrow[0];
-                    const char* sr = srow[0];
-    #pragma unroll
-                    for (int t = 1; t < kRows; t++) {
-                        if (k == t) wr = wrow[t], sr = srow[t];
-                    }
-                    if ((plain_rows >> k) & 1u) {
-                        const float r = plain_row(wr, sr, strip, static_cast<uint32_t>(kv % kVectors));
-    #pragma unroll
-                        for (int t = 0; t < kRows * kVectors; t++) part[t] = t == kv ? r : part[t];
-                    }
-                }
-            }
-    #pragma unroll
-            for (int k = 0; k < kRows * kVectors; k++) acc[k] += lane_holds(strip) ? part[k] : 0.0f;
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
     const auto work = [&](const Chunk& c, uint32_t strip) {
         if constexpr (kWide32) {
             // this lane's values of x
@@ -297,10 +228,6 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
             }
             __builtin_amdgcn_sched_barrier(0);
         } else {
-            if constexpr (kVectors > 1) {
-                work_vectors(c, strip);
-                return;
-            }
             // this lane's values of x, as pairs
             uint32_t xp[kPairs];
     #pragma unroll
@@ -328,7 +255,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
                 if (__builtin_amdgcn_ballot_w64(!tame) != 0) {
     #pragma unroll
                     for (int k = 0; k < kRows; k++)
-                        if (!dev::pairs_scale_is_tame<kF>(c.s[k])) part[k] = plain_row(wrow[k], srow[k], strip, 0);
+                        if (!dev::pairs_scale_is_tame<kF>(c.s[k])) part[k] = plain_row(wrow[k], srow[k], strip);
                 }
             } else {
                 // native encodings: the pairs are the plain arithmetic, every scale goes the same way
@@ -368,15 +295,11 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_stream_kernel(
         }
     }
 #pragma unroll
-    for (int k = 0; k < kRows * kVectors; k++) acc[k] = wave_sum_to_lane63(acc[k]);
+    for (int k = 0; k < kRows; k++) acc[k] = wave_sum_to_lane63(acc[k]);
     if (lane == 63) {
 #pragma unroll
-        for (int k = 0; k < kRows; k++) {
-#pragma unroll
-            for (int v = 0; v < kVectors; v++)
-                if (!idle && static_cast<uint32_t>(k) < nrows && static_cast<uint32_t>(v) < vectors)
-                    store_y(y_dtype, y, static_cast<uint64_t>(v) * y_stride + row0 + k, acc[k * kVectors + v]);
-        }
+        for (int k = 0; k < kRows; k++)
+            if (!idle && static_cast<uint32_t>(k) < nrows) store_y(y_dtype, y, row0 + k, acc[k]);
     }
 }
 
@@ -448,26 +371,26 @@ uint32_t log2_of(uint32_t v) {
 
 constexpr uint32_t values_per_unit(int code) { return code <= 8 ? 128 / code : (code == kCodeE2M1x2 ? 32 : 16); }
 
-// LDS for x: whole strips, 2 bytes per value, times the vectors staged at once
-uint32_t stream_lds_bytes(const GemvArgs& a, uint32_t vectors) {
+// LDS for x: whole strips, 2 bytes per value
+uint32_t stream_lds_bytes(const GemvArgs& a) {
     const uint32_t vals = 128 / a.bits;
-    return (a.cols / vals + 63) / 64 * 64 * vals * (a.dtype == CQ_F32 ? 4 : 2) * vectors;
+    return (a.cols / vals + 63) / 64 * 64 * vals * (a.dtype == CQ_F32 ? 4 : 2);
 }
 
-template <dev::Float kF, class FS, int kBits, int kWaves, int kVectors, int kRows = kStreamRows, int kSegment = 0>
+template <dev::Float kF, class FS, int kBits, int kWaves, int kSegment = 0>
 void launch_stream_waves(hipStream_t s, const GemvArgs& a) {
     constexpr uint32_t kVals = values_per_unit(kBits);
+    constexpr int kRows = kStreamRows;
     const uint32_t units_per_row = a.cols / kVals;
     const dim3 grid((a.rows + kRows * kWaves - 1) / (kRows * kWaves)), block(64 * kWaves);
     const uint32_t strips = (units_per_row + 63) / 64;
-    const uint32_t lds = kSegment > 0 ? (strips < kSegment ? strips : kSegment) * 64 * kVals * (kF == dev::Float::F32 ? 4 : 2) * kVectors
-                                      : stream_lds_bytes(a, 1);
-    hipLaunchKernelGGL((gemv_stream_kernel<kF, FS, kBits, kRows, kWaves, kStreamDepth, kVectors, kSegment>), grid, block,
+    const uint32_t lds = kSegment > 0 ? (strips < kSegment ? strips : kSegment) * 64 * kVals * (kF == dev::Float::F32 ? 4 : 2)
+                                      : stream_lds_bytes(a);
+    hipLaunchKernelGGL((gemv_stream_kernel<kF, FS, kBits, kRows, kWaves, kStreamDepth, kSegment>), grid, block,
                        lds, s, static_cast<const uint32_t*>(a.words),
                        static_cast<const FS*>(a.scales), a.x, a.y, a.y_dtype, a.rows, units_per_row,
                        a.block_rows == 0 ? 31u : log2_of(a.block_cols / kVals), a.block_rows == 0 ? 1u : a.block_rows,
-                       a.word_pitch, static_cast<uint32_t>(a.scale_stride_row), static_cast<uint32_t>(a.scale_stride_col),
-                       a.vectors, static_cast<uint32_t>(a.x_stride), static_cast<uint32_t>(a.y_stride));
+                       a.word_pitch, static_cast<uint32_t>(a.scale_stride_row), static_cast<uint32_t>(a.scale_stride_col));
 }
 
 // Two rows per wave, two strips in flight, four waves (eight rows) per workgroup; eight waves from 16384 columns
@@ -476,63 +399,48 @@ void launch_stream_waves(hipStream_t s, const GemvArgs& a) {
 // [8192, 28672]): 2 / 4 / 2 10.1, 31.3, 9.5, 33.5 us; 2 / 8 / 2 11.2, 33.1, 9.0, 28.9 us; 2 / 4 / 3 10.3, 33.0,
 // 10.1, 33.4 us; 4 / 4 / 2 11.8, 36.5, 10.3, 32.6 us; 1 / 4 / 4 11.4, 34.0, 10.1, 43.3 us; 3 / 4 / 2 10.8, 31.2,
 // 11.7, 34.5 us.
-// Right-hand vectors at once, and the waves of a workgroup that shares their x, rows per wave.  Measured on MI355X,
-// four vectors on 4-bit [28672, 8192] / [14336, 4096] / [4096, 8192] and e4m3 bytes [28672, 8192] (waves / rows):
-// 8 / 2 56.8, 19.3, 12.2, 57.1 us; 16 / 2 63.5, 19.6, 15.3, 67.9 us; 8 / 4 60.0, 20.1, 17.0, 71.7 us; 4 / 2 79.0,
-// 19.6, 13.0, 82.2 us; 16 / 4 68.6, 22.5, 29.6, 68.3 us.
-// Strips of x staged at a time (64 KiB of LDS for four vectors of 4-bit units): 4; with 2, [28672, 8192] took 63.0
-// instead of 57.4 us (e4m3 bytes 72.4 instead of 60.5 us), with 8 (half as many 4-bit workgroups per compute
-// unit) 83.3 us.
-constexpr int kBatch = 4, kBatchWaves = 8, kBatchRows = 2, kBatchSegment = 4;
-constexpr bool batches(int code) { return code != 2; }  // (64 values per unit: their pairs alone would fill the registers)
-
 constexpr int kWideSegment = 16;  // strips of x at a time where a row has more than kStreamMaxColumns values
 
-template <dev::Float kF, class FS, int kBits, bool kBatched>
+// kWide: rows of more than kStreamMaxColumns values, x by segments
+template <dev::Float kF, class FS, int kBits, bool kWide>
 void launch_stream_bits(hipStream_t s, const GemvArgs& a) {
-    if constexpr (kBatched) {
-        if (a.vectors == 1)  // one right-hand side, rows too long for the LDS
-            launch_stream_waves<kF, FS, kBits, 8, 1, kStreamRows,
-                                kWideSegment * int(values_per_unit(4)) / int(values_per_unit(kBits)) / (kF == dev::Float::F32 ? 2 : 1)>(s, a);
-        else if constexpr (batches(kBits) && kF != dev::Float::F32)
-            launch_stream_waves<kF, FS, kBits, kBatchWaves, kBatch, kBatchRows, kBatchSegment>(s, a);
-    } else if (a.cols >= 16384) {
-        launch_stream_waves<kF, FS, kBits, 8, 1>(s, a);
-    } else {
-        launch_stream_waves<kF, FS, kBits, 4, 1>(s, a);
-    }
+    if constexpr (kWide)
+        launch_stream_waves<kF, FS, kBits, 8, kWideSegment * int(values_per_unit(4)) / int(values_per_unit(kBits)) / (kF == dev::Float::F32 ? 2 : 1)>(s, a);
+    else if (a.cols >= 16384)
+        launch_stream_waves<kF, FS, kBits, 8>(s, a);
+    else
+        launch_stream_waves<kF, FS, kBits, 4>(s, a);
 }
 
-template <dev::Float kF, class FS, bool kBatched>
+template <dev::Float kF, class FS, bool kWide>
 void launch_stream_scales(hipStream_t s, const GemvArgs& a) {
     if (a.native == 1)
-        launch_stream_bits<kF, FS, kCodeE4M3, kBatched>(s, a);
+        launch_stream_bits<kF, FS, kCodeE4M3, kWide>(s, a);
     else if (a.native == 2)
-        launch_stream_bits<kF, FS, kCodeE5M2, kBatched>(s, a);
+        launch_stream_bits<kF, FS, kCodeE5M2, kWide>(s, a);
     else if (a.native == 3)
-        launch_stream_bits<kF, FS, kCodeE2M1x2, kBatched>(s, a);
+        launch_stream_bits<kF, FS, kCodeE2M1x2, kWide>(s, a);
     else if (a.bits == 4)
-        launch_stream_bits<kF, FS, 4, kBatched>(s, a);
+        launch_stream_bits<kF, FS, 4, kWide>(s, a);
     else if (a.bits == 8)
-        launch_stream_bits<kF, FS, 8, kBatched>(s, a);
+        launch_stream_bits<kF, FS, 8, kWide>(s, a);
     else
-        launch_stream_bits<kF, FS, 2, kBatched>(s, a);
+        launch_stream_bits<kF, FS, 2, kWide>(s, a);
 }
 
-template <class FS, bool kBatched>
+template <class FS, bool kWide>
 hipError_t launch_stream_floats(hipStream_t s, const GemvArgs& a) {
     if (a.dtype == CQ_BF16)
-        launch_stream_scales<dev::Float::BF16, FS, kBatched>(s, a);
+        launch_stream_scales<dev::Float::BF16, FS, kWide>(s, a);
     else
-        launch_stream_scales<dev::Float::F16, FS, kBatched>(s, a);
+        launch_stream_scales<dev::Float::F16, FS, kWide>(s, a);
     return hipGetLastError();
 }
 
 }  // namespace
 
 // The streaming kernels sit in three objects, so that a process loads the code of the kind it uses (the first launch
-// out of an object loads all of it): one right-hand side with f32 scales, with f16 / bf16 scales, several at once
-// (and rows too long for the LDS), x in f32.
+// out of an object loads all of it): f32 scales, f16 / bf16 scales, rows too long for the LDS, x in f32.
 // CQ_GEMV_PART names the one being compiled; without it everything lands in one object.
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 0
 hipError_t gemv_stream_f32_scales(hipStream_t s, const GemvArgs& a) { return launch_stream_floats<float, false>(s, a); }
@@ -543,7 +451,7 @@ hipError_t gemv_stream_16bit_scales(hipStream_t s, const GemvArgs& a) {
 }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 2
-hipError_t gemv_stream_batched(hipStream_t s, const GemvArgs& a) {
+hipError_t gemv_stream_wide(hipStream_t s, const GemvArgs& a) {
     switch (a.param_dtype) {
         case CQ_F32: return launch_stream_floats<float, true>(s, a);
         case CQ_F16: return launch_stream_floats<_Float16, true>(s, a);
@@ -573,17 +481,22 @@ bool gemv_streams(const GemvArgs& a) {
             a.scale_stride_row >= (1ull << 32) || (a.cols / a.block_cols) * a.scale_stride_col >= (1ull << 29))
             return false;
     }
-    if (a.x_stride >= (1ull << 32) || a.y_stride >= (1ull << 32)) return false;  // the kernels take them as 32-bit numbers
     return a.cols % vals == 0 && a.cols < (1u << 26) && a.word_pitch % 4 == 0 && a.x_aligned16 && a.words_aligned16;
 }
 
 namespace {
 
+hipError_t gemv_batch(hipStream_t s, const GemvArgs& a) {
+    if (a.dtype == CQ_BF16)
+        return a.param_dtype == CQ_F32 ? gemv_batch_bf16_f32(s, a) : a.param_dtype == CQ_F16 ? gemv_batch_bf16_f16(s, a) : gemv_batch_bf16_bf16(s, a);
+    return a.param_dtype == CQ_F32 ? gemv_batch_f16_f32(s, a) : a.param_dtype == CQ_F16 ? gemv_batch_f16_f16(s, a) : gemv_batch_f16_bf16(s, a);
+}
+
 hipError_t launch_one(hipStream_t s, const GemvArgs& a) {
-    if (gemv_mfma_takes(a)) return gemv_mfma(s, a);  // two to four vectors of the common 4-bit layout: matrix cores
+    if (a.vectors > 1) return gemv_batch(s, a);
     if (gemv_streams(a)) {
         if (a.dtype == CQ_F32) return gemv_stream_f32_x(s, a);
-        if (a.vectors > 1 || a.cols > kStreamMaxColumns) return gemv_stream_batched(s, a);
+        if (a.cols > kStreamMaxColumns) return gemv_stream_wide(s, a);
         return a.param_dtype == CQ_F32 ? gemv_stream_f32_scales(s, a) : gemv_stream_16bit_scales(s, a);
     }
     // the N-D layout of the [rows, cols] matrix, as the reference's scales_layout builds it
@@ -605,11 +518,13 @@ uint32_t dtype_bytes(int dtype) { return dtype == CQ_F32 ? 4u : 2u; }
 
 }  // namespace
 
-// How many of the remaining vectors the next launch takes: up to four at once where the streaming kernel applies
-// (all but the 2-bit fields) and every one of them starts on a 16-byte boundary; else one.
+// How many of the remaining vectors the next launch takes: up to sixteen at once on the matrix cores where the streaming
+// kernel's layouts come with x in a 16-bit type (all but the 2-bit fields), every vector starts on a 16-byte boundary and
+// the distances inside sixteen rows (and between the vectors) fit the 32 bits the kernel keeps them in; else one.
 uint32_t gemv_vectors_per_launch(const GemvArgs& a, uint32_t remaining) {
     if (remaining < 2 || !gemv_streams(a) || (a.x_stride * 2) % 16 != 0 || a.bits == 2 || a.dtype == CQ_F32) return 1;
-    return remaining < kBatch ? remaining : kBatch;
+    if (a.rows >= (1u << 31) || a.word_pitch >= (1u << 25) || a.scale_stride_row >= (1u << 25) || a.x_stride >= (1u << 26)) return 1;
+    return remaining < 16 ? remaining : 16;
 }
 
 // an empty sum: every y is zero

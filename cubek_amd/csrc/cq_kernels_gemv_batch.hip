@@ -1,0 +1,385 @@
+// Y = X * dequantize(W)^T for up to sixteen right-hand vectors at once, on the matrix cores: the quantized-input arm of
+// the reference's matmul (crates/cubek-matmul/src/base.rs:309-317; scale lookup
+// components/global/memory/layout.rs:371-455) for a decode step of a batch.  Every weight enters the product as
+// cq_dequantize would store it, F(F(scale) * F(code)) (crates/cubek-quant/src/dequantize.rs:20-79, through
+// include/cubek_quant_device.hpp); products accumulate in f32.
+//
+// A 16 x 16 x 32 matrix instruction wants, in lane (i, g) = (lane % 16, lane / 16), eight values of row i of W and
+// the same eight columns of vector i of x, and the columns of the four g may be any 32 that both operands agree on.
+// Read straight into registers in that order, an instruction touches 64 bytes of each of 16 rows, and such loads cost
+// about 75 cycles of a compute unit each, codes, scales and x alike (28672 x 8192, 4 bits: 47 - 60 us however deep
+// they were issued ahead).  So everything goes through LDS with direct loads of whole lines, a stage of eight 16-byte
+// units per row (128 bytes) at a time, and the next stage is on its way while one is worked on.  The places of a
+// stage are rotated from row to row on their way in, so that the 16 lanes of a read fall on 16 different groups of banks.
+//
+// Bound by instructions beside the loads: 2.4 per 4-bit bf16 weight for the dequantization, 0.5 for the rest; the
+// matrix instructions run beside them.  [28672, 8192] 4 bits, blocks of 32: 32 us for 4 vectors, 38 us for 16 (the
+// streaming kernel took four vectors a launch: 37 and 150 us; a read of the bytes 21 us).
+#include <hip/hip_runtime.h>
+
+#include "../../include/cubek_quant_device.hpp"
+#include "cq_internal.hpp"
+
+namespace cq {
+namespace {
+
+namespace dev = cubek_quant::device;
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kCodeE4M3 = 100, kCodeE5M2 = 101, kCodeE2M1x2 = 102;  // the native encodings; else bits per field
+
+constexpr uint32_t values_per_unit(int code) { return code <= 8 ? 128u / static_cast<uint32_t>(code) : (code == kCodeE2M1x2 ? 32u : 16u); }
+
+template <dev::Float kF>
+__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (kF == dev::Float::BF16) {
+        typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    } else {
+        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    }
+}
+
+// The 4-bit fields of f16 tensors pair up as (0, 4), (1, 5), (2, 6), (3, 7): one mask plants two digits in two
+// halves, without shifting them together; x is brought into the same order.
+template <dev::Float kF, int kCode>
+constexpr bool kCrossPairs = kF == dev::Float::F16 && kCode == 4;
+
+// Eight consecutive values (kVals of a unit / 8 such groups) of a lane's unit as the matrix instruction takes them.
+template <dev::Float kF, int kCode, bool kShort>
+__device__ __forceinline__ u32x4 operand(const u32x4& unit, uint32_t m, float scale) {
+    uint32_t p[8];
+    if constexpr (kCrossPairs<kF, kCode> && kShort) {
+        const uint32_t w = unit[m];
+        const _Float16 sh = static_cast<_Float16>(scale);
+        const f16x2 s2 = {sh, sh};
+        const f16x2 off0 = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-1032.0f)};
+        const f16x2 off1 = {static_cast<_Float16>(-72.0f), static_cast<_Float16>(-72.0f)};
+        const f16x2 sixteenth = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t v = h ? w >> 8 : w;
+            const uint32_t a = (v & 0x000f000fu) ^ 0x64086408u;  // 1024 + digit
+            const uint32_t b = (v & 0x00f000f0u) ^ 0x64806480u;  // 1024 + 16 * digit
+            const f16x2 qa = __builtin_bit_cast(f16x2, a) + off0;                                            // exact
+            const f16x2 qb = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, b), sixteenth, off1);      // exact
+            p[2 * h] = __builtin_bit_cast(uint32_t, s2 * qa);
+            p[2 * h + 1] = __builtin_bit_cast(uint32_t, s2 * qb);
+        }
+        return u32x4{p[0], p[1], p[2], p[3]};
+    } else if constexpr (kCode == 4) {
+        if constexpr (kShort)
+            dev::dequantize_symmetric_packed_value_pairs_tame<kF, 4>(unit[m], scale, p);
+        else
+            dev::dequantize_symmetric_packed_value_pairs<kF, 4>(unit[m], scale, p);
+        if constexpr (kCrossPairs<kF, kCode>)
+            return u32x4{__builtin_amdgcn_perm(p[2], p[0], 0x05040100u), __builtin_amdgcn_perm(p[2], p[0], 0x07060302u),
+                         __builtin_amdgcn_perm(p[3], p[1], 0x05040100u), __builtin_amdgcn_perm(p[3], p[1], 0x07060302u)};
+        else
+            return u32x4{p[0], p[1], p[2], p[3]};
+    } else if constexpr (kCode == 8) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if constexpr (kShort)
+                dev::dequantize_symmetric_packed_value_pairs_tame<kF, 8>(unit[2 * m + j], scale, p + 2 * j);
+            else
+                dev::dequantize_symmetric_packed_value_pairs<kF, 8>(unit[2 * m + j], scale, p + 2 * j);
+        }
+        return u32x4{p[0], p[1], p[2], p[3]};
+    } else if constexpr (kCode == kCodeE2M1x2) {
+        dev::dequantize_symmetric_native_value_pairs<kF, dev::Native::E2M1x2>(unit[m], scale, p);
+        return u32x4{p[0], p[1], p[2], p[3]};
+    } else {
+        constexpr dev::Native kNative = kCode == kCodeE4M3 ? dev::Native::E4M3 : dev::Native::E5M2;
+        dev::dequantize_symmetric_native_value_pairs<kF, kNative>(unit[2 * m], scale, p);
+        dev::dequantize_symmetric_native_value_pairs<kF, kNative>(unit[2 * m + 1], scale, p + 2);
+        return u32x4{p[0], p[1], p[2], p[3]};
+    }
+}
+
+__device__ __forceinline__ void store_y(int dtype, void* y, uint64_t i, float v) {
+    if (dtype == CQ_F32)
+        static_cast<float*>(y)[i] = v;
+    else if (dtype == CQ_F16)
+        static_cast<_Float16*>(y)[i] = static_cast<_Float16>(v);
+    else
+        static_cast<__bf16*>(y)[i] = static_cast<__bf16>(v);
+}
+
+#define CQ_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+
+constexpr uint32_t kU = 8;  // units of a row per stage
+// LDS of a stage: the codes and scales of a wave's 16 rows; the vectors' values (whole loads of 1 KiB)
+constexpr uint32_t kCodeBytes = 16 * kU * 16, kWaveBytes = kCodeBytes + 16 * kU * 4;
+template <int kCode>
+__host__ __device__ constexpr uint32_t x_bytes(uint32_t vectors) {
+    return (vectors * 2u * kU * values_per_unit(kCode) + 1023u) & ~1023u;
+}
+
+// kG groups of 16 rows per workgroup times kS shares of the row's stages (every kS-th one): kG * kS waves.  The waves
+// of a share use its x together; the shares' sums meet in LDS at the end.
+template <dev::Float kF, class FS, int kCode, int kG, int kS>
+__global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
+    const char* __restrict__ words, const char* __restrict__ scales, const char* __restrict__ x, void* __restrict__ y, int y_dtype,
+    uint32_t rows, uint32_t units_per_row, uint32_t units_per_block_log2, uint32_t block_rows, uint64_t row_bytes,
+    uint64_t scale_row_bytes, uint32_t scale_step, uint32_t vectors, uint32_t x_stride_bytes, uint64_t y_stride) {
+    constexpr bool kPacked = kCode <= 8;
+    constexpr uint32_t kM = values_per_unit(kCode) / 8;  // matrix instructions, and pieces of eight values of x, per unit
+    static_assert(kM == 2 || kM == 4, "units of 16 or 32 values");
+    constexpr uint32_t kQ = kU / 4;                      // a lane's units of a stage
+    constexpr uint32_t kPieces = kU * kM;                // a vector's pieces of a stage
+    constexpr uint32_t kCodeLoads = kCodeBytes / 1024, kScaleLoads = kU / 4, kXLoads = (16 * kPieces / 64 + kG - 1) / kG;
+    extern __shared__ char lds[];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t grp = wave % kG, share = wave / kG;
+    const uint32_t i = lane & 15u, g = lane >> 4;
+    const uint32_t x_size = x_bytes<kCode>(vectors);
+    const uint32_t buffer = kS * x_size + kG * kS * kWaveBytes;
+    char* const x_img = lds + share * x_size;
+    char* const code_img = lds + kS * x_size + wave * kWaveBytes;
+    const uint32_t row0 = min((blockIdx.x * kG + grp) * 16u, rows - 1u);
+    const bool idle = (blockIdx.x * kG + grp) * 16u >= rows;  // goes through the motions on the last row
+    const uint32_t stages = (units_per_row + kU - 1u) / kU, steps = (stages + kS - 1) / kS;
+    // scales of a row per stage: 2^slots_log2
+    const uint32_t slots_log2 = 3u - min(units_per_block_log2, 3u);
+    const uint32_t scale_loads = max(1u, (16u << slots_log2) / 64u);
+    const uint32_t my_x_loads = (x_size / 1024u - grp + kG - 1u) / kG;
+
+    // Where a lane's pieces of a stage come from: distances from bases that are uniform (the dispatch sees to it that they
+    // fit).  Codes: place p of row s holds unit (p - rot) % kU, rot = s / 2 (two rows lie side by side across the
+    // banks).  x: place p of vector v's blocks of 16 pieces holds piece (p - v) % 16.  Rows past the last one are the last
+    // one again and never stored.
+    const char* const wbase = words + row0 * row_bytes;
+    const char* const sbase = scales + (row0 / block_rows) * scale_row_bytes;
+    constexpr uint32_t kRowsPerLoad = 64 / kU;
+    uint32_t code_row[kCodeLoads], code_unit[kCodeLoads], scale_row[kScaleLoads], x_at[kXLoads], x_piece[kXLoads];
+#pragma unroll
+    for (uint32_t t = 0; t < kCodeLoads; t++) {
+        const uint32_t s = kRowsPerLoad * t + lane / kU;
+        code_unit[t] = (lane - (s >> 1)) & (kU - 1u);
+        code_row[t] = (min(row0 + s, rows - 1u) - row0) * static_cast<uint32_t>(row_bytes);
+    }
+#pragma unroll
+    for (uint32_t n = 0; n < kScaleLoads; n++)
+        scale_row[n] = (min(row0 + min((64u * n + lane) >> slots_log2, 15u), rows - 1u) / block_rows - row0 / block_rows) * static_cast<uint32_t>(scale_row_bytes);
+    const uint32_t scale_slot = lane & ((1u << slots_log2) - 1u);
+#pragma unroll
+    for (uint32_t n = 0; n < kXLoads; n++) {
+        const uint32_t pl = 64u * (grp + kG * n) + lane, v = min(pl / kPieces, vectors - 1u), in = pl % kPieces;
+        x_piece[n] = (in & ~15u) | ((in - v) & 15u);
+        x_at[n] = v * x_stride_bytes;
+    }
+    const auto load = [&](uint32_t stage, uint32_t into) {
+        const uint32_t unit0 = stage * kU, block0 = unit0 >> units_per_block_log2;
+        const bool partial = unit0 + kU > units_per_row;  // wave-uniform: units past the end are the last one again
+        const uint32_t last_unit = units_per_row - 1u - unit0, last_block = ((units_per_row - 1u) >> units_per_block_log2) - block0;
+        const char* const wfrom = wbase + static_cast<uint64_t>(unit0) * 16u;
+        const char* const sfrom = sbase + static_cast<uint64_t>(block0) * scale_step;
+        const char* const xfrom = x + static_cast<uint64_t>(unit0) * kM * 16u;
+#pragma unroll
+        for (uint32_t t = 0; t < kCodeLoads; t++) {
+            const uint32_t unit = partial ? min(code_unit[t], last_unit) : code_unit[t];
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u)), CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0,
+                                             2 /* nt */);
+        }
+        const uint32_t slot = partial ? min(scale_slot, last_block) : scale_slot;
+#pragma unroll
+        for (uint32_t n = 0; n < kScaleLoads; n++)
+            if (n < scale_loads) {
+                const char* const p = sfrom + (scale_row[n] + slot * scale_step);
+                if constexpr (sizeof(FS) == 4)
+                    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint32_t*>(p), CQ_LDS_PTR(code_img + into + kCodeBytes + n * 256u), 4, 0, 0);
+                else
+                    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint16_t*>(p), CQ_LDS_PTR(code_img + into + kCodeBytes + n * 256u), 2, 0, 0);
+            }
+#pragma unroll
+        for (uint32_t n = 0; n < kXLoads; n++)
+            if (n < my_x_loads) {
+                const uint32_t piece = partial ? min(x_piece[n], last_unit * kM + kM - 1u) : x_piece[n];
+                __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(xfrom + (x_at[n] + piece * 16u)), CQ_LDS_PTR(x_img + into + (grp + kG * n) * 1024u),
+                                                 16, 0, 0);
+            }
+    };
+
+    const uint32_t col = min(i, vectors - 1u);  // columns past the vectors repeat the last one
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    const auto work = [&](uint32_t stage, uint32_t from) {
+        const char* const x_mine = x_img + from + col * (kPieces * 16u);
+        const char* const codes = code_img + from + i * (kU * 16u);
+        const char* const slots = code_img + from + kCodeBytes + (i << (slots_log2 + 2u));
+        // everything a stage needs is asked of LDS at once, in the order of use (a word per scale: 16-bit ones alone in theirs)
+        FS stored[kQ];
+        u32x4 w[kQ], xb[kQ][kM];
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; q++)
+            stored[q] = *reinterpret_cast<const FS*>(slots + ((4u * q + g) >> (3u - slots_log2)) * 4u);
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; q++) {
+            w[q] = *reinterpret_cast<const u32x4*>(codes + ((4u * q + g + (i >> 1)) & (kU - 1u)) * 16u);
+#pragma unroll
+            for (uint32_t m = 0; m < kM; m++) {
+                const uint32_t p = (4u * q + g) * kM + m;
+                xb[q][m] = *reinterpret_cast<const u32x4*>(x_mine + (p >> 4) * 256u + ((p + col) & 15u) * 16u);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (stage * kU + kU > units_per_row) {  // wave-uniform: units past the row's end count nothing
+#pragma unroll
+            for (uint32_t q = 0; q < kQ; q++) {
+                const bool past = stage * kU + 4u * q + g >= units_per_row;
+                w[q] = past ? u32x4{0, 0, 0, 0} : w[q];
+                stored[q] = past ? static_cast<FS>(1.0f) : stored[q];
+#pragma unroll
+                for (uint32_t m = 0; m < kM; m++) xb[q][m] = past ? u32x4{0, 0, 0, 0} : xb[q][m];
+            }
+        }
+        if constexpr (kCrossPairs<kF, kCode>) {
+#pragma unroll
+            for (uint32_t q = 0; q < kQ; q++)
+#pragma unroll
+                for (uint32_t m = 0; m < kM; m++) {
+                    const u32x4 p = xb[q][m];
+                    xb[q][m] = u32x4{__builtin_amdgcn_perm(p[2], p[0], 0x05040100u), __builtin_amdgcn_perm(p[2], p[0], 0x07060302u),
+                                     __builtin_amdgcn_perm(p[3], p[1], 0x05040100u), __builtin_amdgcn_perm(p[3], p[1], 0x07060302u)};
+                }
+        }
+        // The short dequantization serves every scale below 2^100: a sum does not see the sign of a zero product, so unlike
+        // a stored value zero and negative scales may go this way, and digit * s - bias * s is exact down to the denormals.
+        float sc[kQ];
+        uint32_t largest = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kQ; q++) {
+            sc[q] = dev::round_to<kF>(dev::widen(stored[q]));
+            if (kPacked) largest = max(largest, __builtin_bit_cast(uint32_t, sc[q]) & 0x7fffffffu);
+        }
+        if (!kPacked || __builtin_amdgcn_ballot_w64(largest >= 0x71800000u) == 0) {  // ordinary scales all are
+#pragma unroll
+            for (uint32_t q = 0; q < kQ; q++)
+#pragma unroll
+                for (uint32_t m = 0; m < kM; m++) acc[m % 2] = mfma<kF>(operand<kF, kCode, true>(w[q], m, sc[q]), xb[q][m], acc[m % 2]);
+        } else {
+#pragma unroll 1
+            for (uint32_t qm = 0; qm < kQ * kM; qm++) {  // one copy of the general code: its operands are picked out
+                u32x4 word = {0, 0, 0, 0}, b = xb[0][0];
+                float scale = sc[0];
+#pragma unroll
+                for (uint32_t k = 0; k < kQ * kM; k++)
+                    if (qm == k) {
+                        b = xb[k / kM][k % kM], scale = sc[k / kM];
+                        word = kM == 4 ? u32x4{w[k / kM][k % kM], 0, 0, 0} : u32x4{w[k / kM][2 * (k % kM)], w[k / kM][2 * (k % kM) + 1], 0, 0};
+                    }
+                acc[0] = mfma<kF>(operand<kF, kCode, false>(word, 0, scale), b, acc[0]);
+            }
+        }
+    };
+    load(min(share, stages - 1u), 0);
+    for (uint32_t n = 0; n < steps; n++) {
+        const uint32_t from = (n & 1u) * buffer;
+        // stage n is there, and everybody has read the stage before it, whose place the next load takes
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (n + 1 < steps) load(min((n + 1) * kS + share, stages - 1u), buffer - from);
+        if (n * kS + share < stages) work(n * kS + share, from);
+    }
+    f32x4 sum = acc[0] + acc[1];  // sum[r] = (row 4 g + r, vector i)
+    if constexpr (kS > 1) {
+        __syncthreads();
+        float* const part = reinterpret_cast<float*>(lds);  // [share][group][register][lane]
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++)
+            if (share != 0) part[(((share - 1) * kG + grp) * 4u + r) * 64u + lane] = sum[r];
+        __syncthreads();
+        if (share != 0) return;
+#pragma unroll
+        for (uint32_t s = 0; s + 1 < kS; s++)
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) sum[r] += part[((s * kG + grp) * 4u + r) * 64u + lane];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++)
+        if (i < vectors && !idle && row0 + 4u * g + r < rows) store_y(y_dtype, y, i * y_stride + row0 + 4u * g + r, sum[r]);
+}
+
+uint32_t log2_of(uint32_t v) {
+    uint32_t l = 0;
+    while ((1u << l) < v) l++;
+    return l;
+}
+
+template <dev::Float kF, class FS, int kCode, int kG, int kS>
+void launch_shape(hipStream_t s, const GemvArgs& a) {
+    constexpr uint32_t kVals = values_per_unit(kCode);
+    hipLaunchKernelGGL((gemv_batch_kernel<kF, FS, kCode, kG, kS>), dim3((a.rows + 16 * kG - 1) / (16 * kG)),
+                       dim3(64 * kG * kS), 2 * (kS * x_bytes<kCode>(a.vectors) + kG * kS * kWaveBytes), s,
+                       static_cast<const char*>(a.words), static_cast<const char*>(a.scales), static_cast<const char*>(a.x), a.y, a.y_dtype,
+                       a.rows, a.cols / kVals, a.block_rows == 0 ? 31u : log2_of(a.block_cols / kVals), a.block_rows == 0 ? 1u : a.block_rows,
+                       a.word_pitch * 4, a.scale_stride_row * sizeof(FS), static_cast<uint32_t>(a.scale_stride_col * sizeof(FS)), a.vectors,
+                       static_cast<uint32_t>(a.x_stride * 2), a.y_stride);
+}
+
+// How many row groups share a workgroup's x, and how many waves share a row.  x comes from the L2 once per workgroup, so
+// row groups together save L2 traffic; but a launch wants a workgroup per compute unit and eight waves in each, so the
+// groups are as many as leave 256 workgroups, and the waves that are left over split the rows.  Measured on MI355X
+// (kG x kS 4 x 2, 2 x 4, 1 x 4): 4-bit bf16 [28672, 8192], 16 vectors 37.7, 49.6, 64.5 us; [8192, 28672] 67.1, 40.2,
+// 56.5 us; f16 [14336, 4096], 8 vectors 11.3, 10.8, 12.6 us; [4096, 4096], 16 vectors 12.2, 8.1, 7.4 us; e4m3 bytes
+// [14336, 4096], 16 vectors 17.8, 14.8, 21.3 us.  One row group takes eight waves while two workgroups of them fit
+// a compute unit's LDS ([4096, 4096], 4 vectors: 1 x 8 5.6, 1 x 4 6.1 us).
+template <dev::Float kF, class FS, int kCode>
+void launch_code(hipStream_t s, const GemvArgs& a) {
+    const uint32_t groups = (a.rows + 15) / 16;
+    if (groups >= 4 * 256)
+        launch_shape<kF, FS, kCode, 4, 2>(s, a);
+    else if (groups >= 2 * 256)
+        launch_shape<kF, FS, kCode, 2, 4>(s, a);
+    else if (2 * 8 * (x_bytes<kCode>(a.vectors) + kWaveBytes) <= 80 * 1024)
+        launch_shape<kF, FS, kCode, 1, 8>(s, a);
+    else
+        launch_shape<kF, FS, kCode, 1, 4>(s, a);
+}
+
+template <dev::Float kF, class FS>
+hipError_t launch_codes(hipStream_t s, const GemvArgs& a) {
+    if (a.native == 1)
+        launch_code<kF, FS, kCodeE4M3>(s, a);
+    else if (a.native == 2)
+        launch_code<kF, FS, kCodeE5M2>(s, a);
+    else if (a.native == 3)
+        launch_code<kF, FS, kCodeE2M1x2>(s, a);
+    else if (a.bits == 4)
+        launch_code<kF, FS, 4>(s, a);
+    else
+        launch_code<kF, FS, 8>(s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// One object per type of x and of the scales (CQ_GEMV_PART names the one being compiled), so that a process loads the
+// code of the kind it uses.
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 0
+hipError_t gemv_batch_bf16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, float>(s, a); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 1
+hipError_t gemv_batch_bf16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, __bf16>(s, a); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 2
+hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, _Float16>(s, a); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 3
+hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, float>(s, a); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 4
+hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, __bf16>(s, a); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 5
+hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, _Float16>(s, a); }
+#endif
+
+}  // namespace cq

@@ -133,9 +133,8 @@ def test_gemv_native_store_matches_oracle_dequantized_weights(oracle, case):
     check_case(oracle, case, rows * 11 + cols, native=True)
 
 
-# 4-bit fields on blocks of 32 with f32 scales, rows of whole groups of 128 values: two to four vectors at once go to
-# the matrix-core kernel (rows in runs of 2048 or 4096 values; a last run cut short; rows not a multiple of 16; pitched
-# rows; more vectors than four in turns, a last single one on the streaming kernel)
+# 4-bit fields on blocks of 32 with f32 scales: several vectors at once go to the matrix-core kernel (a last stage cut
+# short; rows not a multiple of 16; pitched rows)
 MATRIX_CORE_CASES = [
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 64, 4096, None),
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 77, 4224, None),
@@ -152,6 +151,28 @@ MATRIX_CORE_CASES = [
 @pytest.mark.parametrize("case", MATRIX_CORE_CASES, ids=_id)
 def test_gemv_on_the_matrix_cores(oracle, case, vectors):
     check_case(oracle, case, 3 + vectors, vectors=vectors)
+
+
+# Every split of a workgroup (four, two or one group of 16 rows; rows on two, four or eight waves): rows that end inside a
+# group and leave a workgroup's other groups empty, columns that end inside a stage of eight units or have fewer stages
+# than waves, every width of codes and type of scales, as many vectors as one launch takes and one more.  (Tolerance: as
+# above; the sums go through fewer additions in a row.)
+BATCH_CASES = [
+    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 16401, 288, None, False),       # 4 x 2, a group and a bit
+    (ElemType.F16, QuantValue.Q8S, [32], QuantParam.F16, 16384, 160, None, False),        # 4 x 2, two stages
+    (ElemType.F16, QuantValue.Q4S, [128], QuantParam.F16, 8209, 640, None, False),        # 2 x 4
+    (ElemType.BF16, QuantValue.E4M3, [32, 32], QuantParam.BF16, 8192, 96, None, True),    # 2 x 4, blocks over rows
+    (ElemType.BF16, QuantValue.Q8F, [16], QuantParam.F32, 35, 1040, None, False),         # 1 x 8, a scale per unit
+    (ElemType.BF16, QuantValue.E2M1, [64], QuantParam.F16, 17, 1088, None, True),         # 1 x 4 from five vectors on
+    (ElemType.F16, QuantValue.Q4F, None, QuantParam.BF16, 15, 4128, None, False),         # one scale
+    (ElemType.F16, QuantValue.E5M2, [16], QuantParam.F32, 16, 16, None, True),            # one unit
+]
+
+
+@pytest.mark.parametrize("vectors", [2, 4, 5, 16, 17])
+@pytest.mark.parametrize("case", BATCH_CASES, ids=lambda c: _id(c[:7]))
+def test_gemv_of_a_batch(oracle, case, vectors):
+    check_case(oracle, case[:7], 40 + vectors, native=case[7], vectors=vectors)
 
 
 @pytest.mark.parametrize("vectors", [2, 3, 4, 7, 8, 11])
