@@ -60,7 +60,7 @@ struct FlatArgs {
     int param_dtype;      // cq_dtype of the stored scales
     int encoding;         // 0 two's-complement fields (U32 store, native i8); 1 e4m3, 2 e5m2 bytes; 3 e2m1 nibbles
     Range range;
-    uint32_t whole_grid = 0;  // set between the launchers' objects only: whole tiles of the run to launch
+    uint32_t whole_tiles = 0, whole_grid = 0;  // set between the launchers' objects only: whole tiles of the run, workgroups of the launch
     uint32_t any_group = 0;   // set by the launchers: chunks per block where the lane-wise kernels divide by it (see `block`)
     bool lanes_only = false;  // set by the launchers: no whole-tile kernel exists for this launch (fields that wrap)
 };

@@ -478,7 +478,7 @@ struct LaneSteps {
 //            e2m1 for the native float stores, where kBits is the stored width).
 template <class F, int kBits, int kGroup, int kScaleSrc, int kParam, bool kWide, int kUnroll,
           int kThreads, bool kChecked, int kEnc, class Geo>
-__device__ __forceinline__ void quantize_flat_body(const Geo& geo, int param_dtype_rt, const QuantParams& qp,
+__device__ __forceinline__ void quantize_flat_body(const Geo& geo, uint32_t tile, int param_dtype_rt, const QuantParams& qp,
                                                    uint32_t num_partials) {
     constexpr bool kDynamic = kScaleSrc == kScaleDynamic;
     static_assert(kScaleSrc != kScalePartials || kGroup == 0, "partials feed the per-tensor scale only");
@@ -510,15 +510,6 @@ __device__ __forceinline__ void quantize_flat_body(const Geo& geo, int param_dty
     constexpr bool kWordsLater = Geo::kWaveRuns && !kChecked && kChunkBits < 32 && kUnroll % (32 / (kChunkBits < 32 ? kChunkBits : 32)) == 0;
     [[maybe_unused]] uint32_t words[kUnroll];
     const int param_dtype = kParam != kParamRt ? kParam : param_dtype_rt;
-    // Pass 2 of the per-tensor reduction walks the tiles last to first: pass 1 has just read the
-    // tensor first to last, so what it read last is what the L2 caches still hold.  Groups of
-    // eight consecutive tiles keep their places, because workgroup i runs on XCD i % 8 and tile
-    // i was read there in pass 1 (each XCD has its own L2).
-    uint32_t tile = blockIdx.x;
-    if constexpr (kScaleSrc == kScalePartials) {
-        const uint32_t whole = gridDim.x & ~7u;
-        if (tile < whole) tile = (whole - 8 - (tile & ~7u)) + (tile & 7u);
-    }
     const typename Geo::template Steps<kUnroll, kThreads, kChecked> at(geo, tile);
 
     // Given scales of a whole tile of one run: the 64 / kGroup scales a wave needs in each of its kUnroll steps come
@@ -681,20 +672,42 @@ __device__ __forceinline__ void quantize_flat_body(const Geo& geo, int param_dty
     }
 }
 
-// One contiguous run of whole tiles, parameters typed f32 or like the tensor (kParam): the hot launch.  Ragged
-// ends, other parameter types and rows that are not whole steps run lane by lane (quantize_flat_lanes_kernel),
-// which keeps the number of kernels in the library, and with it its size and load time, down.
+// Pass 2 of the per-tensor reduction walks its `whole` tiles last to first: pass 1 has just read the
+// tensor first to last, so what it read last is what the L2 caches still hold.  Groups of
+// eight consecutive tiles keep their places, because workgroup i runs on XCD i % 8 and tile
+// i was read there in pass 1 (each XCD has its own L2).
+template <int kScaleSrc>
+__device__ __forceinline__ uint32_t tile_order(uint32_t tile, uint32_t tiles) {
+    if constexpr (kScaleSrc == kScalePartials) {
+        const uint32_t whole = tiles & ~7u;
+        if (tile < whole) tile = (whole - 8 - (tile & ~7u)) + (tile & 7u);
+    }
+    return tile;
+}
+
+// One contiguous run, parameters typed f32 or like the tensor (kParam): the hot launch.  Its first `tiles` workgroups take
+// whole tiles and check no bounds; the ragged end behind them, and all of a small tensor, goes in single steps of
+// kThreads chunks, one per workgroup, in the same launch (as a launch of its own the end cost 2 - 5 us, and a few
+// microseconds of host time, on every size that is not a whole number of tiles).  Other parameter types and rows that are
+// not whole steps run lane by lane (quantize_flat_lanes_kernel), which keeps the number of kernels in the library, and
+// with it its size and load time, down.
 template <class F, int kBits, int kGroup, int kScaleSrc, bool kWide, int kUnroll, int kThreads, int kEnc = kEncInt,
           int kParam = CQ_F32>
 __global__ __launch_bounds__(kThreads) void quantize_flat_kernel(
     const u32x4* __restrict__ in, uint32_t* __restrict__ out, const void* __restrict__ scale_in,
-    void* __restrict__ scale_out, uint64_t chunk_begin, uint64_t chunk_end, QuantParams qp, uint32_t num_partials) {
-    const RunGeo geo{in, out, scale_in, scale_out, chunk_begin, chunk_end};
-    if constexpr (F::kPerChunk * kBits < 32) {  // less than a word of codes per chunk
-        const RunGeoWaves waves{geo};
-        quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(waves, kParam, qp, num_partials);
+    void* __restrict__ scale_out, uint32_t tiles, uint64_t num_chunks, QuantParams qp, uint32_t num_partials) {
+    const RunGeo geo{in, out, scale_in, scale_out, 0, num_chunks};
+    if (__builtin_expect(blockIdx.x < tiles, 1)) {
+        const uint32_t tile = tile_order<kScaleSrc>(blockIdx.x, tiles);
+        if constexpr (F::kPerChunk * kBits < 32) {  // less than a word of codes per chunk
+            const RunGeoWaves waves{geo};
+            quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(waves, tile, kParam, qp, num_partials);
+        } else {
+            quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(geo, tile, kParam, qp, num_partials);
+        }
     } else {
-        quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(geo, kParam, qp, num_partials);
+        quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, 1, kThreads, true, kEnc>(
+            geo, tiles * kUnroll + (blockIdx.x - tiles), kParam, qp, num_partials);
     }
 }
 
@@ -707,7 +720,7 @@ __global__ __launch_bounds__(kThreads) void quantize_flat_rows_kernel(
     void* __restrict__ scale_out, uint32_t step_begin, QuantParams qp, uint32_t num_partials, FlatRows rows) {
     const RowsGeo<16, F::kPerChunk * kBits / 8, kGroup> geo{in, out, scale_in, scale_out, step_begin, F::kBytes,
                                                             kParam == CQ_F32 ? 4 : 2, rows};
-    quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(geo, kParam, qp, num_partials);
+    quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParam, kWide, kUnroll, kThreads, false, kEnc>(geo, tile_order<kScaleSrc>(blockIdx.x, gridDim.x), kParam, qp, num_partials);
 }
 
 // Rows found lane by lane (LaneSteps), bounds-checked; the scale type is read at run time.  `tile_begin`:
@@ -718,17 +731,17 @@ __global__ __launch_bounds__(kThreads) void quantize_flat_lanes_kernel(
     void* __restrict__ scale_out, int param_dtype_rt, QuantParams qp, uint32_t num_partials, uint32_t tile_begin,
     LaneRows rows) {
     const LanesGeo geo{in, out, scale_in, scale_out, tile_begin, rows};
-    quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParamRt, kWide, kUnroll, kThreads, true, kEnc>(geo, param_dtype_rt, qp,
-                                                                                               num_partials);
+    quantize_flat_body<F, kBits, kGroup, kScaleSrc, kParamRt, kWide, kUnroll, kThreads, true, kEnc>(
+        geo, tile_order<kScaleSrc>(blockIdx.x, gridDim.x), param_dtype_rt, qp, num_partials);
 }
 
 // `scale_in` of the geometry holds the stored scales
 template <class F, int kBits, int kGroup, int kParam, int kUnroll, int kThreads, bool kChecked, int kEnc, class Geo>
-__device__ __forceinline__ void dequantize_flat_body(const Geo& geo, int param_dtype_rt) {
+__device__ __forceinline__ void dequantize_flat_body(const Geo& geo, uint32_t tile, int param_dtype_rt) {
     const int param_dtype = kParam != kParamRt ? kParam : param_dtype_rt;
     constexpr int kN = F::kPerChunk;
     constexpr int kChunkBits = kN * kBits;
-    const typename Geo::template Steps<kUnroll, kThreads, kChecked> at(geo, blockIdx.x);
+    const typename Geo::template Steps<kUnroll, kThreads, kChecked> at(geo, tile);
 
     // the scales of a wave's kUnroll steps through one load per lane and ds_bpermute (see quantize_flat_body); 16-bit
     // outputs only (f32 [8192, 8192], 2-bit codes on blocks of 64: 45.4 us with it, 44.6 us without)
@@ -797,13 +810,16 @@ __device__ __forceinline__ void dequantize_flat_body(const Geo& geo, int param_d
     }
 }
 
-// whole tiles of one contiguous run, parameters typed f32 or like the tensor (see quantize_flat_kernel)
+// one contiguous run, parameters typed f32 or like the tensor: whole tiles, then single steps (see quantize_flat_kernel)
 template <class F, int kBits, int kGroup, int kUnroll, int kThreads, int kEnc = kEncInt, int kParam = CQ_F32>
 __global__ __launch_bounds__(kThreads) void dequantize_flat_kernel(
-    const uint32_t* __restrict__ in, u32x4* __restrict__ out, const void* __restrict__ params, uint64_t chunk_begin,
-    uint64_t chunk_end) {
-    const RunGeo geo{in, out, params, nullptr, chunk_begin, chunk_end};
-    dequantize_flat_body<F, kBits, kGroup, kParam, kUnroll, kThreads, false, kEnc>(geo, kParam);
+    const uint32_t* __restrict__ in, u32x4* __restrict__ out, const void* __restrict__ params, uint32_t tiles,
+    uint64_t num_chunks) {
+    const RunGeo geo{in, out, params, nullptr, 0, num_chunks};
+    if (__builtin_expect(blockIdx.x < tiles, 1))
+        dequantize_flat_body<F, kBits, kGroup, kParam, kUnroll, kThreads, false, kEnc>(geo, blockIdx.x, kParam);
+    else
+        dequantize_flat_body<F, kBits, kGroup, kParam, 1, kThreads, true, kEnc>(geo, tiles * kUnroll + (blockIdx.x - tiles), kParam);
 }
 // pitched rows of whole steps
 template <class F, int kBits, int kGroup, int kUnroll, int kThreads, int kEnc = kEncInt, int kParam = CQ_F32>
@@ -811,7 +827,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_flat_rows_kernel(
     const uint32_t* __restrict__ in, u32x4* __restrict__ out, const void* __restrict__ params, uint32_t step_begin,
     FlatRows rows) {
     const RowsGeo<F::kPerChunk * kBits / 8, 16, kGroup> geo{in, out, params, nullptr, step_begin, kParam == CQ_F32 ? 4 : 2, 0, rows};
-    dequantize_flat_body<F, kBits, kGroup, kParam, kUnroll, kThreads, false, kEnc>(geo, kParam);
+    dequantize_flat_body<F, kBits, kGroup, kParam, kUnroll, kThreads, false, kEnc>(geo, blockIdx.x, kParam);
 }
 // lane by lane, bounds-checked, parameter type read at run time
 template <class F, int kBits, int kGroup, int kUnroll, int kThreads, int kEnc = kEncInt>
@@ -819,7 +835,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_flat_lanes_kernel(
     const uint32_t* __restrict__ in, u32x4* __restrict__ out, const void* __restrict__ params, int param_dtype_rt,
     uint32_t tile_begin, LaneRows rows) {
     const LanesGeo geo{in, out, params, nullptr, tile_begin, rows};
-    dequantize_flat_body<F, kBits, kGroup, kParamRt, kUnroll, kThreads, true, kEnc>(geo, param_dtype_rt);
+    dequantize_flat_body<F, kBits, kGroup, kParamRt, kUnroll, kThreads, true, kEnc>(geo, blockIdx.x, param_dtype_rt);
 }
 
 // Block abs-max -> scale typed like the input (what quantize takes as `scale`).

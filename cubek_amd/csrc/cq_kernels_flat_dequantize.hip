@@ -26,7 +26,7 @@ hipError_t dequantize_launch_enc(hipStream_t s, const FlatArgs& a) {
     if constexpr (F::kBytes == 2 && whole_tiles_for(kGroup)) {
         hipLaunchKernelGGL((dequantize_flat_kernel<F, kBits, kGroup, kU, kThreads, kEnc, F::kDtype>), dim3(a.whole_grid),
                            dim3(kThreads), 0, s, reinterpret_cast<const uint32_t*>(in), reinterpret_cast<u32x4*>(out), a.scale_in,
-                           0ull, static_cast<uint64_t>(a.whole_grid) * kThreads * kU);
+                           a.whole_tiles, a.num_chunks);
         return hipGetLastError();
     } else {
         return hipErrorInvalidValue;
@@ -35,10 +35,10 @@ hipError_t dequantize_launch_enc(hipStream_t s, const FlatArgs& a) {
     hipError_t same = hipSuccess;
     const hipError_t e = launch_flat(
         a, F::kDtype, kU,
-        [&](uint32_t grid, uint64_t) {
+        [&](uint32_t tiles, uint32_t grid) {
             if (a.param_dtype != CQ_F32) {  // a contiguous run, parameters typed like the tensor
                 FlatArgs b = a;
-                b.whole_grid = grid;
+                b.whole_tiles = tiles, b.whole_grid = grid;
                 same = dequantize_flat_same<F>(s, kBits, b);
             } else if (a.rows > 1) {
                 if constexpr (whole_steps_for(kGroup))
@@ -48,8 +48,8 @@ hipError_t dequantize_launch_enc(hipStream_t s, const FlatArgs& a) {
             } else {
                 if constexpr (whole_tiles_for(kGroup))
                     hipLaunchKernelGGL((dequantize_flat_kernel<F, kBits, kGroup, kU, kThreads, kEnc>), dim3(grid), dim3(kThreads), 0,
-                                       s, reinterpret_cast<const uint32_t*>(in), reinterpret_cast<u32x4*>(out), a.scale_in, 0ull,
-                                       static_cast<uint64_t>(grid) * kThreads * kU);
+                                       s, reinterpret_cast<const uint32_t*>(in), reinterpret_cast<u32x4*>(out), a.scale_in, tiles,
+                                       a.num_chunks);
             }
         },
         [&](const LaneRows& rows, uint32_t tile_begin, uint32_t grid, RunOffsets off) {

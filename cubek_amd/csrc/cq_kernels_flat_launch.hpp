@@ -28,7 +28,7 @@ CQ_DECLARE_QUANTIZE_TU(F16, 1)
 #undef CQ_DECLARE_QUANTIZE_TU
 // The whole-tile kernels of a contiguous run for parameters typed like the float tensor (bf16 scales of a bf16
 // tensor, f16 of f16) live in objects of their own (-DCQ_TU_SAME=1): the runtime loads an object's code on its
-// first launch, so launches with f32 parameters do not pay for them.  FlatArgs::whole_grid tiles, nothing else.
+// first launch, so launches with f32 parameters do not pay for them.  FlatArgs::whole_tiles and the steps behind them, nothing else.
 #ifndef CQ_TU_SAME
 #define CQ_TU_SAME 0
 #endif
@@ -281,15 +281,18 @@ QuantParams quant_params(const Range& r) {
     return p;
 }
 
-// How a flat launch is cut up.  The kernels over whole tiles check no bounds and exist for f32 parameters (a
-// contiguous run, or pitched rows of whole steps) and for parameters typed like the float tensor, `f_dtype` (a
-// contiguous run); everything else is the lane-wise kernel's:
-//   `whole(grid, begin)`                       tiles [begin, begin + grid) of the run / of the rows' steps
+// How a flat launch is cut up.  The kernels over whole tiles exist for f32 parameters (a contiguous run, or pitched
+// rows of whole steps) and for parameters typed like the float tensor, `f_dtype` (a contiguous run); everything else
+// is the lane-wise kernel's:
+//   `whole(tiles, grid)`                       the run: `tiles` whole tiles and grid - tiles steps behind them; the first
+//                                              `tiles` tiles of the rows' steps (grid = tiles)
 //   `lanes(rows, tile_begin, grid, offsets)`   lane by lane; `offsets` = chunks / scales to advance the base
 //                                              pointers by (a contiguous run only)
 struct RunOffsets {
     uint64_t chunks;  // 16-byte chunks of the float tensor
 };
+// Runs of fewer chunks go in single steps altogether: four times the workgroups, each with a quarter of the serial work.
+constexpr uint64_t kSmallRunChunks = 1u << 18;
 template <class WholeFn, class LanesFn>
 hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole, LanesFn lanes) {
     const uint64_t tile = static_cast<uint64_t>(kThreads) * unroll;
@@ -307,7 +310,7 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
         const uint32_t full = p32 && a.any_group == 0 && !a.lanes_only && whole_steps_for(group) && a.num_chunks % kThreads == 0
                                   ? static_cast<uint32_t>(lr.total_chunks / tile) : 0u;
         if (full > 0) {
-            whole(full, 0ull);
+            whole(full, full);
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         if (full < tiles) {
@@ -316,16 +319,17 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
         }
         return e;
     }
-    // one contiguous run
-    const uint64_t full = (p32 || a.param_dtype == f_dtype) && a.any_group == 0 && !a.lanes_only && whole_tiles_for(group) ? a.num_chunks / tile : 0;
-    if (full > 0) {
-        whole(static_cast<uint32_t>(full), 0ull);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+    // one contiguous run (flat_family() answers by the same rule)
+    if ((p32 || a.param_dtype == f_dtype) && a.any_group == 0 && !a.lanes_only && whole_tiles_for(group) && a.num_chunks >= kThreads * 4) {
+        const uint64_t full = a.num_chunks < kSmallRunChunks ? 0 : a.num_chunks / tile;
+        const uint64_t steps = (a.num_chunks - full * tile + kThreads - 1) / kThreads;
+        whole(static_cast<uint32_t>(full), static_cast<uint32_t>(full + steps));
+        return hipGetLastError();
     }
-    // the rest lane by lane, in pieces the 32-bit chunk numbers of those kernels can hold: a multiple of every tile and
+    // lane by lane, in pieces the 32-bit chunk numbers of those kernels can hold: a multiple of every tile and
     // every power-of-two block, or of whole blocks and whole words of codes
     const uint64_t piece = a.any_group == 0 ? (1ull << 30) : (1ull << 30) / (4ull * a.any_group) * (4ull * a.any_group);
-    for (uint64_t begin = full * tile; begin < a.num_chunks; begin += piece) {
+    for (uint64_t begin = 0; begin < a.num_chunks; begin += piece) {
         const uint64_t n = a.num_chunks - begin < piece ? a.num_chunks - begin : piece;
         lanes(lane_rows_of_run(n), 0u, static_cast<uint32_t>((n + tile - 1) / tile), RunOffsets{begin});
         if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -364,8 +368,7 @@ hipError_t quantize_launch_src(hipStream_t s, ScaleSource src, const FlatArgs& a
         if constexpr (kSrc != kScaleStored && F::kBytes == 2 && !kWide && whole_tiles_for(kGroup)) {
             hipLaunchKernelGGL((quantize_flat_kernel<F, kBits, kGroup, kSrc, kWide, kUnrollQ, kThreads, kEnc, F::kDtype>),
                                dim3(a.whole_grid), dim3(kThreads), 0, s, reinterpret_cast<const u32x4*>(in),
-                               reinterpret_cast<uint32_t*>(out), a.scale_in, a.scale_out, 0ull,
-                               static_cast<uint64_t>(a.whole_grid) * kThreads * kUnrollQ, qp, a.num_partials);
+                               reinterpret_cast<uint32_t*>(out), a.scale_in, a.scale_out, a.whole_tiles, a.num_chunks, qp, a.num_partials);
             return hipGetLastError();
         } else {
             return hipErrorInvalidValue;
@@ -374,11 +377,11 @@ hipError_t quantize_launch_src(hipStream_t s, ScaleSource src, const FlatArgs& a
         hipError_t same = hipSuccess;
         const hipError_t e = launch_flat(
             a, F::kDtype, kUnrollQ,
-            [&](uint32_t grid, uint64_t) {
+            [&](uint32_t tiles, uint32_t grid) {
                 if constexpr (kSrc != kScaleStored && !kWide) {  // (fields that wrap: lane by lane only)
                     if (a.param_dtype != CQ_F32) {  // a contiguous run, parameters typed like the tensor
                         FlatArgs b = a;
-                        b.whole_grid = grid;
+                        b.whole_tiles = tiles, b.whole_grid = grid;
                         same = quantize_flat_same<F>(kSrc == kScaleGivenF, s, kBits, src, b);
                     } else if (a.rows > 1) {
                         if constexpr (whole_steps_for(kGroup))
@@ -390,8 +393,7 @@ hipError_t quantize_launch_src(hipStream_t s, ScaleSource src, const FlatArgs& a
                         if constexpr (whole_tiles_for(kGroup))
                             hipLaunchKernelGGL((quantize_flat_kernel<F, kBits, kGroup, kSrc, kWide, kUnrollQ, kThreads, kEnc>),
                                                dim3(grid), dim3(kThreads), 0, s, reinterpret_cast<const u32x4*>(in),
-                                               reinterpret_cast<uint32_t*>(out), a.scale_in, a.scale_out, 0ull,
-                                               static_cast<uint64_t>(grid) * kThreads * kUnrollQ, qp, a.num_partials);
+                                               reinterpret_cast<uint32_t*>(out), a.scale_in, a.scale_out, tiles, a.num_chunks, qp, a.num_partials);
                     }
                 }
             },
