@@ -458,22 +458,28 @@ __device__ __forceinline__ TilePlace tile_place(uint32_t row_tiles, uint32_t col
     return TilePlace{tile % row_tiles, tile / row_tiles, tile < total};
 }
 
-// The quantize tile kernel in steps of 64 columns: thread (row pair, 16 columns), two neighbouring lanes share a
-// block of 32 columns (their maxima meet by DPP), 128 bytes of codes per row and tile.  16 KiB of floats, 18 KiB of
-// words and 4 KiB of scales per workgroup: four workgroups fit a compute unit instead of two.
-constexpr uint32_t kQStepCols = 64, kQPart = 16;
-template <class F, int kBits, int kEnc, int kScale>
+// The quantize tile kernel in steps of 4 * kPart columns: thread (row pair, kPart columns), the lanes that share a block
+// next to each other (their maxima meet by DPP).  kPart 16: 16 KiB of floats, 18 KiB of words and 4 KiB of scales per
+// workgroup: four workgroups fit a compute unit; blocks of 32 and 64 columns, or any multiple of 32 with given scales.
+// kPart 32: blocks of 128 columns, twice the floats.  kWholeTile: 128 bytes of codes per row and tile; else a tile is one
+// step, for launches of few tiles: eight times as many workgroups (4-bit), each with one step's latency.
+// Bound by its stores (runs of 128 and 32 bytes far apart).  Measured against the kernel it replaced for blocks of 64 and
+// 128 and for few tiles (quantize_transposed_quads_kernel, left with runs of 8 bytes): 4 bits, blocks of 64 f16
+// [31072, 1408] 37.8 -> 28.2 us, blocks of 128 [10944, 2816] 30.2 -> 22.8 us, bf16 [117472, 1024] 78.7 -> 67.0 us; few
+// tiles, blocks of 32 [1440, 864] 11.0 -> 5.4 us, [64, 10144] 11.7 -> 5.2 us, 8 bits [5664, 1216] 15.1 -> 8.6 us.
+template <class F, int kBits, int kEnc, int kScale, uint32_t kPart, bool kWholeTile>
 // seg_magic / seg_shift: column / a.segment as a multiplication and a shift (cq_magic_div.hpp; columns below 2^31)
 __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(TransposedArgs a, QuantParams qp, uint32_t seg_magic,
                                                                             uint32_t seg_shift) {
     using U = Unit<F, kBits>;
     constexpr uint32_t kRp = kTileRowsPerThread<F>;
     constexpr uint32_t kTileRows = 64 * kRp;
-    constexpr uint32_t kRowWords = 32;                                // 128 bytes of codes per row and tile
+    constexpr uint32_t kQPart = kPart, kQStepCols = 4 * kPart;
+    constexpr uint32_t kRowWords = kWholeTile ? 32 : kQStepCols / U::kNq;  // of codes per row and tile
     constexpr uint32_t kTileCols = kRowWords * U::kNq;
     constexpr uint32_t kSteps = kTileCols / kQStepCols;
     constexpr uint32_t kPartWords = kQPart / U::kNq;
-    static_assert(kPartWords >= 1, "a thread's sixteen columns are whole words");
+    static_assert(kPartWords >= 1 && kRowWords % 4 == 0, "a thread's columns are whole words, a tile's rows whole stores");
     constexpr uint32_t kStepWords = kQStepCols / U::kNq;
     constexpr uint32_t kRowParts = kTileCols / kTilePart;            // blocks of 32 columns per row and tile
     constexpr uint32_t kPieceRows = 16 / F::kBytes;                  // rows of one 16-byte piece
@@ -496,7 +502,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
     const uint32_t rows_here = a.rows - tile_r0 < kTileRows ? a.rows - tile_r0 : kTileRows;
 
     // loads: piece `piece` (16 bytes of rows) of column i * 16 + t / 16 of the step.  A step's address is a base
-    // that is the same for the whole workgroup plus 32 bits per thread (the launcher checked that 64 columns
+    // that is the same for the whole workgroup plus 32 bits per thread (the launcher checked that a step's columns
     // span less than 4 GiB); threads past the tensor's edge re-read the step's first piece, which nobody stores.
     const uint32_t piece = t & 15u, col_sub = t >> 4;
     const bool rows_live = tile_r0 + piece * kPieceRows < a.rows;    // rows is a multiple of kPieceRows
@@ -516,7 +522,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
         }
         __builtin_amdgcn_sched_barrier(0);  // the loads go out here, a step ahead of their use
     };
-    // arithmetic: rows rp * kRp ..., columns part * 16 ... of the step; lanes 2k and 2k + 1 share a block of 32
+    // arithmetic: rows rp * kRp ..., columns part * kPart ... of the step; two or four neighbouring lanes share a block
     const uint32_t part = t & 3u, rp = t >> 2;
     const uint32_t row0 = tile_r0 + rp * kRp;
     const uint32_t word_of_rows = rp ^ (part << 4);  // this thread's place in every column of its group
@@ -526,7 +532,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
         __syncthreads();  // the previous step's readers are done with the floats
 #pragma unroll
         for (uint32_t i = 0; i < kHeld; i++)
-            *reinterpret_cast<u32x4*>(&lds_floats[(i * 16 + col_sub) * 64 + ((piece * 4) ^ (i << 4))]) = held[i];
+            *reinterpret_cast<u32x4*>(&lds_floats[(i * 16 + col_sub) * 64 + ((piece * 4) ^ ((i / (kPart / 16)) << 4))]) = held[i];
         __syncthreads();
         if (step + 1 < total) load_step(step + 1);
 
@@ -535,11 +541,9 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
         uint32_t raw[kQPart];
 #pragma unroll
         for (uint32_t i = 0; i < kQPart; i++) raw[i] = lds_floats[(part * kQPart + i) * 64 + word_of_rows];
-        // the fused abs-max is launched for blocks of 32 columns only; other block sizes divide by multiplication
-        const uint32_t seg = kScale == 0 ? c0 / kTilePart : magic_div(c0, seg_magic, seg_shift);
-        const uint32_t segment = kScale == 0 ? kTilePart : a.segment;
-        const bool first_part = c0 == seg * segment;
-        const uint32_t scale_slot = seg - (kScale == 0 ? tile_c0 / kTilePart : magic_div(tile_c0, seg_magic, seg_shift));
+        const uint32_t seg = magic_div(c0, seg_magic, seg_shift);
+        const bool first_part = c0 == seg * a.segment;
+        const uint32_t scale_slot = seg - magic_div(tile_c0, seg_magic, seg_shift);
 #pragma unroll
         for (uint32_t j = 0; j < kRp; j++) {
             float v[kQPart];
@@ -555,11 +559,14 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
                 }
             }
             float s_f;
-            if constexpr (kScale == 0) {  // blocks of 32 columns: two lanes
+            if constexpr (kScale == 0) {  // blocks of two lanes' columns or (64 of kPart 16, 128) of four
                 float amax = 0.0f;
 #pragma unroll
                 for (uint32_t i = 0; i < kQPart; i++) amax = fmaxf(amax, fabsf(v[i]));  // NaN elements drop out
-                amax = group_max<2>(amax);
+                if (kPart == 32 || a.segment != 2 * kPart)  // uniform
+                    amax = group_max<4>(amax);
+                else
+                    amax = group_max<2>(amax);
                 const float s32 = absmax_is_tame(amax) ? scale_from_absmax_tame(amax, qp) : scale_from_absmax(amax, qp.width);
                 s_f = F::round(s32);
             } else {
@@ -587,12 +594,14 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
     for (uint32_t idx = t; idx < kTileRows * (kRowWords / 4); idx += kThreads) {
         const uint32_t row = idx / (kRowWords / 4), q = idx % (kRowWords / 4);
         if (row < rows_here && q * 4 < words_here)  // the launcher checked: rows hold a multiple of four words
-            stream_store(*reinterpret_cast<const u32x4*>(&lds_words[row * kRowPitch + q * 4]),
-                         reinterpret_cast<u32x4*>(tile_out + static_cast<uint64_t>(row) * a.vrow + q * 4));
+            // plain stores: runs that are not whole lines meet their neighbours' in the L2, and a re-pack right behind
+            // finds the codes there ([14336, 4096] 4 bits, both launches 45.4 -> 42.5 us)
+            *reinterpret_cast<u32x4*>(tile_out + static_cast<uint64_t>(row) * a.vrow + q * 4) =
+                *reinterpret_cast<const u32x4*>(&lds_words[row * kRowPitch + q * 4]);
     }
     if (a.scale_out != nullptr && !a.tensor_level) {
         const uint32_t tile_seg0 = tile_c0 / a.segment;
-        const uint32_t tile_segs = kRowParts / parts_per_block;
+        const uint32_t tile_segs = kRowParts < parts_per_block ? 1u : kRowParts / parts_per_block;
         const uint32_t segs_here = a.segments - tile_seg0 < tile_segs ? a.segments - tile_seg0 : tile_segs;
 #pragma unroll
         for (uint32_t idx = t; idx < kTileRows * kRowParts; idx += kThreads) {
@@ -890,32 +899,44 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
         const bool scales = a.scale_out != nullptr && !a.tensor_level && a.param_dtype == CQ_F32 && a.sb_col == 1;
         q.staged = (words ? 1u : 0u) | (scales ? 2u : 0u);
     }
-    // Tiles through LDS wherever the runs are 16-byte aligned on both sides (blocks of 32 columns for the fused
-    // abs-max, any multiple of 32 for given scales): 4-bit codes of a transposed bf16 view [28672, 8192],
-    // rotated buffers, against the quads kernel.
+    // Tiles through LDS wherever the runs are 16-byte aligned on both sides (blocks of 32, 64 and 128 columns for the
+    // fused abs-max, any multiple of 32 for given scales).
     const uint32_t cols = a.segments * a.segment;
     uint32_t seg_magic = 0, seg_shift = 0;
     magic_of(a.segment, &seg_magic, &seg_shift);
-    const uint32_t tile_cols = 32u * (32u / static_cast<uint32_t>(bits));  // 128 bytes of codes per row
+    const uint32_t nq = 32u / static_cast<uint32_t>(bits);
+    const uint32_t step_cols = kScale == 0 && a.segment == 128 ? 128u : 64u;
+    const uint32_t row_tiles = (a.rows + 64 * kTileRowsPerThread<F> - 1) / (64 * kTileRowsPerThread<F>);
+    // A tile is 128 bytes of codes per row; where that leaves fewer than two rounds of resident workgroups, a step (figures
+    // at the kernel).
+    const auto tiles_of = [&](uint32_t tile_cols) { return static_cast<uint64_t>(row_tiles) * ((cols + tile_cols - 1) / tile_cols); };
+    const bool whole_tile = tiles_of(32u * nq) * a.batches >= 1024;
+    const uint32_t tile_cols = whole_tile ? 32u * nq : step_cols;
+    const uint64_t tile_count = tiles_of(tile_cols);
     // A tile stores the scales of the blocks that start in it, as one run per row: blocks divide the tile's columns
     // (a block of 96 columns would straddle two tiles of 256; such layouts take the kernels below).
-    bool tiles = cols < (1u << 31) && a.pitch_f * F::kBytes < (1u << 25) && runs_of_16_bytes<F>(a, a.input) && a.segment % kTilePart == 0 && (kScale == 1 || a.segment == kTilePart) &&
-                 (a.tensor_level || tile_cols % a.segment == 0) &&
-                 (reinterpret_cast<uintptr_t>(a.output) & 15u) == 0 && a.vrow % 4 == 0 &&
-                 (cols / (32u / static_cast<uint32_t>(bits))) % 4 == 0 && a.batches <= 65535;
+    bool tiles = cols < (1u << 31) && a.pitch_f * F::kBytes * step_cols < (1ull << 31) && runs_of_16_bytes<F>(a, a.input) && a.segment % kTilePart == 0 &&
+                 (kScale == 1 || a.segment == 32 || a.segment == 64 || a.segment == 128) && (a.tensor_level || tile_cols % a.segment == 0) &&
+                 (reinterpret_cast<uintptr_t>(a.output) & 15u) == 0 && a.vrow % 4 == 0 && (cols / nq) % 4 == 0 && a.batches <= 65535 &&
+                 tile_count < (1u << 31);
     for (uint32_t k = 0; k < a.num_batch_dims; k++) tiles = tiles && a.batch_v[k] % 4 == 0;
-    const uint64_t tile_count = static_cast<uint64_t>((a.rows + 64 * kTileRowsPerThread<F> - 1) / (64 * kTileRowsPerThread<F>)) *
-                                ((cols + tile_cols - 1) / tile_cols);
     const dim3 tile_grid(static_cast<uint32_t>((tile_count + 7) / 8 * 8), 1, a.batches);  // see tile_place()
-    // two rounds of resident workgroups and more; below that the quads kernel's many small workgroups win
-    // (bf16 [4096, 4096], 4-bit: 14.3 us against 16.0 us; [8192, 8192], 2-bit: 43.6 us against 51.1 us)
-    if (tile_count >= (1u << 31) || tile_count * a.batches < 1024) tiles = false;
+#define CQ_TILE(B, E, P, T) \
+    hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale, P, T>), tile_grid, dim3(kThreads), 0, s, a, qp, seg_magic, seg_shift)
 #define CQ_LAUNCH(B, W, E)                                                                                        \
     {                                                                                                             \
-        if (tiles && !W)                                                                                          \
-            hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale>), tile_grid, dim3(kThreads), 0, s, a, qp, \
-                               seg_magic, seg_shift);                                                             \
-        else if (quads)                                                                                           \
+        if (tiles && !W) {                                                                                        \
+            if (kScale == 0 && step_cols == 128) {                                                                \
+                if constexpr (kScale == 0) {                                                                      \
+                    if (whole_tile) CQ_TILE(B, E, 32, true);                                                      \
+                    else CQ_TILE(B, E, 32, false);                                                                \
+                }                                                                                                 \
+            } else if (whole_tile) {                                                                              \
+                CQ_TILE(B, E, 16, true);                                                                          \
+            } else {                                                                                              \
+                CQ_TILE(B, E, 16, false);                                                                         \
+            }                                                                                                     \
+        } else if (quads)                                                                                         \
             hipLaunchKernelGGL((quantize_transposed_quads_kernel<F, B, W, E, kScale>), grid, dim3(kThreads), 0, s, q, qp); \
         else                                                                                                      \
             hipLaunchKernelGGL((quantize_transposed_kernel<F, B, W, E, kScale>), grid, dim3(kThreads), 0, s, a, qp); \
@@ -933,6 +954,7 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
         case kEncE2M1: if (bits == 4) CQ_LAUNCH(4, false, kEncE2M1) break;
     }
 #undef CQ_LAUNCH
+#undef CQ_TILE
     return hipErrorInvalidValue;
 }
 

@@ -300,6 +300,11 @@ LARGE_TRANSPOSED_SCHEMES = {
     "q8s_block96": QuantScheme.default().with_value(QuantValue.Q8S).with_level(QuantLevel.block([96])),
     "q8s_block160": QuantScheme.default().with_value(QuantValue.Q8S).with_level(QuantLevel.block([160])),
     "q2s_block192": QuantScheme.default().with_value(QuantValue.Q2S).with_level(QuantLevel.block([192])),
+    "q4s_block128": QuantScheme.default().with_value(QuantValue.Q4S).with_level(QuantLevel.block([128])),
+    "q8s_block64": QuantScheme.default().with_value(QuantValue.Q8S).with_level(QuantLevel.block([64])),
+    "q8s_block128": QuantScheme.default().with_value(QuantValue.Q8S).with_level(QuantLevel.block([128])),
+    "q2s_block64": QuantScheme.default().with_value(QuantValue.Q2S).with_level(QuantLevel.block([64])),
+    "q2s_block128": QuantScheme.default().with_value(QuantValue.Q2S).with_level(QuantLevel.block([128])),
 }
 
 
@@ -321,6 +326,23 @@ def test_large_transposed_floats_match_the_contiguous_path(gpu, elem, rows, cols
 def test_transposed_tiles_with_ragged_edges_match_the_contiguous_path(gpu, elem, rows, cols, names):
     """Transposed float tensors of thousands of 64 x 256-byte tiles whose last tiles are cut short along both
     axes (the sizes at which whole tiles go through shared memory), against the contiguous kernels."""
+    transposed_against_contiguous(gpu, elem, rows, cols, names)
+
+
+@pytest.mark.parametrize("elem,rows,cols,names", [
+    # few tiles: one step each (rows and the last step cut short; fewer columns than a step; one row group)
+    (ElemType.BF16, 136, 448, ("q4s_block32", "q4s_block64", "q8s_block64", "q2s_block64")),
+    (ElemType.F16, 264, 640, ("q4s_block128", "q8s_block128", "q2s_block128", "e4m3_native_block32")),
+    (ElemType.F32, 68, 384, ("q4s_block96", "q4s_block128", "q8s_block64", "q8s_block32", "q2s_block64", "q8s_tensor")),
+    (ElemType.BF16, 8, 32, ("q4s_block32", "q8s_block32")),
+    # whole tiles of blocks of 64 and 128
+    (ElemType.BF16, 4104, 32896, ("q4s_block128", "q8s_block64")),
+    (ElemType.F16, 2056, 65664, ("q2s_block128", "q8s_block128")),
+    (ElemType.F32, 2052, 16512, ("q4s_block128", "q8s_block64", "q2s_block64")),
+], ids=lambda v: v.name if isinstance(v, ElemType) else v if isinstance(v, str) else str(v) if isinstance(v, int) else "-".join(v))
+def test_transposed_tiles_of_one_step_and_of_long_blocks(gpu, elem, rows, cols, names):
+    """Transposed floats through shared memory where the tiles are few (a tile is one step of 64 or 128 columns) and
+    where a block takes four lanes or a wider step, against the contiguous kernels, bit for bit."""
     transposed_against_contiguous(gpu, elem, rows, cols, names)
 
 
