@@ -56,6 +56,42 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_grouped_kernel(const u32
     }
 }
 
+// ---- rows of a few chunks that are not a power of two: kGroup lanes per row --------------------
+// `loads` (uniform, at most kRowLoads) chunks per lane, all in flight at once; the last one of a row again for lanes past it.
+// Bound by HBM.  With a wave per row most of its lanes had nothing to load: f16 [42651, 328] 13.3 -> 6.2 us, bf16
+// [100000, 136] 26.2 -> 9.4 us, f32 [300000, 24] 57.9 -> 13.3 us.
+constexpr uint32_t kRowLoads = 8;
+template <class F, int kGroup>
+__global__ __launch_bounds__(kThreads) void reduce_rows_lanes_kernel(const u32x4* __restrict__ in, void* __restrict__ out, uint64_t rows,
+                                                                     uint32_t chunks_per_row, uint32_t loads) {
+    const uint64_t row = (static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x) / kGroup;
+    const uint32_t lane = threadIdx.x % kGroup;
+    const u32x4* const p = in + (row < rows ? row : rows - 1) * chunks_per_row;
+    u32x4 raw[kRowLoads];
+#pragma unroll
+    for (uint32_t u = 0; u < kRowLoads; u++) {
+        const uint32_t c = lane + u * kGroup;
+        if (u < loads) raw[u] = stream_load(p + (c < chunks_per_row ? c : chunks_per_row - 1));
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < kRowLoads; u++)
+        if (u < loads) amax = chunk_absmax<F>(raw[u], amax);
+    amax = group_max<kGroup>(amax);
+    if (lane == 0 && row < rows) F::store(out, row, amax);
+}
+
+// Lanes per row for `chunks` chunks in at most kRowLoads loads: the fewest idle slots, more lanes on a tie.
+inline uint32_t row_lanes(uint64_t chunks) {
+    uint32_t best = kWave;
+    for (uint32_t g = kWave; g >= 1; g /= 2) {
+        const uint64_t loads = (chunks + g - 1) / g;
+        if (loads > kRowLoads) break;
+        if (loads * g < (chunks + best - 1) / best * best) best = g;
+    }
+    return best;
+}
+
 // ---- rows, long: one wave per (row, slice) --------------------------------------
 // kPartial: write f32 partials [slice][row] with row pitch `pitch`; otherwise the
 // final value typed F.
@@ -95,13 +131,15 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_wave_kernel(const u32x4*
 }
 
 // ---- columns, wide: one lane per (slice of L, outer, inner chunk) ---------------------
-// kPartial: write f32 partials [slice][output]; otherwise the final chunk typed F.
-template <class F, bool kPartial>
+// Writes one chunk typed F per lane: the result, or a partial [slice][output] (maxima are F numbers, so the partials lose
+// nothing in 16 bits, and their traffic, written and read again, is halved).
+// Bound by HBM; kUnroll loads of 16 bytes per lane in flight.
+template <class F>
 __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __restrict__ in, void* __restrict__ out,
                                                                uint64_t outer, uint64_t len, uint64_t inner_chunks,
                                                                uint32_t slices) {
     constexpr int kN = F::kPerChunk;
-    constexpr int kUnroll = 4;
+    constexpr int kUnroll = 8;
     const uint64_t cols = outer * inner_chunks;  // output chunks
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (t >= cols * slices) return;
@@ -130,13 +168,7 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
             for (int i = 0; i < kN; i++) amax[i] = fmaxf(amax[i], fabsf(v[i]));
         }
     }
-    if constexpr (kPartial) {
-        float* dst = static_cast<float*>(out) + (static_cast<uint64_t>(slice) * cols + col) * kN;
-#pragma unroll
-        for (int i = 0; i < kN; i++) dst[i] = amax[i];
-    } else {
-        static_cast<u32x4*>(out)[col] = F::pack(amax);  // values are F numbers: packing is exact
-    }
+    static_cast<u32x4*>(out)[static_cast<uint64_t>(slice) * cols + col] = F::pack(amax);  // values are F numbers: packing is exact
 }
 
 // ---- columns, few outputs: one workgroup per (outer, column tile, slice of L) ----------
@@ -412,6 +444,10 @@ inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
 constexpr uint64_t kTargetGroups = 2048;
 constexpr uint64_t kTargetLanes = kTargetGroups * kThreads / 2;
 
+// Small tensors along an outer axis, one launch against two: f16 [300, 1024] 8.0 -> 4.6 us, [575, 1792] 8.4 -> 5.2 us, bf16
+// [1000, 4096] 16.3 -> 7.5 us; with 4096 rows the tiles are too few for their work ([4096, 1024] 8.1 -> 17.6 us).
+constexpr uint64_t kOneLaunchLen = 1024, kOneLaunchChunks = 1ull << 20;
+
 // How a contiguous [outer, len, inner] view is cut up; shared by the launcher and
 // by the workspace size query so that the two always agree.
 struct ReducePlan {
@@ -489,15 +525,15 @@ void launch_tile(hipStream_t s, uint32_t cw, uint64_t jobs, const void* in, void
     }
 }
 
-// out[i] = max_s partials[s][i], i < count; partials are f32 with row pitch `pitch`
-template <class F>
+// out[i] = max_s partials[s][i], i < count; partials are typed P (f32 or the output's type) with row pitch `pitch`
+template <class F, class P = F32>
 void launch_fold(hipStream_t s, const void* partials, void* out, uint64_t slices, uint64_t pitch, uint64_t count) {
     constexpr int kFoldThreads = 1024;
-    const uint64_t chunks = pitch / 4;
+    const uint64_t chunks = pitch / P::kPerChunk;
     uint32_t cw = pow2_at_least(chunks, kWave);
     while (cw > 4 && chunks / cw < 128) cw /= 2;  // narrower tiles, more workgroups: the partials sit in L2
     const uint32_t tiles = static_cast<uint32_t>((chunks + cw - 1) / cw);
-    launch_tile<F32, F, kFoldThreads, kTileFinalChecked>(s, cw, tiles, partials, out, slices, chunks, tiles, 1u, 0, count);
+    launch_tile<P, F, kFoldThreads, kTileFinalChecked>(s, cw, tiles, partials, out, slices, chunks, tiles, 1u, 0, count);
 }
 
 // The levels of a strided input with a contiguous last dimension of whole chunks, strides of whole words and
@@ -636,6 +672,21 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         const uint64_t fit = a.workspace == nullptr ? 0 : a.workspace_bytes / (p.pitch * sizeof(float));
         if (slices > fit) slices = fit > 1 ? fit : 1;
     }
+    // A small tensor in one launch: 1024 lanes per tile of up to four chunk columns, the whole axis.  The second launch that
+    // folds slices costs about 4 us, in which a tile's lanes read kOneLaunchLen rows.
+    if ((p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) && slices > 1 && a.len <= kOneLaunchLen &&
+        a.outer * a.len * p.inner_chunks <= kOneLaunchChunks) {
+        const uint32_t cw = pow2_at_least(p.inner_chunks, 4);
+        const uint32_t col_tiles = static_cast<uint32_t>((p.inner_chunks + cw - 1) / cw);
+        const dim3 grid(static_cast<uint32_t>(a.outer * col_tiles));
+        auto src = static_cast<const u32x4*>(a.input);
+        switch (cw) {
+#define CQ_CASE(W) case W: hipLaunchKernelGGL((reduce_tile_kernel<F, F, W, 1024, kTileFinalPacked>), grid, dim3(1024), 0, s, src, a.output, a.len, p.inner_chunks, col_tiles, 1u, 0ull, 0ull); break;
+            CQ_CASE(1) CQ_CASE(2) CQ_CASE(4)
+#undef CQ_CASE
+        }
+        return hipGetLastError();
+    }
     auto in = static_cast<const u32x4*>(a.input);
     switch (p.kind) {
         case ReducePlan::kRowsGrouped: {
@@ -651,6 +702,15 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         }
         case ReducePlan::kRowsWave: {
             dim3 grid = blocks(a.outer * slices, kThreads / kWave);
+            if (slices <= 1 && p.chunks_per_row <= kWave * kRowLoads) {
+                const uint32_t lanes = row_lanes(p.chunks_per_row), loads = static_cast<uint32_t>((p.chunks_per_row + lanes - 1) / lanes);
+                switch (lanes) {
+#define CQ_CASE(G) case G: hipLaunchKernelGGL((reduce_rows_lanes_kernel<F, G>), blocks(a.outer * G, kThreads), dim3(kThreads), 0, s, in, a.output, a.outer, static_cast<uint32_t>(p.chunks_per_row), loads); break;
+                    CQ_CASE(1) CQ_CASE(2) CQ_CASE(4) CQ_CASE(8) CQ_CASE(16) CQ_CASE(32) CQ_CASE(64)
+#undef CQ_CASE
+                }
+                return hipGetLastError();
+            }
             if (slices > 1) {
                 hipLaunchKernelGGL((reduce_rows_wave_kernel<F, true>), grid, dim3(kThreads), 0, s, in, a.workspace, a.outer,
                                    p.chunks_per_row, static_cast<uint32_t>(slices), p.pitch);
@@ -664,11 +724,11 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         case ReducePlan::kCols: {
             dim3 grid = blocks(a.outer * p.inner_chunks * slices, kThreads);
             if (slices > 1) {
-                hipLaunchKernelGGL((reduce_cols_kernel<F, true>), grid, dim3(kThreads), 0, s, in, a.workspace, a.outer, a.len,
+                hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.workspace, a.outer, a.len,
                                    p.inner_chunks, static_cast<uint32_t>(slices));
-                launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
+                launch_fold<F, F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
             } else {
-                hipLaunchKernelGGL((reduce_cols_kernel<F, false>), grid, dim3(kThreads), 0, s, in, a.output, a.outer, a.len,
+                hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.output, a.outer, a.len,
                                    p.inner_chunks, 1u);
             }
             return hipGetLastError();

@@ -61,6 +61,30 @@ def test_reduce_contiguous_all_paths(gpu, oracle, elem):
             assert np.array_equal(got[:n_out].view(np.uint8), want.view(np.uint8)), (shape, axis, use_ws)
 
 
+@pytest.mark.parametrize("elem", ELEMS, ids=lambda e: e.name)
+def test_reduce_short_rows_and_small_outer_axes(gpu, oracle, elem):
+    """Rows of a few chunks that are not a power of two (every width of lane group, the most loads per lane, one chunk
+    more) and axes that one launch takes whole (tiles of 1, 2 and 4 chunk columns, cut short; the longest axis and
+    one more), bit for bit with and without a workspace."""
+    import torch
+
+    rng = np.random.default_rng(int(elem) + 70)
+    n = 4 if elem == ElemType.F32 else 8
+    cases = [((rows, chunks * n), 1) for rows, chunks in ((70, 3), (129, 5), (1, 6), (33, 41), (257, 61), (20000, 17), (9, 130), (300, 511),
+                                                          (40000, 67), (31, 513))]
+    cases += [((length, chunks * n), 0) for length, chunks in ((1024, 300), (1025, 300), (37, 257), (1000, 5), (513, 2), (1023, 1))]
+    cases += [((3, 600, 33 * n), 1)]
+    for shape, axis in cases:
+        x32 = rng.normal(0, 2, shape).astype(np.float32)
+        x32[rng.random(shape) < 0.01] = np.nan
+        x32.reshape(-1)[-1] = np.inf if shape[0] % 2 else -0.0
+        x = oracle.to_bits(x32, elem)
+        want = oracle.reduce_max_abs(x, elem, shape, axis).reshape(-1)
+        for use_ws in (True, False):
+            got, n_out = run(torch, gpu, x, elem, shape, axis, use_workspace=use_ws)
+            assert np.array_equal(got[:n_out].view(np.uint8), want.view(np.uint8)), (shape, axis, use_ws)
+
+
 def test_reduce_strided_views_and_errors(gpu, oracle):
     import torch
 
