@@ -133,20 +133,20 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_wave_kernel(const u32x4*
 // ---- columns, wide: one lane per (slice of L, outer, inner chunk) ---------------------
 // Writes one chunk typed F per lane: the result, or a partial [slice][output] (maxima are F numbers, so the partials lose
 // nothing in 16 bits, and their traffic, written and read again, is halved).
-// Bound by HBM; kUnroll loads of 16 bytes per lane in flight.
+// Bound by HBM; kColsUnroll loads of 16 bytes per lane in flight.  `per_slice`: rows_per_slice().
+constexpr int kColsUnroll = 8;
 template <class F>
 __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __restrict__ in, void* __restrict__ out,
                                                                uint64_t outer, uint64_t len, uint64_t inner_chunks,
-                                                               uint32_t slices) {
+                                                               uint32_t slices, uint64_t per_slice) {
     constexpr int kN = F::kPerChunk;
-    constexpr int kUnroll = 8;
+    constexpr int kUnroll = kColsUnroll;
     const uint64_t cols = outer * inner_chunks;  // output chunks
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (t >= cols * slices) return;
     const uint32_t slice = static_cast<uint32_t>(t / cols);
     const uint64_t col = t % cols;
     const uint64_t o = col / inner_chunks, j = col % inner_chunks;
-    const uint64_t per_slice = (len + slices - 1) / slices;
     const uint64_t begin = slice * per_slice;
     const uint64_t end = begin + per_slice < len ? begin + per_slice : len;
     const u32x4* p = in + o * len * inner_chunks + j;
@@ -448,6 +448,28 @@ constexpr uint64_t kTargetLanes = kTargetGroups * kThreads / 2;
 // [1000, 4096] 16.3 -> 7.5 us; with 4096 rows the tiles are too few for their work ([4096, 1024] 8.1 -> 17.6 us).
 constexpr uint64_t kOneLaunchLen = 1024, kOneLaunchChunks = 1ull << 20;
 
+// Rows per lane of reduce_cols_kernel with at most `most` slices over `cols` columns of chunks.  Its few workgroups all run
+// at once, so a launch lasts as long as the compute unit with the most of them: of two to four workgroups per compute unit
+// the split with the least work there, rows in whole loops of kColsUnroll (a last loop of one row loads eight) and eight rows'
+// worth for a slice's start and end.  The workgroups do not spread evenly, so a round counts 238 of the 256 units: bf16
+// [30000, 3000], workgroups per unit 1.65 34.3, 1.79 33.7, 1.95 39.7, 2.15 38.9, 2.68 35.4 us; [3000, 20008] 1.79 22.6, 2.06
+// 26.8, 2.86 23.5 us.  Against slices of even rows, capped by the partials' bytes alone: bf16 [4093, 11008] 19.1 -> 17.1 us,
+// f16 [1686, 18520] 16.4 -> 14.5 us, bf16 [30000, 3000] 36.6 -> 33.7 us.
+inline uint64_t rows_per_slice(uint64_t len, uint64_t cols, uint64_t most) {
+    constexpr uint64_t kRound = 238 * kThreads, kSliceCost = 8;
+    uint64_t best = len, best_cost = (cols + kRound - 1) / kRound * (len + kSliceCost);
+    for (uint64_t rounds = 2; rounds <= 4; rounds++) {
+        uint64_t n = rounds * kRound / cols;
+        if (n > (len + 15) / 16) n = (len + 15) / 16;
+        if (n > most) n = most;
+        if (n < 2) continue;
+        const uint64_t rows = round_up((len + n - 1) / n, kColsUnroll), slices = (len + rows - 1) / rows;
+        const uint64_t cost = (slices * cols + kRound - 1) / kRound * (rows + kSliceCost);
+        if (cost < best_cost) best = rows, best_cost = cost;
+    }
+    return best;
+}
+
 // How a contiguous [outer, len, inner] view is cut up; shared by the launcher and
 // by the workspace size query so that the two always agree.
 struct ReducePlan {
@@ -722,14 +744,21 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
             return hipGetLastError();
         }
         case ReducePlan::kCols: {
-            dim3 grid = blocks(a.outer * p.inner_chunks * slices, kThreads);
+            uint64_t per_slice = a.len;
+            if (slices > 1) {
+                // the workspace of p.slices in f32 holds twice as many typed in 16 bits
+                const uint64_t fit = a.workspace_bytes / (p.pitch * F::kBytes), most = p.slices * (4 / F::kBytes);
+                per_slice = rows_per_slice(a.len, a.outer * p.inner_chunks, fit < most ? fit : most);
+                slices = (a.len + per_slice - 1) / per_slice;
+            }
+            const dim3 grid = blocks(a.outer * p.inner_chunks * slices, kThreads);
             if (slices > 1) {
                 hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.workspace, a.outer, a.len,
-                                   p.inner_chunks, static_cast<uint32_t>(slices));
+                                   p.inner_chunks, static_cast<uint32_t>(slices), per_slice);
                 launch_fold<F, F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
             } else {
                 hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.output, a.outer, a.len,
-                                   p.inner_chunks, 1u);
+                                   p.inner_chunks, 1u, per_slice);
             }
             return hipGetLastError();
         }

@@ -74,6 +74,8 @@ def test_reduce_short_rows_and_small_outer_axes(gpu, oracle, elem):
                                                           (40000, 67), (31, 513))]
     cases += [((length, chunks * n), 0) for length, chunks in ((1024, 300), (1025, 300), (37, 257), (1000, 5), (513, 2), (1023, 1))]
     cases += [((3, 600, 33 * n), 1)]
+    # slices of whole loops of rows: a last slice of one row, of less than a loop, of a whole one; several outer entries
+    cases += [((length, 256 * n), 0) for length in (4097, 4093, 8200)] + [((2, 1100, 300 * n), 1), ((1500, 2501 * n), 0)]
     for shape, axis in cases:
         x32 = rng.normal(0, 2, shape).astype(np.float32)
         x32[rng.random(shape) < 0.01] = np.nan
