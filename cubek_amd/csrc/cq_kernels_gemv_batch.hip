@@ -281,8 +281,9 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
     load(min(share, stages - 1u), 0);
     for (uint32_t n = 0; n < steps; n++) {
         const uint32_t from = (n & 1u) * buffer;
-        // stage n is there, and everybody has read the stage before it, whose place the next load takes
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // Stage n is there, and everybody has read the stage before it, whose place the next load takes.  The reads are waited
+        // for here and not only where their values are used: nothing else keeps those uses in front of the barrier.
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (n + 1 < steps) load(min((n + 1) * kS + share, stages - 1u), buffer - from);
