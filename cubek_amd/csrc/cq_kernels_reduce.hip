@@ -58,25 +58,42 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_grouped_kernel(const u32
 
 // ---- rows of a few chunks that are not a power of two: kGroup lanes per row --------------------
 // `loads` (uniform, at most kRowLoads) chunks per lane, all in flight at once; the last one of a row again for lanes past it.
-// Bound by HBM.  With a wave per row most of its lanes had nothing to load: f16 [42651, 328] 13.3 -> 6.2 us, bf16
-// [100000, 136] 26.2 -> 9.4 us, f32 [300000, 24] 57.9 -> 13.3 us.
+// One straight piece of code per number of loads: with the loads behind conditions one by one, the compiler waited for each
+// f32 load before the next and kept 238 registers (f32 [42651, 328] 28.8 us, [8192, 512] 9.2, [100000, 24] 6.0).
+// Bound by HBM.  With a wave per row most of its lanes had nothing to load: f32 [42651, 328] 12.8 -> 9.5 us, [8192, 512]
+// 4.8 -> 4.5, [100000, 24] 21.2 -> 4.3; bf16 [42651, 656] 14.2 -> 9.7, [8192, 1024] 4.9 -> 4.6, [100000, 48] 26.0 -> 4.4.
 constexpr uint32_t kRowLoads = 8;
+template <class F, int kGroup, uint32_t kLoads>
+__device__ __forceinline__ float row_share_absmax(const u32x4* row, uint32_t lane, uint32_t chunks_per_row) {
+    u32x4 raw[kLoads];
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; u++) {
+        const uint32_t c = lane + u * kGroup;
+        raw[u] = stream_load(row + (c < chunks_per_row ? c : chunks_per_row - 1));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load ahead of the arithmetic
+    float amax = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; u++) amax = chunk_absmax<F>(raw[u], amax);
+    return amax;
+}
 template <class F, int kGroup>
 __global__ __launch_bounds__(kThreads) void reduce_rows_lanes_kernel(const u32x4* __restrict__ in, void* __restrict__ out, uint64_t rows,
                                                                      uint32_t chunks_per_row, uint32_t loads) {
     const uint64_t row = (static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x) / kGroup;
     const uint32_t lane = threadIdx.x % kGroup;
     const u32x4* const p = in + (row < rows ? row : rows - 1) * chunks_per_row;
-    u32x4 raw[kRowLoads];
-#pragma unroll
-    for (uint32_t u = 0; u < kRowLoads; u++) {
-        const uint32_t c = lane + u * kGroup;
-        if (u < loads) raw[u] = stream_load(p + (c < chunks_per_row ? c : chunks_per_row - 1));
-    }
     float amax = 0.0f;
-#pragma unroll
-    for (uint32_t u = 0; u < kRowLoads; u++)
-        if (u < loads) amax = chunk_absmax<F>(raw[u], amax);
+    switch (loads) {
+        case 1: amax = row_share_absmax<F, kGroup, 1>(p, lane, chunks_per_row); break;
+        case 2: amax = row_share_absmax<F, kGroup, 2>(p, lane, chunks_per_row); break;
+        case 3: amax = row_share_absmax<F, kGroup, 3>(p, lane, chunks_per_row); break;
+        case 4: amax = row_share_absmax<F, kGroup, 4>(p, lane, chunks_per_row); break;
+        case 5: amax = row_share_absmax<F, kGroup, 5>(p, lane, chunks_per_row); break;
+        case 6: amax = row_share_absmax<F, kGroup, 6>(p, lane, chunks_per_row); break;
+        case 7: amax = row_share_absmax<F, kGroup, 7>(p, lane, chunks_per_row); break;
+        case kRowLoads: amax = row_share_absmax<F, kGroup, kRowLoads>(p, lane, chunks_per_row); break;
+    }
     amax = group_max<kGroup>(amax);
     if (lane == 0 && row < rows) F::store(out, row, amax);
 }

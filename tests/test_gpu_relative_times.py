@@ -1,0 +1,45 @@
+"""Calls that move the same bytes in the same way take about the same time, whatever their types: each pair below was once
+two or three times apart, which no comparison of results shows.  The limits leave half as much again for noise."""
+import pytest
+
+from cubek_amd import ComputeClient, ElemType, TensorHandleRef
+from cubek_amd import reduce as rd
+
+pytestmark = pytest.mark.gpu
+
+
+def micros(*calls):
+    """The best time of each call in microseconds, the calls taking turns."""
+    import torch
+
+    best = [float("inf")] * len(calls)
+    for _ in range(8):
+        for i, call in enumerate(calls):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            call()
+            begin.record()
+            for _ in range(20):
+                call()
+            end.record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], begin.elapsed_time(end) * 50)
+    return best
+
+
+def max_abs(elem, rows, cols, axis):
+    """One abs-max over tensors of its own, as a function without arguments."""
+    import torch
+
+    dtype = torch.float32 if elem == ElemType.F32 else torch.bfloat16
+    x = torch.randn((rows, cols), device="cuda").to(dtype)
+    out = torch.empty((1, cols) if axis == 0 else (rows, 1), dtype=dtype, device="cuda")
+    h_x, h_out, client = TensorHandleRef.from_torch(x), TensorHandleRef.from_torch(out), ComputeClient.current()
+    nbytes = rd.workspace_bytes(h_x, axis, elem)
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device="cuda")
+    keep = (x, out, ws)
+    return lambda: (rd.max_abs(client, h_x, h_out, axis, elem, ws.data_ptr(), nbytes), keep)
+
+
+def test_short_rows_of_f32_as_fast_as_of_bf16():
+    f32, bf16 = micros(max_abs(ElemType.F32, 85302, 328, 1), max_abs(ElemType.BF16, 85302, 656, 1))  # 82 chunks of 16 bytes each
+    assert f32 < 1.5 * bf16, (f32, bf16)
