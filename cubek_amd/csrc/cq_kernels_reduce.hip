@@ -461,9 +461,13 @@ inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
 constexpr uint64_t kTargetGroups = 2048;
 constexpr uint64_t kTargetLanes = kTargetGroups * kThreads / 2;
 
-// Small tensors along an outer axis, one launch against two: f16 [300, 1024] 8.0 -> 4.6 us, [575, 1792] 8.4 -> 5.2 us, bf16
-// [1000, 4096] 16.3 -> 7.5 us; with 4096 rows the tiles are too few for their work ([4096, 1024] 8.1 -> 17.6 us).
-constexpr uint64_t kOneLaunchLen = 1024, kOneLaunchChunks = 1ull << 20;
+// Small tensors along an outer axis, one launch against two (two -> one, us): f32 [100, 4000] 8.9 -> 3.7, [512, 4096] 8.4 ->
+// 6.3, bf16 [700, 5600] 11.1 -> 6.2, [1000, 4096] 10.7 -> 7.7.  The lines: at 2^20 chunks it is even (f32 [500, 8192] 9.0 and
+// 9.1, [1000, 4096] 9.2 and 9.0; bf16 [500, 16384] 10.4 and 9.6); with 4096 rows the tiles are too few for their work (f16
+// [4096, 1024] 8.1 -> 17.6); and a tile's workgroup takes its place of 1024 lanes however few rows they share, so more of them
+// than are resident a few times over cost more than the second launch (1024 tiles: f32 [128, 16384] 8.0 -> 7.5; 2048 tiles:
+// [64, 32768] 7.8 -> 11.4, [100, 32768] 8.8 -> 12.2; 4096 tiles: [64, 65536] 8.4 -> 20.8).
+constexpr uint64_t kOneLaunchLen = 1024, kOneLaunchChunks = 1ull << 20, kOneLaunchTiles = 1024;
 
 // Rows per lane of reduce_cols_kernel with at most `most` slices over `cols` columns of chunks.  Its few workgroups all run
 // at once, so a launch lasts as long as the compute unit with the most of them: of two to four workgroups per compute unit
@@ -713,14 +717,14 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
     }
     // A small tensor in one launch: 1024 lanes per tile of up to four chunk columns, the whole axis.  The second launch that
     // folds slices costs about 4 us, in which a tile's lanes read kOneLaunchLen rows.
+    const uint32_t cw = pow2_at_least(p.inner_chunks, 4);
+    const uint64_t col_tiles = (p.inner_chunks + cw - 1) / cw;
     if ((p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) && slices > 1 && a.len <= kOneLaunchLen &&
-        a.outer * a.len * p.inner_chunks <= kOneLaunchChunks) {
-        const uint32_t cw = pow2_at_least(p.inner_chunks, 4);
-        const uint32_t col_tiles = static_cast<uint32_t>((p.inner_chunks + cw - 1) / cw);
+        a.outer * a.len * p.inner_chunks <= kOneLaunchChunks && a.outer * col_tiles <= kOneLaunchTiles) {
         const dim3 grid(static_cast<uint32_t>(a.outer * col_tiles));
         auto src = static_cast<const u32x4*>(a.input);
         switch (cw) {
-#define CQ_CASE(W) case W: hipLaunchKernelGGL((reduce_tile_kernel<F, F, W, 1024, kTileFinalPacked>), grid, dim3(1024), 0, s, src, a.output, a.len, p.inner_chunks, col_tiles, 1u, 0ull, 0ull); break;
+#define CQ_CASE(W) case W: hipLaunchKernelGGL((reduce_tile_kernel<F, F, W, 1024, kTileFinalPacked>), grid, dim3(1024), 0, s, src, a.output, a.len, p.inner_chunks, static_cast<uint32_t>(col_tiles), 1u, 0ull, 0ull); break;
             CQ_CASE(1) CQ_CASE(2) CQ_CASE(4)
 #undef CQ_CASE
         }

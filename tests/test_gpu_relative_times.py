@@ -43,3 +43,8 @@ def max_abs(elem, rows, cols, axis):
 def test_short_rows_of_f32_as_fast_as_of_bf16():
     f32, bf16 = micros(max_abs(ElemType.F32, 85302, 328, 1), max_abs(ElemType.BF16, 85302, 656, 1))  # 82 chunks of 16 bytes each
     assert f32 < 1.5 * bf16, (f32, bf16)
+
+
+def test_few_long_rows_along_the_outer_axis_as_fast_as_many_short_ones():
+    few, many = micros(max_abs(ElemType.F32, 64, 65536, 0), max_abs(ElemType.F32, 2048, 2048, 0))  # 16 MiB each
+    assert few < 1.5 * many, (few, many)
