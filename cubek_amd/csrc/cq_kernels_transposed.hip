@@ -17,6 +17,7 @@
 // dequantize_transposed_kernel.
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 #include "cq_magic_div.hpp"
 
 namespace cq {
@@ -462,7 +463,8 @@ __device__ __forceinline__ TilePlace tile_place(uint32_t row_tiles, uint32_t col
 // next to each other (their maxima meet by DPP).  kPart 16: 16 KiB of floats, 18 KiB of words and 4 KiB of scales per
 // workgroup: four workgroups fit a compute unit; blocks of 32 and 64 columns, or any multiple of 32 with given scales.
 // kPart 32: blocks of 128 columns, twice the floats.  kWholeTile: 128 bytes of codes per row and tile; else a tile is one
-// step, for launches of few tiles: eight times as many workgroups (4-bit), each with one step's latency.
+// step, for launches of few tiles: eight times as many workgroups (4-bit), each with one step's latency
+// (transposed_tile() draws the lines).
 // Bound by its stores (runs of 128 and 32 bytes far apart).  Measured against the kernel it replaced for blocks of 64 and
 // 128 and for few tiles (quantize_transposed_quads_kernel, left with runs of 8 bytes): 4 bits, blocks of 64 f16
 // [31072, 1408] 37.8 -> 28.2 us, blocks of 128 [10944, 2816] 30.2 -> 22.8 us, bf16 [117472, 1024] 78.7 -> 67.0 us; few
@@ -907,15 +909,15 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
     const uint32_t nq = 32u / static_cast<uint32_t>(bits);
     const uint32_t step_cols = kScale == 0 && a.segment == 128 ? 128u : 64u;
     const uint32_t row_tiles = (a.rows + 64 * kTileRowsPerThread<F> - 1) / (64 * kTileRowsPerThread<F>);
-    // A tile is 128 bytes of codes per row; where that leaves fewer than two rounds of resident workgroups, a step (figures
-    // at the kernel).
     const auto tiles_of = [&](uint32_t tile_cols) { return static_cast<uint64_t>(row_tiles) * ((cols + tile_cols - 1) / tile_cols); };
-    const bool whole_tile = tiles_of(32u * nq) * a.batches >= 1024;
+    const TransposedTile tile = transposed_tile(static_cast<uint32_t>(bits), F::kBytes, kScale == 1, a.rows, tiles_of(32u * nq) * a.batches,
+                                                tiles_of(step_cols) * a.batches, step_cols);
+    const bool whole_tile = tile == TransposedTile::kWhole;  // 128 bytes of codes per row; else a step
     const uint32_t tile_cols = whole_tile ? 32u * nq : step_cols;
     const uint64_t tile_count = tiles_of(tile_cols);
     // A tile stores the scales of the blocks that start in it, as one run per row: blocks divide the tile's columns
     // (a block of 96 columns would straddle two tiles of 256; such layouts take the kernels below).
-    bool tiles = cols < (1u << 31) && a.pitch_f * F::kBytes * step_cols < (1ull << 31) && runs_of_16_bytes<F>(a, a.input) && a.segment % kTilePart == 0 &&
+    bool tiles = !(tile == TransposedTile::kRegisters && quads) && cols < (1u << 31) && a.pitch_f * F::kBytes * step_cols < (1ull << 31) && runs_of_16_bytes<F>(a, a.input) && a.segment % kTilePart == 0 &&
                  (kScale == 1 || a.segment == 32 || a.segment == 64 || a.segment == 128) && (a.tensor_level || tile_cols % a.segment == 0) &&
                  (reinterpret_cast<uintptr_t>(a.output) & 15u) == 0 && a.vrow % 4 == 0 && (cols / nq) % 4 == 0 && a.batches <= 65535 &&
                  tile_count < (1u << 31);

@@ -1,0 +1,35 @@
+// Where a launch changes kernel by size: the rules that host tests check, in plain C++.  Times are microseconds of the
+// launch alone on MI355X, buffers rotated.
+#pragma once
+
+#include <stdint.h>
+
+namespace cq {
+
+// The kernel of a transposed quantize whose runs are 16-byte aligned on both sides: the register kernel, the tile kernel
+// with one step of columns per tile, or with 128 bytes of codes per row and tile.  `whole_tiles`, `steps`: how many tiles of
+// either kind the launch has, batches included; `step_cols`: 64, or 128 for a fused abs-max over blocks of 128.
+//
+// From 1024 whole tiles on (two rounds of resident workgroups) those win.  Below:
+// * Steps of 64 columns write a line of codes in pieces (of 16 bytes for 2-bit codes), the next piece of a line coming a
+//   column of tiles later, so with many rows the line has left the L2 before it is full.  Fused abs-max, 2 bits of bf16
+//   (steps, whole tiles, register kernel): [4096, 4096] 12.2, 14.6, 14.5, [8192, 2048] 13.7, 14.9, 14.8, [16384, 1024] 17.9,
+//   15.0, 15.0, [14336, 2048] 24.8, 18.3, 23.4, [14336, 4096] 47.2, 31.7, 36.5; 4 bits [6144, 4096] 17.2, 14.5, 19.0,
+//   [12288, 2048] 22.3, 15.4, 19.3, [2048, 4096] 8.1, 9.8, 10.8.
+// * Given scales read them between the steps: 2 bits of bf16 [4096, 4096] 13.8, 19.8, 16.4, [8192, 2048] 17.0, 20.3, 15.9,
+//   [14336, 1024] 13.9, 20.1, 15.7, [14336, 4096] 54, 44.2, 35.5; 4 bits [8192, 2048] 19.0, 17.0, 15.8, [14336, 1024] 17.4,
+//   15.5, 15.8; wider codes and f32 gain from whole tiles all the same: 8 bits [6144, 2048] 13.8, 12.4, 15.9, 4 bits of f32
+//   [12288, 1024] 19.7, 15.6, 17.2.
+// * A step of 128 columns writes 32 bytes and more: 4 bits of bf16 [1056, 16384] 14.5, 16.8, 19.2, [14336, 2048] 22.0, 22.2, 23.1.
+enum class TransposedTile { kRegisters, kStep, kWhole };
+inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool given_scales, uint64_t rows, uint64_t whole_tiles,
+                                      uint64_t steps, uint32_t step_cols) {
+    if (whole_tiles >= 1024) return TransposedTile::kWhole;
+    if (step_cols == 128) return TransposedTile::kStep;
+    const bool registers_keep_up = given_scales && float_bytes == 2 && bits < 8;
+    if (!registers_keep_up && whole_tiles >= 512) return TransposedTile::kWhole;
+    if (given_scales) return rows <= 6144 || steps <= 1536 || whole_tiles < 256 ? TransposedTile::kStep : TransposedTile::kRegisters;
+    return rows <= 8192 || steps < 2048 ? TransposedTile::kStep : TransposedTile::kWhole;
+}
+
+}  // namespace cq

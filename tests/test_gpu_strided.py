@@ -347,6 +347,19 @@ def test_transposed_tiles_of_one_step_and_of_long_blocks(gpu, elem, rows, cols, 
 
 
 @pytest.mark.parametrize("elem,rows,cols,names", [
+    (ElemType.BF16, 14344, 2240, ("q2s_block64", "q4s_block32")),
+    (ElemType.F16, 16392, 1152, ("q2s_block64", "q4s_block64")),
+    (ElemType.F32, 8196, 1600, ("q2s_block64", "q4s_block32")),
+    (ElemType.BF16, 8200, 2112, ("q2s_block64", "q4s_block64", "q8s_block32")),
+    (ElemType.F16, 6152, 3136, ("q2s_block64", "q4s_block32")),
+], ids=lambda v: v.name if isinstance(v, ElemType) else v if isinstance(v, str) else str(v) if isinstance(v, int) else "-".join(v))
+def test_transposed_tiles_between_few_and_many(gpu, elem, rows, cols, names):
+    """Transposed floats in 256 to 1023 whole tiles, rows and columns cut short: by bits, rows and where the scales come from
+    each of whole tiles, steps and the register kernel, against the contiguous kernels, bit for bit."""
+    transposed_against_contiguous(gpu, elem, rows, cols, names)
+
+
+@pytest.mark.parametrize("elem,rows,cols,names", [
     (ElemType.BF16, 4128, 8640, ("q4s_block96", "q8s_block96", "q8s_block160", "q2s_block192")),
     (ElemType.F32, 2064, 8640, ("q4s_block96", "q8s_block160")),
 ], ids=["bf16", "f32"])

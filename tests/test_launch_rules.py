@@ -1,0 +1,57 @@
+"""Where launches change kernel by size (cubek_amd/csrc/cq_launch_rules.hpp), compiled for the host: on each size below the
+rule has to name the kernel that was the fastest there, or one within 5 % of it."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def answer(tmp_path_factory):
+    """Evaluates C++ expressions over the rules, each to a whole number."""
+    where = tmp_path_factory.mktemp("rules")
+
+    def evaluate(expressions):
+        body = "".join(f'    std::printf("%d\\n", static_cast<int>({e}));\n' for e in expressions)
+        (where / "rules.cpp").write_text('#include <cstdio>\n#include "cq_launch_rules.hpp"\nusing namespace cq;\nint main() {\n' + body + "}\n")
+        build = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", f"-I{os.path.join(ROOT, 'cubek_amd', 'csrc')}",
+                                str(where / "rules.cpp"), "-o", str(where / "rules")], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        assert build.returncode == 0, build.stdout
+        run = subprocess.run([str(where / "rules")], stdout=subprocess.PIPE, text=True)
+        assert run.returncode == 0
+        return [int(line) for line in run.stdout.split()]
+
+    return evaluate
+
+
+REGISTERS, STEP, WHOLE = 0, 1, 2
+
+
+def transposed_tile(bits, float_bytes, given, rows, cols, block=32):
+    row_tiles = -(-rows // (256 // float_bytes))
+    step_cols = 128 if block == 128 and not given else 64
+    whole, steps = row_tiles * -(-cols // (1024 // bits)), row_tiles * -(-cols // step_cols)
+    return f"transposed_tile({bits}, {float_bytes}, {str(given).lower()}, {rows}, {whole}, {steps}, {step_cols})"
+
+
+# (bits, bytes of a float, given scales, rows, columns, block): the kernels that are within 5 % of the fastest
+TRANSPOSED = {
+    (2, 2, False, 14336, 4096, 32): {WHOLE}, (2, 2, False, 31072, 1408, 32): {WHOLE}, (2, 2, False, 14336, 2048, 32): {WHOLE},
+    (2, 2, False, 16384, 1024, 32): {WHOLE, REGISTERS}, (2, 2, False, 4096, 4096, 32): {STEP}, (2, 2, False, 2048, 2048, 64): {STEP},
+    (4, 2, False, 8192, 2048, 32): {WHOLE}, (4, 2, False, 12288, 2048, 32): {WHOLE}, (4, 2, False, 6144, 4096, 64): {WHOLE},
+    (4, 2, False, 2048, 4096, 32): {STEP}, (4, 2, False, 1056, 16384, 128): {STEP}, (8, 2, False, 24576, 512, 32): {WHOLE},
+    (2, 4, False, 12288, 2048, 32): {WHOLE}, (2, 4, False, 4096, 2048, 32): {STEP},
+    (2, 2, True, 14336, 4096, 32): {REGISTERS}, (2, 2, True, 10240, 4096, 64): {REGISTERS}, (2, 2, True, 8192, 2048, 32): {REGISTERS},
+    (2, 2, True, 4096, 4096, 32): {STEP}, (2, 2, True, 14336, 1024, 32): {STEP}, (2, 2, True, 512, 1024, 64): {STEP}, (4, 2, True, 12288, 2048, 32): {REGISTERS, WHOLE},
+    (4, 2, True, 8192, 2048, 32): {REGISTERS}, (4, 2, True, 2048, 4096, 32): {STEP}, (8, 2, True, 6144, 2048, 32): {WHOLE},
+    (4, 4, True, 12288, 1024, 32): {WHOLE}, (2, 4, True, 8192, 3072, 32): {WHOLE}, (2, 4, True, 8192, 1536, 32): {REGISTERS},
+    (4, 2, False, 28672, 8192, 32): {WHOLE}, (8, 2, True, 28672, 8192, 64): {WHOLE},
+}
+
+
+def test_transposed_quantize_takes_the_fastest_of_its_kernels(answer):
+    got = answer([transposed_tile(*case) for case in TRANSPOSED])
+    wrong = {case: g for (case, good), g in zip(TRANSPOSED.items(), got) if g not in good}
+    assert not wrong
