@@ -15,6 +15,8 @@
 // Kernels: quantize_transposed_kernel (given scales or fused abs-max), its variant
 // quantize_transposed_quads_kernel, scales_transposed_kernel (abs-max -> scale only),
 // dequantize_transposed_kernel.
+#include <type_traits>
+
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
 #include "cq_launch_rules.hpp"
@@ -464,12 +466,13 @@ __device__ __forceinline__ TilePlace tile_place(uint32_t row_tiles, uint32_t col
 // workgroup: four workgroups fit a compute unit; blocks of 32 and 64 columns, or any multiple of 32 with given scales.
 // kPart 32: blocks of 128 columns, twice the floats.  kWholeTile: 128 bytes of codes per row and tile; else a tile is one
 // step, for launches of few tiles: eight times as many workgroups (4-bit), each with one step's latency
-// (transposed_tile() draws the lines).
+// (transposed_tile() draws the lines).  kStay: codes through plain stores (transposed_codes_stay(); a branch at the stores
+// instead of a kernel of its own cost 5 - 8 %: 8 bits of bf16 [4096, 4096] 12.3 -> 13.1 us).
 // Bound by its stores (runs of 128 and 32 bytes far apart).  Measured against the kernel it replaced for blocks of 64 and
 // 128 and for few tiles (quantize_transposed_quads_kernel, left with runs of 8 bytes): 4 bits, blocks of 64 f16
 // [31072, 1408] 37.8 -> 28.2 us, blocks of 128 [10944, 2816] 30.2 -> 22.8 us, bf16 [117472, 1024] 78.7 -> 67.0 us; few
 // tiles, blocks of 32 [1440, 864] 11.0 -> 5.4 us, [64, 10144] 11.7 -> 5.2 us, 8 bits [5664, 1216] 15.1 -> 8.6 us.
-template <class F, int kBits, int kEnc, int kScale, uint32_t kPart, bool kWholeTile>
+template <class F, int kBits, int kEnc, int kScale, uint32_t kPart, bool kWholeTile, bool kStay>
 // seg_magic / seg_shift: column / a.segment as a multiplication and a shift (cq_magic_div.hpp; columns below 2^31)
 __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(TransposedArgs a, QuantParams qp, uint32_t seg_magic,
                                                                             uint32_t seg_shift) {
@@ -595,11 +598,14 @@ __global__ __launch_bounds__(kThreads) void quantize_transposed_tile_kernel(Tran
 #pragma unroll
     for (uint32_t idx = t; idx < kTileRows * (kRowWords / 4); idx += kThreads) {
         const uint32_t row = idx / (kRowWords / 4), q = idx % (kRowWords / 4);
-        if (row < rows_here && q * 4 < words_here)  // the launcher checked: rows hold a multiple of four words
-            // plain stores: runs that are not whole lines meet their neighbours' in the L2, and a re-pack right behind
-            // finds the codes there ([14336, 4096] 4 bits, both launches 45.4 -> 42.5 us)
-            *reinterpret_cast<u32x4*>(tile_out + static_cast<uint64_t>(row) * a.vrow + q * 4) =
-                *reinterpret_cast<const u32x4*>(&lds_words[row * kRowPitch + q * 4]);
+        if (row < rows_here && q * 4 < words_here) {  // the launcher checked: rows hold a multiple of four words
+            const u32x4 v = *reinterpret_cast<const u32x4*>(&lds_words[row * kRowPitch + q * 4]);
+            u32x4* const dst = reinterpret_cast<u32x4*>(tile_out + static_cast<uint64_t>(row) * a.vrow + q * 4);
+            if constexpr (kStay)
+                *dst = v;
+            else
+                stream_store(v, dst);
+        }
     }
     if (a.scale_out != nullptr && !a.tensor_level) {
         const uint32_t tile_seg0 = tile_c0 / a.segment;
@@ -923,20 +929,24 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
                  tile_count < (1u << 31);
     for (uint32_t k = 0; k < a.num_batch_dims; k++) tiles = tiles && a.batch_v[k] % 4 == 0;
     const dim3 tile_grid(static_cast<uint32_t>((tile_count + 7) / 8 * 8), 1, a.batches);  // see tile_place()
-#define CQ_TILE(B, E, P, T) \
-    hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale, P, T>), tile_grid, dim3(kThreads), 0, s, a, qp, seg_magic, seg_shift)
+    const bool stay = transposed_codes_stay(static_cast<uint64_t>(a.rows) * (cols / nq) * 4 * a.batches);
+#define CQ_TILE(B, E, P, T, S) \
+    hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale, P, T, S>), tile_grid, dim3(kThreads), 0, s, a, qp, seg_magic, seg_shift)
 #define CQ_LAUNCH(B, W, E)                                                                                        \
     {                                                                                                             \
         if (tiles && !W) {                                                                                        \
             if (kScale == 0 && step_cols == 128) {                                                                \
                 if constexpr (kScale == 0) {                                                                      \
-                    if (whole_tile) CQ_TILE(B, E, 32, true);                                                      \
-                    else CQ_TILE(B, E, 32, false);                                                                \
+                    if (whole_tile && stay) CQ_TILE(B, E, 32, true, true);                                        \
+                    else if (whole_tile) CQ_TILE(B, E, 32, true, false);                                          \
+                    else if constexpr (B < 8) CQ_TILE(B, E, 32, false, true);                                     \
                 }                                                                                                 \
+            } else if (whole_tile && stay) {                                                                      \
+                CQ_TILE(B, E, 16, true, true);                                                                    \
             } else if (whole_tile) {                                                                              \
-                CQ_TILE(B, E, 16, true);                                                                          \
+                CQ_TILE(B, E, 16, true, false);                                                                   \
             } else {                                                                                              \
-                CQ_TILE(B, E, 16, false);                                                                         \
+                CQ_TILE(B, E, 16, false, true);                                                                   \
             }                                                                                                     \
         } else if (quads)                                                                                         \
             hipLaunchKernelGGL((quantize_transposed_quads_kernel<F, B, W, E, kScale>), grid, dim3(kThreads), 0, s, q, qp); \

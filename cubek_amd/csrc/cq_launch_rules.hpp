@@ -25,11 +25,23 @@ enum class TransposedTile { kRegisters, kStep, kWhole };
 inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool given_scales, uint64_t rows, uint64_t whole_tiles,
                                       uint64_t steps, uint32_t step_cols) {
     if (whole_tiles >= 1024) return TransposedTile::kWhole;
-    if (step_cols == 128) return TransposedTile::kStep;
+    if (step_cols == 128) return bits == 8 ? TransposedTile::kWhole : TransposedTile::kStep;  // 8 bits: the same tile
     const bool registers_keep_up = given_scales && float_bytes == 2 && bits < 8;
     if (!registers_keep_up && whole_tiles >= 512) return TransposedTile::kWhole;
     if (given_scales) return rows <= 6144 || steps <= 1536 || whole_tiles < 256 ? TransposedTile::kStep : TransposedTile::kRegisters;
     return rows <= 8192 || steps < 2048 ? TransposedTile::kStep : TransposedTile::kWhole;
 }
+
+// Whether the codes of whole tiles of a transposed quantize leave through plain stores instead of streaming ones (tiles of one
+// step, whose runs are shorter than a line, always take plain ones: the runs have to meet their neighbours' in the L2).
+//
+// After plain stores the codes are in the caches for the kernel that reads them next; the launch itself pays for that
+// (streaming -> plain; the launch alone, with a re-pack behind it, with a dequantize behind it): 8 bits of bf16 [4096, 4096]
+// 17 MB 12.5 -> 13.6, 20.4 -> 20.6, 25.9 -> 24.0; [6144, 4096] 25 MB 19.4 -> 19.1, 29.6 -> 27.8, 37.3 -> 32.9;
+// [14336, 4096] 59 MB 38.4 -> 39.0, 58.9 -> 57.2, 79.9 -> 68.5; [16384, 8192] 134 MB 87.1 -> 86.8, 140 -> 140, 167 -> 153;
+// 4 bits [4096, 4096] 8 MB 11.8 -> 12.8, 17.3 -> 18.1, 23.2 -> 23.1; [14336, 4096] 29 MB 32.2 -> 33.4, 46.7 -> 42.9,
+// 65.6 -> 59.3.  What does not fit the 256 MB of the Infinity Cache pushes itself out: [28672, 16384] 235 MB 225 -> 311 and
+// 312 -> 349, 8 bits [8192, 28672] 235 MB 137 -> 176 and 220 -> 226.
+inline bool transposed_codes_stay(uint64_t bytes) { return bytes >= (20ull << 20) && bytes <= (192ull << 20); }
 
 }  // namespace cq

@@ -55,3 +55,16 @@ def test_transposed_quantize_takes_the_fastest_of_its_kernels(answer):
     got = answer([transposed_tile(*case) for case in TRANSPOSED])
     wrong = {case: g for (case, good), g in zip(TRANSPOSED.items(), got) if g not in good}
     assert not wrong
+
+
+# (rows, columns, bits): whether the codes of whole tiles should stay in the caches
+STAY = {
+    (4096, 4096, 4): False, (4096, 4096, 8): False, (14336, 4096, 2): False, (14336, 4096, 4): True, (16384, 8192, 4): True,
+    (11264, 4096, 8): True, (14336, 4160, 4): True, (16384, 8192, 8): True, (28672, 8256, 4): True, (28672, 16384, 4): False,
+    (28672, 8192, 8): False, (8192, 28672, 8): False, (57344, 8256, 4): False,
+}
+
+
+def test_transposed_codes_stay_in_the_caches_where_they_fit(answer):
+    got = answer([f"transposed_codes_stay({rows * cols * bits // 8}ull)" for rows, cols, bits in STAY])
+    assert got == [int(stay) for stay in STAY.values()], dict(zip(STAY, got))
