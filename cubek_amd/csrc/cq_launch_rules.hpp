@@ -15,7 +15,7 @@ namespace cq {
 //   column of tiles later, so with many rows the line has left the L2 before it is full.  Fused abs-max, 2 bits of bf16
 //   (steps, whole tiles, register kernel): [4096, 4096] 12.2, 14.6, 14.5, [8192, 2048] 13.7, 14.9, 14.8, [16384, 1024] 17.9,
 //   15.0, 15.0, [14336, 2048] 24.8, 18.3, 23.4, [14336, 4096] 47.2, 31.7, 36.5; 4 bits [6144, 4096] 17.2, 14.5, 19.0,
-//   [12288, 2048] 22.3, 15.4, 19.3, [2048, 4096] 8.1, 9.8, 10.8.
+//   [12288, 2048] 22.3, 15.4, 19.3, [14336, 1024] 14.5, 12.3, 14.5, [2048, 4096] 8.1, 9.8, 10.8.
 // * Given scales read them between the steps: 2 bits of bf16 [4096, 4096] 13.8, 19.8, 16.4, [8192, 2048] 17.0, 20.3, 15.9,
 //   [14336, 1024] 13.9, 20.1, 15.7, [14336, 4096] 54, 44.2, 35.5; 4 bits [8192, 2048] 19.0, 17.0, 15.8, [14336, 1024] 17.4,
 //   15.5, 15.8; wider codes and f32 gain from whole tiles all the same: 8 bits [6144, 2048] 13.8, 12.4, 15.9, 4 bits of f32
@@ -28,8 +28,8 @@ inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool 
     if (step_cols == 128) return bits == 8 ? TransposedTile::kWhole : TransposedTile::kStep;  // 8 bits: the same tile
     const bool registers_keep_up = given_scales && float_bytes == 2 && bits < 8;
     if (!registers_keep_up && whole_tiles >= 512) return TransposedTile::kWhole;
-    if (given_scales) return rows <= 6144 || steps <= 1536 || whole_tiles < 256 ? TransposedTile::kStep : TransposedTile::kRegisters;
-    return rows <= 8192 || steps < 2048 ? TransposedTile::kStep : TransposedTile::kWhole;
+    if (rows <= (given_scales ? 6144 : 8192) || steps <= 1536 || whole_tiles < 256) return TransposedTile::kStep;
+    return given_scales ? TransposedTile::kRegisters : TransposedTile::kWhole;
 }
 
 // Whether the codes of whole tiles of a transposed quantize leave through plain stores instead of streaming ones (tiles of one

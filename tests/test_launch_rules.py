@@ -41,6 +41,7 @@ TRANSPOSED = {
     (2, 2, False, 14336, 4096, 32): {WHOLE}, (2, 2, False, 31072, 1408, 32): {WHOLE}, (2, 2, False, 14336, 2048, 32): {WHOLE},
     (2, 2, False, 16384, 1024, 32): {WHOLE, REGISTERS}, (2, 2, False, 4096, 4096, 32): {STEP}, (2, 2, False, 2048, 2048, 64): {STEP},
     (4, 2, False, 8192, 2048, 32): {WHOLE}, (4, 2, False, 12288, 2048, 32): {WHOLE}, (4, 2, False, 6144, 4096, 64): {WHOLE},
+    (4, 2, False, 14336, 1024, 32): {WHOLE}, (2, 2, False, 14336, 1024, 32): {STEP}, (4, 2, False, 11008, 1024, 64): {STEP},
     (4, 2, False, 2048, 4096, 32): {STEP}, (4, 2, False, 1056, 16384, 128): {STEP}, (8, 2, False, 24576, 512, 32): {WHOLE},
     (2, 4, False, 12288, 2048, 32): {WHOLE}, (2, 4, False, 4096, 2048, 32): {STEP},
     (2, 2, True, 14336, 4096, 32): {REGISTERS}, (2, 2, True, 10240, 4096, 64): {REGISTERS}, (2, 2, True, 8192, 2048, 32): {REGISTERS},
