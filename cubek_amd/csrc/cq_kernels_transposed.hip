@@ -929,7 +929,9 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
                  tile_count < (1u << 31);
     for (uint32_t k = 0; k < a.num_batch_dims; k++) tiles = tiles && a.batch_v[k] % 4 == 0;
     const dim3 tile_grid(static_cast<uint32_t>((tile_count + 7) / 8 * 8), 1, a.batches);  // see tile_place()
-    const bool stay = transposed_codes_stay(static_cast<uint64_t>(a.rows) * (cols / nq) * 4 * a.batches);
+    const bool stay = transposed_codes_stay(static_cast<uint64_t>(a.rows) * (cols / nq) * 4 * a.batches,
+                                            a.tensor_level ? 0 : static_cast<uint64_t>(a.rows) * a.segments * a.batches * (a.param_dtype == CQ_F32 ? 4 : 2),
+                                            a.segment);
 #define CQ_TILE(B, E, P, T, S) \
     hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale, P, T, S>), tile_grid, dim3(kThreads), 0, s, a, qp, seg_magic, seg_shift)
 #define CQ_LAUNCH(B, W, E)                                                                                        \
@@ -939,7 +941,7 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
                 if constexpr (kScale == 0) {                                                                      \
                     if (whole_tile && stay) CQ_TILE(B, E, 32, true, true);                                        \
                     else if (whole_tile) CQ_TILE(B, E, 32, true, false);                                          \
-                    else if constexpr (B < 8) CQ_TILE(B, E, 32, false, true);                                     \
+                    else CQ_TILE(B, E, 32, false, true);                                                          \
                 }                                                                                                 \
             } else if (whole_tile && stay) {                                                                      \
                 CQ_TILE(B, E, 16, true, true);                                                                    \
