@@ -929,9 +929,9 @@ hipError_t quantize_transposed(hipStream_t s, int bits, const TransposedArgs& a)
                  tile_count < (1u << 31);
     for (uint32_t k = 0; k < a.num_batch_dims; k++) tiles = tiles && a.batch_v[k] % 4 == 0;
     const dim3 tile_grid(static_cast<uint32_t>((tile_count + 7) / 8 * 8), 1, a.batches);  // see tile_place()
-    const bool stay = transposed_codes_stay(static_cast<uint64_t>(a.rows) * (cols / nq) * 4 * a.batches,
-                                            a.tensor_level ? 0 : static_cast<uint64_t>(a.rows) * a.segments * a.batches * (a.param_dtype == CQ_F32 ? 4 : 2),
-                                            a.segment);
+    const uint64_t row_count = static_cast<uint64_t>(a.rows) * a.batches;
+    const bool stay = transposed_codes_stay(row_count * cols * F::kBytes, row_count * (cols / nq) * 4,
+                                            a.tensor_level ? 0 : row_count * a.segments * (a.param_dtype == CQ_F32 ? 4 : 2), a.segment);
 #define CQ_TILE(B, E, P, T, S) \
     hipLaunchKernelGGL((quantize_transposed_tile_kernel<F, B, E, kScale, P, T, S>), tile_grid, dim3(kThreads), 0, s, a, qp, seg_magic, seg_shift)
 #define CQ_LAUNCH(B, W, E)                                                                                        \

@@ -35,19 +35,20 @@ inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool 
 // Whether the codes of whole tiles of a transposed quantize leave through plain stores instead of streaming ones (tiles of one
 // step always take plain ones: their runs, shorter than a line, have to meet their neighbours' in the L2).
 //
-// After plain stores the codes are in the caches for the kernel that reads them next; the launch itself pays for that
-// (streaming -> plain; the launch alone, with a re-pack behind it, with a dequantize behind it): 4 bits of bf16 [4096, 4096]
-// 8 MB 11.8 -> 12.8, 17.3 -> 18.1, 23.2 -> 23.1; [4096, 5120] 10 MB 14.2 -> 15.2, 20.9 -> 21.6, 32.5 -> 28.9; [8192, 4096]
-// 17 MB 21.6 -> 21.5, 29.2 -> 29.2, 42.9 -> 38.7; [14336, 4096] 29 MB 32.2 -> 33.4, 46.7 -> 42.9, 65.6 -> 59.3; 8 bits
-// [4096, 4096] 17 MB 12.5 -> 13.6, 20.4 -> 20.6, 25.9 -> 24.0; [14336, 4096] 59 MB 38.4 -> 39.0, 58.9 -> 57.2, 79.9 -> 68.5;
-// [16384, 8192] 134 MB 87.1 -> 86.8, 140 -> 140, 167 -> 153.  Once codes and scales come near the 256 MB of the Infinity Cache
-// they push themselves out, blocks of 32 (whose launches are the fastest) first: 8 bits [24576, 8192] 201 + 25 MB 127 -> 135,
-// [28672, 8192] 235 + 29 MB 143 -> 175, 233 -> 255, 279 -> 259; 4 bits [28672, 8192] 117 + 29 MB 114 -> 119, 162 -> 158, 235 ->
-// 226, [28672, 12288] 176 + 44 MB 174 -> 216, 353 -> 333; 2 bits [28672, 16384] 117 + 59 MB 204 -> 234.  Blocks of 64: 8 bits
-// [28672, 8192] 235 + 15 MB 140 -> 145, 238 -> 226, 276 -> 252, [28672, 16384] 470 + 29 MB 298 -> 363, 504 -> 577.
-inline bool transposed_codes_stay(uint64_t code_bytes, uint64_t scale_bytes, uint32_t block) {
-    const uint64_t bytes = code_bytes + scale_bytes;
-    return bytes >= (12ull << 20) && bytes <= (block <= 32 ? 152ull << 20 : 240ull << 20);
+// After plain stores the codes are in the caches for the kernel that reads them next; the launch itself pays for that, and
+// below 52 MiB moved that reader finds much of them there either way (streaming -> plain; the launch alone, with a re-pack
+// behind it, with a dequantize behind it): 4 bits of bf16 [4096, 4096] 8 MB 11.8 -> 12.8, 17.3 -> 18.1, 23.2 -> 23.1; [4096,
+// 5120] 10 MB 14.2 -> 15.2, 20.9 -> 21.6, 32.5 -> 28.9; [8192, 4096] 17 MB 21.6 -> 21.5, 29.2 -> 29.2, 42.9 -> 38.7; [14336,
+// 4096] 29 MB 32.2 -> 33.4, 46.7 -> 42.9, 65.6 -> 59.3; 8 bits [4096, 4096] 17 MB 12.5 -> 13.6, 20.4 -> 20.6, 25.9 -> 24.0;
+// [14336, 4096] 59 MB 38.4 -> 39.0, 58.9 -> 57.2, 79.9 -> 68.5; [16384, 8192] 134 MB 87.1 -> 86.8, 140 -> 140, 167 -> 153.
+// Once codes and scales come near the 256 MB of the Infinity Cache they push themselves out, blocks of 32 (whose launches are
+// the fastest) first: 8 bits [24576, 8192] 201 + 25 MB 127 -> 135, [28672, 8192] 235 + 29 MB 143 -> 175, 233 -> 255, 279 ->
+// 259; 4 bits [28672, 8192] 117 + 29 MB 114 -> 119, 162 -> 158, 235 -> 226, [28672, 12288] 176 + 44 MB 174 -> 216, 353 -> 333;
+// 2 bits [28672, 16384] 117 + 59 MB 204 -> 234.  Blocks of 64: 8 bits [28672, 8192] 235 + 15 MB 140 -> 145, 238 -> 226, 276 ->
+// 252, [28672, 16384] 470 + 29 MB 298 -> 363, 504 -> 577.
+inline bool transposed_codes_stay(uint64_t float_bytes, uint64_t code_bytes, uint64_t scale_bytes, uint32_t block) {
+    const uint64_t kept = code_bytes + scale_bytes;
+    return float_bytes + kept >= (52ull << 20) && kept <= (block <= 32 ? 152ull << 20 : 240ull << 20);
 }
 
 }  // namespace cq

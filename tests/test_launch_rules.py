@@ -58,9 +58,10 @@ def test_transposed_quantize_takes_the_fastest_of_its_kernels(answer):
     assert not wrong
 
 
-# (rows, columns, bits, block): whether the codes of whole tiles should stay in the caches
+# (rows, columns of a 16-bit type, bits, block): whether the codes of whole tiles should stay in the caches
 STAY = {
-    (4096, 4096, 4, 32): False, (8192, 4096, 2, 64): False, (4096, 5120, 4, 32): True, (4096, 4096, 8, 32): True,
+    (4096, 4096, 4, 32): False, (4096, 5120, 4, 32): True, (4096, 4096, 8, 32): False,
+    (65536, 256, 8, 128): False, (4096, 5120, 8, 32): True, (8192, 4096, 4, 32): True,
     (14336, 4096, 4, 32): True, (16384, 8192, 4, 64): True, (11264, 4096, 8, 32): True, (14336, 4160, 4, 32): True,
     (16384, 8192, 8, 32): True, (28672, 8192, 4, 32): True, (28672, 8192, 8, 64): True, (28672, 8192, 8, 128): True,
     (24576, 8192, 8, 32): False, (28672, 8192, 8, 32): False, (8192, 28672, 8, 32): False, (28672, 12288, 4, 32): False,
@@ -69,5 +70,5 @@ STAY = {
 
 
 def test_transposed_codes_stay_in_the_caches_where_they_fit(answer):
-    got = answer([f"transposed_codes_stay({rows * cols * bits // 8}ull, {rows * cols // block * 4}ull, {block})" for rows, cols, bits, block in STAY])
+    got = answer([f"transposed_codes_stay({rows * cols * 2}ull, {rows * cols * bits // 8}ull, {rows * cols // block * 4}ull, {block})" for rows, cols, bits, block in STAY])
     assert got == [int(stay) for stay in STAY.values()], dict(zip(STAY, got))
