@@ -7,6 +7,7 @@
 #include "cq_device.hpp"
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 #include "cq_magic_div.hpp"
 
 #include <cstring>
@@ -166,7 +167,8 @@ __device__ __forceinline__ void transpose_fields(uint32_t (&a)[kP]) {
 
 // kTileWords: input word columns per tile (a multiple of 4, at most 64);
 // kTileCols: output word columns per tile (input rows / kP).
-template <int kP, int kTileWords, int kTileCols>
+// kStay: plain stores (repack_stays()).
+template <int kP, int kTileWords, int kTileCols, bool kStay>
 __global__ __launch_bounds__(kTileWords / 4 * kTileCols) void repack_tile_kernel(TileArgs a) {
     constexpr int kQuads = kTileWords / 4;   // 16-byte word quads per tile row of the input
     constexpr int kT = kQuads * kTileCols;   // threads
@@ -223,10 +225,11 @@ __global__ __launch_bounds__(kTileWords / 4 * kTileCols) void repack_tile_kernel
         if (p < static_cast<uint64_t>(a.wp) * kP && lw0 + c4 < a.wl) {
             const uint32_t col = (c4 + (row / (4 * kP)) * kRot) % kTileCols;
             const u32x4 v = *reinterpret_cast<const u32x4*>(&lds[row * kTileCols + col]);
-            // A plain store, not a streaming one: rows that do not start on a line cut a tile's runs into parts of lines,
-            // which meet their neighbours' in the L2 before they leave (4-bit codes of [1024, 117472] 54.2 -> 23.0 us,
-            // of [512, 201376] 46.1 -> 20.0 us; rows of whole lines, [4096, 14336] 14.4 -> 10.0 us).
-            *reinterpret_cast<u32x4*>(a.out + out_base + p * a.out_p_stride + lw0 + c4) = v;
+            u32x4* const dst = reinterpret_cast<u32x4*>(a.out + out_base + p * a.out_p_stride + lw0 + c4);
+            if constexpr (kStay)
+                *dst = v;
+            else
+                stream_store(v, dst);
         }
     }
 }
@@ -307,11 +310,19 @@ hipError_t launch_repack(hipStream_t s, const RepackArgs& bytes_or_words) {
     // both sides move whole 128-byte lines (64-byte segments measured at two thirds of this)
     const uint32_t tile_words = a.packing == 4 ? 64 : 32;
     if (plan_tiles(a, &t, &tile_grid, tile_words, 32)) {
+        bool whole_lines = (reinterpret_cast<uintptr_t>(t.out) & 127u) == 0 && t.out_p_stride % 32 == 0;
+        for (uint32_t d = 0; d < t.num_batch_dims; d++) whole_lines = whole_lines && t.batch_out[d] % 32 == 0;
+        const bool stay = repack_stays(a.num_out * 4, whole_lines);
+#define CQ_TILES(P, W, T) \
+    if (stay) hipLaunchKernelGGL((repack_tile_kernel<P, W, 32, true>), tile_grid, dim3(T), 0, s, t); \
+    else hipLaunchKernelGGL((repack_tile_kernel<P, W, 32, false>), tile_grid, dim3(T), 0, s, t); \
+    break;
         switch (a.packing) {
-            case 4: hipLaunchKernelGGL((repack_tile_kernel<4, 64, 32>), tile_grid, dim3(512), 0, s, t); break;
-            case 8: hipLaunchKernelGGL((repack_tile_kernel<8, 32, 32>), tile_grid, dim3(256), 0, s, t); break;
-            default: hipLaunchKernelGGL((repack_tile_kernel<16, 32, 32>), tile_grid, dim3(256), 0, s, t); break;
+            case 4: CQ_TILES(4, 64, 512)
+            case 8: CQ_TILES(8, 32, 256)
+            default: CQ_TILES(16, 32, 256)
         }
+#undef CQ_TILES
         return hipGetLastError();
     }
     // the same packing on both sides: strided rows, copied in 16-byte units where everything is aligned

@@ -51,4 +51,17 @@ inline bool transposed_codes_stay(uint64_t float_bytes, uint64_t code_bytes, uin
     return float_bytes + kept >= (52ull << 20) && kept <= (block <= 32 ? 152ull << 20 : 240ull << 20);
 }
 
+// Whether the tiles of a re-pack leave through plain stores instead of streaming ones.  `whole_lines`: the output's rows start on
+// lines of 128 bytes.
+//
+// Rows that do not, cut a tile's runs into parts of lines, which have to meet their neighbours' in the L2 before they leave
+// (streaming -> plain, us): 4 bits [4096, 14400] 17.8 -> 15.6, [1024, 117472] 51 -> 29, [8192, 28704] 103 -> 51.  Whole lines
+// gain from plain stores only in the middle: 4 bits 8 MB 4.7 -> 5.7, 29 MB 13.3 -> 15.4, 34 MB 16.1 -> 16.6, 67 MB 29.9 -> 26.8,
+// 84 MB 33.8 -> 31.9; 8 bits 17 MB 6.8 -> 7.9, 46 MB 19.1 -> 18.2, 67 MB 26.5 -> 24.9, 235 MB 84.9 -> 90.7.  Above, a quantize
+// that left the codes in the caches and the output push each other out: 4 bits 117 MB 45.7 -> 41.9 alone, but both launches
+// 158 -> 176; 8 bits 134 MB both 128 -> 135.
+inline bool repack_stays(uint64_t bytes, bool whole_lines) {
+    return !whole_lines || (bytes >= (32ull << 20) && bytes <= (96ull << 20));
+}
+
 }  // namespace cq

@@ -84,6 +84,24 @@ def test_quantize_transposed_then_repack_equals_quantize_of_transpose(gpu, oracl
     assert np.array_equal(got, codes_kn.reshape(k, n // 8))
 
 
+@pytest.mark.parametrize("rows,cols", [(8192, 5120), (8192, 5136), (4096, 3072)])
+def test_bytes_of_large_and_small_outputs(rows, cols):
+    """8-bit fields packed along the first dimension: re-packing transposes bytes.  40 MiB of whole lines, of rows that start
+    inside lines, and 12 MiB of whole lines."""
+    import torch
+
+    from cubek_amd import TensorHandleRef
+
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    src = torch.randint(0, 256, (cols, rows), dtype=torch.uint8, device="cuda", generator=g)
+    dst = torch.zeros((rows, cols // 4), dtype=torch.int32, device="cuda")
+    words = src.view(torch.int32)  # [cols, rows / 4]
+    cq_contiguous.into_contiguous_packed_ref(ComputeClient.current(), TensorHandleRef(words.data_ptr(), (rows // 4, cols), (1, rows // 4), 4),
+                                             TensorHandleRef.from_torch(dst), (rows, cols), 4)
+    torch.cuda.synchronize()
+    assert torch.equal(dst.view(torch.uint8), src.t().contiguous())
+
+
 def test_into_contiguous_packed_errors(gpu):
     import torch
 

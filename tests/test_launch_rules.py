@@ -72,3 +72,15 @@ STAY = {
 def test_transposed_codes_stay_in_the_caches_where_they_fit(answer):
     got = answer([f"transposed_codes_stay({rows * cols * 2}ull, {rows * cols * bits // 8}ull, {rows * cols // block * 4}ull, {block})" for rows, cols, bits, block in STAY])
     assert got == [int(stay) for stay in STAY.values()], dict(zip(STAY, got))
+
+
+# (bytes of the output, rows on whole lines): whether a re-pack's output should leave through plain stores
+REPACK = {
+    (8 << 20, True): False, (28 << 20, True): False, (64 << 20, True): True, (80 << 20, True): True, (112 << 20, True): False,
+    (224 << 20, True): False, (15 << 20, False): True, (112 << 20, False): True,
+}
+
+
+def test_repacked_words_stay_in_the_caches_where_lines_are_shared_or_both_launches_fit(answer):
+    got = answer([f"repack_stays({n}ull, {str(lines).lower()})" for n, lines in REPACK])
+    assert got == [int(stay) for stay in REPACK.values()], dict(zip(REPACK, got))
