@@ -15,7 +15,8 @@ namespace cq {
 //   column of tiles later, so with many rows the line has left the L2 before it is full.  Fused abs-max, 2 bits of bf16
 //   (steps, whole tiles, register kernel): [4096, 4096] 12.2, 14.6, 14.5, [8192, 2048] 13.7, 14.9, 14.8, [16384, 1024] 17.9,
 //   15.0, 15.0, [14336, 2048] 24.8, 18.3, 23.4, [14336, 4096] 47.2, 31.7, 36.5; 4 bits [6144, 4096] 17.2, 14.5, 19.0,
-//   [12288, 2048] 22.3, 15.4, 19.3, [14336, 1024] 14.5, 12.3, 14.5, [2048, 4096] 8.1, 9.8, 10.8.
+//   [12288, 2048] 22.3, 15.4, 19.3, [14336, 1024] 14.5, 12.3, 14.5, [2048, 4096] 8.1, 9.8, 10.8, [1024, 28672] 18.9,
+//   20.4, 23.2.
 // * Given scales read them between the steps: 2 bits of bf16 [4096, 4096] 13.8, 19.8, 16.4, [8192, 2048] 17.0, 20.3, 15.9,
 //   [14336, 1024] 13.9, 20.1, 15.7, [14336, 4096] 54, 44.2, 35.5; 4 bits [8192, 2048] 19.0, 17.0, 15.8, [14336, 1024] 17.4,
 //   15.5, 15.8; wider codes and f32 gain from whole tiles all the same: 8 bits [6144, 2048] 13.8, 12.4, 15.9, 4 bits of f32
@@ -27,7 +28,8 @@ inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool 
     if (whole_tiles >= 1024) return TransposedTile::kWhole;
     if (step_cols == 128) return TransposedTile::kStep;
     const bool registers_keep_up = given_scales && float_bytes == 2 && bits < 8;
-    if (!registers_keep_up && whole_tiles >= 512) return TransposedTile::kWhole;
+    const bool few_rows = !given_scales && rows <= 1280;
+    if (!registers_keep_up && !few_rows && whole_tiles >= 512) return TransposedTile::kWhole;
     if (rows <= (given_scales ? 6144 : 8192) || steps <= 1536 || whole_tiles < 256) return TransposedTile::kStep;
     return given_scales ? TransposedTile::kRegisters : TransposedTile::kWhole;
 }
@@ -36,7 +38,7 @@ inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool 
 // step always take plain ones: their runs, shorter than a line, have to meet their neighbours' in the L2).
 //
 // After plain stores the codes are in the caches for the kernel that reads them next; the launch itself pays for that, and
-// below 52 MiB moved that reader finds much of them there either way (streaming -> plain; the launch alone, with a re-pack
+// below 51 MiB moved that reader finds much of them there either way (streaming -> plain; the launch alone, with a re-pack
 // behind it, with a dequantize behind it): 4 bits of bf16 [4096, 4096] 8 MB 11.8 -> 12.8, 17.3 -> 18.1, 23.2 -> 23.1; [4096,
 // 5120] 10 MB 14.2 -> 15.2, 20.9 -> 21.6, 32.5 -> 28.9; [8192, 4096] 17 MB 21.6 -> 21.5, 29.2 -> 29.2, 42.9 -> 38.7; [14336,
 // 4096] 29 MB 32.2 -> 33.4, 46.7 -> 42.9, 65.6 -> 59.3; 8 bits [4096, 4096] 17 MB 12.5 -> 13.6, 20.4 -> 20.6, 25.9 -> 24.0;
@@ -48,7 +50,7 @@ inline TransposedTile transposed_tile(uint32_t bits, uint32_t float_bytes, bool 
 // 252, [28672, 16384] 470 + 29 MB 298 -> 363, 504 -> 577.
 inline bool transposed_codes_stay(uint64_t float_bytes, uint64_t code_bytes, uint64_t scale_bytes, uint32_t block) {
     const uint64_t kept = code_bytes + scale_bytes;
-    return float_bytes + kept >= (52ull << 20) && kept <= (block <= 32 ? 152ull << 20 : 240ull << 20);
+    return float_bytes + kept >= (51ull << 20) && kept <= (block <= 32 ? 152ull << 20 : 240ull << 20);
 }
 
 // Whether the tiles of a re-pack leave through plain stores instead of streaming ones.  `whole_lines`: the output's rows start on

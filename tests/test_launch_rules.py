@@ -42,7 +42,7 @@ TRANSPOSED = {
     (2, 2, False, 16384, 1024, 32): {WHOLE, REGISTERS}, (2, 2, False, 4096, 4096, 32): {STEP}, (2, 2, False, 2048, 2048, 64): {STEP},
     (4, 2, False, 8192, 2048, 32): {WHOLE}, (4, 2, False, 12288, 2048, 32): {WHOLE}, (4, 2, False, 6144, 4096, 64): {WHOLE},
     (4, 2, False, 14336, 1024, 32): {WHOLE}, (2, 2, False, 14336, 1024, 32): {STEP}, (4, 2, False, 11008, 1024, 64): {STEP},
-    (4, 2, False, 2048, 4096, 32): {STEP}, (4, 2, False, 1056, 16384, 128): {STEP}, (8, 2, False, 24576, 512, 32): {WHOLE},
+    (4, 2, False, 1024, 28672, 32): {STEP}, (4, 2, False, 2048, 8192, 32): {WHOLE, STEP}, (4, 2, False, 2048, 4096, 32): {STEP}, (4, 2, False, 1056, 16384, 128): {STEP}, (8, 2, False, 24576, 512, 32): {WHOLE},
     (2, 4, False, 12288, 2048, 32): {WHOLE}, (2, 4, False, 4096, 2048, 32): {STEP},
     (2, 2, True, 14336, 4096, 32): {REGISTERS}, (2, 2, True, 10240, 4096, 64): {REGISTERS}, (2, 2, True, 8192, 2048, 32): {REGISTERS},
     (2, 2, True, 4096, 4096, 32): {STEP}, (2, 2, True, 14336, 1024, 32): {STEP}, (2, 2, True, 512, 1024, 64): {STEP}, (4, 2, True, 12288, 2048, 32): {REGISTERS, WHOLE},
@@ -61,7 +61,7 @@ def test_transposed_quantize_takes_the_fastest_of_its_kernels(answer):
 # (rows, columns of a 16-bit type, bits, block): whether the codes of whole tiles should stay in the caches
 STAY = {
     (4096, 4096, 4, 32): False, (4096, 5120, 4, 32): True, (4096, 4096, 8, 32): False,
-    (65536, 256, 8, 128): False, (4096, 5120, 8, 32): True, (8192, 4096, 4, 32): True,
+    (1056, 16384, 8, 32): True, (65536, 256, 8, 128): False, (4096, 5120, 8, 32): True, (8192, 4096, 4, 32): True,
     (14336, 4096, 4, 32): True, (16384, 8192, 4, 64): True, (11264, 4096, 8, 32): True, (14336, 4160, 4, 32): True,
     (16384, 8192, 8, 32): True, (28672, 8192, 4, 32): True, (28672, 8192, 8, 64): True, (28672, 8192, 8, 128): True,
     (24576, 8192, 8, 32): False, (28672, 8192, 8, 32): False, (8192, 28672, 8, 32): False, (28672, 12288, 4, 32): False,
