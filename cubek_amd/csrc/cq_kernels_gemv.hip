@@ -481,6 +481,9 @@ bool gemv_streams(const GemvArgs& a) {
             a.scale_stride_row >= (1ull << 32) || (a.cols / a.block_cols) * a.scale_stride_col >= (1ull << 29))
             return false;
     }
+    // rows of x and y so far apart that 32 bits do not hold it: the native store refuses such a call, the U32 store
+    // has the general kernel for it
+    if (a.x_stride >= (1ull << 32) || a.y_stride >= (1ull << 32)) return false;
     return a.cols % vals == 0 && a.cols < (1u << 26) && a.word_pitch % 4 == 0 && a.x_aligned16 && a.words_aligned16;
 }
 

@@ -196,3 +196,26 @@ def test_extension_value_runs_on_the_streaming_kernels():
     for store in (QuantStore.U32, QuantStore.Native):
         got = kinds(scheme_of(QuantValue.E2M1_OCP, [32], store=store), BF16, (28672, 8192))
         assert set(got.values()) == {"flat"}, (store, got)
+
+
+def test_product_with_vectors_beyond_32_bits_apart():
+    """Rows of x or y 2^32 elements apart or more: the native store refuses the call, the U32 store takes the general kernel;
+    one element less streams."""
+    rows, cols = 128, 4096
+    for x_stride, y_stride, near in ((1 << 32, rows, False), (cols, 1 << 32, False), ((1 << 32) - 8, (1 << 32) - 1, True)):
+        x = TensorHandleRef(0x10000000, (2, cols), (x_stride, 1), 2)
+        y = TensorHandleRef(0x50000000, (2, rows), (y_stride, 1), 2)
+        for value, store, elem_size in ((QuantValue.Q4S, QuantStore.U32, 4), (QuantValue.Q8S, QuantStore.Native, 1), (QuantValue.E4M3, QuantStore.Native, 1)):
+            scheme = scheme_of(value, [32], store=store)
+            packed, blocks = scheme.packed_shape((rows, cols)), scheme.scales_shape((rows, cols))
+            values = TensorHandleRef(0x20000000, packed, (packed[1], 1), elem_size)
+            params = TensorHandleRef(0x30000000, blocks, (blocks[1], 1), 4)
+            ask = lambda: _ffi.plan_kind(_ffi.OP_GEMV, x, values, params, y, scheme, BF16)
+            if near:
+                assert ask() == "flat"
+            elif store == QuantStore.U32:
+                assert ask() == "rows"
+            else:
+                with pytest.raises(_ffi.QuantError) as e:
+                    ask()
+                assert e.value.status == _ffi.ERR_UNSUPPORTED_SCHEME
