@@ -169,8 +169,8 @@ def test_gpu_f32_near_midpoints(gpu, oracle):
 @pytest.mark.parametrize("elem", ELEMS, ids=lambda e: e.name)
 @pytest.mark.parametrize("block", [None, (16,), (32,), (128,), (24,), (4, 32), (2, 3, 16)], ids=str)
 def test_gpu_seeded_vs_oracle(gpu, oracle, elem, block):
-    """Contiguous tensors on every kernel family that a block shape selects (whole tiles, lanes, odd blocks, 2-D blocks,
-    per element), both stores, given scales, fused dynamic quantize and dequantize."""
+    """Contiguous tensors on every kernel family that a block shape selects (single steps of a run, lanes, odd blocks, 2-D
+    blocks, per element), both stores, given scales, fused dynamic quantize and dequantize."""
     shape = (6, 96, 768) if block and len(block) == 3 else (192, 768)
     rng = np.random.default_rng(len(shape) * 131 + int(elem) + (sum(block) if block else 0))
     x32 = rng.normal(0, 1.0, shape).astype(np.float32)
@@ -190,3 +190,20 @@ def test_gpu_seeded_vs_oracle(gpu, oracle, elem, block):
             assert same_bits(gpu.dequantize(w_ref, shape, os_ref, elem, scheme), y_ref), (store, param)
             if store == QuantStore.U32:
                 assert {1, 3} <= set((nibbles(w_ref) & 7).tolist())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("elem", ELEMS, ids=lambda e: e.name)
+def test_gpu_whole_tiles_vs_oracle(gpu, oracle, elem):
+    """2^18 chunks of 16 bytes and a ragged end: whole tiles without bounds checks, single steps behind them."""
+    shape = (2051, 512 if elem == ElemType.F32 else 1024)
+    x = oracle.to_bits(np.random.default_rng(77 + int(elem)).normal(0, 1.0, shape).astype(np.float32), elem)
+    for store in (QuantStore.U32, QuantStore.Native):
+        scheme = ocp(store, (32,), QuantParam.F32)
+        s_ref = oracle.compute_scales(x, elem, shape, scheme)
+        w_ref, os_ref = oracle.quantize(x, elem, shape, s_ref, scheme)
+        w_gpu, os_gpu = gpu.quantize(x, elem, shape, s_ref, scheme)
+        assert same_bits(w_gpu, w_ref) and same_bits(os_gpu, os_ref), (store, "given")
+        w_dyn, os_dyn = gpu.quantize_dynamic(x, elem, shape, scheme)
+        assert same_bits(w_dyn, w_ref) and same_bits(os_dyn, os_ref), (store, "dynamic")
+        assert same_bits(gpu.dequantize(w_ref, shape, os_ref, elem, scheme), oracle.dequantize(w_ref, shape, os_ref, elem, scheme)), store

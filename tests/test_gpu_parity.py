@@ -130,8 +130,9 @@ def test_param_dtypes(gpu, oracle, elem, param):
 
 @pytest.mark.parametrize("elem", [ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
 def test_params_typed_like_the_tensor_on_whole_tiles(gpu, oracle, elem):
-    """bf16 scales of a bf16 tensor, f16 of f16: a contiguous tensor runs kernels compiled for that parameter
-    type over its whole tiles (four of them here) and the lane-wise kernels over the ragged rest."""
+    """bf16 scales of a bf16 tensor, f16 of f16: a contiguous tensor runs kernels compiled for that parameter type, a small
+    one like this in single steps with bounds checks (test_runs_of_whole_tiles has the whole tiles); blocks of 8 and 16
+    go lane by lane."""
     param = QuantParam.BF16 if elem == ElemType.BF16 else QuantParam.F16
     rng = np.random.default_rng(4100 + int(elem))
     shape = (33, 1024)
@@ -156,6 +157,57 @@ def test_params_typed_like_the_tensor_on_whole_tiles(gpu, oracle, elem):
         assert np.array_equal(w_dyn, w_ref) and same_floats(os_dyn, os_ref, pe), (value, level)
         assert same_floats(gpu.dequantize(w_ref, shape, os_ref, elem, scheme),
                            oracle.dequantize(w_ref, shape, os_ref, elem, scheme), elem), (value, level)
+
+
+# Contiguous runs of 2^18 chunks of 16 bytes and more: whole tiles without bounds checks, and single steps behind them where
+# the run does not end with a tile.  A tile is 1024 chunks on the quantize side, 512 or 1024 on the dequantize side.
+WHOLE_TILE_SCHEMES = [
+    (QuantValue.Q8S, QuantLevel.block([32]), QuantStore.U32),
+    (QuantValue.Q4S, QuantLevel.block([64]), QuantStore.U32),
+    (QuantValue.Q2S, QuantLevel.block([32]), QuantStore.U32),
+    (QuantValue.Q2S, QuantLevel.block([128]), QuantStore.U32),
+    (QuantValue.E2M1, QuantLevel.block([32]), QuantStore.U32),
+    (QuantValue.Q4F, QuantLevel.block([128]), QuantStore.U32),
+    (QuantValue.Q8F, QuantLevel.Tensor, QuantStore.U32),
+    (QuantValue.Q2F, QuantLevel.Tensor, QuantStore.U32),
+    (QuantValue.E4M3, QuantLevel.block([32]), QuantStore.Native),
+    (QuantValue.E5M2, QuantLevel.Tensor, QuantStore.Native),
+    (QuantValue.E2M1, QuantLevel.block([64]), QuantStore.Native),
+    (QuantValue.Q8S, QuantLevel.block([128]), QuantStore.Native),
+]
+
+
+def check_run(gpu, oracle, elem, param, rows, schemes, seed):
+    per_row = 512 if elem == ElemType.F32 else 1024  # 128 chunks
+    shape = (rows, per_row)
+    x = rand_input(np.random.default_rng(seed), shape, elem, oracle, sigma=2.0)
+    x[-1, -256:] = 0
+    for value, level, store in schemes:
+        scheme = QuantScheme.default().with_value(value).with_level(level).with_store(store).with_param(param)
+        tag, pe = (value, level, store, rows), gpu.param_elem(scheme)
+        s_ref = oracle.compute_scales(x, elem, shape, scheme)
+        w_ref, os_ref = oracle.quantize(x, elem, shape, s_ref, scheme)
+        w_gpu, os_gpu = gpu.quantize(x, elem, shape, s_ref, scheme)
+        assert np.array_equal(w_gpu, w_ref) and same_floats(os_gpu, os_ref, pe), tag + ("given",)
+        w_dyn, os_dyn = gpu.quantize_dynamic(x, elem, shape, scheme)
+        assert np.array_equal(w_dyn, w_ref) and same_floats(os_dyn, os_ref, pe), tag + ("dynamic",)
+        assert same_floats(gpu.dequantize(w_ref, shape, os_ref, elem, scheme),
+                           oracle.dequantize(w_ref, shape, os_ref, elem, scheme), elem), tag + ("dequantize",)
+
+
+@pytest.mark.parametrize("elem,param", [(ElemType.BF16, QuantParam.F32), (ElemType.F16, QuantParam.F32), (ElemType.F32, QuantParam.F32),
+                                        (ElemType.BF16, QuantParam.BF16), (ElemType.F16, QuantParam.F16)], ids=lambda v: v.name)
+def test_runs_of_whole_tiles(gpu, oracle, elem, param):
+    """Whole tiles and a ragged end of a step and a half, for every width, encoding and scale source."""
+    check_run(gpu, oracle, elem, param, 2051, WHOLE_TILE_SCHEMES, 5100 + int(elem) + int(param))
+
+
+@pytest.mark.parametrize("rows", [2047, 2048, 2049, 2052], ids=lambda r: f"{r}rows")
+@pytest.mark.parametrize("elem,param", [(ElemType.BF16, QuantParam.F32), (ElemType.F32, QuantParam.F32), (ElemType.F16, QuantParam.F16)],
+                         ids=lambda v: v.name)
+def test_runs_that_end_around_whole_tiles(gpu, oracle, elem, param, rows):
+    """The last run in single steps, the first of whole tiles alone, one half step and one whole dequantize tile behind them."""
+    check_run(gpu, oracle, elem, param, rows, [WHOLE_TILE_SCHEMES[k] for k in (0, 2, 6)], 5200 + rows)
 
 
 # ---------------------------------------------------------------- adversarial arithmetic
