@@ -230,7 +230,9 @@ __device__ __forceinline__ bool pairs_scale_is_tame(FS scale) {
     return (__builtin_bit_cast(uint32_t, s) - 0x0d800000u) < (0x71800000u - 0x0d800000u);
 }
 
-// Precondition: pairs_scale_is_tame<kF>(scale).
+// Precondition: pairs_scale_is_tame<kF>(scale).  Where the sign of a zero does not matter (the values enter a sum), any scale
+// of size below 2^100 after rounding to kF will do for 4- and 8-bit fields, negative, zero and denormal ones too: digit * s -
+// bias * s stays exact down to the denormals, and only a zero value may come out with the other sign.
 template <Float kF, int kBits, class FS>
 __device__ __forceinline__ void dequantize_symmetric_packed_value_pairs_tame(uint32_t word, FS scale, uint32_t* out) {
     static_assert(kF != Float::F32, "pairs are for the 16-bit types");

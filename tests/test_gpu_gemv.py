@@ -180,7 +180,7 @@ def test_gemv_of_a_batch(oracle, case, vectors):
                                   "e5m2-native", "q2-in-turns"])
 def test_gemv_with_several_right_hand_sides(oracle, kind, vectors):
     """x [vectors, cols] -> y [vectors, rows]: every row of y is the product with that row of x, whichever way the
-    vectors are taken (up to four or eight at once by the streaming kernel, in turns otherwise)."""
+    vectors are taken (up to sixteen at once on the matrix cores, in turns otherwise)."""
     import torch
 
     elem, value, block, param, native, rows, cols = {
@@ -270,8 +270,9 @@ def test_gemv_random_configurations(oracle):
 
 @pytest.mark.parametrize("elem", [ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
 def test_gemv_scales_of_every_kind(oracle, elem):
-    """Negative, zero, tiny and huge scales among ordinary ones (the streaming kernel sends their lanes down a
-    plain path): same tolerance against the oracle's dequantized weights."""
+    """Negative, zero, tiny and huge scales among ordinary ones (the streaming kernel of one vector sends their lanes down a
+    plain path; several vectors at once take all of these the short way): same tolerance against the oracle's
+    dequantized weights."""
     import torch
 
     rows, cols = 96, 4096
@@ -299,9 +300,74 @@ def test_gemv_scales_of_every_kind(oracle, elem):
         assert np.all(np.abs(got - want) <= 2e-5 * mag + 1e-30), (vectors, float(np.max(np.abs(got - want) / (mag + 1e-30))))
 
 
+# Several vectors at once: the short dequantization takes every scale below 2^100 in size, of either sign, zero and denormal
+# ones as well; a larger one sends its wave's stage through the general code, whose operands are picked out one by one (4-bit
+# f16 weights and x in another order than elsewhere, 8-bit words in pairs).  (Tolerance: as above.)
+SCALE_CASES = {
+    "bf16": [-0.01, 0.0, -0.0, 1e-36, -3.0, 2.0 ** -110, 3000.0, -1e-30, 1e-39, 2.0 ** 99, -(2.0 ** 99)],
+    "bf16-large": [-0.01, 0.0, 2.0 ** 100, -(2.0 ** 101), 2.0 ** 110],
+    "f16": [-0.01, 0.0, -0.0, 1e-36, -3.0, 1e-7, -6e-8, 400.0, 2.0 ** -110],
+    "f16-infinite": [1e6, 65520.0, np.inf],   # infinite once they are f16
+    "bf16-infinite": [np.inf],
+}
+
+
+@pytest.mark.parametrize("vectors", [2, 5, 16])
+@pytest.mark.parametrize("value", [QuantValue.Q4S, QuantValue.Q8S, QuantValue.E4M3, QuantValue.E2M1], ids=lambda v: v.name)
+@pytest.mark.parametrize("kind", list(SCALE_CASES))
+def test_gemv_of_a_batch_scales_of_every_kind(oracle, kind, value, vectors):
+    """Odd scales in one block in twenty, and in a row's last one; an infinite one stands on codes of one sign against ones
+    in x, so that its row sums to that infinity and every other row stays finite."""
+    import torch
+
+    elem = ElemType.F16 if kind.startswith("f16") else ElemType.BF16
+    infinite = kind.endswith("infinite")
+    native = value in (QuantValue.E4M3, QuantValue.E2M1)
+    scheme = QuantScheme.default().with_value(value).with_level(QuantLevel.block([32]))
+    if native:
+        scheme = scheme.with_store(QuantStore.Native)
+    rows, cols = 83, 1312   # 41 blocks: a last stage cut short for every width
+    rng = np.random.default_rng(31 + vectors)
+    bits = {QuantValue.Q8S: 8, QuantValue.E4M3: 8}.get(value, 4)
+    codes = rng.integers(0, 256, (rows, cols * bits // 8), dtype=np.uint8)
+    if value == QuantValue.E4M3:
+        codes &= 0xBF   # no NaN, and 1.9 at most
+    scales = rng.uniform(0.001, 0.02, (rows, cols // 32)).astype(np.float32)
+    odd = np.array(SCALE_CASES[kind], np.float32)
+    xb = oracle.to_bits(rng.normal(0, 1, (vectors, cols)).astype(np.float32), elem).reshape(vectors, cols)
+    if infinite:
+        for k, (row, block) in enumerate(((2, 0), (17, 20), (40, cols // 32 - 1), (82, 7))):
+            scales[row, block] = odd[k % len(odd)]
+            at = slice(block * 32 * bits // 8, (block + 1) * 32 * bits // 8)
+            codes[row, at] = 0x33 if bits == 4 else 0x38
+            xb[:, block * 32:(block + 1) * 32] = oracle.to_bits(np.ones(32, np.float32), elem)
+    else:
+        at = rng.random(scales.shape) < 0.05
+        at[:, -1] |= rng.random(rows) < 0.3
+        scales[at] = rng.choice(odd, int(at.sum()))
+    stored = codes if native else codes.view(np.uint32)
+    deq = oracle.from_bits(oracle.dequantize(stored, (rows, cols), scales, elem, scheme), elem).astype(np.float64)
+    assert infinite or np.all(np.isfinite(deq))
+    x64 = oracle.from_bits(xb, elem).astype(np.float64).reshape(vectors, cols)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want, mag = x64 @ deq.T, np.abs(x64) @ np.abs(deq).T
+    h = TensorHandleRef.from_torch
+    d_stored = torch.from_numpy(stored if native else stored.view(np.int32)).cuda()
+    d_scales, d_x = torch.from_numpy(scales).cuda(), torch.from_numpy(xb.view(np.int16)).cuda()
+    y = torch.zeros((vectors, rows), dtype=torch.float32, device="cuda")
+    matvec.launch_ref(ComputeClient.current(), h(d_stored), h(d_scales), scheme, h(d_x), h(y), elem, ElemType.F32)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().astype(np.float64)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.flatnonzero(~finite[0]), [2, 17, 40, 82] if infinite else []) and not np.any(np.isnan(want))
+    assert np.array_equal(got[~finite], want[~finite])
+    err = np.abs(got[finite] - want[finite])
+    assert np.all(err <= 2e-5 * mag[finite] + 1e-30), float(np.max(err / (mag[finite] + 1e-30)))
+
+
 def test_gemv_scales_with_strides(oracle):
-    """The scales of a [rows, blocks] layout stored column by column (strides (1, rows)) and with a row pitch:
-    the streaming kernel addresses them through both strides."""
+    """The scales of a [rows, blocks] layout stored column by column (strides (1, rows)) and with a row pitch: the kernels of
+    one vector and of several address them through both strides."""
     import torch
 
     rows, cols = 37, 2304
@@ -310,9 +376,9 @@ def test_gemv_scales_with_strides(oracle):
     words = rng.integers(0, 2**32, (rows, cols // 8), dtype=np.uint64).astype(np.uint32)
     scales = rng.uniform(0.001, 0.02, (rows, cols // 32)).astype(np.float32)
     deq = oracle.from_bits(oracle.dequantize(words, (rows, cols), scales, ElemType.BF16, scheme), ElemType.BF16).astype(np.float64)
-    xb = oracle.to_bits(rng.normal(0, 1, cols).astype(np.float32), ElemType.BF16)
-    x64 = oracle.from_bits(xb, ElemType.BF16).astype(np.float64)
-    want, mag = deq @ x64, np.abs(deq) @ np.abs(x64)
+    xb = oracle.to_bits(rng.normal(0, 1, (6, cols)).astype(np.float32), ElemType.BF16).reshape(6, cols)
+    x64 = oracle.from_bits(xb, ElemType.BF16).astype(np.float64).reshape(6, cols)
+    want, mag = x64 @ deq.T, np.abs(x64) @ np.abs(deq).T
     d_words = torch.from_numpy(words.view(np.int32)).cuda()
     d_x = torch.from_numpy(xb.view(np.int16)).cuda()
     h = TensorHandleRef.from_torch
@@ -322,11 +388,51 @@ def test_gemv_scales_with_strides(oracle):
     pitched[:, :nb] = torch.from_numpy(scales).cuda()
     for name, h_scales in (("column-major", TensorHandleRef(col_major.data_ptr(), (rows, nb), (1, rows), 4)),
                            ("pitched", TensorHandleRef(pitched.data_ptr(), (rows, nb), (nb + 5, 1), 4))):
-        y = torch.full((rows,), float("nan"), dtype=torch.float32, device="cuda")
-        matvec.launch_ref(ComputeClient.current(), h(d_words), h_scales, scheme, h(d_x), h(y), ElemType.BF16, ElemType.F32)
+        for vectors in (1, 6):
+            y = torch.full((vectors, rows), float("nan"), dtype=torch.float32, device="cuda")
+            hx, hy = (h(d_x), h(y)) if vectors > 1 else (h(d_x[0]), h(y[0]))
+            matvec.launch_ref(ComputeClient.current(), h(d_words), h_scales, scheme, hx, hy, ElemType.BF16, ElemType.F32)
+            torch.cuda.synchronize()
+            got = y.cpu().numpy().astype(np.float64)
+            assert np.all(np.abs(got - want[:vectors]) <= 2e-5 * mag[:vectors] + 1e-30), (name, vectors)
+
+
+@pytest.mark.parametrize("case", [
+    (ElemType.F16, QuantValue.Q4S, [128], QuantParam.F16, False), (ElemType.BF16, QuantValue.Q8S, [16], QuantParam.BF16, False),
+    (ElemType.F16, QuantValue.E2M1, [64], QuantParam.F32, True), (ElemType.BF16, QuantValue.E4M3, [4, 32], QuantParam.F16, True)],
+    ids=lambda c: f"{c[0].name}-{c[1].name}-{c[3].name}")
+def test_gemv_of_a_batch_scales_with_strides(oracle, case):
+    """Several vectors: scales column by column, pitched, and every third entry of a larger tensor, in each of their types."""
+    import torch
+
+    elem, value, block, param, native = case
+    rows, cols, vectors = 52, 1408, 3
+    scheme = QuantScheme.default().with_value(value).with_level(QuantLevel.block(block)).with_param(param)
+    if native:
+        scheme = scheme.with_store(QuantStore.Native)
+    rng = np.random.default_rng(77)
+    wb = oracle.to_bits(rng.normal(0, 0.02, (rows, cols)).astype(np.float32), elem)
+    words, stored_scales = oracle.quantize(wb, elem, (rows, cols), oracle.compute_scales(wb, elem, (rows, cols), scheme), scheme)
+    deq = oracle.from_bits(oracle.dequantize(words, (rows, cols), stored_scales, elem, scheme), elem).astype(np.float64)
+    xb = oracle.to_bits(rng.normal(0, 1, (vectors, cols)).astype(np.float32), elem).reshape(vectors, cols)
+    x64 = oracle.from_bits(xb, elem).astype(np.float64).reshape(vectors, cols)
+    want, mag = x64 @ deq.T, np.abs(x64) @ np.abs(deq).T
+    words = words.reshape(rows, -1)
+    d_words = torch.from_numpy(words if native else words.view(np.int32)).cuda()
+    d_x = torch.from_numpy(xb.view(np.int16)).cuda()
+    shape = scheme.scales_shape((rows, cols))
+    scales = stored_scales.reshape(shape)
+    h = TensorHandleRef.from_torch
+    for strides in ((1, shape[0]), (shape[1] + 3, 1), (3 * shape[1], 3)):
+        room = np.zeros((shape[0] - 1) * strides[0] + (shape[1] - 1) * strides[1] + 1, scales.dtype)
+        np.lib.stride_tricks.as_strided(room, shape, tuple(n * room.itemsize for n in strides))[...] = scales
+        d_scales = torch.from_numpy(room.view(np.int16) if room.dtype == np.uint16 else room).cuda()
+        y = torch.full((vectors, rows), float("nan"), dtype=torch.float32, device="cuda")
+        matvec.launch_ref(ComputeClient.current(), h(d_words), TensorHandleRef(d_scales.data_ptr(), shape, strides, room.itemsize), scheme,
+                          h(d_x), h(y), elem, ElemType.F32)
         torch.cuda.synchronize()
         got = y.cpu().numpy().astype(np.float64)
-        assert np.all(np.abs(got - want) <= 2e-5 * mag + 1e-30), name
+        assert np.all(np.abs(got - want) <= 2e-5 * mag + 1e-30), strides
 
 
 @pytest.mark.parametrize("kind", ["e4m3-native", "q4-f32-x", "q4-bf16", "q4-bf16-four-vectors"])
