@@ -12,9 +12,17 @@
 // units per row (128 bytes) at a time, and the next stage is on its way while one is worked on.  The places of a
 // stage are rotated from row to row on their way in, so that the 16 lanes of a read fall on 16 different groups of banks.
 //
-// Bound by instructions beside the loads: 2.4 per 4-bit bf16 weight for the dequantization, 0.5 for the rest; the
-// matrix instructions run beside them.  [28672, 8192] 4 bits, blocks of 32: 32 us for 4 vectors, 38 us for 16 (the
-// streaming kernel took four vectors a launch: 37 and 150 us; a read of the bytes 21 us).
+// Bound by instructions beside the loads where a weight of 4 bits fills the chip: 2.4 per bf16 weight for the
+// dequantization, 0.5 for the rest; at 4 cycles each they issue for more than half of the time ([28672, 8192], blocks of 32:
+// 34 us for 4 vectors, 38 us for 16; a read of the bytes 21 us), the matrix instructions for a tenth beside them.  With 8
+// bits and e4m3 bytes ([28672, 8192] 8 bits, 16 vectors 57 us), and in launches of a few rounds ([14336, 4096] f16, 8 vectors
+// 11 us), they issue for 35 - 43 %, and the waves spend about half of theirs waiting for a stage; few rows ([1024, 28672],
+// 64 workgroups, 28 us) are a chain of stages on a quarter of the chip.
+//
+// Against the kernels of two to four vectors a launch before it, us: [28672, 8192] 4 bits bf16 2 vectors 35.0 -> 34.1, 16
+// vectors 140 -> 39, f16 2 vectors 54 -> 31, 8 bits 57 -> 51, e4m3 56 -> 50; [14336, 4096] bf16 2 vectors 12.5 -> 11.7, f16
+// blocks of 128 20.0 -> 10.5; [1024, 28672] 2 vectors 30 -> 17.8, 16 vectors 141 -> 28.6.  The one size that lost is
+// [8192, 28672] in e4m3 bytes with 3 vectors, 54.2 -> 56.5.
 #include <hip/hip_runtime.h>
 
 #include "../../include/cubek_quant_device.hpp"
@@ -331,7 +339,10 @@ void launch_shape(hipStream_t s, const GemvArgs& a) {
 // (kG x kS 4 x 2, 2 x 4, 1 x 4): 4-bit bf16 [28672, 8192], 16 vectors 37.7, 49.6, 64.5 us; [8192, 28672] 67.1, 40.2,
 // 56.5 us; f16 [14336, 4096], 8 vectors 11.3, 10.8, 12.6 us; [4096, 4096], 16 vectors 12.2, 8.1, 7.4 us; e4m3 bytes
 // [14336, 4096], 16 vectors 17.8, 14.8, 21.3 us.  One row group takes eight waves while two workgroups of them fit
-// a compute unit's LDS ([4096, 4096], 4 vectors: 1 x 8 5.6, 1 x 4 6.1 us).
+// a compute unit's LDS, 80 KiB each (1 x 8, 1 x 4): 4-bit bf16 [4096, 4096], 4 vectors, 72 KiB 6.0, 6.4 us; [4096, 14336]
+// 12.1, 14.2 us.  Past that one workgroup of eight is resident, which costs where there are two for a compute unit
+// ([8192, 4096], 5 vectors, 88 KiB 10.5, 8.0 us; these take 2 x 4) and gains where there is one at most ([4096, 14336],
+// 5 vectors 12.6, 14.7 us; [1024, 28672] 18.9, 25.0 us): the line is on the safe side there.
 template <dev::Float kF, class FS, int kCode>
 void launch_code(hipStream_t s, const GemvArgs& a) {
     const uint32_t groups = (a.rows + 15) / 16;

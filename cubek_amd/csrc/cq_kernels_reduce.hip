@@ -7,17 +7,23 @@
 // A contiguous tensor is viewed as [outer, L, inner] around the reduced axis.
 //   inner == 1 (innermost axis):  rows of L contiguous elements
 //        rows that are 1..64 chunks long (power of two): lane groups + DPP butterfly
-//        otherwise one wave per (row, slice) with 16-byte lane-strided loads
+//        other rows of up to 512 chunks: lane groups with up to eight loads per lane
+//        longer ones: one wave per (row, slice) with 16-byte lane-strided loads
 //   inner a multiple of one 16-byte chunk:
 //        wide or many: one lane per (outer, inner chunk) walking L with stride `inner`
 //        narrow, few:  one workgroup per (outer, tile of chunk columns, slice of L);
 //                      its lanes form a [row phase][chunk column] grid, so a step
 //                      reads whole rows of the tile, and combine through LDS
+//        small tensors whose axis would be sliced: one launch of the tile kernel
 // When the outputs alone give too few workgroups to fill the GPU, L is cut into
-// slices whose f32 partial maxima go to a caller-provided workspace
-// ([slice][output]) and a second kernel folds them (the same tile kernel over the
-// partials).  Anything else (strided tensors, odd inner sizes) takes a
-// one-wave-per-output (long axis) or one-thread-per-output fallback.
+// slices whose partial maxima go to a caller-provided workspace ([slice][output])
+// and a second kernel folds them (the same tile kernel over the partials).
+// Partials are f32, except that those of the contiguous one-lane-per-column kernel
+// are typed like the tensor (a maximum is a number of it), so that twice as many
+// slices of a 16-bit tensor fit.  Strided tensors with a contiguous last dimension
+// of whole chunks have kernels of their own on the same plan; anything else (odd
+// inner sizes, strided last dimension) takes a one-wave-per-output (long axis) or
+// one-thread-per-output fallback.
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
 #include "cq_magic_div.hpp"
@@ -499,12 +505,13 @@ struct ReducePlan {
     uint32_t cw = 1, col_tiles = 1;
     uint64_t slices = 1;  // wanted; the launcher lowers it to what the workspace holds
     uint64_t lane_slices = 1;  // kTile on a strided input (one lane per output chunk and slice instead): wanted there
-    uint64_t pitch = 0;   // floats per slice of partials
+    uint64_t pitch = 0;   // partials per slice
 };
 
 ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN) {
     ReducePlan p;
-    // partials (f32 per output and slice) stay below 1/32 of the bytes read
+    // f32 partials of all slices stay below 1/32 of the bytes read; the workspace is sized for these (partials typed like
+    // a 16-bit tensor are twice as many in the same bytes)
     const uint64_t traffic_cap = len * (16 / kN) / 128 > 0 ? len * (16 / kN) / 128 : 1;
     if (len == 0 || outer == 0 || inner == 0) return p;
     if (inner == 1 && len % kN == 0) {
