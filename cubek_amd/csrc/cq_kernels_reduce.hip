@@ -8,21 +8,22 @@
 //   inner == 1 (innermost axis):  rows of L contiguous elements
 //        rows that are 1..64 chunks long (power of two): lane groups + DPP butterfly
 //        other rows of up to 512 chunks: lane groups with up to eight loads per lane
-//        longer ones: one wave per (row, slice) with 16-byte lane-strided loads
-//   inner a multiple of one 16-byte chunk:
+//        few long ones: a workgroup per row; others: one wave per (row, slice) with 16-byte lane-strided loads
+//        rows that are not whole chunks: the same, over the aligned chunks inside each row
+//   inner of at least one 16-byte chunk (a ragged end overlaps the chunk before it):
 //        wide or many: one lane per (outer, inner chunk) walking L with stride `inner`
 //        narrow, few:  one workgroup per (outer, tile of chunk columns, slice of L);
 //                      its lanes form a [row phase][chunk column] grid, so a step
 //                      reads whole rows of the tile, and combine through LDS
-//        small tensors whose axis would be sliced: one launch of the tile kernel
+//        short axes: one launch of the tile kernel
 // When the outputs alone give too few workgroups to fill the GPU, L is cut into
 // slices whose partial maxima go to a caller-provided workspace ([slice][output])
 // and a second kernel folds them (the same tile kernel over the partials).
 // Partials are f32, except that those of the contiguous one-lane-per-column kernel
 // are typed like the tensor (a maximum is a number of it), so that twice as many
 // slices of a 16-bit tensor fit.  Strided tensors with a contiguous last dimension
-// of whole chunks have kernels of their own on the same plan; anything else (odd
-// inner sizes, strided last dimension) takes a one-wave-per-output (long axis) or
+// of whole chunks have kernels of their own on the same plan; anything else (less than a
+// chunk of columns, strided last dimension) takes a one-wave-per-output (long axis) or
 // one-thread-per-output fallback.
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
@@ -115,6 +116,98 @@ inline uint32_t row_lanes(uint64_t chunks) {
     return best;
 }
 
+// ---- rows that start anywhere -------------------------------------------------------------------
+// A row of `len` elements at any element: its whole aligned chunks, and the fewer than two chunks' worth of elements beside
+// them.  Every access is aligned, so nothing is read twice and nothing outside the row.
+template <class F>
+struct RowSpan {
+    const char* begin;
+    const u32x4* body;   // the first aligned chunk inside the row
+    uint32_t len, head, chunks;  // elements; elements in front of the body; whole chunks inside (at least one: len >= 2 chunks)
+    __device__ __forceinline__ RowSpan(const void* in, uint64_t row, uint32_t row_len) : len(row_len) {
+        begin = static_cast<const char*>(in) + row * row_len * F::kBytes;
+        const uint32_t off = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(begin)) & 15u;
+        head = off == 0 ? 0 : (16 - off) / F::kBytes;
+        body = reinterpret_cast<const u32x4*>(begin + head * F::kBytes);
+        chunks = (len - head) / F::kPerChunk;
+    }
+    // the elements beside the body, dealt out to kLanes lanes
+    template <int kLanes>
+    __device__ __forceinline__ float edges(uint32_t lane) const {
+        float amax = 0.0f;
+        const uint32_t tail = head + chunks * F::kPerChunk;  // elements from here on
+#pragma unroll
+        for (uint32_t u = 0; u < (2 * F::kPerChunk + kLanes - 1) / kLanes; u++) {
+            const uint32_t i = lane + u * kLanes;
+            const uint32_t e = i < F::kPerChunk ? i : tail + i - F::kPerChunk;
+            const bool mine = i < F::kPerChunk ? e < head : e < len;
+            amax = fmaxf(amax, fabsf(F::load(begin, mine ? e : 0)));  // the row's first element again where there is none
+        }
+        return amax;
+    }
+};
+
+// Short ones: kGroup lanes per row, all loads in flight at once (reduce_rows_lanes_kernel).
+template <class F, int kGroup>
+__global__ __launch_bounds__(kThreads) void reduce_ragged_rows_lanes_kernel(const void* __restrict__ in, void* __restrict__ out, uint64_t rows,
+                                                                            uint32_t len, uint32_t loads) {
+    const uint64_t row = (static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x) / kGroup;
+    const uint32_t lane = threadIdx.x % kGroup;
+    const RowSpan<F> r(in, row < rows ? row : rows - 1, len);
+    float amax = r.template edges<kGroup>(lane);
+    switch (loads) {
+#define CQ_CASE(N) case N: amax = fmaxf(amax, row_share_absmax<F, kGroup, N>(r.body, lane, r.chunks)); break;
+        CQ_CASE(1) CQ_CASE(2) CQ_CASE(3) CQ_CASE(4) CQ_CASE(5) CQ_CASE(6) CQ_CASE(7) CQ_CASE(8)
+#undef CQ_CASE
+    }
+    static_assert(kRowLoads == 8, "the cases above");
+    amax = group_max<kGroup>(amax);
+    if (lane == 0 && row < rows) F::store(out, row, amax);
+}
+
+// Long ones: kLanes lanes (a wave, or a workgroup of 1024) per row and slice of it; slice 0 takes the elements beside the
+// body.  kPartial as in reduce_rows_wave_kernel.
+template <class F, int kLanes, bool kPartial>
+__global__ __launch_bounds__(kLanes > kThreads ? kLanes : kThreads) void reduce_rows_span_kernel(const void* __restrict__ in, void* __restrict__ out,
+                                                                                                 uint64_t rows, uint32_t len, uint32_t slices,
+                                                                                                 uint64_t pitch) {
+    constexpr int kT = kLanes > kThreads ? kLanes : kThreads;
+    constexpr uint32_t kUnroll = 4;
+    const uint32_t lane = threadIdx.x % kLanes;
+    const uint64_t job = static_cast<uint64_t>(blockIdx.x) * (kT / kLanes) + threadIdx.x / kLanes;
+    if (job >= rows * slices) return;  // whole waves (kLanes of 64) leave together; a workgroup of one job never does
+    const uint64_t row = job / slices;
+    const uint32_t slice = static_cast<uint32_t>(job % slices);
+    const RowSpan<F> r(in, row, len);
+    const uint32_t per_slice = (r.chunks + slices - 1) / slices;
+    const uint32_t begin = slice * per_slice;
+    const uint32_t end = begin + per_slice < r.chunks ? begin + per_slice : r.chunks;
+    float amax = slice == 0 ? r.template edges<kLanes>(lane) : 0.0f;
+    for (uint32_t c0 = begin + lane; c0 < end; c0 += kLanes * kUnroll) {
+        u32x4 raw[kUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kUnroll; u++) {
+            const uint32_t c = c0 + u * kLanes;
+            raw[u] = stream_load(r.body + (c < end ? c : end - 1));
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kUnroll; u++) amax = chunk_absmax<F>(raw[u], amax);
+    }
+    amax = group_max<64>(amax);
+    if constexpr (kLanes > kWave) {
+        __shared__ float wave_max[kLanes / kWave];
+        if (threadIdx.x % kWave == 0) wave_max[threadIdx.x / kWave] = amax;
+        __syncthreads();
+        amax = group_max<kLanes / kWave>(wave_max[threadIdx.x % (kLanes / kWave)]);
+    }
+    if (lane == 0) {
+        if constexpr (kPartial)
+            static_cast<float*>(out)[static_cast<uint64_t>(slice) * pitch + row] = amax;
+        else
+            F::store(out, row, amax);
+    }
+}
+
 // ---- rows, long: one wave per (row, slice) --------------------------------------
 // kPartial: write f32 partials [slice][row] with row pitch `pitch`; otherwise the
 // final value typed F.
@@ -153,17 +246,40 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_wave_kernel(const u32x4*
     }
 }
 
+// (Ragged rows, one wave or thread per output of single elements -> these kernels, us: axis 0 bf16 [43625, 2348] 386 -> 44.7,
+// [7995, 5226] 119 -> 20.6, f16 [120, 1553] 13.4 -> 3.7; axis 1 f16 [2996, 29565] 202 -> 29.8, f32 [6153, 15671] 133 -> 63.)
+// The chunks of kN columns along `inner`.  kRagged: `inner` is not a whole number of chunks, or the tensor does not start on
+// one: accesses of 16 bytes at any element (global memory takes them), and the last chunk lies over the one before it, so
+// that it ends with the row: its columns are reduced twice, to the same bits, and stored twice.
+template <class F, bool kRagged>
+struct ColumnChunks {
+    uint64_t row_bytes;
+    uint64_t at;  // bytes from a row's start to the lane's chunk
+    __device__ __forceinline__ ColumnChunks(uint64_t inner, uint64_t j) : row_bytes(inner * F::kBytes), at(j * 16) {
+        if (kRagged && at + 16 > row_bytes) at = row_bytes - 16;
+    }
+    __device__ __forceinline__ const char* rows(const void* in, uint64_t first) const { return static_cast<const char*>(in) + first * row_bytes + at; }
+    __device__ __forceinline__ const u32x4* row(const char* p, uint64_t l) const { return reinterpret_cast<const u32x4*>(p + l * row_bytes); }
+    __device__ __forceinline__ void store(char* outputs, u32x4 v) const {
+        if constexpr (kRagged)
+            __builtin_memcpy(outputs + at, &v, 16);
+        else
+            *reinterpret_cast<u32x4*>(outputs + at) = v;
+    }
+};
+
 // ---- columns, wide: one lane per (slice of L, outer, inner chunk) ---------------------
 // Writes one chunk typed F per lane: the result, or a partial [slice][output] (maxima are F numbers, so the partials lose
 // nothing in 16 bits, and their traffic, written and read again, is halved).
 // Bound by HBM; kColsUnroll loads of 16 bytes per lane in flight.  `per_slice`: rows_per_slice().
 constexpr int kColsUnroll = 8;
-template <class F>
+template <class F, bool kRagged>
 __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __restrict__ in, void* __restrict__ out,
-                                                               uint64_t outer, uint64_t len, uint64_t inner_chunks,
-                                                               uint32_t slices, uint64_t per_slice) {
+                                                               uint64_t outer, uint64_t len, uint64_t inner,
+                                                               uint32_t slices, uint64_t per_slice, uint64_t pitch) {
     constexpr int kN = F::kPerChunk;
     constexpr int kUnroll = kColsUnroll;
+    const uint64_t inner_chunks = (inner + kN - 1) / kN;
     const uint64_t cols = outer * inner_chunks;  // output chunks
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (t >= cols * slices) return;
@@ -172,7 +288,8 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
     const uint64_t o = col / inner_chunks, j = col % inner_chunks;
     const uint64_t begin = slice * per_slice;
     const uint64_t end = begin + per_slice < len ? begin + per_slice : len;
-    const u32x4* p = in + o * len * inner_chunks + j;
+    const ColumnChunks<F, kRagged> at(inner, j);
+    const char* p = at.rows(in, o * len);
     float amax[kN];
 #pragma unroll
     for (int i = 0; i < kN; i++) amax[i] = 0.0f;
@@ -181,7 +298,7 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
             const uint64_t l = l0 + u < end ? l0 + u : end - 1;
-            raw[u] = stream_load(p + l * inner_chunks);
+            raw[u] = stream_load(at.row(p, l));
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
@@ -191,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
             for (int i = 0; i < kN; i++) amax[i] = fmaxf(amax[i], fabsf(v[i]));
         }
     }
-    static_cast<u32x4*>(out)[static_cast<uint64_t>(slice) * cols + col] = F::pack(amax);  // values are F numbers: packing is exact
+    at.store(static_cast<char*>(out) + (static_cast<uint64_t>(slice) * pitch + o * inner) * F::kBytes, F::pack(amax));  // values are F numbers: packing is exact
 }
 
 // ---- columns, few outputs: one workgroup per (outer, column tile, slice of L) ----------
@@ -199,9 +316,9 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
 // (F32 when folding partials), FOut the type of the final result.
 enum TileOut { kTileFinalPacked = 0, kTilePartial = 1, kTileFinalChecked = 2 };
 
-template <class FIn, class FOut, int kCW, int kT, int kMode>
+template <class FIn, class FOut, int kCW, int kT, int kMode, bool kRagged>
 __global__ __launch_bounds__(kT) void reduce_tile_kernel(const u32x4* __restrict__ in, void* __restrict__ out,
-                                                         uint64_t len, uint64_t inner_chunks, uint32_t col_tiles,
+                                                         uint64_t len, uint64_t inner, uint32_t col_tiles,
                                                          uint32_t slices, uint64_t pitch, uint64_t count) {
     static_assert(kCW >= 1 && kCW <= kWave && kT % kWave == 0, "a tile row fits in one wave");
     constexpr int kN = FIn::kPerChunk;
@@ -219,7 +336,9 @@ __global__ __launch_bounds__(kT) void reduce_tile_kernel(const u32x4* __restrict
     const uint64_t per_slice = (len + slices - 1) / slices;
     const uint64_t begin = slice * per_slice;
     const uint64_t end = begin + per_slice < len ? begin + per_slice : len;
-    const u32x4* p = in + o * len * inner_chunks + (j < inner_chunks ? j : inner_chunks - 1);
+    const uint64_t inner_chunks = (inner + kN - 1) / kN;
+    const ColumnChunks<FIn, kRagged> at(inner, j < inner_chunks ? j : inner_chunks - 1);
+    const char* p = at.rows(in, o * len);
     float amax[kN];
 #pragma unroll
     for (int i = 0; i < kN; i++) amax[i] = 0.0f;
@@ -228,7 +347,7 @@ __global__ __launch_bounds__(kT) void reduce_tile_kernel(const u32x4* __restrict
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
             const uint64_t l = l0 + static_cast<uint64_t>(u) * kRH;
-            raw[u] = stream_load(p + (l < end ? l : end - 1) * inner_chunks);
+            raw[u] = stream_load(at.row(p, l < end ? l : end - 1));
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; u++) {
@@ -257,17 +376,17 @@ __global__ __launch_bounds__(kT) void reduce_tile_kernel(const u32x4* __restrict
 #pragma unroll
         for (int i = 0; i < kN; i++) amax[i] = fmaxf(amax[i], lds[w][cx][i]);
     }
-    const uint64_t col = o * inner_chunks + j;
+    const uint64_t first = o * inner + at.at / FIn::kBytes;  // output element of amax[0]
     if constexpr (kMode == kTilePartial) {
-        float* dst = static_cast<float*>(out) + static_cast<uint64_t>(slice) * pitch + col * kN;
+        float* dst = static_cast<float*>(out) + static_cast<uint64_t>(slice) * pitch + first;
 #pragma unroll
         for (int i = 0; i < kN; i++) dst[i] = amax[i];
     } else if constexpr (kMode == kTileFinalPacked) {
-        static_cast<u32x4*>(out)[col] = FOut::pack(amax);
+        at.store(static_cast<char*>(out) + o * inner * FOut::kBytes, FOut::pack(amax));
     } else {
 #pragma unroll
         for (int i = 0; i < kN; i++)
-            if (col * kN + i < count) FOut::store(out, col * kN + i, amax[i]);
+            if (first + i < count) FOut::store(out, first + i, amax[i]);
     }
 }
 
@@ -467,13 +586,33 @@ inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
 constexpr uint64_t kTargetGroups = 2048;
 constexpr uint64_t kTargetLanes = kTargetGroups * kThreads / 2;
 
-// Small tensors along an outer axis, one launch against two (two -> one, us): f32 [100, 4000] 8.9 -> 3.7, [512, 4096] 8.4 ->
-// 6.3, bf16 [700, 5600] 11.1 -> 6.2, [1000, 4096] 10.7 -> 7.7.  The lines: at 2^20 chunks it is even (f32 [500, 8192] 9.0 and
-// 9.1, [1000, 4096] 9.2 and 9.0; bf16 [500, 16384] 10.4 and 9.6); with 4096 rows the tiles are too few for their work (f16
-// [4096, 1024] 8.1 -> 17.6); and a tile's workgroup takes its place of 1024 lanes however few rows they share, so more of them
-// than are resident a few times over cost more than the second launch (1024 tiles: f32 [128, 16384] 8.0 -> 7.5; 2048 tiles:
-// [64, 32768] 7.8 -> 11.4, [100, 32768] 8.8 -> 12.2; 4096 tiles: [64, 65536] 8.4 -> 20.8).
-constexpr uint64_t kOneLaunchLen = 1024, kOneLaunchChunks = 1ull << 20, kOneLaunchTiles = 1024;
+// An outer axis in one launch of tiles (OneLaunch below) against slices and a fold.  A tile's lanes walk the whole axis, so
+// its workgroup lasts len * cw / (4 * 512) loads' latency; a second launch costs about 4 us.  (slices and fold -> one launch,
+// us; without a fold where the partials' bytes allowed one slice only, as in the first two.)
+//   f16 [115, 21256] 14.6 -> 4.1, bf16 [60, 30000] 8.7 -> 3.5, [337, 19272] 10.7 -> 6.2, [600, 8448] 10.5 -> 5.7, [1041, 9088]
+//   11.0 -> 6.8, [1036, 4835] 11.8 -> 8.3, f16 [391, 296] 6.3 -> 3.8, f32 [250, 32000] 9.9 -> 7.2, [83, 1184] 8.9 -> 3.0
+// Chunk columns per tile: a line of 128 bytes is eight of them, but fewer tiles than half of the compute units leave the
+// others idle: 605 columns 4 (bf16 [1036, 4835] 4, 8: 8.3, 9.9), 832 - 2048 columns 8 ([4093, 11008] 4, 8, 16: 38.5, 19.1,
+// 26.2), more 16 ([752, 19680] 4, 8, 16: 12.3, 11.1, 9.0).  512 lanes were the best or within 5 % of it throughout; up to 128
+// rows 256 of them start and end sooner (f32 [37, 15360] 3.2 -> 3.0).
+// The lines: past 1280 rows a tile's walk costs more than the fold (bf16 [1893, 1150] 8.6 -> 10.2, [2443, 4469] 12.2 -> 14.4,
+// [3726, 6656] 15.3 -> 19.1).  Where rows are whole lines no tile reads half of one, and the walk may be longer: [4093, 11008]
+// 20.5 -> 19.1, [3000, 16384] 21.6 -> 19.4, [2048, 32768] 27.3 -> 22.2; others of that size lose (f32 [1468, 29424] 31.4 ->
+// 33.9, bf16 [2874, 18205] 23.7 -> 29.7).  Fewer than eight rows are a loop of reduce_cols_kernel (f16 [5, 25600] 2.8 -> 3.1).
+struct OneLaunch {
+    bool take;
+    uint32_t cw;  // chunk columns per tile
+    uint64_t col_tiles;
+};
+inline OneLaunch one_launch(uint64_t outer, uint64_t len, uint64_t inner_chunks, bool whole_lines) {
+    const uint64_t cols = outer * inner_chunks;
+    const uint32_t cw = pow2_at_least(inner_chunks, cols >= 2200 ? 16 : cols >= 800 ? 8 : 4);
+    const uint64_t col_tiles = (inner_chunks + cw - 1) / cw;
+    const bool lines = whole_lines && cw >= 8;
+    const bool take = len >= 8 && outer * col_tiles <= 2048 &&
+                      (lines ? len <= 4096 && len * cw <= 32768 && cols * len <= (1ull << 23) : len <= 1280 && cols * len <= (1ull << 21));
+    return {take, cw, col_tiles};
+}
 
 // Rows per lane of reduce_cols_kernel with at most `most` slices over `cols` columns of chunks.  Its few workgroups all run
 // at once, so a launch lasts as long as the compute unit with the most of them: of two to four workgroups per compute unit
@@ -497,11 +636,19 @@ inline uint64_t rows_per_slice(uint64_t len, uint64_t cols, uint64_t most) {
     return best;
 }
 
+// Rows so few that they would be sliced, with a workgroup to each instead: one launch, no fold (sliced -> one launch, us):
+// f16 [6, 25952] 5.7 -> 3.2, f32 [237, 29888] 10.1 -> 6.6, [1500, 32768] 39.5 -> 32.4, bf16 [439, 5504] 6.9 -> 4.0, [500,
+// 131072] 26.8 -> 22.9.  Not where one workgroup would read for longer than the fold takes: bf16 [32, 131072] 6.1 -> 7.1,
+// [64, 2^20] 26.8 -> 45.0.  256 lanes up to 2048 chunks: of 1024 lanes with four loads each most would read a chunk again.
+inline bool block_per_row(uint64_t rows, uint64_t chunks) { return chunks <= 8192 || (chunks <= 16384 && rows >= 256); }
+constexpr uint64_t kNarrowBlockRowChunks = 2048;
+
 // How a contiguous [outer, len, inner] view is cut up; shared by the launcher and
 // by the workspace size query so that the two always agree.
 struct ReducePlan {
     enum Kind { kFallback, kRowsGrouped, kRowsWave, kCols, kTile } kind = kFallback;
-    uint64_t chunks_per_row = 0, inner_chunks = 0;
+    bool ragged = false;  // rows, or rows of columns, that are not whole chunks
+    uint64_t chunks_per_row = 0, inner_chunks = 0;  // ragged: whole chunks of a row; chunks that cover the columns
     uint32_t cw = 1, col_tiles = 1;
     uint64_t slices = 1;  // wanted; the launcher lowers it to what the workspace holds
     uint64_t lane_slices = 1;  // kTile on a strided input (one lane per output chunk and slice instead): wanted there
@@ -514,9 +661,11 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
     // a 16-bit tensor are twice as many in the same bytes)
     const uint64_t traffic_cap = len * (16 / kN) / 128 > 0 ? len * (16 / kN) / 128 : 1;
     if (len == 0 || outer == 0 || inner == 0) return p;
-    if (inner == 1 && len % kN == 0) {
+    p.ragged = (inner == 1 ? len : inner) % kN != 0;
+    if (inner == 1) {
+        if (len < 2 * kN && p.ragged) return p;
         p.chunks_per_row = len / kN;
-        if (p.chunks_per_row <= 64 && (p.chunks_per_row & (p.chunks_per_row - 1)) == 0) {
+        if (!p.ragged && p.chunks_per_row <= 64 && (p.chunks_per_row & (p.chunks_per_row - 1)) == 0) {
             p.kind = ReducePlan::kRowsGrouped;
             return p;
         }
@@ -530,12 +679,12 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
         }
         return p;
     }
-    if (inner % kN != 0) return p;
-    p.inner_chunks = inner / kN;
+    if (inner < kN) return p;
+    p.inner_chunks = (inner + kN - 1) / kN;
     const uint64_t cols = outer * p.inner_chunks;
     if (cols >= kTargetLanes || p.inner_chunks >= kThreads) {
         p.kind = ReducePlan::kCols;
-        p.pitch = outer * inner;
+        p.pitch = round_up(outer * inner, kN);
         if (cols < kTargetLanes) {
             p.slices = kTargetLanes / cols;
             const uint64_t max_slices = (len + 15) / 16;  // at least 16 rows per slice
@@ -551,7 +700,7 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
     if (p.lane_slices < 1) p.lane_slices = 1;
     p.cw = pow2_at_least(p.inner_chunks, kWave);
     p.col_tiles = static_cast<uint32_t>((p.inner_chunks + p.cw - 1) / p.cw);
-    p.pitch = outer * inner;  // a multiple of kN, hence of 4
+    p.pitch = round_up(outer * inner, kN);  // whole chunks of partials
     const uint64_t base = outer * p.col_tiles;
     if (base < kTargetGroups) {
         p.slices = kTargetGroups / base;
@@ -564,14 +713,16 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
 }
 
 template <class FIn, class FOut, int kT, int kMode>
-void launch_tile(hipStream_t s, uint32_t cw, uint64_t jobs, const void* in, void* out, uint64_t len,
-                 uint64_t inner_chunks, uint32_t col_tiles, uint32_t slices, uint64_t pitch, uint64_t count) {
+void launch_tile(hipStream_t s, bool ragged, uint32_t cw, uint64_t jobs, const void* in, void* out, uint64_t len,
+                 uint64_t inner, uint32_t col_tiles, uint32_t slices, uint64_t pitch, uint64_t count) {
     auto src = static_cast<const u32x4*>(in);
     dim3 grid(static_cast<uint32_t>(jobs));
-    switch (cw) {
-#define CQ_CASE(W) case W: hipLaunchKernelGGL((reduce_tile_kernel<FIn, FOut, W, kT, kMode>), grid, dim3(kT), 0, s, src, out, len, inner_chunks, col_tiles, slices, pitch, count); break;
+    switch (cw * 2 + (ragged ? 1 : 0)) {
+#define CQ_TILE(W, R) hipLaunchKernelGGL((reduce_tile_kernel<FIn, FOut, W, kT, kMode, R>), grid, dim3(kT), 0, s, src, out, len, inner, col_tiles, slices, pitch, count)
+#define CQ_CASE(W) case W * 2: CQ_TILE(W, false); break; case W * 2 + 1: if constexpr (kMode != kTileFinalChecked) CQ_TILE(W, true); break;
         CQ_CASE(1) CQ_CASE(2) CQ_CASE(4) CQ_CASE(8) CQ_CASE(16) CQ_CASE(32) CQ_CASE(64)
 #undef CQ_CASE
+#undef CQ_TILE
     }
 }
 
@@ -583,7 +734,7 @@ void launch_fold(hipStream_t s, const void* partials, void* out, uint64_t slices
     uint32_t cw = pow2_at_least(chunks, kWave);
     while (cw > 4 && chunks / cw < 128) cw /= 2;  // narrower tiles, more workgroups: the partials sit in L2
     const uint32_t tiles = static_cast<uint32_t>((chunks + cw - 1) / cw);
-    launch_tile<P, F, kFoldThreads, kTileFinalChecked>(s, cw, tiles, partials, out, slices, chunks, tiles, 1u, 0, count);
+    launch_tile<P, F, kFoldThreads, kTileFinalChecked>(s, false, cw, tiles, partials, out, slices, pitch, tiles, 1u, 0, count);
 }
 
 // The levels of a strided input with a contiguous last dimension of whole chunks, strides of whole words and
@@ -661,12 +812,19 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         }
     }
     ReducePlan p;
-    if (a.contiguous && (reinterpret_cast<uintptr_t>(a.input) & 15u) == 0) p = plan_reduce(a.outer, a.len, a.inner, kN);
+    if (a.contiguous && (reinterpret_cast<uintptr_t>(a.input) & (F::kBytes - 1)) == 0) {
+        p = plan_reduce(a.outer, a.len, a.inner, kN);
+        if ((reinterpret_cast<uintptr_t>(a.input) & 15u) != 0) {  // whole chunks, none of them aligned
+            p.ragged = true;
+            if (p.kind == ReducePlan::kRowsGrouped) p.kind = a.len < 2 * kN ? ReducePlan::kFallback : ReducePlan::kRowsWave;
+        }
+    }
     ReduceLevels levels;
     uint64_t len_stride = 0;
     if (!a.contiguous && a.out_contiguous && strided_levels<F>(a, &levels, &len_stride)) {
         // the plan of the contiguous tensor of this shape, with kernels that look up where rows and columns lie
         p = plan_reduce(a.outer, a.len, a.inner, kN);
+        if (p.ragged) p.kind = ReducePlan::kFallback;
         const bool rows = p.kind == ReducePlan::kRowsGrouped || p.kind == ReducePlan::kRowsWave;
         const bool cols = p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile;
         if ((rows && a.axis != a.rank - 1) || (cols && (a.axis == a.rank - 1 || (reinterpret_cast<uintptr_t>(a.output) & 15u) != 0)))
@@ -706,7 +864,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
             if (slices > 1) {
                 hipLaunchKernelGGL((reduce_cols_strided_kernel<F, true>), grid, dim3(kThreads), 0, s, in, a.workspace, levels,
                                    out_chunks, a.len, len_stride, static_cast<uint32_t>(slices));
-                launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
+                launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);  // whole chunks: no padding
             } else {
                 hipLaunchKernelGGL((reduce_cols_strided_kernel<F, false>), grid, dim3(kThreads), 0, s, in, a.output, levels,
                                    out_chunks, a.len, len_stride, 1u);
@@ -715,27 +873,26 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         }
         p = ReducePlan{};
     }
-    if ((p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) && (reinterpret_cast<uintptr_t>(a.output) & 15u) != 0)
-        p.kind = ReducePlan::kFallback;
+    if ((p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) && (reinterpret_cast<uintptr_t>(a.output) & 15u) != 0) {
+        p.ragged = true;  // the kernels whose stores need not be aligned either
+        if ((reinterpret_cast<uintptr_t>(a.output) & (F::kBytes - 1)) != 0) p.kind = ReducePlan::kFallback;
+    }
     uint64_t slices = p.slices;
     if (slices > 1) {
         const uint64_t fit = a.workspace == nullptr ? 0 : a.workspace_bytes / (p.pitch * sizeof(float));
         if (slices > fit) slices = fit > 1 ? fit : 1;
     }
-    // A small tensor in one launch: 1024 lanes per tile of up to four chunk columns, the whole axis.  The second launch that
-    // folds slices costs about 4 us, in which a tile's lanes read kOneLaunchLen rows.
-    const uint32_t cw = pow2_at_least(p.inner_chunks, 4);
-    const uint64_t col_tiles = (p.inner_chunks + cw - 1) / cw;
-    if ((p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) && slices > 1 && a.len <= kOneLaunchLen &&
-        a.outer * a.len * p.inner_chunks <= kOneLaunchChunks && a.outer * col_tiles <= kOneLaunchTiles) {
-        const dim3 grid(static_cast<uint32_t>(a.outer * col_tiles));
-        auto src = static_cast<const u32x4*>(a.input);
-        switch (cw) {
-#define CQ_CASE(W) case W: hipLaunchKernelGGL((reduce_tile_kernel<F, F, W, 1024, kTileFinalPacked>), grid, dim3(1024), 0, s, src, a.output, a.len, p.inner_chunks, static_cast<uint32_t>(col_tiles), 1u, 0ull, 0ull); break;
-            CQ_CASE(1) CQ_CASE(2) CQ_CASE(4)
-#undef CQ_CASE
+    if (p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) {
+        const OneLaunch one = one_launch(a.outer, a.len, p.inner_chunks, !p.ragged && a.inner * F::kBytes % 128 == 0);
+        if (one.take) {
+            const uint64_t tiles = a.outer * one.col_tiles;
+            const uint32_t col_tiles = static_cast<uint32_t>(one.col_tiles);
+            if (a.len <= 128)
+                launch_tile<F, F, 256, kTileFinalPacked>(s, p.ragged, one.cw, tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+            else
+                launch_tile<F, F, 512, kTileFinalPacked>(s, p.ragged, one.cw, tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+            return hipGetLastError();
         }
-        return hipGetLastError();
     }
     auto in = static_cast<const u32x4*>(a.input);
     switch (p.kind) {
@@ -752,6 +909,35 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         }
         case ReducePlan::kRowsWave: {
             dim3 grid = blocks(a.outer * slices, kThreads / kWave);
+            const uint32_t len = static_cast<uint32_t>(a.len);
+            if (p.slices > 1 && block_per_row(a.outer, p.chunks_per_row)) {
+                const dim3 rows(static_cast<uint32_t>(a.outer));
+                if (p.chunks_per_row <= kNarrowBlockRowChunks)
+                    hipLaunchKernelGGL((reduce_rows_span_kernel<F, 256, false>), rows, dim3(256), 0, s, a.input, a.output, a.outer, len, 1u, 0);
+                else
+                    hipLaunchKernelGGL((reduce_rows_span_kernel<F, 1024, false>), rows, dim3(1024), 0, s, a.input, a.output, a.outer, len, 1u, 0);
+                return hipGetLastError();
+            }
+            if (p.ragged) {
+                if (slices > 1) {
+                    hipLaunchKernelGGL((reduce_rows_span_kernel<F, kWave, true>), grid, dim3(kThreads), 0, s, a.input, a.workspace, a.outer,
+                                       len, static_cast<uint32_t>(slices), p.pitch);
+                    launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, a.outer);
+                } else if (p.chunks_per_row <= kWave * kRowLoads) {
+                    uint32_t lanes = row_lanes(p.chunks_per_row);
+                    if (lanes < 8) lanes = 8;
+                    const uint32_t loads = static_cast<uint32_t>((p.chunks_per_row + lanes - 1) / lanes);
+                    switch (lanes) {
+#define CQ_CASE(G) case G: hipLaunchKernelGGL((reduce_ragged_rows_lanes_kernel<F, G>), blocks(a.outer * G, kThreads), dim3(kThreads), 0, s, a.input, a.output, a.outer, len, loads); break;
+                        CQ_CASE(8) CQ_CASE(16) CQ_CASE(32) CQ_CASE(64)
+#undef CQ_CASE
+                    }
+                } else {
+                    hipLaunchKernelGGL((reduce_rows_span_kernel<F, kWave, false>), grid, dim3(kThreads), 0, s, a.input, a.output, a.outer, len,
+                                       1u, 0);
+                }
+                return hipGetLastError();
+            }
             if (slices <= 1 && p.chunks_per_row <= kWave * kRowLoads) {
                 const uint32_t lanes = row_lanes(p.chunks_per_row), loads = static_cast<uint32_t>((p.chunks_per_row + lanes - 1) / lanes);
                 switch (lanes) {
@@ -780,25 +966,24 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                 slices = (a.len + per_slice - 1) / per_slice;
             }
             const dim3 grid = blocks(a.outer * p.inner_chunks * slices, kThreads);
-            if (slices > 1) {
-                hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.workspace, a.outer, a.len,
-                                   p.inner_chunks, static_cast<uint32_t>(slices), per_slice);
-                launch_fold<F, F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
-            } else {
-                hipLaunchKernelGGL((reduce_cols_kernel<F>), grid, dim3(kThreads), 0, s, in, a.output, a.outer, a.len,
-                                   p.inner_chunks, 1u, per_slice);
-            }
+            void* const dst = slices > 1 ? a.workspace : a.output;
+            if (p.ragged)
+                hipLaunchKernelGGL((reduce_cols_kernel<F, true>), grid, dim3(kThreads), 0, s, in, dst, a.outer, a.len, a.inner,
+                                   static_cast<uint32_t>(slices), per_slice, p.pitch);
+            else
+                hipLaunchKernelGGL((reduce_cols_kernel<F, false>), grid, dim3(kThreads), 0, s, in, dst, a.outer, a.len, a.inner,
+                                   static_cast<uint32_t>(slices), per_slice, p.pitch);
+            if (slices > 1) launch_fold<F, F>(s, a.workspace, a.output, slices, p.pitch, a.outer * a.inner);
             return hipGetLastError();
         }
         case ReducePlan::kTile: {
             const uint64_t jobs = a.outer * p.col_tiles * slices;
+            const uint32_t n = static_cast<uint32_t>(slices);
             if (slices > 1) {
-                launch_tile<F, F, kThreads, kTilePartial>(s, p.cw, jobs, a.input, a.workspace, a.len, p.inner_chunks,
-                                                          p.col_tiles, static_cast<uint32_t>(slices), p.pitch, 0);
-                launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, p.pitch);
+                launch_tile<F, F, kThreads, kTilePartial>(s, p.ragged, p.cw, jobs, a.input, a.workspace, a.len, a.inner, p.col_tiles, n, p.pitch, 0);
+                launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, a.outer * a.inner);
             } else {
-                launch_tile<F, F, kThreads, kTileFinalPacked>(s, p.cw, jobs, a.input, a.output, a.len, p.inner_chunks,
-                                                              p.col_tiles, 1u, 0, 0);
+                launch_tile<F, F, kThreads, kTileFinalPacked>(s, p.ragged, p.cw, jobs, a.input, a.output, a.len, a.inner, p.col_tiles, 1u, 0, 0);
             }
             return hipGetLastError();
         }

@@ -88,6 +88,43 @@ def test_reduce_short_rows_and_small_outer_axes(gpu, oracle, elem):
             assert np.array_equal(got[:n_out].view(np.uint8), want.view(np.uint8)), (shape, axis, use_ws)
 
 
+@pytest.mark.parametrize("elem", ELEMS, ids=lambda e: e.name)
+def test_reduce_ragged_rows_and_columns(gpu, oracle, elem):
+    """Rows and rows of columns that are not whole 16-byte chunks, and whole ones in tensors that start one element behind
+    a chunk: every kernel's smallest and largest size and the ones beside them, with and without a workspace."""
+    import torch
+
+    rng = np.random.default_rng(int(elem) + 700)
+    n = 4 if elem == ElemType.F32 else 8
+    rows = [(1, 2 * n + 1), (3, 2 * n - 1), (257, 2 * n + 1), (300, 16 * n + n - 1), (70, 129), (4100, 512 * n + 1), (4100, 513 * n - 1),
+            (33, 513 * n + 1), (300, 2049 * n - 1), (7, 2049 * n + 1), (3, 8193 * n + 3), (2, 40000 * n + 1)]
+    cols = [(7, 3 * n + 1), (8, n + 1), (40, n - 1), (128, 2300 * n + 1), (129, 2200 * n - 1), (1280, 257 * n + 1), (1281, 300 * n + 3),
+            (4093, 256 * n + 1), (9000, n + 3), (5, 801 * n + 1), (1400, 832 * n)]
+    cases = [(shape, 1) for shape in rows] + [(shape, 0) for shape in cols] + [((3, 600, 41 * n + 1), 1), ((2, 3, 2 * n + 3), 0), ((5, 9, 3 * n + 1), 2)]
+    for shape, axis in cases:
+        size = 4 if elem == ElemType.F32 else 2
+        x32 = rng.normal(0, 2, shape).astype(np.float32)
+        x32[rng.random(shape) < 0.01] = np.nan
+        x32.reshape(-1)[-1] = np.inf if shape[0] % 2 else -0.0
+        x = oracle.to_bits(x32, elem)
+        want = oracle.reduce_max_abs(x, elem, shape, axis).reshape(-1)
+        out_shape = tuple(1 if d == axis else s for d, s in enumerate(shape))
+        for first_in, first_out in ((0, 0), (1, 0), (0, 1)):  # elements in front of the tensor and of its result
+            dx = gpu.to_dev(np.concatenate([np.zeros(first_in, x.dtype), x.reshape(-1)]))
+            dout = torch.zeros(want.size + 2, dtype=gpu.storage_dtype(elem), device="cuda")
+            hin = TensorHandleRef(dx.data_ptr() + first_in * size, shape, gpu.contiguous_strides(shape), size)
+            hout = TensorHandleRef(dout.data_ptr() + first_out * size, out_shape, gpu.contiguous_strides(out_shape), size)
+            nbytes = cq_reduce.workspace_bytes(hin, axis, elem)
+            for ws_bytes in (nbytes, 0):
+                dout.zero_()
+                ws = torch.full((max(nbytes, 16),), 0x7f, dtype=torch.uint8, device="cuda")
+                cq_reduce.max_abs(ComputeClient.current(), hin, hout, axis, elem, ws.data_ptr() if ws_bytes else 0, ws_bytes)
+                torch.cuda.synchronize()
+                got = gpu.to_host(dout)
+                assert np.array_equal(got[first_out:first_out + want.size].view(np.uint8), want.view(np.uint8)), (shape, axis, first_in, first_out, ws_bytes)
+                assert not got[:first_out].any() and not got[first_out + want.size:].any(), (shape, axis, "past the result")
+
+
 def test_reduce_strided_views_and_errors(gpu, oracle):
     import torch
 
