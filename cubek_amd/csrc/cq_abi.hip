@@ -1184,20 +1184,14 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
     const uint64_t chunk_elems = per_chunk > 32u / p.bits ? per_chunk : 32u / p.bits;
     const uint64_t flat_chunks = flat ? (p.n / chunk_elems) * chunk_elems / per_chunk : 0;
     if (p.tensor_level && flat_chunks > 0) {
-        // per tensor, two-pass grid reduction: pass 1 leaves one abs-max per workgroup in
+        // per tensor: large ones in one pass that keeps them on the chip; others by a two-pass grid reduction: pass 1 leaves one abs-max per workgroup in
         // the workspace; pass 2 (the quantize kernel) reduces those, derives the scale,
         // writes out_scale[0] and quantizes
         if (!workspace || workspace_bytes < cq::kMaxPartials * sizeof(float)) return CQ_ERR_WORKSPACE_TOO_SMALL;
         if (!aligned(workspace, 4)) return CQ_ERR_INVALID_ARGUMENT;
-        uint32_t num_partials = 0;
-        st = CQ_RUN_AUX(CQ_FAMILY_FLAT, cq::launch_absmax_partials(stream, input_dtype, input->ptr, p.n,
-                                                   static_cast<float*>(workspace), &num_partials));
-        if (st != CQ_OK) return st;
         cq::FlatArgs a{};
         a.input = input->ptr;
         a.output = output->ptr;
-        a.scale_in = workspace;
-        a.num_partials = num_partials;
         a.scale_out = out_scale->ptr;
         a.num_chunks = flat_chunks;
         a.lanes_only = wraps;
@@ -1205,7 +1199,17 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
         a.param_dtype = pd;
         a.encoding = flat_encoding(scheme);
         a.range = p.range;
-        st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_flat(stream, input_dtype, p.bits, cq::ScaleSource::Partials, a));
+        if (!wraps && cq::quantize_resident(static_cast<int>(p.bits), a)) {
+            st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_resident(stream, input_dtype, static_cast<int>(p.bits), a, p.n, workspace));
+        } else {
+            uint32_t num_partials = 0;
+            st = CQ_RUN_AUX(CQ_FAMILY_FLAT, cq::launch_absmax_partials(stream, input_dtype, input->ptr, p.n,
+                                                       static_cast<float*>(workspace), &num_partials));
+            if (st != CQ_OK) return st;
+            a.scale_in = workspace;
+            a.num_partials = num_partials;
+            st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_flat(stream, input_dtype, p.bits, cq::ScaleSource::Partials, a));
+        }
         if (st != CQ_OK) return st;
         flat_words = flat_chunks * per_chunk / p.nq;
     } else if (p.tensor_level && (flat_rows_ok(p, scheme, input_dtype, input, output, out_scale, dtype_size(pd), nullptr, 0, false, &fr) ||

@@ -559,6 +559,46 @@ __device__ __forceinline__ void quantize_pack_f16_tame(const float* x, float d, 
     }
 }
 
+// quantize_values_neg + pack_chunk_neg for a chunk of bf16 and a tame divisor.  The clamped quotients, rounded to bf16, are
+// f16 numbers too (8 of 11 significant bits; what is below the normal f16 range rounds to zero either way), and adding 1536
+// rounds two of them at a time to whole numbers, to the nearest even, in the low bits of the sums: 5.8 instructions per 8-bit
+// code against 7.5.
+template <int kBits>
+__device__ __forceinline__ void quantize_pack_bf16_tame(const float* x, float d, float lo, float hi, uint32_t* w) {
+    static_assert(kBits == 2 || kBits == 4 || kBits == 8, "2, 4 or 8 bits per value");
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const float nr = -__builtin_amdgcn_rcpf(d);
+    const float nhi = -hi, nlo = -lo;
+    float qn[8];  // negated
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const uint32_t p = BF16::pack2(neg_clamp_of_neg(x[i] * nr, nhi, nlo), neg_clamp_of_neg(x[i + 1] * nr, nhi, nlo));
+        qn[i] = bits_f32(p << 16);
+        qn[i + 1] = bits_f32(p & 0xffff0000u);
+    }
+    constexpr uint32_t kBias = kBits == 8 ? 0u : 1u << (kBits - 1);
+    constexpr _Float16 kMagic = static_cast<_Float16>(1536.0f + static_cast<float>(kBias));  // 0x6600 + kBias
+    const f16x2 magic = {kMagic, kMagic};
+    const auto codes = [&](int a, int b) { return __builtin_bit_cast(u16x2, magic - __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(qn[a], qn[b]))); };
+    if constexpr (kBits == 8) {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            w[j] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, codes(4 * j + 1, 4 * j + 3)),
+                                         __builtin_bit_cast(uint32_t, codes(4 * j, 4 * j + 2)), 0x06020400u);
+    } else {
+        // sums of biased fields, elements 0 - 3 in the low half and 4 - 7 in the high one; what the 0x6600 add up to is known
+        constexpr uint16_t kUp = 1u << kBits, kAll = static_cast<uint16_t>(0x6600u * (1u + kUp + kUp * kUp + kUp * kUp * kUp));
+        u16x2 sum = codes(3, 7);
+#pragma unroll
+        for (int k = 2; k >= 0; k--) sum = sum * u16x2{kUp, kUp} + codes(k, k + 4);
+        const uint32_t v = __builtin_bit_cast(uint32_t, sum - u16x2{kAll, kAll});
+        if constexpr (kBits == 4)
+            w[0] = v ^ field_bias<4>(32);
+        else
+            w[0] = ((v | (v >> 8)) & 0xffffu) ^ field_bias<2>(16);
+    }
+}
+
 // Sign-extended field i of a word (v_bfe_i32).
 template <int kBits>
 __device__ __forceinline__ float unpack_field(uint32_t w, int i) {

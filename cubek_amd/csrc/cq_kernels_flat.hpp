@@ -21,6 +21,7 @@
 #pragma once
 
 #include "cq_device.hpp"
+#include "cq_internal.hpp"
 #include "cq_magic_div.hpp"
 
 #ifndef CQ_WAVE_SCALES
@@ -28,6 +29,17 @@
 #endif
 
 namespace cq {
+
+constexpr uint64_t kKeepOutputBytes = 192ull << 20;  // QuantParams::keep: outputs up to this size
+inline QuantParams quant_params(const Range& r) {
+    QuantParams p;
+    p.lo = r.lo;
+    p.hi = r.hi;
+    p.width = r.hi - r.lo;
+    p.rwidth = 1.0f / p.width;  // IEEE division on the host: correctly rounded
+    p.unrounded = r.unrounded;
+    return p;
+}
 
 // Where a chunk's scale comes from.
 enum ScaleSrc : int {

@@ -270,17 +270,6 @@ LaneRows lane_rows_of_rows(const FlatArgs& a) {
     return r;
 }
 
-constexpr uint64_t kKeepOutputBytes = 192ull << 20;  // QuantParams::keep: outputs up to this size
-QuantParams quant_params(const Range& r) {
-    QuantParams p;
-    p.lo = r.lo;
-    p.hi = r.hi;
-    p.width = r.hi - r.lo;
-    p.rwidth = 1.0f / p.width;  // IEEE division on the host: correctly rounded
-    p.unrounded = r.unrounded;
-    return p;
-}
-
 // How a flat launch is cut up.  The kernels over whole tiles exist for f32 parameters (a contiguous run, or pitched
 // rows of whole steps) and for parameters typed like the float tensor, `f_dtype` (a contiguous run); everything else
 // is the lane-wise kernel's:

@@ -66,4 +66,13 @@ inline bool repack_stays(uint64_t bytes, bool whole_lines) {
     return !whole_lines || (bytes >= (32ull << 20) && bytes <= (96ull << 20));
 }
 
+// Whether a quantize with one scale per tensor keeps the tensor on the chip between its abs-max and its codes (one read,
+// cq_kernels_resident.hip) instead of reading it twice.  Below, its launch, its wait for the maxima of all workgroups and its
+// idle registers cost more than the second read, which the L2s and the Infinity Cache serve there.  Narrower codes have less to
+// write, and the arithmetic of the one pass, which nothing overlaps with, counts for more (two passes -> one, us): 8 bits of
+// bf16 48 MiB 23.3 -> 23.4, 64 MiB 30.9 -> 27.0, of f32 64 MiB 26.1 -> 24.6, e4m3 of f16 64 MiB 34.9 -> 33.6; 4 bits of bf16
+// 64 MiB 27.1 -> 27.7, 128 MiB 52.9 -> 48.5, of f32 64 MiB 24.3 -> 24.9, 128 MiB 46.3 -> 38.4; 2 bits of bf16 100 MiB 37.5 ->
+// 37.4, of f32 100 MiB 35.5 -> 32.7; e2m1 of bf16 100 MiB 41.3 -> 35.7.
+inline bool quantize_stays_resident(uint64_t chunks, int bits) { return chunks >= (bits == 8 ? 60ull << 16 : 96ull << 16); }
+
 }  // namespace cq

@@ -1,0 +1,154 @@
+"""One scale for a large tensor, quantized in one read of it (cq_kernels_resident.hip), against the two calls that share no
+kernel with it: compute_scales, then quantize with the given scale.  Codes and scale bit for bit."""
+import numpy as np
+import pytest
+
+from cubek_amd import ComputeClient, ElemType, QuantParam, QuantScheme, QuantStore, QuantValue, TensorHandleRef
+from cubek_amd import quantize as qz
+
+pytestmark = pytest.mark.gpu
+H = TensorHandleRef.from_torch
+ROUND = 512 * 256  # chunks that all workgroups read in a step each
+
+
+def dtype_of(torch, elem):
+    return {ElemType.F32: torch.float32, ElemType.F16: torch.float16, ElemType.BF16: torch.bfloat16}[elem]
+
+
+def scheme_of(value, store=QuantStore.U32, param=QuantParam.F32):
+    return QuantScheme.default().with_value(value).with_store(store).with_param(param)
+
+
+class Call:
+    """A tensor of `n` values and the two results: of the fused call and of the two calls."""
+
+    def __init__(self, torch, x, elem, scheme, fill=0xFF):
+        n = x.numel()
+        per = scheme.num_quants()
+        self.torch, self.x, self.elem, self.scheme = torch, x, elem, scheme
+        kind = torch.uint8 if scheme.store == QuantStore.Native else torch.int32
+        self.codes = torch.zeros(n // per + 4, dtype=kind, device="cuda")  # four more, which have to stay zero
+        self.shape = scheme.packed_shape((n,))
+        param = {QuantParam.F32: torch.float32, QuantParam.F16: torch.float16, QuantParam.BF16: torch.bfloat16}[scheme.param]
+        self.scale = torch.full((1,), -1.0, dtype=param, device="cuda")
+        self.ws = torch.full((1024,), fill, dtype=torch.uint8, device="cuda")
+
+    def fused(self):
+        qz.launch_dynamic(ComputeClient.current(), H(self.x), H(self.codes[:self.shape[0]]), H(self.scale), self.scheme, self.elem,
+                          self.ws.data_ptr(), 1024)
+
+    def check(self, what):
+        torch = self.torch
+        given = torch.zeros(1, dtype=self.x.dtype, device="cuda")
+        codes, scale, ws = torch.zeros_like(self.codes), torch.zeros_like(self.scale), torch.empty(1024, dtype=torch.uint8, device="cuda")
+        client = ComputeClient.current()
+        qz.compute_scales(client, H(self.x), H(given), self.scheme, self.elem, ws.data_ptr(), 1024)
+        qz.launch_ref(client, H(self.x), H(codes[:self.shape[0]]), H(given), H(scale), self.scheme, self.elem)
+        torch.cuda.synchronize()
+        assert torch.equal(self.scale.view(torch.uint8), scale.view(torch.uint8)), (what, self.scale, scale)
+        assert torch.equal(self.codes, codes), what
+
+
+def values(torch, n, elem, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(n, generator=gen, device="cuda") * 0.02).to(dtype_of(torch, elem))
+
+
+KINDS = [(QuantValue.Q8S, QuantStore.U32, 60), (QuantValue.Q8F, QuantStore.U32, 61), (QuantValue.E4M3, QuantStore.Native, 64),
+         (QuantValue.E5M2, QuantStore.Native, 65), (QuantValue.Q8S, QuantStore.Native, 48 + 13), (QuantValue.Q4S, QuantStore.U32, 96),
+         (QuantValue.Q4F, QuantStore.U32, 113), (QuantValue.Q2S, QuantStore.U32, 97), (QuantValue.E2M1, QuantStore.Native, 96),
+         (QuantValue.E2M1_OCP, QuantStore.U32, 96)]
+
+
+@pytest.mark.parametrize("elem", [ElemType.F32, ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
+@pytest.mark.parametrize("value,store,mib", KINDS, ids=lambda v: getattr(v, "name", str(v)))
+def test_every_kind_of_code(elem, value, store, mib):
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    scheme = scheme_of(value, store)
+    for chunks in (mib << 16, (mib << 16) + 4 * 77):  # whole rounds where the size is one; a cut step
+        call = Call(torch, values(torch, chunks * per, elem, int(value) + chunks), elem, scheme)
+        call.fused()
+        call.check((elem.name, value.name, store.name, chunks))
+
+
+# chunks: the fewest; on both sides of what registers, registers and LDS hold; one chunk in the last step; more than is held
+SIZES = [60 << 16, 47 * ROUND + 1, 48 * ROUND, 48 * ROUND + 5, 64 * ROUND - 511, 64 * ROUND, 64 * ROUND + 1, 65 * ROUND + 512, 72 * ROUND + 13, 81 * ROUND - 1]
+
+
+@pytest.mark.parametrize("elem,value,store,param", [(ElemType.BF16, QuantValue.Q8S, QuantStore.U32, QuantParam.F32),
+                                                    (ElemType.F16, QuantValue.E4M3, QuantStore.Native, QuantParam.F16),
+                                                    (ElemType.F32, QuantValue.Q8F, QuantStore.Native, QuantParam.BF16),
+                                                    (ElemType.BF16, QuantValue.Q8S, QuantStore.Native, QuantParam.F16)],
+                         ids=lambda v: getattr(v, "name", str(v)))
+def test_sizes_and_ends(elem, value, store, param):
+    """Every number of rounds that changes the kernel's way, with elements behind the last chunk (native store), the largest
+    value in the first, in the last and in a middle place, a workspace of any content."""
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    for i, chunks in enumerate(SIZES):
+        n = chunks * per + (3 if store == QuantStore.Native else 0)
+        x = values(torch, n, elem, i)
+        x[(0, n - 1, n // 2)[i % 3]] = -0.75
+        call = Call(torch, x, elem, scheme_of(value, store, param), fill=(0, 0x3F, 0x7F, 0xFF)[i % 4])
+        call.fused()
+        call.check((elem.name, chunks))
+        assert float(call.scale) > 0.001
+
+
+@pytest.mark.parametrize("elem", [ElemType.F32, ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
+def test_values_that_divide(elem):
+    """Zeros, an infinity, abs-maxima whose divisor is no ordinary number, NaN elements, every 16-bit pattern."""
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    n = ((60 << 16) + 7) * per
+    dt = dtype_of(torch, elem)
+    base = values(torch, n, elem, 5)
+    tiny = 2.0 ** -22 if elem == ElemType.F16 else 2.0 ** -124
+    variants = [torch.zeros(n, dtype=dt, device="cuda"), (base.float().sign() * tiny).to(dt), base.clone(), base.clone(), base.clone()]
+    variants[2][n // 3] = float("inf")
+    variants[3][::1001] = float("nan")
+    variants[3][n - 1] = float("nan")
+    if per == 8:
+        patterns = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(dt)
+        finite = torch.where(patterns.float().abs() < 3.0, patterns, torch.zeros_like(patterns))
+        variants[4][:65536] = finite
+        variants[4][n - 65536:] = finite
+    for i, x in enumerate(variants):
+        for value in (QuantValue.Q8S, QuantValue.Q8F):
+            call = Call(torch, x, elem, scheme_of(value))
+            call.fused()
+            call.check((elem.name, i, value.name))
+
+
+def test_streams_and_graphs():
+    """Launches on two streams at once, each with its workspace (their workgroups share the compute units, and none waits for
+    one that has not started), and a captured launch replayed on new values."""
+    import torch
+
+    n = (64 << 16) * 8
+    scheme = scheme_of(QuantValue.Q8S)
+    calls = [Call(torch, values(torch, n + 8 * 64 * i, ElemType.BF16, i), ElemType.BF16, scheme) for i in range(4)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for i, call in enumerate(calls):
+            with torch.cuda.stream(streams[i % 2]):
+                call.fused()
+    torch.cuda.synchronize()
+    for i, call in enumerate(calls):
+        call.check(i)
+    call, graph = calls[0], torch.cuda.CUDAGraph()
+    with torch.cuda.stream(streams[0]):
+        with torch.cuda.graph(graph, stream=streams[0]):
+            call.fused()
+    for seed in (7, 8, 9):
+        call.x.copy_(values(torch, n, ElemType.BF16, seed) * (seed - 6))
+        call.codes.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        call.check(seed)
