@@ -1184,9 +1184,9 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
     const uint64_t chunk_elems = per_chunk > 32u / p.bits ? per_chunk : 32u / p.bits;
     const uint64_t flat_chunks = flat ? (p.n / chunk_elems) * chunk_elems / per_chunk : 0;
     if (p.tensor_level && flat_chunks > 0) {
-        // per tensor: large ones in one pass that keeps them on the chip; others by a two-pass grid reduction: pass 1 leaves one abs-max per workgroup in
-        // the workspace; pass 2 (the quantize kernel) reduces those, derives the scale,
-        // writes out_scale[0] and quantizes
+        // per tensor: in one pass that keeps it on the chip, or by a two-pass grid reduction: pass 1 leaves one abs-max
+        // per workgroup in the workspace; pass 2 (the quantize kernel) reduces those, derives the scale, writes
+        // out_scale[0] and quantizes
         if (!workspace || workspace_bytes < cq::kMaxPartials * sizeof(float)) return CQ_ERR_WORKSPACE_TOO_SMALL;
         if (!aligned(workspace, 4)) return CQ_ERR_INVALID_ARGUMENT;
         cq::FlatArgs a{};
@@ -1199,8 +1199,9 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
         a.param_dtype = pd;
         a.encoding = flat_encoding(scheme);
         a.range = p.range;
-        if (!wraps && cq::quantize_resident(static_cast<int>(p.bits), a)) {
-            st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_resident(stream, input_dtype, static_cast<int>(p.bits), a, p.n, workspace));
+        const cq::ResidentWay way = wraps || g_probe.on ? cq::ResidentWay::kNone : cq::quantize_resident(stream, static_cast<int>(p.bits), a);
+        if (way != cq::ResidentWay::kNone) {
+            st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_resident(stream, way, input_dtype, static_cast<int>(p.bits), a, p.n, workspace));
         } else {
             uint32_t num_partials = 0;
             st = CQ_RUN_AUX(CQ_FAMILY_FLAT, cq::launch_absmax_partials(stream, input_dtype, input->ptr, p.n,

@@ -83,9 +83,11 @@ constexpr uint32_t kMaxPartials = 256;
 hipError_t launch_absmax_partials(hipStream_t s, int dtype, const void* input, uint64_t num_elems,
                                   float* partials, uint32_t* num_partials);
 // One scale per tensor in one read of it (cq_kernels_resident.hip): abs-max of `num_elems` elements, codes of a.num_chunks
-// chunks, out_scale[0].  `slots`: kMaxPartials words of workspace.  quantize_resident(): whether it is the faster way.
-bool quantize_resident(int bits, const FlatArgs& a);
-hipError_t launch_quantize_resident(hipStream_t s, int dtype, int bits, const FlatArgs& a, uint64_t num_elems, void* slots);
+// chunks, out_scale[0].  quantize_resident(): whether it is the faster way, and whether `slots` (kMaxPartials words of
+// workspace) are needed, as in a captured launch.
+enum class ResidentWay { kNone, kNumbered, kCaptured };
+ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& a);
+hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& a, uint64_t num_elems, void* slots);
 // Per-tensor scale from the partials: out_dtype(f_dtype(2*absmax/(hi-lo))) stored at out[0].
 hipError_t launch_tensor_scale(hipStream_t s, int f_dtype, int out_dtype, const float* partials,
                                uint32_t num_partials, Range range, void* out);

@@ -1,22 +1,28 @@
 // One scale for a whole contiguous tensor, quantized in one read of it: every workgroup keeps its share of the tensor in
 // registers and LDS while the abs-max of the others arrives.
 //
-// The two-pass quantize (absmax_partials_kernel, then quantize_flat_kernel) reads the tensor twice, and from 64 MB on the
-// second read comes from memory again.  The register files and the LDS of the 256 compute units hold 168 MiB.  A workgroup of 512
-// lanes with all 256 registers each fills one compute unit; it takes every 256th step of 512 chunks, loads up to 64 of
-// them at once (48 stay in registers, 16 in LDS: 128 MiB), publishes the abs-max of what it read, waits for the other
-// workgroups', and quantizes what it holds.  What a tensor has beyond that (its first steps) is read twice as before, in
-// loops in front of and behind the resident part.
+// The two-pass quantize (absmax_partials_kernel, then quantize_flat_kernel) reads the tensor twice, from 64 MB on both times from
+// memory, and is two launches, which for small tensors is all of its time.  The register files and the LDS of the 256 compute
+// units hold 168 MiB.  A workgroup of 512 lanes with all 256 registers each fills one compute unit; it takes every 256th step of
+// 512 chunks, loads up to 64 of them at once (48 stay in registers, 16 in LDS: 128 MiB), publishes the abs-max of what it read,
+// waits for the other workgroups', and quantizes what it holds.  What a tensor has beyond that (its first steps) is read twice
+// as before, in loops in front of and behind the resident part.  Up to 2 or 8 chunks per lane go through kernels of their own,
+// without loops, and up to 8 steps through one workgroup.
 //
-// Waiting.  A slot per workgroup holds its abs-max, or kUnset as the launch before this one leaves it.  No workgroup depends
+// Waiting.  A slot per workgroup holds the launch's number and the workgroup's abs-max; launches take turns at kRegions regions
+// of slots.  Numbers differ until 2^32 launches have gone by, and every launch writes all slots of its region, so what
+// a slot held before is never taken for this launch's.  A replay of a captured launch would bring the same number again:
+// captured launches have their slots in the caller's workspace, where a launch before them leaves kUnset.  No workgroup depends
 // on another one running: one that has waited for kPatience polls works out the missing shares itself, one by one, from
-// memory, and publishes them (the same bits, whoever does), so that it goes on after at most 256 of them whatever else
-// occupies the GPU, and workgroups that start late find everything there.
+// memory, and keeps them (the same bits, whoever does), so that it goes on after at most 256 of them whatever else
+// occupies the GPU and whoever takes its slots; it publishes them too, for workgroups that start late.
 //
-// Bound by its phases one after the other.  bf16 128 MiB to 8 bits, 41 us: 4 of the two launches, the read 19.5 (6.9 TB/s), 4
-// from the first published maximum to the last one seen, the arithmetic 11.5, which the stores overlap with (39.1 without
-// them).  Two passes -> one, us: bf16 8 bits 64 MiB 30.9 -> 27.0, 112 MiB 52.9 -> 37.2, 128 MiB 60.3 -> 41.2, 256 MiB 116 -> 98;
-// f32 8 bits 64 MiB 26.1 -> 24.6, 128 MiB 50.6 -> 37.4, 512 MiB 199 -> 181; f16 to e4m3 128 MiB 64.8 -> 50.3.
+// Bound by its phases one after the other.  bf16 128 MiB to 8 bits, 38 us: 2 of the launch, the read 19.5 (6.9 TB/s), 4
+// from the first published maximum to the last one seen, the arithmetic 11.5, which the stores overlap with.  Two passes -> one,
+// us: bf16 8 bits 32 KiB 5.6 -> 4.2, 1 MiB 5.9 -> 5.1, 4 MiB 6.3 -> 5.5, 16 MiB 8.7 -> 8.1, 64 MiB 25.0 -> 21.7, 112 MiB 50.6 -> 34.4,
+// 128 MiB 58.6 -> 38.0, 192 MiB 86.3 -> 66.5; f32 8 bits 64 MiB 22.3 -> 19.5, 128 MiB 45.4 -> 33.9; f16 to e4m3 128 MiB 60.1 -> 45.2.
+#include <atomic>
+
 #include "cq_internal.hpp"
 #include "cq_kernels_flat.hpp"
 #include "cq_launch_rules.hpp"
@@ -25,25 +31,31 @@ namespace cq {
 namespace {
 
 constexpr int kThreads = 512;
-constexpr uint32_t kGroups = 256;  // workgroups = slots
-static_assert(kGroups <= kMaxPartials, "the slots are the caller's workspace");
+constexpr uint32_t kGroups = 256;  // most workgroups = slots
+static_assert(kGroups <= kMaxPartials, "a captured launch's slots are the caller's workspace");
 constexpr uint32_t kUnset = 0xffffffffu;  // no abs-max: NaN elements are ignored
 constexpr uint32_t kPatience = 64;        // polls, about a microsecond each
 typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
 constexpr uint32_t kPerVector = 8;  // chunks
-constexpr uint32_t kInRegisters = 48, kInLds = 16, kResident = kInRegisters + kInLds;  // chunks per lane
+
+// Slots of launches outside a graph: regions of kGroups, taken in turn, so that up to kRegions launches at once have one
+// each.  A slot holds a launch's number beside an abs-max.
+constexpr uint32_t kRegions = 64;
+__device__ uint64_t g_slots[kRegions * kGroups];
 
 __global__ __launch_bounds__(kGroups) void unset_slots_kernel(uint32_t* __restrict__ slots) { slots[threadIdx.x] = kUnset; }
 
 struct ResidentArgs {
     const void* in;
     void* out;
-    uint32_t* slots;
+    uint32_t* slots;     // of a captured launch
     void* scale_out;
     uint64_t chunks;     // whole chunks that the launch quantizes
     uint64_t num_elems;  // elements of the tensor: the abs-max covers those behind the chunks too
-    uint32_t rounds;     // steps of the busiest workgroup
+    uint32_t groups;     // workgroups, a power of two
+    uint32_t rounds;     // steps of the busiest one
     uint32_t streamed;   // the first of them, read twice
+    uint32_t number;     // of the launch; 0: a captured one, with slots in the workspace
     int param_dtype;
     QuantParams qp;
 };
@@ -51,8 +63,10 @@ struct ResidentArgs {
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 constexpr int kAuxStream = 2, kAuxKeep = 17;  // nt; sc0 sc1 (output_store)
 
-template <class F, int kBits, int kEnc>
+// kInRegisters, kInLds: chunks that a lane keeps
+template <class F, int kBits, int kEnc, uint32_t kInRegisters, uint32_t kInLds>
 struct Resident {
+    static constexpr uint32_t kResident = kInRegisters + kInLds;
     static constexpr int kN = F::kPerChunk;
     static constexpr int kChunkBits = kN * kBits;
     const ResidentArgs& a;
@@ -62,8 +76,8 @@ struct Resident {
     struct Window {
         Rsrc in, out;
         __device__ __forceinline__ Window(const ResidentArgs& a, uint32_t first, uint32_t rounds) {
-            const uint64_t skip = static_cast<uint64_t>(first) * kRoundChunks, left = a.chunks > skip ? a.chunks - skip : 0;
-            const uint32_t most = rounds * kRoundChunks, n = left < most ? static_cast<uint32_t>(left) : most;
+            const uint64_t skip = static_cast<uint64_t>(first) * (a.groups * kThreads), left = a.chunks > skip ? a.chunks - skip : 0;
+            const uint32_t most = rounds * (a.groups * kThreads), n = left < most ? static_cast<uint32_t>(left) : most;
             in = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(a.in)) + skip * 16, 0, static_cast<int>(n * 16), 0x00027000);
             out = __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(a.out) + skip * kChunkBits / 8, 0, static_cast<int>(n * kChunkBits / 8), 0x00027000);
         }
@@ -71,8 +85,7 @@ struct Resident {
             return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(in, static_cast<int>(chunk * 16), 0, kAuxStream));
         }
     };
-    static constexpr uint32_t kRoundChunks = kGroups * kThreads;
-    __device__ __forceinline__ static uint32_t chunk_of(uint32_t group, uint32_t round) { return round * kRoundChunks + group * kThreads + threadIdx.x; }
+    __device__ __forceinline__ uint32_t chunk_of(uint32_t group, uint32_t round) const { return (round * a.groups + group) * kThreads + threadIdx.x; }
     // the chunks of rounds [first, first + kUnroll) before `end`, under way
     template <uint32_t kUnroll>
     struct Batch {
@@ -81,7 +94,7 @@ struct Resident {
         __device__ __forceinline__ Batch(const Resident& r, uint32_t group, uint32_t first, uint32_t end)
             : window(r.a, first, first < end ? (end - first < kUnroll ? end - first : kUnroll) : 0) {
 #pragma unroll
-            for (uint32_t u = 0; u < kUnroll; u++) raw[u] = window.load(chunk_of(group, u));
+            for (uint32_t u = 0; u < kUnroll; u++) raw[u] = window.load(r.chunk_of(group, u));
         }
     };
     __device__ __forceinline__ static float absmax(u32x4 raw, float acc) {
@@ -126,15 +139,29 @@ struct Resident {
         __syncthreads();
         return group_max<kThreads / kWave>(wave_max[threadIdx.x % (kThreads / kWave)]);
     }
+    // Slots behind those of the launch's workgroups are written too, so that no slot keeps a number until the count of
+    // launches comes round to it.
     __device__ __forceinline__ void publish(uint32_t group, float amax) const {
-        if (threadIdx.x == 0) __hip_atomic_store(a.slots + group, f32_bits(amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.number == 0) {
+            if (threadIdx.x == 0) __hip_atomic_store(a.slots + group, f32_bits(amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (threadIdx.x < kGroups && threadIdx.x % a.groups == group) {
+            const uint64_t slot = static_cast<uint64_t>(a.number) << 32 | f32_bits(amax);
+            __hip_atomic_store(region() + threadIdx.x, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    __device__ __forceinline__ uint64_t* region() const { return g_slots + a.number % kRegions * kGroups; }
+    __device__ __forceinline__ uint32_t poll(uint32_t group) const {
+        if (a.number == 0) return __hip_atomic_load(a.slots + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t slot = __hip_atomic_load(region() + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return slot >> 32 == a.number ? static_cast<uint32_t>(slot) : kUnset;
     }
     // the abs-max of all shares
     __device__ __forceinline__ float collect() const {
         __shared__ uint32_t missing;
-        uint32_t mine = 0;
+        __shared__ float found;
+        uint32_t mine = threadIdx.x < a.groups ? kUnset : 0;
         for (uint32_t polls = 0;; polls++) {
-            if (threadIdx.x < kGroups) mine = __hip_atomic_load(a.slots + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (mine == kUnset) mine = poll(threadIdx.x);
             if (!__syncthreads_or(mine == kUnset)) break;
             if (polls < kPatience) {
                 __builtin_amdgcn_s_sleep(2);
@@ -147,10 +174,14 @@ struct Resident {
             if (mine == kUnset) atomicMin(&missing, place);
             __syncthreads();
             const uint32_t share = (missing + blockIdx.x * 2) % kGroups;
-            publish(share, group_absmax(share_absmax(share)));
+            const float amax = group_absmax(share_absmax(share));
+            publish(share, amax);
+            // kept here as well: a launch kRegions later may have taken the slot
+            if (threadIdx.x == 0) found = amax;
             __syncthreads();
+            if (threadIdx.x == share) mine = f32_bits(found);
         }
-        return group_absmax(threadIdx.x < kGroups ? bits_f32(mine) : 0.0f);
+        return group_absmax(bits_f32(mine));
     }
     template <bool kTame>
     __device__ __forceinline__ void quantize(u32x4 raw, const Window& to, uint32_t chunk, float d) const {
@@ -191,9 +222,49 @@ struct Resident {
             now = next;
         }
     }
+    // the divisor, from the abs-max of what the workgroup read; block 0 stores the scale
+    __device__ __forceinline__ float divisor(float amax) const {
+        amax = group_absmax(amax);
+        if (a.groups > 1) {
+            publish(blockIdx.x, amax);
+            amax = collect();
+        }
+        // the scale as quantize_flat_body derives it
+        const float s_f = F::round(scale_from_absmax(amax, a.qp.width));
+        const bool fs_rounds = a.param_dtype != CQ_F32 && a.param_dtype != F::kDtype;
+        const float s_fs = fs_rounds ? round_to_dtype(a.param_dtype, s_f) : s_f;
+        if (blockIdx.x == 0 && threadIdx.x == 0) store_dtype(a.param_dtype, a.scale_out, 0, s_fs);
+        return fs_rounds ? F::round(s_fs) : s_f;
+    }
+    // divisions, for the divisors that need them: all of the share from memory again
+    __device__ __forceinline__ void quantize_exact(float d) const {
+#pragma unroll 1
+        for (uint32_t k = 0; k < a.rounds; k++) {
+            const Window again(a, k, 1);
+            quantize<false>(again.load(chunk_of(blockIdx.x, 0)), again, chunk_of(blockIdx.x, 0), d);
+        }
+    }
+    // few chunks
+    __device__ __forceinline__ void run_small() const {
+        const Window w(a, 0, kResident);
+        u32x4 raw[kInRegisters];
+#pragma unroll
+        for (uint32_t u = 0; u < kInRegisters; u++) raw[u] = w.load(chunk_of(blockIdx.x, u));
+        float amax = tail_absmax(blockIdx.x, 0.0f);
+#pragma unroll
+        for (uint32_t u = 0; u < kInRegisters; u++) amax = absmax(raw[u], amax);
+        const float d = divisor(amax);
+        if (!__builtin_amdgcn_readfirstlane(divisor_is_tame(d))) return quantize_exact(d);
+#pragma unroll
+        for (uint32_t u = 0; u < kInRegisters; u++) {
+            if (u >= a.rounds) break;
+            quantize<true>(raw[u], w, chunk_of(blockIdx.x, u), d);
+        }
+    }
     __device__ __forceinline__ void run() const {
         __shared__ u32x4 lds[kInLds][kThreads];
-        float amax = streamed_absmax(blockIdx.x, a.streamed, 0.0f);
+        float amax = 0.0f;
+        if (a.streamed) amax = streamed_absmax(blockIdx.x, a.streamed, amax);
         amax = tail_absmax(blockIdx.x, amax);
         const Window w(a, a.streamed, kResident);
         const uint32_t held = a.rounds - a.streamed;  // of the kResident chunks: the others read as zeros, and are skipped
@@ -208,8 +279,9 @@ struct Resident {
             for (uint32_t i = 0; i < 4; i++) kept[u / kPerVector][u % kPerVector * 4 + i] = raw[i];
         };
         const auto held_chunk = [&](uint32_t v, uint32_t u) { return u32x4{kept[v][u * 4], kept[v][u * 4 + 1], kept[v][u * 4 + 2], kept[v][u * 4 + 3]}; };
-        // the chunks for LDS come first, and the last registers are loaded in their place
-        {
+        // vectors that the share does not reach are not loaded; the chunks for LDS come first, and the last registers are loaded
+        // in their place
+        if (held > kInRegisters) {
             u32x4 raw[kInLds];
 #pragma unroll
             for (uint32_t u = 0; u < kInLds; u++) raw[u] = load(kInRegisters + u);
@@ -222,6 +294,14 @@ struct Resident {
                 hold(kInRegisters - kInLds + u, load(kInRegisters - kInLds + u));
                 __builtin_amdgcn_sched_barrier(0);
             }
+        } else {
+#pragma unroll
+            for (uint32_t v = 0; v < kInRegisters; v += kPerVector) {
+                if (v < held) {
+#pragma unroll
+                    for (uint32_t u = 0; u < kPerVector; u++) hold(v + u, load(v + u));
+                }
+            }
         }
 #pragma unroll
         for (uint32_t u = 0; u < kInRegisters; u += 4) {
@@ -231,22 +311,8 @@ struct Resident {
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        publish(blockIdx.x, group_absmax(amax));
-        amax = collect();
-        // the scale as quantize_flat_body derives it
-        const float s_f = F::round(scale_from_absmax(amax, a.qp.width));
-        const bool fs_rounds = a.param_dtype != CQ_F32 && a.param_dtype != F::kDtype;
-        const float s_fs = fs_rounds ? round_to_dtype(a.param_dtype, s_f) : s_f;
-        if (blockIdx.x == 0 && threadIdx.x == 0) store_dtype(a.param_dtype, a.scale_out, 0, s_fs);
-        const float d = fs_rounds ? F::round(s_fs) : s_f;
-        if (!__builtin_amdgcn_readfirstlane(divisor_is_tame(d))) {  // divisions: all of it from memory again
-#pragma unroll 1
-            for (uint32_t k = 0; k < a.rounds; k++) {
-                const Window again(a, k, 1);
-                quantize<false>(again.load(chunk_of(blockIdx.x, 0)), again, chunk_of(blockIdx.x, 0), d);
-            }
-            return;
-        }
+        const float d = divisor(amax);
+        if (!__builtin_amdgcn_readfirstlane(divisor_is_tame(d))) return quantize_exact(d);
         // a loop over the chunks of a vector, each picked by the vector index register: 48 copies of the code for one chunk
         // would take as long (bf16 128 MiB 41.2 and 42.4 us), in five times the bytes
 #pragma unroll
@@ -257,23 +323,35 @@ struct Resident {
         }
 #pragma unroll 1
         for (uint32_t u = 0; kInRegisters + u < held; u++) quantize<true>(lds[u][threadIdx.x], w, chunk_of(blockIdx.x, kInRegisters + u), d);
-        quantize_streamed(a.streamed, d);
+        if (a.streamed) quantize_streamed(a.streamed, d);
     }
 };
 
-template <class F, int kBits, int kEnc>
+constexpr uint32_t kFew = 2, kSome = 8, kMostRegisters = 48, kMostLds = 16;  // chunks per lane
+
+template <class F, int kBits, int kEnc, uint32_t kInRegisters, uint32_t kInLds>
 __global__ __launch_bounds__(kThreads, 2) void quantize_resident_kernel(ResidentArgs a) {
-    const Resident<F, kBits, kEnc> r{a};
-    r.run();
+    const Resident<F, kBits, kEnc, kInRegisters, kInLds> r{a};
+    if constexpr (kInLds == 0)
+        r.run_small();
+    else
+        r.run();
 }
 
 template <class F, int kBits, int kEnc>
 hipError_t launch(hipStream_t s, ResidentArgs a) {
     const uint64_t steps = (a.chunks + kThreads - 1) / kThreads;
-    a.rounds = static_cast<uint32_t>((steps + kGroups - 1) / kGroups);
-    a.streamed = a.rounds > kResident ? a.rounds - kResident : 0;
-    hipLaunchKernelGGL(unset_slots_kernel, dim3(1), dim3(kGroups), 0, s, a.slots);
-    hipLaunchKernelGGL((quantize_resident_kernel<F, kBits, kEnc>), dim3(kGroups), dim3(kThreads), 0, s, a);
+    a.groups = 1;
+    if (steps > kSome)  // up to there a workgroup alone has nothing to wait for
+        while (a.groups < kGroups && a.groups < steps) a.groups *= 2;
+    a.rounds = static_cast<uint32_t>((steps + a.groups - 1) / a.groups);
+    constexpr uint32_t kMost = kMostRegisters + kMostLds;
+    a.streamed = a.rounds > kMost ? a.rounds - kMost : 0;
+    if (a.number == 0) hipLaunchKernelGGL(unset_slots_kernel, dim3(1), dim3(kGroups), 0, s, a.slots);
+    const auto kernel = a.rounds <= kFew    ? quantize_resident_kernel<F, kBits, kEnc, kFew, 0>
+                        : a.rounds <= kSome ? quantize_resident_kernel<F, kBits, kEnc, kSome, 0>
+                                            : quantize_resident_kernel<F, kBits, kEnc, kMostRegisters, kMostLds>;
+    hipLaunchKernelGGL(kernel, dim3(a.groups), dim3(kThreads), 0, s, a);
     return hipGetLastError();
 }
 
@@ -296,14 +374,21 @@ hipError_t launch_encoding(hipStream_t s, int bits, int encoding, const Resident
 
 }  // namespace
 
-bool quantize_resident(int bits, const FlatArgs& f) {
-    if (!quantize_stays_resident(f.num_chunks, bits)) return false;
+ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& f) {
+    const bool captured_too = quantize_stays_resident(f.num_chunks, bits, true);
+    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, false)) return ResidentWay::kNone;
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
-    return hipGetDevice(&device) == hipSuccess && hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-           units >= static_cast<int>(kGroups);
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        units < static_cast<int>(kGroups))
+        return ResidentWay::kNone;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return ResidentWay::kNumbered;
+    (void)hipGetLastError();  // the default stream during another one's capture: an error, for the launch to report
+    return captured_too ? ResidentWay::kCaptured : ResidentWay::kNone;
 }
 
-hipError_t launch_quantize_resident(hipStream_t s, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {
+hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {
+    static std::atomic<uint32_t> launches{0};
     ResidentArgs a{};
     a.in = f.input;
     a.out = f.output;
@@ -313,6 +398,7 @@ hipError_t launch_quantize_resident(hipStream_t s, int dtype, int bits, const Fl
     a.num_elems = num_elems;
     a.param_dtype = f.param_dtype;
     a.qp = quant_params(f.range);
+    while (way == ResidentWay::kNumbered && a.number == 0) a.number = launches.fetch_add(1, std::memory_order_relaxed) + 1;
     switch (dtype) {
         case CQ_F32: return launch_encoding<F32>(s, bits, f.encoding, a);
         case CQ_BF16: return launch_encoding<BF16>(s, bits, f.encoding, a);

@@ -66,13 +66,21 @@ inline bool repack_stays(uint64_t bytes, bool whole_lines) {
     return !whole_lines || (bytes >= (32ull << 20) && bytes <= (96ull << 20));
 }
 
-// Whether a quantize with one scale per tensor keeps the tensor on the chip between its abs-max and its codes (one read,
-// cq_kernels_resident.hip) instead of reading it twice.  Below, its launch, its wait for the maxima of all workgroups and its
-// idle registers cost more than the second read, which the L2s and the Infinity Cache serve there.  Narrower codes have less to
-// write, and the arithmetic of the one pass, which nothing overlaps with, counts for more (two passes -> one, us): 8 bits of
-// bf16 48 MiB 23.3 -> 23.4, 64 MiB 30.9 -> 27.0, of f32 64 MiB 26.1 -> 24.6, e4m3 of f16 64 MiB 34.9 -> 33.6; 4 bits of bf16
-// 64 MiB 27.1 -> 27.7, 128 MiB 52.9 -> 48.5, of f32 64 MiB 24.3 -> 24.9, 128 MiB 46.3 -> 38.4; 2 bits of bf16 100 MiB 37.5 ->
-// 37.4, of f32 100 MiB 35.5 -> 32.7; e2m1 of bf16 100 MiB 41.3 -> 35.7.
-inline bool quantize_stays_resident(uint64_t chunks, int bits) { return chunks >= (bits == 8 ? 60ull << 16 : 96ull << 16); }
+// Whether a quantize with one scale per tensor keeps the tensor on the chip between its abs-max and its codes (one read and
+// one launch, cq_kernels_resident.hip) instead of reading it twice in two.  Small tensors gain the launch; from 8 chunks per lane
+// on (16 MiB) the larger kernel's phases, with idle registers between them, cost more than a second read that the
+// L2s and the Infinity Cache serve, until that read comes from memory again.  Narrower codes have less to write, and the arithmetic
+// of the one pass, which nothing overlaps with, counts for more.  Two passes -> one, us: 8 bits of bf16 8 MiB 6.5 -> 6.3, 16 MiB
+// 8.7 -> 8.1, 17 MiB 9.6 -> 9.6, 24 MiB 10.8 -> 10.9, 32 MiB 12.6 -> 12.7, 48 MiB 18.8 -> 17.3; of f32 16 MiB 8.0 -> 7.8, 32 MiB
+// 11.4 -> 11.7, 48 MiB 17.4 -> 15.7; 4 bits of bf16 16 MiB 8.6 -> 8.2, 24 MiB 10.8 -> 11.1, 48 MiB 17.8 -> 17.9, 60 MiB 22.1 -> 21.4;
+// e4m3 of f16 48 MiB 20.3 -> 20.1.
+//
+// Captured launches need one more in front, which marks their slots: from 60 MiB on (8 bits of bf16 48 MiB 23.3 -> 23.4,
+// 64 MiB 30.9 -> 27.0, of f32 64 MiB 26.1 -> 24.6), narrower codes from 96 MiB on (4 bits of bf16 64 MiB 27.1 -> 27.7, 128 MiB 52.9
+// -> 48.5, 2 bits of bf16 100 MiB 37.5 -> 37.4, of f32 100 MiB 35.5 -> 32.7, e2m1 of bf16 100 MiB 41.3 -> 35.7).
+inline bool quantize_stays_resident(uint64_t chunks, int bits, bool captured) {
+    if (captured) return chunks >= (bits == 8 ? 60ull << 16 : 96ull << 16);
+    return chunks <= 16ull << 16 || chunks >= (bits == 8 ? 48ull << 16 : 56ull << 16);
+}
 
 }  // namespace cq

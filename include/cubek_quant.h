@@ -19,8 +19,10 @@
  *     clamp() is max(lo, min(x, hi)) with minNum/maxNum, so a NaN quotient (NaN element, NaN scale, 0/0)
  *     quantizes to q_max; abs-max ignores NaN elements; a zero result keeps the sign IEEE gives it;
  *   - calls are re-entrant and thread safe.  The library's state is the per-thread code behind
- *     cq_last_hip_error() and, for cq_quantize_dynamic_static only, one scratch array per GPU inside the
- *     library's device code, shared by all calls of that entry point on that GPU (see there).
+ *     cq_last_hip_error(); one array per GPU inside the library's device code (128 KiB) through which the
+ *     workgroups of a launch exchange abs-maxima, with a count of such launches (launches at once, on any
+ *     streams, do not disturb one another's results); and, for cq_quantize_dynamic_static only, one scratch
+ *     array per GPU, shared by all calls of that entry point on that GPU (see there).
  */
 #ifndef CUBEK_QUANT_H
 #define CUBEK_QUANT_H

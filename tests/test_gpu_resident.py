@@ -1,4 +1,4 @@
-"""One scale for a large tensor, quantized in one read of it (cq_kernels_resident.hip), against the two calls that share no
+"""One scale for a tensor, quantized in one read of it (cq_kernels_resident.hip), against the two calls that share no
 kernel with it: compute_scales, then quantize with the given scale.  Codes and scale bit for bit."""
 import numpy as np
 import pytest
@@ -52,6 +52,62 @@ class Call:
 def values(torch, n, elem, seed):
     gen = torch.Generator(device="cuda").manual_seed(seed)
     return (torch.randn(n, generator=gen, device="cuda") * 0.02).to(dtype_of(torch, elem))
+
+
+# chunks: single words, a cut step, the most for one workgroup and one more, both ends of 2 and of 8 chunks per lane, and one
+# more than 8 (read twice); 48 MiB, where one read begins again for codes of 8 bits
+SMALL = [4, 8, 508, 512, 516, 8 * 512, 8 * 512 + 4, 33 * 512 + 8, 2 * ROUND, 2 * ROUND + 4, 8 * ROUND - 4, 8 * ROUND, 8 * ROUND + 4, 24 * ROUND]
+
+
+@pytest.mark.parametrize("elem", [ElemType.F32, ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
+@pytest.mark.parametrize("value,store", [(QuantValue.Q8S, QuantStore.U32), (QuantValue.Q4F, QuantStore.U32), (QuantValue.Q2S, QuantStore.U32),
+                                         (QuantValue.E4M3, QuantStore.Native), (QuantValue.E2M1, QuantStore.Native)],
+                         ids=lambda v: v.name)
+def test_small_sizes(elem, value, store):
+    """The sizes at which the kernel's way changes; elements behind the last chunk where codes are bytes."""
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    for i, chunks in enumerate(SMALL):
+        n = chunks * per + (3 if value == QuantValue.E4M3 else 0)
+        x = values(torch, n, elem, i)
+        x[(0, n - 1, n // 2)[i % 3]] = -0.75
+        call = Call(torch, x, elem, scheme_of(value, store, QuantParam(i % 3)), fill=(0, 0x7F, 0xFF)[i % 3])
+        call.fused()
+        call.check((elem.name, value.name, chunks))
+
+
+def test_many_small_launches():
+    """More launches than there are regions of slots, on four streams, each with its workspace; then
+    captured ones, replayed on new values between launches outside the graph."""
+    import torch
+
+    scheme = scheme_of(QuantValue.Q8S)
+    calls = [Call(torch, values(torch, 8 * (512 * (3 + i) + 4), ElemType.BF16, i) * (i + 1), ElemType.BF16, scheme) for i in range(100)]
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for i, call in enumerate(calls):
+            with torch.cuda.stream(streams[i % 4]):
+                call.fused()
+    torch.cuda.synchronize()
+    for i, call in enumerate(calls):
+        call.check(i)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(streams[0]):
+        with torch.cuda.graph(graph, stream=streams[0]):
+            for call in calls[:3]:
+                call.fused()
+    for seed in (7, 8, 9):
+        for i, call in enumerate(calls[:4]):
+            call.x.copy_(values(torch, call.x.numel(), ElemType.BF16, seed + i) * (seed - 6))
+            call.codes.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        calls[3].fused()
+        torch.cuda.synchronize()
+        for call in calls[:4]:
+            call.check(seed)
 
 
 KINDS = [(QuantValue.Q8S, QuantStore.U32, 60), (QuantValue.Q8F, QuantStore.U32, 61), (QuantValue.E4M3, QuantStore.Native, 64),
