@@ -82,7 +82,7 @@ uint32_t flat_family(const FlatArgs& a, int f_dtype);
 constexpr uint32_t kMaxPartials = 256;
 hipError_t launch_absmax_partials(hipStream_t s, int dtype, const void* input, uint64_t num_elems,
                                   float* partials, uint32_t* num_partials);
-// One scale per tensor in one read of it (cq_kernels_resident.hip): abs-max of `num_elems` elements, codes of a.num_chunks
+// One scale per tensor in one read of it (cq_kernels_resident.hpp): abs-max of `num_elems` elements, codes of a.num_chunks
 // chunks, out_scale[0].  quantize_resident(): whether it is the faster way, and whether `slots` (kMaxPartials words of
 // workspace) are needed, as in a captured launch.
 enum class ResidentWay { kNone, kNumbered, kCaptured };

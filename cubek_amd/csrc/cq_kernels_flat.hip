@@ -1,7 +1,9 @@
-// Launchers of the flat (contiguous) kernels: block scales, the per-tensor abs-max, and the dispatch of
+// Launchers of the flat (contiguous) kernels: block scales, the per-tensor abs-max, one scale in one read
+// (cq_kernels_resident.hpp), and the dispatch of
 // quantize and dequantize to the per-type launchers of cq_kernels_flat_quantize.hip and
 // cq_kernels_flat_dequantize.hip.
 #include "cq_kernels_flat_launch.hpp"
+#include "cq_kernels_resident.hpp"
 
 namespace cq {
 namespace {

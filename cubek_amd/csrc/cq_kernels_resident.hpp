@@ -21,6 +21,8 @@
 // from the first published maximum to the last one seen, the arithmetic 11.5, which the stores overlap with.  Two passes -> one,
 // us: bf16 8 bits 32 KiB 5.6 -> 4.2, 1 MiB 5.9 -> 5.1, 4 MiB 6.3 -> 5.5, 16 MiB 8.7 -> 8.1, 64 MiB 25.0 -> 21.7, 112 MiB 50.6 -> 34.4,
 // 128 MiB 58.6 -> 38.0, 192 MiB 86.3 -> 66.5; f32 8 bits 64 MiB 22.3 -> 19.5, 128 MiB 45.4 -> 33.9; f16 to e4m3 128 MiB 60.1 -> 45.2.
+#pragma once
+
 #include <atomic>
 
 #include "cq_internal.hpp"
@@ -28,7 +30,7 @@
 #include "cq_launch_rules.hpp"
 
 namespace cq {
-namespace {
+namespace resident {
 
 constexpr int kThreads = 512;
 constexpr uint32_t kGroups = 256;  // most workgroups = slots
@@ -41,7 +43,7 @@ constexpr uint32_t kPerVector = 8;  // chunks
 // Slots of launches outside a graph: regions of kGroups, taken in turn, so that up to kRegions launches at once have one
 // each.  A slot holds a launch's number beside an abs-max.
 constexpr uint32_t kRegions = 64;
-__device__ uint64_t g_slots[kRegions * kGroups];
+static __device__ uint64_t g_slots[kRegions * kGroups];
 
 __global__ __launch_bounds__(kGroups) void unset_slots_kernel(uint32_t* __restrict__ slots) { slots[threadIdx.x] = kUnset; }
 
@@ -372,14 +374,14 @@ hipError_t launch_encoding(hipStream_t s, int bits, int encoding, const Resident
     return hipErrorInvalidValue;
 }
 
-}  // namespace
+}  // namespace resident
 
 ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& f) {
     const bool captured_too = quantize_stays_resident(f.num_chunks, bits, true);
     if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, false)) return ResidentWay::kNone;
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        units < static_cast<int>(kGroups))
+        units < static_cast<int>(resident::kGroups))
         return ResidentWay::kNone;
     hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
     if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return ResidentWay::kNumbered;
@@ -389,7 +391,7 @@ ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& f) {
 
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {
     static std::atomic<uint32_t> launches{0};
-    ResidentArgs a{};
+    resident::ResidentArgs a{};
     a.in = f.input;
     a.out = f.output;
     a.slots = static_cast<uint32_t*>(slots);
@@ -400,9 +402,9 @@ hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, i
     a.qp = quant_params(f.range);
     while (way == ResidentWay::kNumbered && a.number == 0) a.number = launches.fetch_add(1, std::memory_order_relaxed) + 1;
     switch (dtype) {
-        case CQ_F32: return launch_encoding<F32>(s, bits, f.encoding, a);
-        case CQ_BF16: return launch_encoding<BF16>(s, bits, f.encoding, a);
-        case CQ_F16: return launch_encoding<F16>(s, bits, f.encoding, a);
+        case CQ_F32: return resident::launch_encoding<F32>(s, bits, f.encoding, a);
+        case CQ_BF16: return resident::launch_encoding<BF16>(s, bits, f.encoding, a);
+        case CQ_F16: return resident::launch_encoding<F16>(s, bits, f.encoding, a);
         default: return hipErrorInvalidValue;
     }
 }

@@ -67,7 +67,7 @@ inline bool repack_stays(uint64_t bytes, bool whole_lines) {
 }
 
 // Whether a quantize with one scale per tensor keeps the tensor on the chip between its abs-max and its codes (one read and
-// one launch, cq_kernels_resident.hip) instead of reading it twice in two.  Small tensors gain the launch; from 8 chunks per lane
+// one launch, cq_kernels_resident.hpp) instead of reading it twice in two.  Small tensors gain the launch; from 8 chunks per lane
 // on (16 MiB) the larger kernel's phases, with idle registers between them, cost more than a second read that the
 // L2s and the Infinity Cache serve, until that read comes from memory again.  Narrower codes have less to write, and the arithmetic
 // of the one pass, which nothing overlaps with, counts for more.  Two passes -> one, us: 8 bits of bf16 8 MiB 6.5 -> 6.3, 16 MiB

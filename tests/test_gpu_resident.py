@@ -1,4 +1,4 @@
-"""One scale for a tensor, quantized in one read of it (cq_kernels_resident.hip), against the two calls that share no
+"""One scale for a tensor, quantized in one read of it (cq_kernels_resident.hpp), against the two calls that share no
 kernel with it: compute_scales, then quantize with the given scale.  Codes and scale bit for bit."""
 import numpy as np
 import pytest
