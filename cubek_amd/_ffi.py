@@ -51,6 +51,7 @@ OK, ERR_INVALID_ARGUMENT, ERR_UNSUPPORTED_SCHEME, ERR_BLOCK_NOT_DIVISIBLE, ERR_S
     ERR_SCRATCH_TOO_SMALL = range(11)
 
 _lib = None
+_calls = None
 
 
 def lib() -> ctypes.CDLL:
@@ -102,6 +103,24 @@ def lib() -> ctypes.CDLL:
                                             ctypes.c_uint32]
     _lib = L
     return L
+
+
+def calls():
+    """The module of the package's calls (csrc/py_call.cpp): each takes the Python objects of a call and returns its status."""
+    global _calls
+    if _calls is None:
+        lib()
+        try:
+            from . import _call
+        except ImportError as e:
+            raise RuntimeError("native module not built: there is no fallback path. "
+                               "Build it with `make -C cubek_amd/csrc` (needs hipcc and Python's headers).") from e
+        from .scheme import QuantScheme
+        from .tensor import TensorHandleRef
+
+        _call.bind(TensorHandleRef, QuantScheme)
+        _calls = _call
+    return _calls
 
 
 def check(status: int) -> None:

@@ -4,7 +4,6 @@ Executed by gfx950 kernels behind the C ABI; the caller provides the output.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Sequence
 
 from . import _ffi
@@ -16,8 +15,6 @@ def into_contiguous_packed_ref(client: ComputeClient, input: TensorHandleRef, ou
     """``shape`` is the logical (unpacked) shape; ``input`` holds ``packing`` values per
     stored element along its rightmost stride-1 dimension, ``output`` is contiguous with
     the last dimension of ``shape`` divided by ``packing``."""
-    c_shape = (ctypes.c_uint64 * len(shape))(*shape)
-    rc = _ffi.lib().cq_into_contiguous_packed(client.stream, input.as_c(), output.as_c(), c_shape, len(shape),
-                                              packing)
+    rc = _ffi.calls().repack(client.stream, input, output, shape, packing)
     if rc:
         _ffi.check(rc)

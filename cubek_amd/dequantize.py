@@ -10,7 +10,6 @@ def launch_ref(client: ComputeClient, values: TensorHandleRef, output: TensorHan
                params: TensorHandleRef, scheme: QuantScheme, input_dtype: ElemType) -> None:
     """Convert the quantized ``values`` back to floats of type ``input_dtype``
     (the reference names the output float type ``input_dtype``)."""
-    rc = _ffi.lib().cq_dequantize(client.stream, values.as_c(), output.as_c(), params.as_c(),
-                                  scheme.to_c(), int(input_dtype))
+    rc = _ffi.calls().dequantize(client.stream, values, output, params, scheme, input_dtype)
     if rc:
         _ffi.check(rc)

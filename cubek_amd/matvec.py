@@ -12,7 +12,6 @@ def launch_ref(client: ComputeClient, values: TensorHandleRef, params: TensorHan
                x: TensorHandleRef, y: TensorHandleRef, elem: ElemType, y_elem: ElemType) -> None:
     """``values``: packed [rows, cols / num_quants]; ``params``: the scales; ``x``: [cols] of ``elem``;
     ``y``: [rows] of ``y_elem``.  Each weight enters as the value dequantize would store for ``elem``."""
-    rc = _ffi.lib().cq_gemv_quantized(client.stream, values.as_c(), params.as_c(), scheme.to_c(), x.as_c(), y.as_c(),
-                                      int(elem), int(y_elem))
+    rc = _ffi.calls().gemv(client.stream, values, params, scheme, x, y, elem, y_elem)
     if rc:
         _ffi.check(rc)

@@ -15,8 +15,7 @@ def launch_ref(client: ComputeClient, input: TensorHandleRef, output: TensorHand
                input_elem: ElemType) -> None:
     """Quantize ``input`` with the given ``scale`` tensor (typed like the input)
     into ``output`` and copy the scales, cast to ``scheme.param``, into ``out_scale``."""
-    rc = _ffi.lib().cq_quantize(client.stream, input.as_c(), output.as_c(), scale.as_c(), out_scale.as_c(),
-                                scheme.to_c(), int(input_elem))
+    rc = _ffi.calls().quantize(client.stream, input, output, scale, out_scale, scheme, input_elem)
     if rc:
         _ffi.check(rc)
 
@@ -30,8 +29,7 @@ def compute_scales(client: ComputeClient, input: TensorHandleRef, scales: Tensor
                    workspace_bytes: int = 0) -> None:
     """scale = 2*absmax/(q_max-q_min) per block or tensor, typed like the input
     (the rule of crates/cubek-quant/tests/suite/symmetric.rs:35-38,156-179)."""
-    rc = _ffi.lib().cq_compute_scales(client.stream, input.as_c(), scales.as_c(), scheme.to_c(),
-                                      int(input_elem), workspace, workspace_bytes)
+    rc = _ffi.calls().compute_scales(client.stream, input, scales, scheme, input_elem, workspace, workspace_bytes)
     if rc:
         _ffi.check(rc)
 
@@ -40,8 +38,8 @@ def launch_dynamic(client: ComputeClient, input: TensorHandleRef, output: Tensor
                    out_scale: TensorHandleRef, scheme: QuantScheme, input_elem: ElemType,
                    workspace: int = 0, workspace_bytes: int = 0) -> None:
     """Fused abs-max + scale + quantize; same results as compute_scales + launch_ref."""
-    rc = _ffi.lib().cq_quantize_dynamic(client.stream, input.as_c(), output.as_c(), out_scale.as_c(),
-                                        scheme.to_c(), int(input_elem), workspace, workspace_bytes)
+    rc = _ffi.calls().quantize_dynamic(client.stream, input, output, out_scale, scheme, input_elem, workspace,
+                                       workspace_bytes)
     if rc:
         _ffi.check(rc)
 
@@ -50,7 +48,6 @@ def launch_dynamic_static(client: ComputeClient, input: TensorHandleRef, output:
                           out_scale: TensorHandleRef, scheme: QuantScheme, input_elem: ElemType) -> None:
     """launch_dynamic for callers that cannot allocate a workspace: the scratch memory is an array
     inside the library (one per GPU, shared by all calls on that GPU)."""
-    rc = _ffi.lib().cq_quantize_dynamic_static(client.stream, input.as_c(), output.as_c(), out_scale.as_c(),
-                                               scheme.to_c(), int(input_elem))
+    rc = _ffi.calls().quantize_dynamic_static(client.stream, input, output, out_scale, scheme, input_elem)
     if rc:
         _ffi.check(rc)

@@ -19,7 +19,6 @@ def max_abs(client: ComputeClient, input: TensorHandleRef, output: TensorHandleR
     """``output`` has the input's shape with extent 1 on ``axis`` (else QuantError
     ERR_SHAPE_MISMATCH, the reference's ReduceError::MismatchShape; an axis >= rank
     gives ERR_INVALID_AXIS, its ReduceError::InvalidAxis)."""
-    rc = _ffi.lib().cq_reduce_max_abs(client.stream, input.as_c(), output.as_c(), axis, int(elem),
-                                      workspace, workspace_size)
+    rc = _ffi.calls().max_abs(client.stream, input, output, axis, elem, workspace, workspace_size)
     if rc:
         _ffi.check(rc)
