@@ -10,16 +10,20 @@ namespace {
 
 template <class F, int kGroup>
 hipError_t scales_launch(hipStream_t s, const FlatArgs& a) {
-    dim3 grid(grid_for(a.num_chunks, kUnrollQ)), block(kThreads);
+    dim3 block(kThreads);
     if (a.lanes.levels > 0) {
-        hipLaunchKernelGGL((scales_flat_lanes_kernel<F, kGroupRt, kUnrollQ, kThreads>), dim3(lanes_grid(a, kUnrollQ)), block, 0, s,
+        const bool one = a.rows * a.num_chunks < kSmallLaneChunks;
+        const auto kernel = one ? scales_flat_lanes_kernel<F, kGroupRt, 1, kThreads> : scales_flat_lanes_kernel<F, kGroupRt, kUnrollQ, kThreads>;
+        hipLaunchKernelGGL(kernel, dim3(lanes_grid(a, one ? 1 : kUnrollQ)), block, 0, s,
                            static_cast<const u32x4*>(a.input), a.scale_out, quant_params(a.range), with_group(lane_rows(a), kGroup));
     } else if (a.rows > 1) {
         const FlatRows rows = flat_rows(a);
         hipLaunchKernelGGL((scales_flat_rows_kernel<F, kGroup, kUnrollQ, kThreads>), dim3((rows.total_steps + kUnrollQ - 1) / kUnrollQ),
                            block, 0, s, static_cast<const u32x4*>(a.input), a.scale_out, quant_params(a.range), rows);
     } else {
-        hipLaunchKernelGGL((scales_flat_kernel<F, kGroup, kUnrollQ, kThreads>), grid, block, 0, s,
+        const bool one = a.num_chunks < kSmallRunChunks;
+        const auto kernel = one ? scales_flat_kernel<F, kGroup, 1, kThreads> : scales_flat_kernel<F, kGroup, kUnrollQ, kThreads>;
+        hipLaunchKernelGGL(kernel, dim3(grid_for(a.num_chunks, one ? 1 : kUnrollQ)), block, 0, s,
                            static_cast<const u32x4*>(a.input), a.scale_out, a.num_chunks,
                            quant_params(a.range));
     }

@@ -443,31 +443,38 @@ struct LaneSteps {
                                     : static_cast<char*>(g.scale_out) + scale_row * static_cast<uint32_t>(r.scale_out[0]);
                 continue;
             }
-            uint64_t in = 0, out = 0, scale_in = 0, scale_out = 0;
+            const auto walk = [&](auto zero) {  // offsets in the type of `zero`
+                using Offset = decltype(zero);
+                Offset in = 0, out = 0, scale_in = 0, scale_out = 0;
 #pragma unroll  // a loop over l would index the launch's arguments at run time, which sends all of them through scratch memory
-            for (int l = 0; l < kMaxLaneLevels; l++) {
-                if (l < static_cast<int>(r.levels)) {
-                    uint32_t index = row;
-                    if (l + 1 < static_cast<int>(r.levels)) {
-                        const uint32_t q = magic_div(row, r.magic[l], r.shift[l]);
-                        index = row - q * r.count[l];
-                        row = q;
+                for (int l = 0; l < kMaxLaneLevels; l++) {
+                    if (l < static_cast<int>(r.levels)) {
+                        uint32_t index = row;
+                        if (l + 1 < static_cast<int>(r.levels)) {
+                            const uint32_t q = magic_div(row, r.magic[l], r.shift[l]);
+                            index = row - q * r.count[l];
+                            row = q;
+                        }
+                        in += index * static_cast<Offset>(r.in[l]);
+                        out += index * static_cast<Offset>(r.out[l]);
+                        uint32_t scale_index = index;
+                        if (l == 0 && r.scale_rows > 1) {
+                            scale_index = magic_div(index, r.scale_magic, r.scale_shift);
+                            block_row_[u] = index == scale_index * r.scale_rows;
+                        }
+                        scale_in += scale_index * static_cast<Offset>(r.scale_in[l]);
+                        scale_out += scale_index * static_cast<Offset>(r.scale_out[l]);
                     }
-                    in += index * r.in[l];
-                    out += index * r.out[l];
-                    uint32_t scale_index = index;
-                    if (l == 0 && r.scale_rows > 1) {
-                        scale_index = magic_div(index, r.scale_magic, r.scale_shift);
-                        block_row_[u] = index == scale_index * r.scale_rows;
-                    }
-                    scale_in += scale_index * r.scale_in[l];
-                    scale_out += scale_index * r.scale_out[l];
                 }
-            }
-            in_[u] = static_cast<const char*>(g.in) + in;
-            out_[u] = static_cast<char*>(g.out) + out;
-            scale_in_[u] = static_cast<const char*>(g.scale_in) + scale_in;
-            scale_out_[u] = g.scale_out == nullptr ? nullptr : static_cast<char*>(g.scale_out) + scale_out;
+                in_[u] = static_cast<const char*>(g.in) + in;
+                out_[u] = static_cast<char*>(g.out) + out;
+                scale_in_[u] = static_cast<const char*>(g.scale_in) + scale_in;
+                scale_out_[u] = g.scale_out == nullptr ? nullptr : static_cast<char*>(g.scale_out) + scale_out;
+            };
+            if (r.narrow)
+                walk(uint32_t{0});
+            else
+                walk(uint64_t{0});
         }
     }
     __device__ __forceinline__ Index chunk(int u) const { return col_[u]; }

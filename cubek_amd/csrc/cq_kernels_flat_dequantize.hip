@@ -52,9 +52,10 @@ hipError_t dequantize_launch_enc(hipStream_t s, const FlatArgs& a) {
                                        a.num_chunks);
             }
         },
-        [&](const LaneRows& rows, uint32_t tile_begin, uint32_t grid, RunOffsets off) {
-            hipLaunchKernelGGL((dequantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), kU, kThreads, kEnc>), dim3(grid), dim3(kThreads), 0,
-                               s, reinterpret_cast<const uint32_t*>(in + off.chunks * kInChunk),
+        [&](const LaneRows& rows, uint32_t tile_begin, uint32_t grid, RunOffsets off, bool one) {
+            const auto kernel = one ? dequantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), 1, kThreads, kEnc>
+                                    : dequantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), kU, kThreads, kEnc>;
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, reinterpret_cast<const uint32_t*>(in + off.chunks * kInChunk),
                                reinterpret_cast<u32x4*>(out + off.chunks * 16),
                                static_cast<const char*>(a.scale_in) + off.chunks / div * param_bytes, a.param_dtype, tile_begin,
                                with_group(rows, kGroup, a.any_group));

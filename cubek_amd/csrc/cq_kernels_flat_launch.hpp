@@ -275,8 +275,8 @@ LaneRows lane_rows_of_rows(const FlatArgs& a) {
 // is the lane-wise kernel's:
 //   `whole(tiles, grid)`                       the run: `tiles` whole tiles and grid - tiles steps behind them; the first
 //                                              `tiles` tiles of the rows' steps (grid = tiles)
-//   `lanes(rows, tile_begin, grid, offsets)`   lane by lane; `offsets` = chunks / scales to advance the base
-//                                              pointers by (a contiguous run only)
+//   `lanes(rows, tile_begin, grid, offsets, one)`  lane by lane; `offsets` = chunks / scales to advance the base
+//                                              pointers by (a contiguous run only); `one`: tiles of one step
 struct RunOffsets {
     uint64_t chunks;  // 16-byte chunks of the float tensor
 };
@@ -286,6 +286,13 @@ struct RunOffsets {
 // 300 000 chunks 4.5 and 3.4, 5.6 and 4.5, 2.95 and 2.99, 6.3 and 6.1; 2^19 4.85 and 4.26, 6.0 and 5.8, 3.4 and 3.9, 7.4 and
 // 7.5.  One line for all four, where the dequantize has nothing to gain any more.
 constexpr uint64_t kSmallRunChunks = 1u << 18;
+// Lane by lane the same: tiles of one step, a chunk per lane, for launches of fewer chunks.  There a tile of four steps is a few
+// workgroups' serial work, every step with a walk of its own over the levels.  Quantize and dequantize, us, tiles of several steps
+// and of one: f16 [16, 8, 3, 128] behind permuted dimensions 8.3 and 5.2, 120 tokens 9.5 and 6.7, 250 (512 000 chunks) 10.4 and 9.7,
+// 500 14.3 and 14.2; 4 bits of bf16 [16, 8, 500, 80] (640 000) 13.5 and 12.4, 1200 tokens 19.2 and 19.4, [20, 4, 980, 128] 14.5 and
+// 15.0; runs of 4 bits, blocks of 16, [1024, 1024] 7.4 and 5.0, [4096, 1024] 9.5 and 8.0; of 8 bits, blocks of 24, [2048, 1536] 8.3
+// and 8.1, [4096, 1536] (786 432) 11.3 and 11.6.
+constexpr uint64_t kSmallLaneChunks = 3u << 18;
 template <class WholeFn, class LanesFn>
 hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole, LanesFn lanes) {
     const uint64_t tile = static_cast<uint64_t>(kThreads) * unroll;
@@ -293,7 +300,8 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
     const int group = group_of(f_dtype, a.block);
     hipError_t e = hipSuccess;
     if (a.lanes.levels > 0) {
-        lanes(lane_rows(a, unroll), 0u, lanes_grid(a, unroll), RunOffsets{0});
+        const bool one = a.rows * a.num_chunks < kSmallLaneChunks;
+        lanes(lane_rows(a, one ? 1 : unroll), 0u, lanes_grid(a, one ? 1 : unroll), RunOffsets{0}, one);
         return hipGetLastError();
     }
     if (a.rows > 1) {
@@ -307,7 +315,8 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         if (full < tiles) {
-            lanes(lr, full, tiles - full, RunOffsets{0});
+            const bool one = full == 0 && lr.total_chunks < kSmallLaneChunks;
+            lanes(lr, full, one ? grid_for(lr.total_chunks, 1) : tiles - full, RunOffsets{0}, one);
             e = hipGetLastError();
         }
         return e;
@@ -324,7 +333,8 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
     const uint64_t piece = a.any_group == 0 ? (1ull << 30) : (1ull << 30) / (4ull * a.any_group) * (4ull * a.any_group);
     for (uint64_t begin = 0; begin < a.num_chunks; begin += piece) {
         const uint64_t n = a.num_chunks - begin < piece ? a.num_chunks - begin : piece;
-        lanes(lane_rows_of_run(n), 0u, static_cast<uint32_t>((n + tile - 1) / tile), RunOffsets{begin});
+        const bool one = n < kSmallLaneChunks;
+        lanes(lane_rows_of_run(n), 0u, grid_for(n, one ? 1 : unroll), RunOffsets{begin}, one);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return e;
@@ -390,12 +400,13 @@ hipError_t quantize_launch_src(hipStream_t s, ScaleSource src, const FlatArgs& a
                     }
                 }
             },
-            [&](const LaneRows& rows, uint32_t tile_begin, uint32_t grid, RunOffsets off) {
+            [&](const LaneRows& rows, uint32_t tile_begin, uint32_t grid, RunOffsets off, bool one) {
                 const uint64_t scales = off.chunks / div;
                 const void* scale_in = a.scale_in == nullptr ? nullptr : static_cast<const char*>(a.scale_in) + scales * scale_in_bytes;
                 void* scale_out = a.scale_out == nullptr ? nullptr : static_cast<char*>(a.scale_out) + scales * scale_out_bytes;
-                hipLaunchKernelGGL((quantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), kSrc, kWide, kUnrollQ, kThreads, kEnc>),
-                                   dim3(grid), dim3(kThreads), 0, s, reinterpret_cast<const u32x4*>(in + off.chunks * 16),
+                const auto kernel = one ? quantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), kSrc, kWide, 1, kThreads, kEnc>
+                                        : quantize_flat_lanes_kernel<F, kBits, lanes_group(kGroup), kSrc, kWide, kUnrollQ, kThreads, kEnc>;
+                hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, reinterpret_cast<const u32x4*>(in + off.chunks * 16),
                                    reinterpret_cast<uint32_t*>(out + off.chunks * kOutChunk), scale_in, scale_out,
                                    a.param_dtype, qp, a.num_partials, tile_begin, with_group(rows, kGroup, a.any_group));
             });
