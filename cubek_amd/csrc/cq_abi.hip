@@ -1140,11 +1140,14 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
 
     // blocks over the last two dimensions (or 1-D blocks on layouts the flat kernel refuses): one
     // launch that owns whole blocks
-    // Blocks of 8 - 64 rows on rows of at most 1 KiB leave the fused block kernel too few lanes along the row
+    // Blocks of 8 - 64 rows, not all powers of two, on rows of at most 1 KiB leave the fused block kernel too few lanes along the row
     // (18 - 35 % of HBM peak).  Two launches take half the time there: the blocks' scales as FS(F(scale)) into
     // out_scale, then the flat body, lane by lane, reading them back (the divisor F(FS(scale)) is the same either way).
+    cq::RowArgs rb;
+    const bool blocks = !wraps && !p.tensor_level && scales_rows_ok(p) && rows_args(p, scheme, input_dtype, input, output, &rb) &&
+                        cq::blocks_dynamic_supported(input_dtype, static_cast<int>(p.bits), rb);
     if (!p.tensor_level && p.rank >= 2 && scales_rows_ok(p) && p.layout.block[p.rank - 2] >= 8 && p.layout.block[p.rank - 2] <= 64 &&
-        p.shape[p.rank - 1] * dtype_size(input_dtype) <= 1024) {
+        p.shape[p.rank - 1] * dtype_size(input_dtype) <= 1024 && !(blocks && cq::block_tiles_supported(input_dtype, static_cast<int>(p.bits), rb))) {
         cq::FlatArgs f2{};
         if (lane_rows_ok(p, scheme, input_dtype, input, output, out_scale, dtype_size(pd), nullptr, 0, true, &f2)) {
             st = produce_scales(stream, p, scheme, input, input_dtype, out_scale, pd, workspace, workspace_bytes);
@@ -1161,9 +1164,7 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
         }
     }
 
-    cq::RowArgs rb;
-    if (!wraps && !p.tensor_level && scales_rows_ok(p) && rows_args(p, scheme, input_dtype, input, output, &rb) &&
-        cq::blocks_dynamic_supported(input_dtype, static_cast<int>(p.bits), rb)) {
+    if (blocks) {
         rb.input = input->ptr;
         rb.output = output->ptr;
         rb.scale_out = out_scale->ptr;

@@ -269,6 +269,7 @@ struct QuantParams {
     uint32_t keep = 0;    // the flat quantize kernels: codes leave through output_store(keep = true): they stay in the
                           // Infinity Cache for the kernel that reads them next
 };
+constexpr uint64_t kKeepOutputBytes = 192ull << 20;  // QuantParams::keep: outputs up to this size
 // A store that streams past the caches, or one that is written through the L2 at system scope (sc0 sc1): it leaves
 // no dirty line behind in the L2, as a plain store would (which costs the launch 4 - 8 %), but unlike the streaming
 // store it leaves the data in the memory-side Infinity Cache.  `keep` is the same for the whole launch: a scalar

@@ -30,7 +30,6 @@
 
 namespace cq {
 
-constexpr uint64_t kKeepOutputBytes = 192ull << 20;  // QuantParams::keep: outputs up to this size
 inline QuantParams quant_params(const Range& r) {
     QuantParams p;
     p.lo = r.lo;

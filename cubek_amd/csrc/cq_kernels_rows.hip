@@ -15,6 +15,7 @@
 //   quantize_rows_kernel / dequantize_rows_kernel   scales given / stored
 //   scales_rows_kernel        abs-max of BR x BC blocks -> scales
 //   quantize_blocks_kernel    abs-max + scale + quantize of BR x BC blocks in one launch
+//   quantize_block_tiles_kernel  the same for blocks of powers of two
 //   absmax_rows_kernel        per-tensor abs-max partials over strided rows
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
@@ -23,6 +24,7 @@ namespace cq {
 namespace {
 
 constexpr int kThreads = 256;
+bool aligned8(const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; }
 
 template <class F, int kBits>
 struct Unit {
@@ -381,6 +383,118 @@ __global__ __launch_bounds__(kThreads) void quantize_blocks_kernel(RowArgs a, Bl
     }
 }
 
+// The same for blocks of a power of two of rows and of chunk columns, which a workgroup holds whole: 2^tj_log2 lanes along the
+// row (whole blocks), kT >> tj_log2 rows at a time, kR times.  BlockTilesGeom comes with nothing to divide by, a block's lanes
+// in a wave meet by DPP and shuffles, its waves in one step through LDS.
+// quantize_blocks_kernel spends small launches on divisions and on a walk over the block's phases in LDS one by one, and large ones
+// on column bounds and 8 - 16 chunks per lane; here 2 or 4 chunks a lane leave more waves to hide the loads, and codes stay in the
+// caches for their reader (QuantParams::keep).  Bound by HBM where it is large.  Quantize and dequantize, us, old -> this: e4m3 of
+// bf16 [14336, 4096], 128 x 128 64.4 -> 54.6 (its bytes at a copy's rate 57.8), [512, 2048] 9.4 -> 6.6; 8 bits, 32 x 32 [2048, 4096]
+// 14.4 -> 12.1, [128, 512] (two launches) 10.6 -> 5.3, f32 64 x 64 [14336, 4096] 97.5 -> 89.8, 4 bits of f16, 64 x 64 [65536, 512]
+// 47.8 -> 31.8.  Also faster where the last tile of a row is a quarter full: bf16 [65536, 288] 32.5 -> 24.5.
+struct BlockTilesGeom {
+    uint32_t tj_log2, cpb_log2, chunks_per_row;
+    uint32_t pairs;  // codes on 8-byte boundaries: chunks of two words are stored at once
+};
+
+template <class F, int kBits, int kEnc, int kT, int kR>
+__global__ __launch_bounds__(kT) void quantize_block_tiles_kernel(RowArgs a, BlockTilesGeom g, QuantParams qp) {
+    constexpr int kN = F::kPerChunk;
+    constexpr int kChunkBits = kN * kBits;
+    constexpr uint32_t kWaves = kT / kWave;
+    __shared__ float met[kWaves][kWave];
+    const int last = static_cast<int>(a.rank) - 1;
+    const uint32_t tj = 1u << g.tj_log2, rows_at_once = kT >> g.tj_log2;
+    const uint32_t row = threadIdx.x >> g.tj_log2, jl = threadIdx.x & (tj - 1);
+    const uint32_t jc = blockIdx.x * tj + jl;
+    const bool live = jc < g.chunks_per_row;  // the same for every lane of a block and of a word
+    const uint32_t from = live ? jc : g.chunks_per_row - 1;
+    RowPos pos{};
+    if (a.rank == 2) {
+        const uint64_t first = static_cast<uint64_t>(blockIdx.y) * (rows_at_once * kR);
+        pos.f = first * a.fstride[0];
+        pos.v = first * a.vstride[0];
+        pos.sb = blockIdx.y * a.sb[0];
+    } else {
+        pos = row_pos(a, blockIdx.y * (rows_at_once * kR));
+    }
+    const uint64_t pitch_f = a.fstride[last - 1] / kN, pitch_v = a.vstride[last - 1];
+    const u32x4* at = static_cast<const u32x4*>(a.input) + pos.f / kN + row * pitch_f + from;
+    u32x4 raw[kR];
+#pragma unroll
+    for (int k = 0; k < kR; k++) raw[k] = stream_load(at + k * (rows_at_once * pitch_f));
+    __builtin_amdgcn_sched_barrier(0);
+    float amax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kR; k++) {
+        float v[kN];
+        F::unpack(raw[k], v);
+#pragma unroll
+        for (int i = 0; i < kN; i++) amax = fmaxf(amax, fabsf(v[i]));  // NaN elements drop out
+    }
+    amax = group_max_rt(amax, g.cpb_log2);
+    if (g.tj_log2 <= 4) amax = fmaxf(amax, __shfl_xor(amax, 16, kWave));
+    if (g.tj_log2 <= 5) amax = fmaxf(amax, __shfl_xor(amax, 32, kWave));
+    const uint32_t block = jl >> g.cpb_log2;
+    if (threadIdx.x % kWave < tj) met[threadIdx.x / kWave][block] = amax;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; w++) amax = fmaxf(amax, met[w][block]);
+    const float s32 = absmax_is_tame(amax) ? scale_from_absmax_tame(amax, qp) : scale_from_absmax(amax, qp.width);
+    const float s_fs = round_to_dtype(a.param_dtype, F::round(s32));
+    if (live && row == 0 && (jl & ((1u << g.cpb_log2) - 1u)) == 0)
+        store_dtype(a.param_dtype, a.scale_out, pos.sb + static_cast<uint64_t>(jc >> g.cpb_log2) * a.sb[last], s_fs);
+    const float d = F::round(s_fs);
+    const bool tame = divisor_is_tame(d);
+    const bool keep = qp.keep != 0;
+    uint32_t* dst = static_cast<uint32_t*>(a.output) + pos.v + row * pitch_v;
+#pragma unroll
+    for (int k = 0; k < kR; k++, dst += rows_at_once * pitch_v) {
+        float v[kN];
+        F::unpack(raw[k], v);
+        uint32_t w[2] = {0, 0};
+        const auto by_value = [&](bool d_tame) {
+            float qn[kN];
+            quantize_codes<F, kN, kEnc>(v, d, d_tame, qp.lo, qp.hi, qp.unrounded != 0, qn);
+            if constexpr (kEnc == kEncInt)
+                pack_chunk_neg<kBits, kN, false>(qn, w);
+            else
+                encode_chunk<kEnc, kN>(qn, w);
+        };
+        if constexpr (kEnc == kEncInt && F::kDtype == CQ_F16) {
+            if (tame)
+                quantize_pack_f16_tame<kBits>(v, d, qp.lo, qp.hi, w);
+            else
+                by_value(false);
+        } else if constexpr (kEnc == kEncInt && F::kDtype == CQ_BF16) {
+            if (tame)
+                quantize_pack_bf16_tame<kBits>(v, d, qp.lo, qp.hi, w);
+            else
+                by_value(false);
+        } else {
+            by_value(tame);
+        }
+        if constexpr (kChunkBits == 64) {
+            uint32_t* const p = dst + 2 * static_cast<uint64_t>(jc);
+            if (!live) continue;
+            if (g.pairs) {
+                output_store(keep, u32x2{w[0], w[1]}, reinterpret_cast<u32x2*>(p));
+            } else {
+                output_store(keep, w[0], p);
+                output_store(keep, w[1], p + 1);
+            }
+        } else if constexpr (kChunkBits == 32) {
+            if (live) output_store(keep, w[0], dst + jc);
+        } else {
+            // neighbouring lanes (same row) hold the other parts of the word
+            constexpr int kLanesPerWord = 32 / kChunkBits;
+            const uint32_t sub = jc & (kLanesPerWord - 1);
+            const uint32_t word = group_or<kLanesPerWord>(w[0] << (sub * kChunkBits));
+            if (live && sub == 0) output_store(keep, word, dst + jc / kLanesPerWord);
+        }
+    }
+}
+
 // Per-tensor abs-max, pass 1, over strided rows: gridDim.x <= kMaxPartials workgroups of 1024
 // threads stride over the (row tile, chunk tile) pairs; one f32 partial per workgroup.  A
 // maximum does not mind seeing an element twice: indices beyond the end are clamped to the
@@ -569,6 +683,45 @@ bool blocks_geom(uint32_t per_chunk, uint32_t bits, const RowArgs& a, BlocksGeom
     return tiles < (1ull << 31);
 }
 
+// Whether quantize_block_tiles_kernel takes the launch: its lanes along the row, and how many chunks of a block's column each
+// lane would hold in a workgroup of 256.
+bool block_tiles_geom(uint32_t per_chunk, const RowArgs& a, BlockTilesGeom* g, uint32_t* per_lane) {
+    if (a.rank < 2) return false;
+    const uint32_t last = a.rank - 1, br = a.block[last - 1], cpb = a.block[last] / per_chunk;
+    if ((br & (br - 1)) != 0 || (cpb & (cpb - 1)) != 0 || cpb > 64 || a.rows / br > 65535) return false;
+    g->chunks_per_row = a.shape[last] / per_chunk;
+    g->cpb_log2 = g->tj_log2 = 0;
+    while ((1u << g->cpb_log2) < cpb) g->cpb_log2++;
+    while ((1u << g->tj_log2) < cpb || g->tj_log2 < 4 || (br << g->tj_log2) < kThreads) g->tj_log2++;
+    if (g->tj_log2 > 6 || g->chunks_per_row < (1u << g->tj_log2) || (br << g->tj_log2) > 4096) return false;
+    *per_lane = (br << g->tj_log2) / kThreads;
+    g->pairs = aligned8(a.output);
+    for (uint32_t d = 0; d < last; d++) g->pairs = g->pairs && a.vstride[d] % 2 == 0;
+    return true;
+}
+
+template <class F, int kBits, int kEnc, int kT, int kR>
+hipError_t block_tiles_variant(hipStream_t s, const RowArgs& a, const BlockTilesGeom& g, const QuantParams& qp) {
+    const uint32_t last = a.rank - 1;
+    const dim3 grid((g.chunks_per_row + (1u << g.tj_log2) - 1) >> g.tj_log2, static_cast<uint32_t>(a.rows / a.block[last - 1]));
+    hipLaunchKernelGGL((quantize_block_tiles_kernel<F, kBits, kEnc, kT, kR>), grid, dim3(kT), 0, s, a, g, qp);
+    return hipGetLastError();
+}
+
+template <class F, int kBits, int kEnc>
+hipError_t block_tiles(hipStream_t s, const RowArgs& a, const BlockTilesGeom& g, uint32_t per_lane, const QuantParams& qp) {
+    // 512 lanes from four chunks on: quantize and dequantize of bf16 [512, 2048], 128 x 128, 256 x 8, 512 x 4, 1024 x 2: 7.0, 6.6, 6.7 us,
+    // [14336, 4096] 55.3, 54.5, 58.5; 64 x 64, 256 x 4, 512 x 2, 1024 x 1: 6.2, 6.0, 7.0 and 54.4, 54.5, 82.5.  Not for two: 32 x 32,
+    // 256 x 2, 512 x 1: 6.0, 6.2 and 54.1, 77.3.
+    switch (per_lane) {
+        case 1: return block_tiles_variant<F, kBits, kEnc, 256, 1>(s, a, g, qp);
+        case 2: return block_tiles_variant<F, kBits, kEnc, 256, 2>(s, a, g, qp);
+        case 4: return block_tiles_variant<F, kBits, kEnc, 512, 2>(s, a, g, qp);
+        case 8: return block_tiles_variant<F, kBits, kEnc, 512, 4>(s, a, g, qp);
+        default: return block_tiles_variant<F, kBits, kEnc, 1024, 4>(s, a, g, qp);
+    }
+}
+
 template <class F, int kBits, bool kWide, int kEnc, int kRows, int kCols>
 hipError_t quantize_blocks_variant(hipStream_t s, const RowArgs& a, const BlocksGeom& g, const QuantParams& qp) {
     hipLaunchKernelGGL((quantize_blocks_kernel<F, kBits, kWide, kEnc, kRows, kCols>), dim3(g.tiles), dim3(kThreads), 0, s, a,
@@ -578,6 +731,9 @@ hipError_t quantize_blocks_variant(hipStream_t s, const RowArgs& a, const Blocks
 
 template <class F, int kBits, bool kWide, int kEnc>
 hipError_t quantize_blocks_rows(hipStream_t s, const RowArgs& a, const BlocksGeom& g, const QuantParams& qp) {
+    BlockTilesGeom tiles;
+    uint32_t per_lane;
+    if (block_tiles_geom(F::kPerChunk, a, &tiles, &per_lane)) return block_tiles<F, kBits, kEnc>(s, a, tiles, per_lane, qp);
     if (g.rows_per_thread <= 1) return quantize_blocks_variant<F, kBits, kWide, kEnc, 1, 4>(s, a, g, qp);
     if (g.rows_per_thread <= 2) return quantize_blocks_variant<F, kBits, kWide, kEnc, 2, 4>(s, a, g, qp);
     if (g.rows_per_thread <= 4) return quantize_blocks_variant<F, kBits, kWide, kEnc, 4, 2>(s, a, g, qp);
@@ -598,6 +754,7 @@ hipError_t quantize_blocks(hipStream_t s, int bits, const RowArgs& a) {
     qp.width = a.range.hi - a.range.lo;
     qp.rwidth = 1.0f / qp.width;  // IEEE division on the host: correctly rounded
     qp.unrounded = a.range.unrounded;
+    qp.keep = a.rows * a.shape[a.rank - 1] * static_cast<uint64_t>(bits) / 8 <= kKeepOutputBytes ? 1u : 0u;
     const bool wide = a.range.hi > 127.0f || a.range.lo < -128.0f;
     switch (a.encoding) {
         case kEncInt:
@@ -622,6 +779,12 @@ bool blocks_dynamic_supported(int dtype, int bits, const RowArgs& a) {
     if (bc % per_chunk) return false;
     BlocksGeom g;
     return a.rows != 0 && a.shape[a.rank - 1] != 0 && blocks_geom(per_chunk, static_cast<uint32_t>(bits), a, &g);
+}
+
+bool block_tiles_supported(int dtype, int bits, const RowArgs& a) {
+    BlockTilesGeom g;
+    uint32_t per_lane;
+    return blocks_dynamic_supported(dtype, bits, a) && block_tiles_geom(dtype == CQ_F32 ? 4 : 8, a, &g, &per_lane);
 }
 
 hipError_t launch_quantize_blocks_dynamic(hipStream_t s, int dtype, int bits, const RowArgs& a) {
