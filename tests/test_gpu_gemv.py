@@ -175,6 +175,39 @@ def test_gemv_of_a_batch(oracle, case, vectors):
     check_case(oracle, case[:7], 40 + vectors, native=case[7], vectors=vectors)
 
 
+# (rows, cols) on both sides of each line that the split of a launch over row groups and waves is drawn at: 256, 512, 768, 1024 and 1536
+# groups of 16 rows, rows of 8, 12 and 48 units of 32 (4 bits) values and just more
+SPLITS = [(17, 288), (4096, 256), (4096, 288), (1000, 384), (1000, 416), (4097, 416), (8192, 320), (8193, 320), (12288, 320), (12289, 320),
+          (16384, 288), (16385, 1504), (16385, 1536), (24576, 1568), (24577, 1568)]
+
+
+@pytest.mark.parametrize("vectors", [2, 5, 12, 16])
+@pytest.mark.parametrize("value", [QuantValue.Q4S, QuantValue.Q8S, QuantValue.E4M3], ids=lambda v: v.name)
+def test_gemv_of_a_batch_splits(value, vectors):
+    """Against the float64 product of the dequantized weights (held against the oracle elsewhere); tolerance as above."""
+    import torch
+
+    from cubek_amd import dequantize, quantize
+
+    H, client = TensorHandleRef.from_torch, ComputeClient.current()
+    store = QuantStore.Native if value == QuantValue.E4M3 else QuantStore.U32
+    for i, (rows, cols) in enumerate(SPLITS):
+        elem, dtype = ((ElemType.BF16, torch.bfloat16), (ElemType.F16, torch.float16))[i % 2]
+        scheme = QuantScheme.default().with_value(value).with_store(store).with_level(QuantLevel.block([32]))
+        gen = torch.Generator(device="cuda").manual_seed(rows + vectors)
+        w = (torch.randn((rows, cols), generator=gen, device="cuda") * 0.02).to(dtype)
+        x = torch.randn((vectors, cols), generator=gen, device="cuda").to(dtype)
+        codes = torch.empty(scheme.packed_shape(w.shape), dtype=torch.uint8 if store == QuantStore.Native else torch.int32, device="cuda")
+        scales = torch.empty(scheme.scales_shape(w.shape), device="cuda")
+        y = torch.full((vectors, rows), float("nan"), device="cuda")
+        quantize.launch_dynamic(client, H(w), H(codes), H(scales), scheme, elem)
+        dequantize.launch_ref(client, H(codes), H(w), H(scales), scheme, elem)
+        matvec.launch_ref(client, H(codes), H(scales), scheme, H(x), H(y), elem, ElemType.F32)
+        w64, x64 = w.double(), x.double()
+        want, mag = x64 @ w64.t().contiguous(), x64.abs() @ w64.abs().t().contiguous()
+        assert torch.all((y.double() - want).abs() <= 2e-5 * mag), (rows, cols)
+
+
 @pytest.mark.parametrize("vectors", [2, 3, 4, 7, 8, 11])
 @pytest.mark.parametrize("kind", ["q4-b32", "q8-b64-f16", "e4m3-native", "q4-general", "q4-wide", "e2m1-native-wide",
                                   "e5m2-native", "q2-in-turns"])
