@@ -27,6 +27,7 @@
 // one-thread-per-output fallback.
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 #include "cq_magic_div.hpp"
 
 namespace cq {
@@ -576,43 +577,10 @@ inline uint64_t packed_outputs_bytes(uint64_t num_out, uint64_t elem_bytes) { re
 
 inline dim3 blocks(uint64_t n, uint64_t per_block) { return dim3(static_cast<uint32_t>((n + per_block - 1) / per_block)); }
 inline uint64_t round_up(uint64_t v, uint64_t m) { return (v + m - 1) / m * m; }
-inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
-    uint32_t p = 1;
-    while (p < v && p < cap) p <<= 1;
-    return p;
-}
 
 // enough workgroups / lanes to keep 256 CUs busy
 constexpr uint64_t kTargetGroups = 2048;
 constexpr uint64_t kTargetLanes = kTargetGroups * kThreads / 2;
-
-// An outer axis in one launch of tiles (OneLaunch below) against slices and a fold.  A tile's lanes walk the whole axis, so
-// its workgroup lasts len * cw / (4 * 512) loads' latency; a second launch costs about 4 us.  (slices and fold -> one launch,
-// us; without a fold where the partials' bytes allowed one slice only, as in the first two.)
-//   f16 [115, 21256] 14.6 -> 4.1, bf16 [60, 30000] 8.7 -> 3.5, [337, 19272] 10.7 -> 6.2, [600, 8448] 10.5 -> 5.7, [1041, 9088]
-//   11.0 -> 6.8, [1036, 4835] 11.8 -> 8.3, f16 [391, 296] 6.3 -> 3.8, f32 [250, 32000] 9.9 -> 7.2, [83, 1184] 8.9 -> 3.0
-// Chunk columns per tile: a line of 128 bytes is eight of them, but fewer tiles than half of the compute units leave the
-// others idle: 605 columns 4 (bf16 [1036, 4835] 4, 8: 8.3, 9.9), 832 - 2048 columns 8 ([4093, 11008] 4, 8, 16: 38.5, 19.1,
-// 26.2), more 16 ([752, 19680] 4, 8, 16: 12.3, 11.1, 9.0).  512 lanes were the best or within 5 % of it throughout; up to 128
-// rows 256 of them start and end sooner (f32 [37, 15360] 3.2 -> 3.0).
-// The lines: past 1280 rows a tile's walk costs more than the fold (bf16 [1893, 1150] 8.6 -> 10.2, [2443, 4469] 12.2 -> 14.4,
-// [3726, 6656] 15.3 -> 19.1).  Where rows are whole lines no tile reads half of one, and the walk may be longer: [4093, 11008]
-// 20.5 -> 19.1, [3000, 16384] 21.6 -> 19.4, [2048, 32768] 27.3 -> 22.2; others of that size lose (f32 [1468, 29424] 31.4 ->
-// 33.9, bf16 [2874, 18205] 23.7 -> 29.7).  Fewer than eight rows are a loop of reduce_cols_kernel (f16 [5, 25600] 2.8 -> 3.1).
-struct OneLaunch {
-    bool take;
-    uint32_t cw;  // chunk columns per tile
-    uint64_t col_tiles;
-};
-inline OneLaunch one_launch(uint64_t outer, uint64_t len, uint64_t inner_chunks, bool whole_lines) {
-    const uint64_t cols = outer * inner_chunks;
-    const uint32_t cw = pow2_at_least(inner_chunks, cols >= 2200 ? 16 : cols >= 800 ? 8 : 4);
-    const uint64_t col_tiles = (inner_chunks + cw - 1) / cw;
-    const bool lines = whole_lines && cw >= 8;
-    const bool take = len >= 8 && outer * col_tiles <= 2048 &&
-                      (lines ? len <= 4096 && len * cw <= 32768 && cols * len <= (1ull << 23) : len <= 1280 && cols * len <= (1ull << 21));
-    return {take, cw, col_tiles};
-}
 
 // Rows per lane of reduce_cols_kernel with at most `most` slices over `cols` columns of chunks.  Its few workgroups all run
 // at once, so a launch lasts as long as the compute unit with the most of them: of two to four workgroups per compute unit
@@ -883,15 +851,23 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         if (slices > fit) slices = fit > 1 ? fit : 1;
     }
     if (p.kind == ReducePlan::kCols || p.kind == ReducePlan::kTile) {
-        const OneLaunch one = one_launch(a.outer, a.len, p.inner_chunks, !p.ragged && a.inner * F::kBytes % 128 == 0);
-        if (one.take) {
-            const uint64_t tiles = a.outer * one.col_tiles;
-            const uint32_t col_tiles = static_cast<uint32_t>(one.col_tiles);
-            if (a.len <= 128)
-                launch_tile<F, F, 256, kTileFinalPacked>(s, p.ragged, one.cw, tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
-            else
-                launch_tile<F, F, 512, kTileFinalPacked>(s, p.ragged, one.cw, tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
-            return hipGetLastError();
+        ReduceColumns c{};
+        c.outer = a.outer, c.len = a.len, c.inner = a.inner, c.per_chunk = kN;
+        c.ragged = p.ragged, c.tiles = p.kind == ReducePlan::kTile ? a.outer * p.col_tiles : 0;
+        c.wanted = p.slices, c.slices = slices;
+        const ReduceTile tile = reduce_tile(c);
+        switch (reduce_way(c)) {
+            case ReduceWay::kOneLaunch: {
+                // 512 lanes were the best or within 5 % of it throughout; up to 128 rows 256 of them start and end sooner (f32
+                // [37, 15360] 3.2 -> 3.0 us)
+                const uint32_t col_tiles = static_cast<uint32_t>(tile.col_tiles);
+                if (a.len <= 128)
+                    launch_tile<F, F, 256, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+                else
+                    launch_tile<F, F, 512, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+                return hipGetLastError();
+            }
+            case ReduceWay::kPlan: break;
         }
     }
     auto in = static_cast<const u32x4*>(a.input);

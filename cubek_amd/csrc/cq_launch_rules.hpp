@@ -83,4 +83,56 @@ inline bool quantize_stays_resident(uint64_t chunks, int bits, bool captured) {
     return chunks <= 16ull << 16 || chunks >= (bits == 8 ? 48ull << 16 : 56ull << 16);
 }
 
+inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
+    uint32_t p = 1;
+    while (p < v && p < cap) p <<= 1;
+    return p;
+}
+
+// Abs-max along an outer axis of a contiguous [outer, len, inner] tensor (cq_kernels_reduce.hip): the plan of slices and a fold, or
+// one launch of tiles whose workgroups walk the whole axis.  "->" below is from the former to the latter.
+struct ReduceColumns {
+    uint64_t outer, len, inner;  // elements
+    uint64_t per_chunk;          // elements of a 16-byte chunk
+    bool ragged;                 // rows that are not whole aligned chunks
+    uint64_t tiles;              // workgroups of the plan's tiles before it cuts the axis; 0: the plan is a lane per chunk of columns
+    uint64_t wanted, slices;     // slices that the plan wants, and what the workspace holds
+};
+// Chunk columns per tile of the one launch: a line of 128 bytes is eight of them, but fewer tiles than half of the compute units
+// leave the others idle: 605 columns 4 (bf16 [1036, 4835] 4, 8: 8.3, 9.9), 832 - 2048 columns 8 ([4093, 11008] 4, 8, 16: 38.5,
+// 19.1, 26.2), more 16 ([752, 19680] 4, 8, 16: 12.3, 11.1, 9.0).
+struct ReduceTile {
+    uint32_t cw;
+    uint64_t col_tiles;
+};
+inline ReduceTile reduce_tile(const ReduceColumns& c) {
+    const uint64_t chunks = (c.inner + c.per_chunk - 1) / c.per_chunk, cols = c.outer * chunks;
+    const uint32_t cw = pow2_at_least(chunks, cols >= 2200 ? 16 : cols >= 800 ? 8 : 4);
+    return {cw, (chunks + cw - 1) / cw};
+}
+
+enum class ReduceWay { kPlan, kOneLaunch };
+inline ReduceWay reduce_way(const ReduceColumns& c) {
+    const uint64_t cols = c.outer * ((c.inner + c.per_chunk - 1) / c.per_chunk), tiles = c.outer * reduce_tile(c).col_tiles;
+    // Without room for half of the slices, the columns alone are too few lanes (bf16 [43625, 2348] 4160 -> 158, [20000, 4097] 2133 -> 85,
+    // [2000, 301] 36.5 -> 5.8, [4096, 4096] 394 -> 17.9).
+    if (c.wanted > 2 * c.slices) return ReduceWay::kOneLaunch;
+    // Tiles that want two slices and have room for one: they are wide, and few rows each (bf16 [2, 155, 128] 2.7 -> 2.9).
+    if (c.slices < c.wanted && c.tiles != 0 && !c.ragged) return ReduceWay::kPlan;
+    if (c.len < 8) return ReduceWay::kPlan;  // a loop of a lane per chunk (f16 [5, 25600] 2.8 -> 3.1)
+    // A tile's lanes walk the whole axis, so its workgroup lasts len * cw / (4 * 512) loads' latency; a second launch costs about 4
+    // us.  (Without a fold where the partials' bytes allowed one slice only, as in the first two.)
+    //   f16 [115, 21256] 14.6 -> 4.1, bf16 [60, 30000] 8.7 -> 3.5, [337, 19272] 10.7 -> 6.2, [600, 8448] 10.5 -> 5.7, [1041, 9088]
+    //   11.0 -> 6.8, [1036, 4835] 11.8 -> 8.3, f16 [391, 296] 6.3 -> 3.8, f32 [250, 32000] 9.9 -> 7.2, [83, 1184] 8.9 -> 3.0
+    // Past 1280 rows the walk costs more than the fold (bf16 [2443, 4469] 12.2 -> 14.4, f32 [1468, 29424] 31.4 -> 33.9).
+    if (tiles > 2048) return ReduceWay::kPlan;
+    bool one = c.len <= 1280 && cols * c.len <= (1ull << 21);
+    // Where rows are whole lines no tile reads half of one, and the walk may be longer: [4093, 11008] 20.5 -> 19.1, [3000, 16384] 21.6 ->
+    // 19.4, [2048, 32768] 27.3 -> 22.2.
+    const uint32_t cw = reduce_tile(c).cw;
+    if (!c.ragged && c.inner % (8 * c.per_chunk) == 0 && cw >= 8)
+        one = c.len <= 4096 && c.len * cw <= 32768 && cols * c.len <= (1u << 23);
+    return one ? ReduceWay::kOneLaunch : ReduceWay::kPlan;
+}
+
 }  // namespace cq

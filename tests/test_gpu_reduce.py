@@ -65,8 +65,8 @@ def test_reduce_contiguous_all_paths(gpu, oracle, elem):
 def test_reduce_short_rows_and_small_outer_axes(gpu, oracle, elem):
     """Rows of a few chunks that are not a power of two (every width of lane group, the most loads per lane, one chunk
     more) and axes that one launch takes whole (tiles of 1, 2 and 4 chunk columns, cut short; the longest axis and
-    one more), bit for bit; without a workspace the outer axes are not sliced, so they take the kernels of one lane per
-    column or one workgroup per tile instead of the one launch."""
+    one more), bit for bit; without a workspace the outer axes are not sliced, so those that a workspace would cut into
+    slices take tiles over the whole axis too."""
     import torch
 
     rng = np.random.default_rng(int(elem) + 70)

@@ -84,3 +84,30 @@ REPACK = {
 def test_repacked_words_stay_in_the_caches_where_lines_are_shared_or_both_launches_fit(answer):
     got = answer([f"repack_stays({n}ull, {str(lines).lower()})" for n, lines in REPACK])
     assert got == [int(stay) for stay in REPACK.values()], dict(zip(REPACK, got))
+
+
+ONE, PLAN = "kOneLaunch", "kPlan"
+
+
+def reduce_way(outer, length, inner, elem_bytes, ragged, tiles, wanted, room):
+    """`tiles`: of the plan (0: a lane per chunk of columns); slices that the plan wants and that the workspace has room for."""
+    return (f"[] {{ ReduceColumns c{{}}; c.outer = {outer}, c.len = {length}, c.inner = {inner}, c.per_chunk = {16 // elem_bytes}, c.ragged = {str(ragged).lower()}, "
+            f"c.tiles = {tiles}, c.wanted = {wanted}, c.slices = {room}; return reduce_way(c); }}()")
+
+
+# the arguments of reduce_way(): the way that was the faster one, or within 5 % of it
+REDUCE = {
+    # no workspace, or too little
+    (1, 43625, 2348, 2, True, 0, 681, 1): ONE, (1, 20000, 4097, 2, True, 0, 312, 1): ONE, (1, 2000, 301, 2, True, 1, 31, 1): ONE,
+    (16, 3000, 77, 2, True, 16, 46, 1): ONE, (1, 4096, 4096, 2, False, 0, 64, 1): ONE, (1, 5000, 801, 2, True, 2, 78, 30): ONE,
+    (1, 5000, 801, 2, True, 2, 78, 40): PLAN, (2, 155, 128, 2, False, 2, 2, 1): PLAN,
+    # a workspace
+    (1, 1041, 9088, 2, False, 0, 16, 16): ONE, (1, 250, 32000, 4, False, 0, 7, 7): ONE, (1, 20000, 4097, 2, True, 0, 312, 312): PLAN,
+    (1, 2443, 4469, 2, True, 0, 38, 38): PLAN, (1, 5, 25600, 2, False, 0, 1, 1): PLAN,
+}
+
+
+def test_reductions_along_an_outer_axis_take_the_faster_way(answer):
+    got = answer([f"{reduce_way(*case)} == ReduceWay::{way}" for case, way in REDUCE.items()])
+    wrong = [case for case, right in zip(REDUCE, got) if not right]
+    assert not wrong
