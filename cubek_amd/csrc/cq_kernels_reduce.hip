@@ -619,6 +619,7 @@ struct ReducePlan {
     uint64_t chunks_per_row = 0, inner_chunks = 0;  // ragged: whole chunks of a row; chunks that cover the columns
     uint32_t cw = 1, col_tiles = 1;
     uint64_t slices = 1;  // wanted; the launcher lowers it to what the workspace holds
+    bool long_axis = false;  // columns: more slices than one, if the partials' bytes allow them
     uint64_t lane_slices = 1;  // kTile on a strided input (one lane per output chunk and slice instead): wanted there
     uint64_t pitch = 0;   // partials per slice
 };
@@ -657,6 +658,7 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
             p.slices = kTargetLanes / cols;
             const uint64_t max_slices = (len + 15) / 16;  // at least 16 rows per slice
             if (p.slices > max_slices) p.slices = max_slices;
+            p.long_axis = p.slices > 1;
             if (p.slices > traffic_cap) p.slices = traffic_cap;
         }
         return p;
@@ -675,6 +677,7 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
         const uint64_t rows_per_step = kThreads / p.cw * 4;  // rows one workgroup reads per loop trip
         const uint64_t max_slices = (len + 2 * rows_per_step - 1) / (2 * rows_per_step);
         if (p.slices > max_slices) p.slices = max_slices;
+        p.long_axis = p.slices > 1;
         if (p.slices > traffic_cap) p.slices = traffic_cap;
     }
     return p;
@@ -854,7 +857,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         ReduceColumns c{};
         c.outer = a.outer, c.len = a.len, c.inner = a.inner, c.per_chunk = kN;
         c.ragged = p.ragged, c.tiles = p.kind == ReducePlan::kTile ? a.outer * p.col_tiles : 0;
-        c.wanted = p.slices, c.slices = slices;
+        c.long_axis = p.long_axis, c.wanted = p.slices, c.slices = slices;
         const ReduceTile tile = reduce_tile(c);
         switch (reduce_way(c)) {
             case ReduceWay::kOneLaunch: {
@@ -867,6 +870,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                     launch_tile<F, F, 512, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
                 return hipGetLastError();
             }
+            case ReduceWay::kPerOutput: p.kind = ReducePlan::kFallback; break;
             case ReduceWay::kPlan: break;
         }
     }

@@ -90,12 +90,13 @@ inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {
 }
 
 // Abs-max along an outer axis of a contiguous [outer, len, inner] tensor (cq_kernels_reduce.hip): the plan of slices and a fold, or
-// one launch of tiles whose workgroups walk the whole axis.  "->" below is from the former to the latter.
+// one launch of tiles whose workgroups walk the whole axis, or a lane or wave per output (the kernel for any strides).  "->" below is from the former to the latter.
 struct ReduceColumns {
     uint64_t outer, len, inner;  // elements
     uint64_t per_chunk;          // elements of a 16-byte chunk
     bool ragged;                 // rows that are not whole aligned chunks
     uint64_t tiles;              // workgroups of the plan's tiles before it cuts the axis; 0: the plan is a lane per chunk of columns
+    bool long_axis;              // the plan wants slices, whatever the bytes of their partials
     uint64_t wanted, slices;     // slices that the plan wants, and what the workspace holds
 };
 // Chunk columns per tile of the one launch: a line of 128 bytes is eight of them, but fewer tiles than half of the compute units
@@ -111,15 +112,33 @@ inline ReduceTile reduce_tile(const ReduceColumns& c) {
     return {cw, (chunks + cw - 1) / cw};
 }
 
-enum class ReduceWay { kPlan, kOneLaunch };
+enum class ReduceWay { kPerOutput, kPlan, kOneLaunch };
 inline ReduceWay reduce_way(const ReduceColumns& c) {
     const uint64_t cols = c.outer * ((c.inner + c.per_chunk - 1) / c.per_chunk), tiles = c.outer * reduce_tile(c).col_tiles;
+    const bool f32 = c.per_chunk == 4;
+    // Ragged rows, few elements per output: a workgroup per tile is mostly idle lanes and costs a large launch 1.5 ns each, a lane per
+    // output 0.1 us per element of the axis, or 1 ns per thousand elements of the tensor (tiles -> per output: f16 [34978, 9, 23]
+    // 53.8 -> 5.9, [13557, 2, 125] 15.2 -> 6.1, bf16 [10812, 76, 11] 23.1 -> 10.2; [4485, 225, 11] 13.2 -> 22.9, [3905, 8, 431] 9.4 ->
+    // 14.6).  Below four elements (twelve in rows of less than 32 that are not f32) also against a lane per chunk, whose loads and
+    // stores overlap and are not aligned (f16 [155, 2, 949] 2.7 -> 2.3, [620, 12, 11] 3.5 -> 2.9, f32 [200000, 3, 5] 5.7 -> 4.9), as
+    // long as the launch is small (f32 [3038, 1, 365] 4.0 -> 4.7, [166490, 1, 11] 5.1 -> 6.6).
+    if (c.ragged && !c.long_axis && c.len < 256) {
+        if (c.len * 50 + 100 < c.tiles && c.outer * c.len * c.inner < c.tiles * 1800) return ReduceWay::kPerOutput;
+        if (f32 ? c.len <= 4 && c.inner < 8 : c.inner < 32 ? c.len <= 12 : c.len <= 4 && c.outer * c.inner * c.len <= (1u << 19))
+            return ReduceWay::kPerOutput;
+    }
+    // From 256 elements on an output has a wave, which for few of them ends before the tiles' 8 columns a lane have met (bf16
+    // [631, 47] 4.0 -> 3.3, [325, 11] 3.4 -> 2.6, [901, 423] 3.6 -> 4.1; of f32, with 4, [452, 47] 2.2 -> 3.1).
+    if (c.ragged && !f32 && c.len >= 256 && c.len <= 768 && c.outer * c.inner <= 1280) return ReduceWay::kPerOutput;
     // Without room for half of the slices, the columns alone are too few lanes (bf16 [43625, 2348] 4160 -> 158, [20000, 4097] 2133 -> 85,
     // [2000, 301] 36.5 -> 5.8, [4096, 4096] 394 -> 17.9).
     if (c.wanted > 2 * c.slices) return ReduceWay::kOneLaunch;
     // Tiles that want two slices and have room for one: they are wide, and few rows each (bf16 [2, 155, 128] 2.7 -> 2.9).
     if (c.slices < c.wanted && c.tiles != 0 && !c.ragged) return ReduceWay::kPlan;
-    if (c.len < 8) return ReduceWay::kPlan;  // a loop of a lane per chunk (f16 [5, 25600] 2.8 -> 3.1)
+    // An axis that is too short for slices is short for the plan's wider tiles too (f16 [15, 832] 1.8 -> 2.4, bf16 [20, 1640] 2.2 -> 2.5,
+    // f16 [8, 24256] 2.0 -> 2.4, bf16 [212, 14, 799] 2.6 -> 4.5), except where a lane per ragged chunk would walk it (f32
+    // [15, 11951] 2.7 -> 2.3).
+    if (!c.long_axis && !(c.ragged && c.tiles == 0 && c.len > 8 && tiles <= 256)) return ReduceWay::kPlan;
     // A tile's lanes walk the whole axis, so its workgroup lasts len * cw / (4 * 512) loads' latency; a second launch costs about 4
     // us.  (Without a fold where the partials' bytes allowed one slice only, as in the first two.)
     //   f16 [115, 21256] 14.6 -> 4.1, bf16 [60, 30000] 8.7 -> 3.5, [337, 19272] 10.7 -> 6.2, [600, 8448] 10.5 -> 5.7, [1041, 9088]

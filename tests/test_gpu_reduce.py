@@ -125,6 +125,27 @@ def test_reduce_ragged_rows_and_columns(gpu, oracle, elem):
                 assert not got[:first_out].any() and not got[first_out + want.size:].any(), (shape, axis, "past the result")
 
 
+@pytest.mark.parametrize("elem", ELEMS, ids=lambda e: e.name)
+def test_reduce_short_axes_and_few_outputs(gpu, oracle, elem):
+    """Axes along which slices would be too short, with the lengths and widths on both sides of those that a lane or wave per
+    output, a lane per chunk, the plan's tiles and the one launch's tiles take."""
+    import torch
+
+    rng = np.random.default_rng(int(elem) + 7000)
+    n = 4 if elem == ElemType.F32 else 8
+    cases = [(700, 3, n + 1), (700, 13, 2 * n - 1), (40, 12, 31), (40, 13, 31), (300, 2, 33), (300, 5, 33), (3, 4, 949), (3, 5, 949), (2000, 9, 23), (2000, 40, 23),
+             (1, 8, 2201), (1, 9, 2201), (1, 16, 300 * n), (1, 16, 104 * n), (30, 7, 41 * n), (1, 255, 37), (1, 256, 37), (1, 768, 1280 - 1), (1, 769, 37), (3, 300, 427)]
+    for shape in cases:
+        x32 = rng.normal(0, 2, shape).astype(np.float32)
+        x32[rng.random(shape) < 0.01] = np.nan
+        x32.reshape(-1)[-1] = np.inf if shape[2] % 2 else -0.0
+        x = oracle.to_bits(x32, elem)
+        want = oracle.reduce_max_abs(x, elem, shape, 1).reshape(-1)
+        for use_ws in (True, False):
+            got, n_out = run(torch, gpu, x, elem, shape, 1, use_workspace=use_ws)
+            assert np.array_equal(got[:n_out].view(np.uint8), want.view(np.uint8)), (shape, use_ws)
+
+
 def test_reduce_strided_views_and_errors(gpu, oracle):
     import torch
 

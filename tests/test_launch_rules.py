@@ -86,13 +86,14 @@ def test_repacked_words_stay_in_the_caches_where_lines_are_shared_or_both_launch
     assert got == [int(stay) for stay in REPACK.values()], dict(zip(REPACK, got))
 
 
-ONE, PLAN = "kOneLaunch", "kPlan"
+ONE, PLAN, OUTPUTS = "kOneLaunch", "kPlan", "kPerOutput"
 
 
-def reduce_way(outer, length, inner, elem_bytes, ragged, tiles, wanted, room):
-    """`tiles`: of the plan (0: a lane per chunk of columns); slices that the plan wants and that the workspace has room for."""
+def reduce_way(outer, length, inner, elem_bytes, ragged, tiles, wanted, room, long_axis=True):
+    """`tiles`: of the plan (0: a lane per chunk of columns); slices that the plan wants and that the workspace has room for;
+    `long_axis`: whether it would want any, were their partials no bytes."""
     return (f"[] {{ ReduceColumns c{{}}; c.outer = {outer}, c.len = {length}, c.inner = {inner}, c.per_chunk = {16 // elem_bytes}, c.ragged = {str(ragged).lower()}, "
-            f"c.tiles = {tiles}, c.wanted = {wanted}, c.slices = {room}; return reduce_way(c); }}()")
+            f"c.tiles = {tiles}, c.wanted = {wanted}, c.slices = {room}, c.long_axis = {str(long_axis).lower()}; return reduce_way(c); }}()")
 
 
 # the arguments of reduce_way(): the way that was the faster one, or within 5 % of it
@@ -103,7 +104,17 @@ REDUCE = {
     (1, 5000, 801, 2, True, 2, 78, 40): PLAN, (2, 155, 128, 2, False, 2, 2, 1): PLAN,
     # a workspace
     (1, 1041, 9088, 2, False, 0, 16, 16): ONE, (1, 250, 32000, 4, False, 0, 7, 7): ONE, (1, 20000, 4097, 2, True, 0, 312, 312): PLAN,
-    (1, 2443, 4469, 2, True, 0, 38, 38): PLAN, (1, 5, 25600, 2, False, 0, 1, 1): PLAN,
+    (1, 2443, 4469, 2, True, 0, 38, 38): PLAN, (1, 5, 25600, 2, False, 0, 1, 1, False): PLAN,
+    # axes too short for slices
+    (1, 15, 832, 2, False, 2, 1, 1, False): PLAN, (1, 20, 1640, 2, False, 4, 1, 1, False): PLAN, (1, 8, 24256, 2, False, 0, 1, 1, False): PLAN,
+    (3, 89, 64, 2, False, 3, 1, 1, False): PLAN, (212, 14, 799, 2, True, 424, 1, 1, False): PLAN, (5, 12, 10885, 4, True, 0, 1, 1, False): PLAN,
+    (1, 15, 11951, 4, True, 0, 1, 1, False): ONE, (3905, 8, 431, 2, True, 3905, 1, 1, False): PLAN, (4485, 225, 11, 2, True, 4485, 1, 1, False): PLAN,
+    (34978, 9, 23, 2, True, 34978, 1, 1, False): OUTPUTS, (13557, 2, 125, 2, True, 13557, 1, 1, False): OUTPUTS,
+    (10812, 76, 11, 2, True, 10812, 1, 1, False): OUTPUTS, (1248, 17, 89, 2, True, 1248, 1, 1, False): OUTPUTS, (8141, 1, 29, 2, True, 8141, 1, 1, False): OUTPUTS,
+    (155, 2, 949, 2, True, 310, 1, 1, False): OUTPUTS, (620, 12, 11, 2, True, 620, 1, 1, False): OUTPUTS, (200000, 3, 5, 4, True, 0, 1, 1, False): OUTPUTS,
+    (3038, 1, 365, 4, True, 0, 1, 1, False): PLAN, (166490, 1, 11, 4, True, 0, 1, 1, False): PLAN,
+    # few outputs
+    (1, 631, 47, 2, True, 1, 9, 9): OUTPUTS, (1, 325, 11, 2, True, 1, 1, 1, False): OUTPUTS, (1, 901, 423, 2, True, 1, 14, 14): ONE, (1, 452, 47, 4, True, 1, 7, 7): ONE,
 }
 
 
