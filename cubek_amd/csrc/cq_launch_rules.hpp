@@ -146,11 +146,21 @@ inline ReduceWay reduce_way(const ReduceColumns& c) {
     // Past 1280 rows the walk costs more than the fold (bf16 [2443, 4469] 12.2 -> 14.4, f32 [1468, 29424] 31.4 -> 33.9).
     if (tiles > 2048) return ReduceWay::kPlan;
     bool one = c.len <= 1280 && cols * c.len <= (1ull << 21);
-    // Where rows are whole lines no tile reads half of one, and the walk may be longer: [4093, 11008] 20.5 -> 19.1, [3000, 16384] 21.6 ->
-    // 19.4, [2048, 32768] 27.3 -> 22.2.
+    // Where rows are whole lines no tile reads half of one, and the walk may be longer, as long as the compute units without
+    // a tile are few: they count for nothing in the one launch and read with the others in the plan's.  Calls in a row on
+    // rotated buffers: 104 tiles bf16 [1600, 6656] 10.7 -> 9.7, [2048, 6656] 11.2 -> 11.0, [3000, 6656] 13.2 -> 15.1, f32 [1600, 3328] 9.1 ->
+    // 9.2, [2048, 3328] 9.6 -> 10.7; 128 bf16 [2560, 8192] 13.7 -> 12.9, [3726, 8192] 15.5 -> 17.7, f32 [2400, 4096] 12.3 -> 12.0, [3000,
+    // 4096] 13.4 -> 14.2; 144 and 160 [3000, 9216] 15.2 -> 15.1, [2400, 10240] 14.6 -> 14.8, [3000, 10240] 15.5 -> 17.5; 172 and more
+    // [4093, 11008] 19.8 -> 18.3, f32 [4093, 5504] 18.5 -> 18.1, bf16 [4093, 14336] 24.2 -> 22.1, [3726, 16384] 27.0 -> 22.4; a second round
+    // of a few, 274, [1281, 17536] 14.0 -> 12.0, [1600, 17536] 14.4 -> 14.9, [2560, 17536] 19.5 -> 21.3.
+    // Tiles of 16 columns are twice the work each: up to 256 of them bf16 [2048, 20480] 18.2 -> 17.2, [2048, 32768] 26.4 -> 21.6; 272 [500, 34816]
+    // 11.6 -> 10.0, [900, 34816] 15.1 -> 16.0; 384 [900, 49152] 19.5 -> 17.7; 512 [900, 65536] 24.7 -> 21.5.
     const uint32_t cw = reduce_tile(c).cw;
-    if (!c.ragged && c.inner % (8 * c.per_chunk) == 0 && cw >= 8)
-        one = c.len <= 4096 && c.len * cw <= 32768 && cols * c.len <= (1u << 23);
+    if (!c.ragged && c.inner % (8 * c.per_chunk) == 0 && cw >= 8) {
+        const uint64_t longest = cw == 8 ? (tiles < 128 ? 1700 : tiles < 171 ? 2400 : tiles <= 256 ? 4096 : 1400)
+                                         : (tiles <= 256 ? 2048 : tiles <= 320 ? 768 : tiles < 512 ? 1152 : 2048);
+        one = c.len <= longest && cols * c.len <= (1u << 23);
+    }
     return one ? ReduceWay::kOneLaunch : ReduceWay::kPlan;
 }
 

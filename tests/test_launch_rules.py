@@ -113,6 +113,14 @@ REDUCE = {
     (10812, 76, 11, 2, True, 10812, 1, 1, False): OUTPUTS, (1248, 17, 89, 2, True, 1248, 1, 1, False): OUTPUTS, (8141, 1, 29, 2, True, 8141, 1, 1, False): OUTPUTS,
     (155, 2, 949, 2, True, 310, 1, 1, False): OUTPUTS, (620, 12, 11, 2, True, 620, 1, 1, False): OUTPUTS, (200000, 3, 5, 4, True, 0, 1, 1, False): OUTPUTS,
     (3038, 1, 365, 4, True, 0, 1, 1, False): PLAN, (166490, 1, 11, 4, True, 0, 1, 1, False): PLAN,
+    # rows of whole lines: the longest axes of one launch by the number of its tiles, 104, 128, 160, 172, 224, 256, 274, then of 16 columns
+    (1, 1600, 6656, 2, False, 0, 20, 20): ONE, (1, 3000, 6656, 2, False, 0, 40, 40): PLAN, (1, 4096, 6656, 2, False, 0, 64, 64): PLAN,
+    (1, 2048, 3328, 4, False, 0, 64, 64): PLAN, (1, 2048, 8192, 2, False, 0, 32, 32): ONE, (1, 3726, 8192, 2, False, 0, 58, 58): PLAN,
+    (1, 2048, 4096, 4, False, 0, 64, 64): ONE, (1, 3726, 4096, 4, False, 0, 116, 116): PLAN, (1, 2048, 10240, 2, False, 0, 32, 32): ONE,
+    (1, 3000, 10240, 2, False, 0, 46, 46): PLAN, (1, 4093, 11008, 2, False, 0, 63, 63): ONE, (1, 4093, 5504, 4, False, 0, 127, 127): ONE,
+    (1, 4093, 14336, 2, False, 0, 63, 63): ONE, (1, 4093, 16384, 2, False, 0, 63, 63): ONE, (1, 1281, 17536, 2, False, 0, 20, 20): ONE,
+    (1, 2048, 17536, 2, False, 0, 32, 32): PLAN, (1, 2048, 32768, 2, False, 0, 32, 32): ONE, (1, 500, 34816, 2, False, 0, 7, 7): ONE,
+    (1, 1281, 34816, 2, False, 0, 20, 20): PLAN, (1, 900, 49152, 2, False, 0, 14, 14): ONE, (1, 900, 65536, 2, False, 0, 14, 14): ONE,
     # few outputs
     (1, 631, 47, 2, True, 1, 9, 9): OUTPUTS, (1, 325, 11, 2, True, 1, 1, 1, False): OUTPUTS, (1, 901, 423, 2, True, 1, 14, 14): ONE, (1, 452, 47, 4, True, 1, 7, 7): ONE,
 }
