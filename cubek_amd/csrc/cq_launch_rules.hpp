@@ -117,13 +117,13 @@ inline ReduceWay reduce_way(const ReduceColumns& c) {
     const uint64_t cols = c.outer * ((c.inner + c.per_chunk - 1) / c.per_chunk), tiles = c.outer * reduce_tile(c).col_tiles;
     const bool f32 = c.per_chunk == 4;
     // Ragged rows, few elements per output: a workgroup per tile is mostly idle lanes and costs a large launch 1.5 ns each, a lane per
-    // output 0.1 us per element of the axis, or 1 ns per thousand elements of the tensor (tiles -> per output: f16 [34978, 9, 23]
-    // 53.8 -> 5.9, [13557, 2, 125] 15.2 -> 6.1, bf16 [10812, 76, 11] 23.1 -> 10.2; [4485, 225, 11] 13.2 -> 22.9, [3905, 8, 431] 9.4 ->
+    // output 0.1 us per element of the axis, 0.2 of f32, or 1 ns per thousand elements of the tensor (tiles -> per output: f16 [34978, 9, 23]
+    // 53.8 -> 5.9, [13557, 2, 125] 15.2 -> 6.1, bf16 [10812, 76, 11] 23.1 -> 10.2; [4485, 225, 11] 13.2 -> 22.9, f32 [7362, 85, 9] 10.6 -> 18.9, bf16 [3905, 8, 431] 9.4 ->
     // 14.6).  Below four elements (twelve in rows of less than 32 that are not f32) also against a lane per chunk, whose loads and
     // stores overlap and are not aligned (f16 [155, 2, 949] 2.7 -> 2.3, [620, 12, 11] 3.5 -> 2.9, f32 [200000, 3, 5] 5.7 -> 4.9), as
     // long as the launch is small (f32 [3038, 1, 365] 4.0 -> 4.7, [166490, 1, 11] 5.1 -> 6.6).
     if (c.ragged && !c.long_axis && c.len < 256) {
-        if (c.len * 50 + 100 < c.tiles && c.outer * c.len * c.inner < c.tiles * 1800) return ReduceWay::kPerOutput;
+        if (c.len * (f32 ? 100 : 50) + 100 < c.tiles && c.outer * c.len * c.inner < c.tiles * 1800) return ReduceWay::kPerOutput;
         if (f32 ? c.len <= 4 && c.inner < 8 : c.inner < 32 ? c.len <= 12 : c.len <= 4 && c.outer * c.inner * c.len <= (1u << 19))
             return ReduceWay::kPerOutput;
     }
@@ -138,7 +138,7 @@ inline ReduceWay reduce_way(const ReduceColumns& c) {
     // An axis that is too short for slices is short for the plan's wider tiles too (f16 [15, 832] 1.8 -> 2.4, bf16 [20, 1640] 2.2 -> 2.5,
     // f16 [8, 24256] 2.0 -> 2.4, bf16 [212, 14, 799] 2.6 -> 4.5), except where a lane per ragged chunk would walk it (f32
     // [15, 11951] 2.7 -> 2.3).
-    if (!c.long_axis && !(c.ragged && c.tiles == 0 && c.len > 8 && tiles <= 256)) return ReduceWay::kPlan;
+    if (!c.long_axis && !(c.ragged && c.tiles == 0 && c.len > 8 && tiles <= 512)) return ReduceWay::kPlan;
     // A tile's lanes walk the whole axis, so its workgroup lasts len * cw / (4 * 512) loads' latency; a second launch costs about 4
     // us.  (Without a fold where the partials' bytes allowed one slice only, as in the first two.)
     //   f16 [115, 21256] 14.6 -> 4.1, bf16 [60, 30000] 8.7 -> 3.5, [337, 19272] 10.7 -> 6.2, [600, 8448] 10.5 -> 5.7, [1041, 9088]
@@ -146,6 +146,9 @@ inline ReduceWay reduce_way(const ReduceColumns& c) {
     // Past 1280 rows the walk costs more than the fold (bf16 [2443, 4469] 12.2 -> 14.4, f32 [1468, 29424] 31.4 -> 33.9).
     if (tiles > 2048) return ReduceWay::kPlan;
     bool one = c.len <= 1280 && cols * c.len <= (1ull << 21);
+    // Slices of few ragged rows cost more than those of whole chunks: f32 [1283, 115] 5.5 -> 3.0, [1748, 5] 5.0 -> 2.5, [2213, 61] 5.0 ->
+    // 3.5, bf16 [1557, 1751] 8.5 -> 6.8, [1524, 9] 5.6 -> 4.1; f16 [2160, 73] 5.6 -> 6.5, f32 [2442, 501] 6.6 -> 9.0.
+    if (c.ragged && c.len <= (f32 ? 2304 : 1920) && cols * c.len <= (1u << 19)) one = true;
     // Where rows are whole lines no tile reads half of one, and the walk may be longer, as long as the compute units without
     // a tile are few: they count for nothing in the one launch and read with the others in the plan's.  Calls in a row on
     // rotated buffers: 104 tiles bf16 [1600, 6656] 10.7 -> 9.7, [2048, 6656] 11.2 -> 11.0, [3000, 6656] 13.2 -> 15.1, f32 [1600, 3328] 9.1 ->

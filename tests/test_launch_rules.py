@@ -111,7 +111,7 @@ REDUCE = {
     (1, 15, 11951, 4, True, 0, 1, 1, False): ONE, (3905, 8, 431, 2, True, 3905, 1, 1, False): PLAN, (4485, 225, 11, 2, True, 4485, 1, 1, False): PLAN,
     (34978, 9, 23, 2, True, 34978, 1, 1, False): OUTPUTS, (13557, 2, 125, 2, True, 13557, 1, 1, False): OUTPUTS,
     (10812, 76, 11, 2, True, 10812, 1, 1, False): OUTPUTS, (1248, 17, 89, 2, True, 1248, 1, 1, False): OUTPUTS, (8141, 1, 29, 2, True, 8141, 1, 1, False): OUTPUTS,
-    (155, 2, 949, 2, True, 310, 1, 1, False): OUTPUTS, (620, 12, 11, 2, True, 620, 1, 1, False): OUTPUTS, (200000, 3, 5, 4, True, 0, 1, 1, False): OUTPUTS,
+    (7362, 85, 9, 4, True, 7362, 1, 1, False): PLAN, (6, 13, 2901, 2, True, 0, 1, 1, False): ONE, (155, 2, 949, 2, True, 310, 1, 1, False): OUTPUTS, (620, 12, 11, 2, True, 620, 1, 1, False): OUTPUTS, (200000, 3, 5, 4, True, 0, 1, 1, False): OUTPUTS,
     (3038, 1, 365, 4, True, 0, 1, 1, False): PLAN, (166490, 1, 11, 4, True, 0, 1, 1, False): PLAN,
     # rows of whole lines: the longest axes of one launch by the number of its tiles, 104, 128, 160, 172, 224, 256, 274, then of 16 columns
     (1, 1600, 6656, 2, False, 0, 20, 20): ONE, (1, 3000, 6656, 2, False, 0, 40, 40): PLAN, (1, 4096, 6656, 2, False, 0, 64, 64): PLAN,
@@ -121,6 +121,9 @@ REDUCE = {
     (1, 4093, 14336, 2, False, 0, 63, 63): ONE, (1, 4093, 16384, 2, False, 0, 63, 63): ONE, (1, 1281, 17536, 2, False, 0, 20, 20): ONE,
     (1, 2048, 17536, 2, False, 0, 32, 32): PLAN, (1, 2048, 32768, 2, False, 0, 32, 32): ONE, (1, 500, 34816, 2, False, 0, 7, 7): ONE,
     (1, 1281, 34816, 2, False, 0, 20, 20): PLAN, (1, 900, 49152, 2, False, 0, 14, 14): ONE, (1, 900, 65536, 2, False, 0, 14, 14): ONE,
+    # ragged rows, few columns
+    (1, 1283, 115, 4, True, 1, 11, 11): ONE, (1, 1748, 5, 4, True, 1, 2, 2): ONE, (1, 2213, 61, 4, True, 1, 9, 9): ONE, (1, 1557, 1751, 2, True, 4, 24, 24): ONE,
+    (1, 2160, 73, 2, True, 1, 17, 17): PLAN, (1, 2442, 501, 4, True, 2, 76, 76): PLAN, (1, 1900, 4469, 2, True, 0, 29, 29): PLAN, (1, 1800, 1752, 2, False, 4, 28, 28): PLAN,
     # few outputs
     (1, 631, 47, 2, True, 1, 9, 9): OUTPUTS, (1, 325, 11, 2, True, 1, 1, 1, False): OUTPUTS, (1, 901, 423, 2, True, 1, 14, 14): ONE, (1, 452, 47, 4, True, 1, 7, 7): ONE,
 }
