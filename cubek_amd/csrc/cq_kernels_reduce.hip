@@ -117,6 +117,9 @@ inline uint32_t row_lanes(uint64_t chunks) {
     return best;
 }
 
+// The same for rows with edges, which are dealt out to the lanes too.
+inline uint32_t ragged_row_lanes(uint64_t chunks) { return row_lanes(chunks) < 8 ? 8 : row_lanes(chunks); }
+
 // ---- rows that start anywhere -------------------------------------------------------------------
 // A row of `len` elements at any element: its whole aligned chunks, and the fewer than two chunks' worth of elements beside
 // them.  Every access is aligned, so nothing is read twice and nothing outside the row.
@@ -529,13 +532,13 @@ struct StridedReduce {
     uint64_t out_strides[CQ_MAX_RANK];
 };
 
-// kLanes lanes per output element (1 or a whole wave)
+// kLanes lanes per output element (1 or a whole wave), from element `first` on
 template <class F, int kLanes>
 __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(const void* __restrict__ in,
                                                                   void* __restrict__ out, StridedReduce r,
-                                                                  uint64_t num_out) {
+                                                                  uint64_t first, uint64_t num_out) {
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    const uint64_t i = t / kLanes;
+    const uint64_t i = first + t / kLanes;
     const uint32_t lane = static_cast<uint32_t>(t % kLanes);
     if (i >= num_out) return;  // kLanes divides the wave: whole groups leave together
     uint64_t rem = i, in_off = 0, out_off = 0;
@@ -553,11 +556,11 @@ __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(const void* __
     if (lane == 0) F::store(out, out_off, m);
 }
 
-// Output element i of a contiguous result -> its place in a strided output tensor.
+// Output element i (`first` and on) of a contiguous result -> its place in a strided output tensor.
 template <class F>
 __global__ __launch_bounds__(kThreads) void scatter_outputs_kernel(const void* __restrict__ packed, void* __restrict__ out,
-                                                                   StridedReduce r, uint64_t num_out) {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+                                                                   StridedReduce r, uint64_t first, uint64_t num_out) {
+    const uint64_t i = first + static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= num_out) return;
     uint64_t rem = i, out_off = 0;
     for (int d = static_cast<int>(r.rank) - 1; d >= 0; d--) {
@@ -577,6 +580,10 @@ inline uint64_t packed_outputs_bytes(uint64_t num_out, uint64_t elem_bytes) { re
 
 inline dim3 blocks(uint64_t n, uint64_t per_block) { return dim3(static_cast<uint32_t>((n + per_block - 1) / per_block)); }
 inline uint64_t round_up(uint64_t v, uint64_t m) { return (v + m - 1) / m * m; }
+
+// The runtime counts a launch's lanes in 32 bits and drops what is above, without an error.
+constexpr uint64_t kMostLanes = 1ull << 32;
+inline uint64_t lanes_of_piece(uint64_t left) { return left < kMostLanes - kThreads ? left : kMostLanes - kThreads; }
 
 // enough workgroups / lanes to keep 256 CUs busy
 constexpr uint64_t kTargetGroups = 2048;
@@ -777,8 +784,9 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                 r.shape[d] = static_cast<uint32_t>(a.shape[d]);
                 r.out_strides[d] = a.out_strides[d];
             }
-            hipLaunchKernelGGL((scatter_outputs_kernel<F>), blocks(num_out, kThreads), dim3(kThreads), 0, s, a.workspace, a.output, r,
-                               num_out);
+            for (uint64_t first = 0; first < num_out; first += kMostLanes - kThreads)
+                hipLaunchKernelGGL((scatter_outputs_kernel<F>), blocks(lanes_of_piece(num_out - first), kThreads), dim3(kThreads), 0, s, a.workspace,
+                                   a.output, r, first, num_out);
             return hipGetLastError();
         }
     }
@@ -874,6 +882,9 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
             case ReduceWay::kPlan: break;
         }
     }
+    if (p.kind == ReducePlan::kRowsWave && p.chunks_per_row <= kWave * kRowLoads &&
+        a.outer * (p.ragged ? ragged_row_lanes(p.chunks_per_row) : row_lanes(p.chunks_per_row)) >= kMostLanes)
+        p.kind = ReducePlan::kFallback;  // one lane for each of so many short rows
     auto in = static_cast<const u32x4*>(a.input);
     switch (p.kind) {
         case ReducePlan::kRowsGrouped: {
@@ -904,8 +915,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                                        len, static_cast<uint32_t>(slices), p.pitch);
                     launch_fold<F>(s, a.workspace, a.output, slices, p.pitch, a.outer);
                 } else if (p.chunks_per_row <= kWave * kRowLoads) {
-                    uint32_t lanes = row_lanes(p.chunks_per_row);
-                    if (lanes < 8) lanes = 8;
+                    const uint32_t lanes = ragged_row_lanes(p.chunks_per_row);
                     const uint32_t loads = static_cast<uint32_t>((p.chunks_per_row + lanes - 1) / lanes);
                     switch (lanes) {
 #define CQ_CASE(G) case G: hipLaunchKernelGGL((reduce_ragged_rows_lanes_kernel<F, G>), blocks(a.outer * G, kThreads), dim3(kThreads), 0, s, a.input, a.output, a.outer, len, loads); break;
@@ -980,12 +990,14 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         if (d != a.axis) num_out *= a.shape[d];
     }
     if (num_out == 0) return hipSuccess;
-    if (a.shape[a.axis] >= 256)
-        hipLaunchKernelGGL((reduce_strided_kernel<F, kWave>), blocks(num_out * kWave, kThreads), dim3(kThreads), 0, s,
-                           a.input, a.output, r, num_out);
-    else
-        hipLaunchKernelGGL((reduce_strided_kernel<F, 1>), blocks(num_out, kThreads), dim3(kThreads), 0, s, a.input,
-                           a.output, r, num_out);
+    const uint64_t lanes = a.shape[a.axis] >= 256 ? kWave : 1;
+    for (uint64_t first = 0; first < num_out; first += (kMostLanes - kThreads) / lanes) {
+        const dim3 grid = blocks(lanes_of_piece((num_out - first) * lanes), kThreads);
+        if (lanes == kWave)
+            hipLaunchKernelGGL((reduce_strided_kernel<F, kWave>), grid, dim3(kThreads), 0, s, a.input, a.output, r, first, num_out);
+        else
+            hipLaunchKernelGGL((reduce_strided_kernel<F, 1>), grid, dim3(kThreads), 0, s, a.input, a.output, r, first, num_out);
+    }
     return hipGetLastError();
 }
 

@@ -106,3 +106,29 @@ def test_offsets_beyond_32_bits(oracle):
     for c0 in range(0, COLS, 8192):
         assert torch.equal(xt[c0:c0 + 8192].t().contiguous().view(torch.int16),
                            y[:, c0:c0 + 8192].contiguous().view(torch.int16)), c0
+
+
+@pytest.mark.parametrize("rows,cols,axis_last", [((1 << 29) + 3, 9, True), (3, ((1 << 32) + 40) // 3, False)], ids=["short_rows", "many_outputs"])
+def test_more_lanes_than_a_launch_counts(rows, cols, axis_last):
+    """2^29 rows that would have eight lanes each; 2^32 outputs that have a lane each (a tensor whose rows lie two elements apart)."""
+    import torch
+
+    client = ComputeClient.current()
+    if axis_last:
+        x = torch.zeros((rows, cols), device="cuda")
+        x[-1, 4], x[5, 8] = -3.0, 2.0
+        out = torch.full((rows, 1), -1.0, device="cuda")
+        h_x, axis = TensorHandleRef.from_torch(x), 1
+    else:
+        store = torch.zeros((2 * cols * rows,), dtype=torch.bfloat16, device="cuda")
+        x = store.view(1, rows, cols, 2)[..., 0]
+        x[0, -1, -1], x[0, 0, 5] = -3.0, 2.0
+        out = torch.full((1, rows, cols), -1.0, dtype=torch.bfloat16, device="cuda")
+        h_x, axis = TensorHandleRef.from_torch(x), 0
+    cq_reduce.max_abs(client, h_x, TensorHandleRef.from_torch(out), axis, ElemType.F32 if axis_last else ElemType.BF16)
+    torch.cuda.synchronize()
+    flat = out.view(-1)
+    assert flat[-1].item() == 3.0 and flat[5].item() == 2.0
+    flat[-1] = flat[5] = 0.0
+    for begin in range(0, flat.numel(), 1 << 30):
+        assert not flat[begin:begin + (1 << 30)].any(), begin
