@@ -8,6 +8,14 @@
 
 namespace cq {
 
+// The runtime counts a launch's lanes in 32 bits and drops what is above, without an error.  launch(first, last) for pieces of
+// [begin, end) that have a lane per element, or `lanes` of them, and fit.
+constexpr uint64_t kMostLanes = (1ull << 32) - 1024;
+template <class Launch>
+void in_pieces(uint64_t begin, uint64_t end, uint64_t lanes, Launch launch) {
+    for (uint64_t first = begin; first < end; first += kMostLanes / lanes) launch(first, end - first < kMostLanes / lanes ? end : first + kMostLanes / lanes);
+}
+
 // Scale addressing of one launch, the data of the reference's
 // ScalesLayout::{PerTensor,BlockScaled} (crates/cubek-quant/src/layout/scales.rs:15-195).
 struct Layout {

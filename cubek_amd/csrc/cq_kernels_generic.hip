@@ -115,11 +115,11 @@ __global__ __launch_bounds__(kThreads) void dequantize_generic_kernel(GenericArg
     }
 }
 
-// One thread per block: abs-max over the block's N-D box.
+// One thread per block, from block `first` on: abs-max over the block's N-D box.
 template <class F>
-__global__ __launch_bounds__(kThreads) void scales_generic_kernel(GenericArgs a, int out_dtype,
+__global__ __launch_bounds__(kThreads) void scales_generic_kernel(GenericArgs a, int out_dtype, uint64_t first,
                                                                   uint64_t num_blocks) {
-    uint64_t b = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    uint64_t b = first + static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (b >= num_blocks) return;
     const Layout& L = a.layout;
     // block coordinates (row-major over shape/block) and the box origin
@@ -245,6 +245,17 @@ __global__ __launch_bounds__(kThreads) void absmax_partials_strided_kernel(Gener
 
 inline dim3 grid_for(uint64_t n) { return dim3(static_cast<uint32_t>((n + kThreads - 1) / kThreads)); }
 
+// launch(args of a piece of the words)
+template <class Launch>
+hipError_t words_in_pieces(GenericArgs a, Launch launch) {
+    in_pieces(a.word_begin, a.word_end, 1, [&](uint64_t first, uint64_t last) {
+        a.word_begin = first;
+        a.word_end = last;
+        launch(a);
+    });
+    return hipGetLastError();
+}
+
 #define CQ_SWITCH_DTYPE(D, ...)                          \
     switch (D) {                                         \
         case CQ_F32: { using kF = F32; __VA_ARGS__; }    \
@@ -256,24 +267,22 @@ inline dim3 grid_for(uint64_t n) { return dim3(static_cast<uint32_t>((n + kThrea
 }  // namespace
 
 hipError_t launch_quantize_generic(hipStream_t s, int dtype, int bits, const GenericArgs& a) {
-    if (a.word_end <= a.word_begin) return hipSuccess;
-    CQ_SWITCH_DTYPE(dtype, hipLaunchKernelGGL((quantize_generic_kernel<kF>), grid_for(a.word_end - a.word_begin),
-                                              dim3(kThreads), 0, s, a, bits);
-                    return hipGetLastError())
+    CQ_SWITCH_DTYPE(dtype, return words_in_pieces(a, [&](const GenericArgs& piece) {
+                        hipLaunchKernelGGL((quantize_generic_kernel<kF>), grid_for(piece.word_end - piece.word_begin), dim3(kThreads), 0, s, piece, bits);
+                    }))
 }
 
 hipError_t launch_dequantize_generic(hipStream_t s, int dtype, int bits, const GenericArgs& a) {
-    if (a.word_end <= a.word_begin) return hipSuccess;
-    CQ_SWITCH_DTYPE(dtype, hipLaunchKernelGGL((dequantize_generic_kernel<kF>), grid_for(a.word_end - a.word_begin),
-                                              dim3(kThreads), 0, s, a, bits);
-                    return hipGetLastError())
+    CQ_SWITCH_DTYPE(dtype, return words_in_pieces(a, [&](const GenericArgs& piece) {
+                        hipLaunchKernelGGL((dequantize_generic_kernel<kF>), grid_for(piece.word_end - piece.word_begin), dim3(kThreads), 0, s, piece, bits);
+                    }))
 }
 
 hipError_t launch_scales_generic(hipStream_t s, int dtype, int out_dtype, const GenericArgs& a,
                                  uint64_t num_blocks) {
-    if (num_blocks == 0) return hipSuccess;
-    CQ_SWITCH_DTYPE(dtype, hipLaunchKernelGGL((scales_generic_kernel<kF>), grid_for(num_blocks), dim3(kThreads), 0, s,
-                                              a, out_dtype, num_blocks);
+    CQ_SWITCH_DTYPE(dtype, in_pieces(0, num_blocks, 1, [&](uint64_t first, uint64_t last) {
+                        hipLaunchKernelGGL((scales_generic_kernel<kF>), grid_for(last - first), dim3(kThreads), 0, s, a, out_dtype, first, last);
+                    });
                     return hipGetLastError())
 }
 
@@ -288,17 +297,15 @@ hipError_t launch_absmax_partials_strided(hipStream_t s, int dtype, const Generi
 }
 
 hipError_t launch_quantize_native(hipStream_t s, int dtype, const GenericArgs& a) {
-    if (a.word_end <= a.word_begin) return hipSuccess;
-    CQ_SWITCH_DTYPE(dtype, hipLaunchKernelGGL((quantize_native_kernel<kF>), grid_for(a.word_end - a.word_begin),
-                                              dim3(kThreads), 0, s, a);
-                    return hipGetLastError())
+    CQ_SWITCH_DTYPE(dtype, return words_in_pieces(a, [&](const GenericArgs& piece) {
+                        hipLaunchKernelGGL((quantize_native_kernel<kF>), grid_for(piece.word_end - piece.word_begin), dim3(kThreads), 0, s, piece);
+                    }))
 }
 
 hipError_t launch_dequantize_native(hipStream_t s, int dtype, const GenericArgs& a) {
-    if (a.word_end <= a.word_begin) return hipSuccess;
-    CQ_SWITCH_DTYPE(dtype, hipLaunchKernelGGL((dequantize_native_kernel<kF>), grid_for(a.word_end - a.word_begin),
-                                              dim3(kThreads), 0, s, a);
-                    return hipGetLastError())
+    CQ_SWITCH_DTYPE(dtype, return words_in_pieces(a, [&](const GenericArgs& piece) {
+                        hipLaunchKernelGGL((dequantize_native_kernel<kF>), grid_for(piece.word_end - piece.word_begin), dim3(kThreads), 0, s, piece);
+                    }))
 }
 
 }  // namespace cq

@@ -532,7 +532,7 @@ struct StridedReduce {
     uint64_t out_strides[CQ_MAX_RANK];
 };
 
-// kLanes lanes per output element (1 or a whole wave), from element `first` on
+// kLanes lanes per output element (1 or a whole wave), elements [first, num_out)
 template <class F, int kLanes>
 __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(const void* __restrict__ in,
                                                                   void* __restrict__ out, StridedReduce r,
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(const void* __
     if (lane == 0) F::store(out, out_off, m);
 }
 
-// Output element i (`first` and on) of a contiguous result -> its place in a strided output tensor.
+// Output element i, first <= i < num_out, of a contiguous result -> its place in a strided output tensor.
 template <class F>
 __global__ __launch_bounds__(kThreads) void scatter_outputs_kernel(const void* __restrict__ packed, void* __restrict__ out,
                                                                    StridedReduce r, uint64_t first, uint64_t num_out) {
@@ -580,10 +580,6 @@ inline uint64_t packed_outputs_bytes(uint64_t num_out, uint64_t elem_bytes) { re
 
 inline dim3 blocks(uint64_t n, uint64_t per_block) { return dim3(static_cast<uint32_t>((n + per_block - 1) / per_block)); }
 inline uint64_t round_up(uint64_t v, uint64_t m) { return (v + m - 1) / m * m; }
-
-// The runtime counts a launch's lanes in 32 bits and drops what is above, without an error.
-constexpr uint64_t kMostLanes = 1ull << 32;
-inline uint64_t lanes_of_piece(uint64_t left) { return left < kMostLanes - kThreads ? left : kMostLanes - kThreads; }
 
 // enough workgroups / lanes to keep 256 CUs busy
 constexpr uint64_t kTargetGroups = 2048;
@@ -784,9 +780,9 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                 r.shape[d] = static_cast<uint32_t>(a.shape[d]);
                 r.out_strides[d] = a.out_strides[d];
             }
-            for (uint64_t first = 0; first < num_out; first += kMostLanes - kThreads)
-                hipLaunchKernelGGL((scatter_outputs_kernel<F>), blocks(lanes_of_piece(num_out - first), kThreads), dim3(kThreads), 0, s, a.workspace,
-                                   a.output, r, first, num_out);
+            in_pieces(0, num_out, 1, [&](uint64_t first, uint64_t last) {
+                hipLaunchKernelGGL((scatter_outputs_kernel<F>), blocks(last - first, kThreads), dim3(kThreads), 0, s, a.workspace, a.output, r, first, last);
+            });
             return hipGetLastError();
         }
     }
@@ -883,7 +879,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
         }
     }
     if (p.kind == ReducePlan::kRowsWave && p.chunks_per_row <= kWave * kRowLoads &&
-        a.outer * (p.ragged ? ragged_row_lanes(p.chunks_per_row) : row_lanes(p.chunks_per_row)) >= kMostLanes)
+        a.outer * (p.ragged ? ragged_row_lanes(p.chunks_per_row) : row_lanes(p.chunks_per_row)) > kMostLanes)
         p.kind = ReducePlan::kFallback;  // one lane for each of so many short rows
     auto in = static_cast<const u32x4*>(a.input);
     switch (p.kind) {
@@ -991,13 +987,10 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
     }
     if (num_out == 0) return hipSuccess;
     const uint64_t lanes = a.shape[a.axis] >= 256 ? kWave : 1;
-    for (uint64_t first = 0; first < num_out; first += (kMostLanes - kThreads) / lanes) {
-        const dim3 grid = blocks(lanes_of_piece((num_out - first) * lanes), kThreads);
-        if (lanes == kWave)
-            hipLaunchKernelGGL((reduce_strided_kernel<F, kWave>), grid, dim3(kThreads), 0, s, a.input, a.output, r, first, num_out);
-        else
-            hipLaunchKernelGGL((reduce_strided_kernel<F, 1>), grid, dim3(kThreads), 0, s, a.input, a.output, r, first, num_out);
-    }
+    in_pieces(0, num_out, lanes, [&](uint64_t first, uint64_t last) {
+        const auto kernel = lanes == kWave ? reduce_strided_kernel<F, kWave> : reduce_strided_kernel<F, 1>;
+        hipLaunchKernelGGL(kernel, blocks((last - first) * lanes, kThreads), dim3(kThreads), 0, s, a.input, a.output, r, first, last);
+    });
     return hipGetLastError();
 }
 

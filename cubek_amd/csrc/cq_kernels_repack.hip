@@ -17,10 +17,10 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// One thread per output element, any rank and strides.
+// One thread per output element, from element `first` on, any rank and strides.
 template <class W>
-__global__ __launch_bounds__(kThreads) void repack_generic_kernel(RepackArgs a) {
-    const uint64_t pos = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
+__global__ __launch_bounds__(kThreads) void repack_generic_kernel(RepackArgs a, uint64_t first) {
+    const uint64_t pos = first + static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (pos >= a.num_out) return;
     const int last = static_cast<int>(a.rank) - 1;
     const W* in = static_cast<const W*>(a.input);
@@ -339,11 +339,10 @@ hipError_t launch_repack(hipStream_t s, const RepackArgs& bytes_or_words) {
                            static_cast<const uint32_t*>(g.input), static_cast<uint32_t*>(g.output), levels, total);
         return hipGetLastError();
     }
-    const dim3 grid(static_cast<uint32_t>((g.num_out + kThreads - 1) / kThreads));
-    if (g.elem_bytes == 4)
-        hipLaunchKernelGGL((repack_generic_kernel<uint32_t>), grid, dim3(kThreads), 0, s, g);
-    else
-        hipLaunchKernelGGL((repack_generic_kernel<uint8_t>), grid, dim3(kThreads), 0, s, g);
+    in_pieces(0, g.num_out, 1, [&](uint64_t first, uint64_t last) {
+        const auto kernel = g.elem_bytes == 4 ? repack_generic_kernel<uint32_t> : repack_generic_kernel<uint8_t>;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((last - first + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, g, first);
+    });
     return hipGetLastError();
 }
 

@@ -132,3 +132,48 @@ def test_more_lanes_than_a_launch_counts(rows, cols, axis_last):
     flat[-1] = flat[5] = 0.0
     for begin in range(0, flat.numel(), 1 << 30):
         assert not flat[begin:begin + (1 << 30)].any(), begin
+
+
+def test_per_element_kernels_of_more_lanes_than_a_launch_counts():
+    """2^32 bytes that have a lane each: quantized from and dequantized into floats two elements apart, and copied out of rows of an
+    odd pitch."""
+    import torch
+
+    from cubek_amd import QuantParam, QuantStore, _ffi, contiguous
+
+    client, h = ComputeClient.current(), TensorHandleRef.from_torch
+    rows, cols = 3, ((1 << 32) + 100) // 3
+    floats = torch.zeros((rows, cols, 2), dtype=torch.bfloat16, device="cuda")[..., 0]
+    ends = [(0, 5, 7), (1, 11, -9), (2, cols - 1, 3)]
+    for r, c, v in ends:
+        floats[r, c] = v * 0.5
+    scheme = QuantScheme.default().with_value(QuantValue.Q8S).with_store(QuantStore.Native).with_param(QuantParam.F32)
+    given = torch.full((1,), 0.5, dtype=torch.bfloat16, device="cuda")
+    scale = torch.zeros((1,), device="cuda")
+    codes = torch.full((rows, cols), 99, dtype=torch.uint8, device="cuda")
+    assert _ffi.plan_kind(_ffi.OP_QUANTIZE, h(floats), h(codes), h(given), h(scale), scheme, ELEM) == "per_element"
+    qz.launch_ref(client, h(floats), h(codes), h(given), h(scale), scheme, ELEM)
+
+    def check(t, back):
+        torch.cuda.synchronize()
+        for r, c, v in ends:
+            assert back(t[r, c].item()) == v, (r, c)
+            t[r, c] = 0
+        for row in t:
+            for begin in range(0, cols, 1 << 28):
+                assert not row[begin:begin + (1 << 28)].any(), begin
+        for r, c, v in ends:
+            t[r, c] = v % 256 if t.dtype == torch.uint8 else v * 0.5
+
+    signed = lambda b: b - 256 if b > 127 else b  # noqa: E731
+    check(codes, signed)
+    floats.fill_(4.0)
+    assert _ffi.plan_kind(_ffi.OP_DEQUANTIZE, h(floats), h(codes), h(scale), None, scheme, ELEM) == "per_element"
+    dq.launch_ref(client, h(codes), h(floats), h(scale), scheme, ELEM)
+    check(floats, lambda v: v * 2)
+    del floats
+    pitched = torch.zeros((rows, cols + 1 + cols % 2), dtype=torch.uint8, device="cuda")[:, :cols]
+    pitched.copy_(codes)
+    codes.fill_(99)
+    contiguous.into_contiguous_packed_ref(client, h(pitched), h(codes), (rows, cols), 1)
+    check(codes, signed)
