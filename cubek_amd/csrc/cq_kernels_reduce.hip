@@ -686,14 +686,15 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
     return p;
 }
 
-template <class FIn, class FOut, int kT, int kMode>
+// kWidest: of the tiles that the caller asks for
+template <class FIn, class FOut, int kT, int kMode, int kWidest = kWave>
 void launch_tile(hipStream_t s, bool ragged, uint32_t cw, uint64_t jobs, const void* in, void* out, uint64_t len,
                  uint64_t inner, uint32_t col_tiles, uint32_t slices, uint64_t pitch, uint64_t count) {
     auto src = static_cast<const u32x4*>(in);
     dim3 grid(static_cast<uint32_t>(jobs));
     switch (cw * 2 + (ragged ? 1 : 0)) {
 #define CQ_TILE(W, R) hipLaunchKernelGGL((reduce_tile_kernel<FIn, FOut, W, kT, kMode, R>), grid, dim3(kT), 0, s, src, out, len, inner, col_tiles, slices, pitch, count)
-#define CQ_CASE(W) case W * 2: CQ_TILE(W, false); break; case W * 2 + 1: if constexpr (kMode != kTileFinalChecked) CQ_TILE(W, true); break;
+#define CQ_CASE(W) case W * 2: if constexpr (W <= kWidest) CQ_TILE(W, false); break; case W * 2 + 1: if constexpr (W <= kWidest && kMode != kTileFinalChecked) CQ_TILE(W, true); break;
         CQ_CASE(1) CQ_CASE(2) CQ_CASE(4) CQ_CASE(8) CQ_CASE(16) CQ_CASE(32) CQ_CASE(64)
 #undef CQ_CASE
 #undef CQ_TILE
@@ -871,7 +872,7 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                 if (a.len <= 128)
                     launch_tile<F, F, 256, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
                 else
-                    launch_tile<F, F, 512, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+                    launch_tile<F, F, 512, kTileFinalPacked, kWidestReduceTile>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
                 return hipGetLastError();
             }
             case ReduceWay::kPerOutput: p.kind = ReducePlan::kFallback; break;

@@ -102,13 +102,14 @@ struct ReduceColumns {
 // Chunk columns per tile of the one launch: a line of 128 bytes is eight of them, but fewer tiles than half of the compute units
 // leave the others idle: 605 columns 4 (bf16 [1036, 4835] 4, 8: 8.3, 9.9), 832 - 2048 columns 8 ([4093, 11008] 4, 8, 16: 38.5,
 // 19.1, 26.2), more 16 ([752, 19680] 4, 8, 16: 12.3, 11.1, 9.0).
+constexpr uint32_t kWidestReduceTile = 16;
 struct ReduceTile {
     uint32_t cw;
     uint64_t col_tiles;
 };
 inline ReduceTile reduce_tile(const ReduceColumns& c) {
     const uint64_t chunks = (c.inner + c.per_chunk - 1) / c.per_chunk, cols = c.outer * chunks;
-    const uint32_t cw = pow2_at_least(chunks, cols >= 2200 ? 16 : cols >= 800 ? 8 : 4);
+    const uint32_t cw = pow2_at_least(chunks, cols >= 2200 ? kWidestReduceTile : cols >= 800 ? 8 : 4);
     return {cw, (chunks + cw - 1) / cw};
 }
 
