@@ -9,13 +9,16 @@
 // as before, in loops in front of and behind the resident part.  Up to 2 or 8 chunks per lane go through kernels of their own,
 // without loops, and up to 8 steps through one workgroup.
 //
-// Waiting.  A slot per workgroup holds the launch's number and the workgroup's abs-max; launches take turns at kRegions regions
-// of slots.  Numbers differ until 2^32 launches have gone by, and every launch writes all slots of its region, so what
-// a slot held before is never taken for this launch's.  A replay of a captured launch would bring the same number again:
-// captured launches have their slots in the caller's workspace, where a launch before them leaves kUnset.  No workgroup depends
-// on another one running: one that has waited for kPatience polls works out the missing shares itself, one by one, from
-// memory, and keeps them (the same bits, whoever does), so that it goes on after at most 256 of them whatever else
-// occupies the GPU and whoever takes its slots; it publishes them too, for workgroups that start late.
+// Waiting.  A slot per workgroup holds the launch's number and kStarted (in the large kernel), then the workgroup's abs-max; launches of
+// several workgroups take turns at kRegions regions of slots.  Numbers differ until 2^32 such launches have gone by on a device, and each of
+// them writes all slots of its region, so what a slot held before is never taken for this launch's.  A replay of a captured
+// launch would bring the same number again: captured launches have their slots in the caller's workspace, where a launch before
+// them leaves kUnset.
+// No workgroup depends on another one running.  Where other launches have taken compute units, or the stream has few, some
+// workgroups start only when others end: after kGrace polls those that wait work out such a share from memory, each another one
+// (it marks the slot as started), and publish it for all, itself included if the slots go to a later launch meanwhile.  One that has
+// started runs and will publish; all the same a workgroup waits for kPatience polls at most, and then works out
+// whatever is missing, so that it goes on after at most 256 shares.
 //
 // Bound by its phases one after the other.  bf16 128 MiB to 8 bits, 38 us: 2 of the launch, the read 19.5 (6.9 TB/s), 4
 // from the first published maximum to the last one seen, the arithmetic 11.5, which the stores overlap with.  Two passes -> one,
@@ -35,8 +38,8 @@ namespace resident {
 constexpr int kThreads = 512;
 constexpr uint32_t kGroups = 256;  // most workgroups = slots
 static_assert(kGroups <= kMaxPartials, "a captured launch's slots are the caller's workspace");
-constexpr uint32_t kUnset = 0xffffffffu;  // no abs-max: NaN elements are ignored
-constexpr uint32_t kPatience = 64;        // polls, about a microsecond each
+constexpr uint32_t kUnset = 0xffffffffu, kStarted = 0xfffffffeu;  // no abs-maxima: NaN elements are ignored
+constexpr uint32_t kGrace = 8, kGraceOfSmall = 32, kPatience = 1024, kBySize = 0xffffffffu;  // polls
 typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
 constexpr uint32_t kPerVector = 8;  // chunks
 
@@ -58,6 +61,7 @@ struct ResidentArgs {
     uint32_t rounds;     // steps of the busiest one
     uint32_t streamed;   // the first of them, read twice
     uint32_t number;     // of the launch; 0: a captured one, with slots in the workspace
+    uint32_t grace = kBySize, patience = kPatience;
     int param_dtype;
     QuantParams qp;
 };
@@ -125,11 +129,17 @@ struct Resident {
         if (group == 0 && e < a.num_elems) acc = fmaxf(acc, fabsf(F::load(a.in, e)));
         return acc;
     }
-    // another workgroup's share
+    // another workgroup's share, a few loads at a time: the registers are full
     __device__ __forceinline__ float share_absmax(uint32_t group) const {
+        constexpr uint32_t kUnroll = kInRegisters < 4 ? kInRegisters : 4;
         float acc = 0.0f;
 #pragma unroll 1
-        for (uint32_t k = 0; k < a.rounds; k++) acc = absmax(Window(a, k, 1).load(chunk_of(group, 0)), acc);
+        for (uint32_t k0 = 0; k0 < a.rounds; k0 += kUnroll) {
+            const Batch<kUnroll> now(*this, group, k0, a.rounds);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t u = 0; u < kUnroll; u++) acc = absmax(now.raw[u], acc);
+        }
         return tail_absmax(group, acc);
     }
     // the abs-max of the workgroup's lanes, in lane 0 of the workgroup
@@ -143,41 +153,55 @@ struct Resident {
     }
     // Slots behind those of the launch's workgroups are written too, so that no slot keeps a number until the count of
     // launches comes round to it.
-    __device__ __forceinline__ void publish(uint32_t group, float amax) const {
+    __device__ __forceinline__ void publish(uint32_t group, uint32_t what) const {
         if (a.number == 0) {
-            if (threadIdx.x == 0) __hip_atomic_store(a.slots + group, f32_bits(amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (threadIdx.x == 0) __hip_atomic_store(a.slots + group, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else if (threadIdx.x < kGroups && threadIdx.x % a.groups == group) {
-            const uint64_t slot = static_cast<uint64_t>(a.number) << 32 | f32_bits(amax);
-            __hip_atomic_store(region() + threadIdx.x, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(region() + threadIdx.x, tagged(what), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __device__ __forceinline__ uint64_t* region() const { return g_slots + a.number % kRegions * kGroups; }
+    __device__ __forceinline__ uint64_t tagged(uint32_t what) const { return static_cast<uint64_t>(a.number) << 32 | what; }
     __device__ __forceinline__ uint32_t poll(uint32_t group) const {
         if (a.number == 0) return __hip_atomic_load(a.slots + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint64_t slot = __hip_atomic_load(region() + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return slot >> 32 == a.number ? static_cast<uint32_t>(slot) : kUnset;
     }
+    // Marks a share that has not started; false: it has meanwhile.
+    __device__ __forceinline__ bool claim(uint32_t group) const {
+        if (a.number == 0) {
+            uint32_t seen = kUnset;
+            return __hip_atomic_compare_exchange_strong(a.slots + group, &seen, kStarted, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        uint64_t seen = __hip_atomic_load(region() + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return seen >> 32 != a.number &&
+               __hip_atomic_compare_exchange_strong(region() + group, &seen, tagged(kStarted), __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     // the abs-max of all shares
     __device__ __forceinline__ float collect() const {
-        __shared__ uint32_t missing;
+        __shared__ uint32_t missing, claimed;
         __shared__ float found;
         uint32_t mine = threadIdx.x < a.groups ? kUnset : 0;
         for (uint32_t polls = 0;; polls++) {
-            if (mine == kUnset) mine = poll(threadIdx.x);
-            if (!__syncthreads_or(mine == kUnset)) break;
-            if (polls < kPatience) {
+            if (mine >= kStarted) mine = poll(threadIdx.x);
+            if (!__syncthreads_or(mine >= kStarted)) break;
+            const bool impatient = polls >= a.patience, help = impatient ? mine >= kStarted : mine == kUnset;
+            if (!(impatient || (polls >= a.grace && __syncthreads_or(help)))) {
                 __builtin_amdgcn_s_sleep(2);
                 continue;
             }
-            // the first share missing from this workgroup's place on, so that those who help start at different ones
+            // the first one from this workgroup's place on, so that those who help start at different ones
             if (threadIdx.x == 0) missing = kGroups;
             __syncthreads();
             const uint32_t place = (threadIdx.x - blockIdx.x * 2) % kGroups;
-            if (mine == kUnset) atomicMin(&missing, place);
+            if (help) atomicMin(&missing, place);
             __syncthreads();
             const uint32_t share = (missing + blockIdx.x * 2) % kGroups;
+            if (threadIdx.x == share) claimed = impatient || claim(share);
+            __syncthreads();
+            if (!claimed) continue;
             const float amax = group_absmax(share_absmax(share));
-            publish(share, amax);
+            publish(share, f32_bits(amax));
             // kept here as well: a launch kRegions later may have taken the slot
             if (threadIdx.x == 0) found = amax;
             __syncthreads();
@@ -228,7 +252,7 @@ struct Resident {
     __device__ __forceinline__ float divisor(float amax) const {
         amax = group_absmax(amax);
         if (a.groups > 1) {
-            publish(blockIdx.x, amax);
+            publish(blockIdx.x, f32_bits(amax));
             amax = collect();
         }
         // the scale as quantize_flat_body derives it
@@ -265,6 +289,7 @@ struct Resident {
     }
     __device__ __forceinline__ void run() const {
         __shared__ u32x4 lds[kInLds][kThreads];
+        publish(blockIdx.x, kStarted);
         float amax = 0.0f;
         if (a.streamed) amax = streamed_absmax(blockIdx.x, a.streamed, amax);
         amax = tail_absmax(blockIdx.x, amax);
@@ -340,8 +365,17 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_resident_kernel(Resident
         r.run();
 }
 
+// The number of a launch of several workgroups; not 0.
+inline uint32_t next_number(int device) {
+    static std::atomic<uint32_t> counts[16];
+    uint32_t n;
+    do n = counts[device % 16].fetch_add(1, std::memory_order_relaxed) + 1;
+    while (n == 0);
+    return n;
+}
+
 template <class F, int kBits, int kEnc>
-hipError_t launch(hipStream_t s, ResidentArgs a) {
+hipError_t launch(hipStream_t s, ResidentWay way, ResidentArgs a) {
     const uint64_t steps = (a.chunks + kThreads - 1) / kThreads;
     a.groups = 1;
     if (steps > kSome)  // up to there a workgroup alone has nothing to wait for
@@ -349,7 +383,16 @@ hipError_t launch(hipStream_t s, ResidentArgs a) {
     a.rounds = static_cast<uint32_t>((steps + a.groups - 1) / a.groups);
     constexpr uint32_t kMost = kMostRegisters + kMostLds;
     a.streamed = a.rounds > kMost ? a.rounds - kMost : 0;
-    if (a.number == 0) hipLaunchKernelGGL(unset_slots_kernel, dim3(1), dim3(kGroups), 0, s, a.slots);
+    if (a.grace == kBySize) a.grace = a.rounds > kSome ? kGrace : kGraceOfSmall;
+    if (a.groups > 1) {
+        int device = 0;
+        if (way == ResidentWay::kCaptured)
+            hipLaunchKernelGGL(unset_slots_kernel, dim3(1), dim3(kGroups), 0, s, a.slots);
+        else if (const hipError_t e = hipGetDevice(&device); e != hipSuccess)
+            return e;
+        else
+            a.number = next_number(device);
+    }
     const auto kernel = a.rounds <= kFew    ? quantize_resident_kernel<F, kBits, kEnc, kFew, 0>
                         : a.rounds <= kSome ? quantize_resident_kernel<F, kBits, kEnc, kSome, 0>
                                             : quantize_resident_kernel<F, kBits, kEnc, kMostRegisters, kMostLds>;
@@ -358,18 +401,18 @@ hipError_t launch(hipStream_t s, ResidentArgs a) {
 }
 
 template <class F>
-hipError_t launch_encoding(hipStream_t s, int bits, int encoding, const ResidentArgs& a) {
+hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encoding, const ResidentArgs& a) {
     switch (encoding) {
         case kEncInt:
             switch (bits) {
-                case 2: return launch<F, 2, kEncInt>(s, a);
-                case 4: return launch<F, 4, kEncInt>(s, a);
-                case 8: return launch<F, 8, kEncInt>(s, a);
+                case 2: return launch<F, 2, kEncInt>(s, way, a);
+                case 4: return launch<F, 4, kEncInt>(s, way, a);
+                case 8: return launch<F, 8, kEncInt>(s, way, a);
             }
             break;
-        case kEncE4M3: return launch<F, 8, kEncE4M3>(s, a);
-        case kEncE5M2: return launch<F, 8, kEncE5M2>(s, a);
-        case kEncE2M1: return launch<F, 4, kEncE2M1>(s, a);
+        case kEncE4M3: return launch<F, 8, kEncE4M3>(s, way, a);
+        case kEncE5M2: return launch<F, 8, kEncE5M2>(s, way, a);
+        case kEncE2M1: return launch<F, 4, kEncE2M1>(s, way, a);
     }
     return hipErrorInvalidValue;
 }
@@ -390,7 +433,6 @@ ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& f) {
 }
 
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {
-    static std::atomic<uint32_t> launches{0};
     resident::ResidentArgs a{};
     a.in = f.input;
     a.out = f.output;
@@ -400,11 +442,10 @@ hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, i
     a.num_elems = num_elems;
     a.param_dtype = f.param_dtype;
     a.qp = quant_params(f.range);
-    while (way == ResidentWay::kNumbered && a.number == 0) a.number = launches.fetch_add(1, std::memory_order_relaxed) + 1;
     switch (dtype) {
-        case CQ_F32: return resident::launch_encoding<F32>(s, bits, f.encoding, a);
-        case CQ_BF16: return resident::launch_encoding<BF16>(s, bits, f.encoding, a);
-        case CQ_F16: return resident::launch_encoding<F16>(s, bits, f.encoding, a);
+        case CQ_F32: return resident::launch_encoding<F32>(s, way, bits, f.encoding, a);
+        case CQ_BF16: return resident::launch_encoding<BF16>(s, way, bits, f.encoding, a);
+        case CQ_F16: return resident::launch_encoding<F16>(s, way, bits, f.encoding, a);
         default: return hipErrorInvalidValue;
     }
 }

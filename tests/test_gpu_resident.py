@@ -1,5 +1,8 @@
 """One scale for a tensor, quantized in one read of it (cq_kernels_resident.hpp), against the two calls that share no
 kernel with it: compute_scales, then quantize with the given scale.  Codes and scale bit for bit."""
+import ctypes
+import os
+
 import numpy as np
 import pytest
 
@@ -208,3 +211,38 @@ def test_streams_and_graphs():
         graph.replay()
         torch.cuda.synchronize()
         call.check(seed)
+
+
+@pytest.fixture(scope="module")
+def waits():
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "libcq_resident_test.so"))
+    lib.cq_test_resident.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 5 + [ctypes.c_uint64] * 2 + [ctypes.c_uint32] * 2
+    return lib.cq_test_resident
+
+
+@pytest.mark.parametrize("kind,elem,value,store", [(0, ElemType.BF16, QuantValue.Q8S, QuantStore.U32), (1, ElemType.F32, QuantValue.Q4S, QuantStore.U32),
+                                                   (2, ElemType.F16, QuantValue.E4M3, QuantStore.Native)], ids=["bf16-q8", "f32-q4", "f16-e4m3"])
+def test_workgroups_that_work_out_the_shares_of_others(waits, kind, elem, value, store):
+    """No grace: shares that have not started when a workgroup has read its own; no patience: every share that has not arrived.  Numbered
+    launches and ones with slots in the workspace, of a few, some and many steps, beyond what the chip holds, with elements
+    behind the last chunk."""
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    for chunks in (9 * 512, 100 * 512 + 8, 2 * ROUND, 5 * ROUND + 4, 20 * ROUND + 4, 66 * ROUND + 516):
+        n = chunks * per + (3 if store == QuantStore.Native else 0)
+        call = Call(torch, values(torch, n, elem, chunks), elem, scheme_of(value, store))
+        call.x[n - 1] = -0.75
+        for grace, patience in ((0, 1024), (0, 0), (8, 1024)):
+            for slots in (None, call.ws.data_ptr()):
+                call.codes.zero_()
+                call.scale.fill_(-1.0)
+                rc = waits(kind, torch.cuda.current_stream().cuda_stream, call.x.data_ptr(), call.codes.data_ptr(), call.scale.data_ptr(), slots,
+                           chunks, n, grace, patience)
+                assert rc == 0
+                if store == QuantStore.Native:  # the bytes behind the last chunk are another kernel's
+                    tail = slice(chunks * per, n)
+                    assert not call.codes[tail].any()
+                    given = call.scale.to(call.x.dtype)
+                    qz.launch_ref(ComputeClient.current(), H(call.x[tail]), H(call.codes[tail]), H(given), H(torch.empty_like(call.scale)), call.scheme, elem)
+                call.check((chunks, grace, patience, slots is None))
