@@ -94,7 +94,7 @@ hipError_t launch_absmax_partials(hipStream_t s, int dtype, const void* input, u
 // chunks, out_scale[0].  quantize_resident(): whether it is the faster way, and whether `slots` (kMaxPartials words of
 // workspace) are needed, as in a captured launch.
 enum class ResidentWay { kNone, kNumbered, kCaptured };
-ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& a);
+ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, const FlatArgs& a);
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& a, uint64_t num_elems, void* slots);
 // Per-tensor scale from the partials: out_dtype(f_dtype(2*absmax/(hi-lo))) stored at out[0].
 hipError_t launch_tensor_scale(hipStream_t s, int f_dtype, int out_dtype, const float* partials,

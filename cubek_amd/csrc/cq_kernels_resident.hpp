@@ -419,9 +419,9 @@ hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encodin
 
 }  // namespace resident
 
-ResidentWay quantize_resident(hipStream_t stream, int bits, const FlatArgs& f) {
-    const bool captured_too = quantize_stays_resident(f.num_chunks, bits, true);
-    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, false)) return ResidentWay::kNone;
+ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, const FlatArgs& f) {
+    const bool captured_too = quantize_stays_resident(f.num_chunks, bits, float_bytes, true);
+    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, float_bytes, false)) return ResidentWay::kNone;
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         units < static_cast<int>(resident::kGroups))

@@ -78,7 +78,12 @@ inline bool repack_stays(uint64_t bytes, bool whole_lines) {
 // Captured launches need one more in front, which marks their slots: from 60 MiB on (8 bits of bf16 48 MiB 23.3 -> 23.4,
 // 64 MiB 30.9 -> 27.0, of f32 64 MiB 26.1 -> 24.6), narrower codes from 96 MiB on (4 bits of bf16 64 MiB 27.1 -> 27.7, 128 MiB 52.9
 // -> 48.5, 2 bits of bf16 100 MiB 37.5 -> 37.4, of f32 100 MiB 35.5 -> 32.7, e2m1 of bf16 100 MiB 41.3 -> 35.7).
-inline bool quantize_stays_resident(uint64_t chunks, int bits, bool captured) {
+//
+// What is beyond the chip's 128 MiB is read twice here too, by fewer waves than the two passes have, which cost more than the one read
+// saves from 448 MiB on with a byte of codes for two of a tensor, from 768 MiB with one for four (8 bits of bf16 384 MiB 174 -> 154, 512 MiB 208 ->
+// 211, 4 GiB 1770 -> 1990; of f32 512 MiB 201 -> 171, 1 GiB 378 -> 377; 4 bits of bf16 512 MiB 201 -> 178, 1 GiB 380 -> 387).
+inline bool quantize_stays_resident(uint64_t chunks, int bits, int float_bytes, bool captured) {
+    if (chunks > (bits == 8 && float_bytes == 2 ? 448ull << 16 : 768ull << 16)) return false;
     if (captured) return chunks >= (bits == 8 ? 60ull << 16 : 96ull << 16);
     return chunks <= 16ull << 16 || chunks >= (bits == 8 ? 48ull << 16 : 56ull << 16);
 }

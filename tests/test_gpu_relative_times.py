@@ -2,7 +2,8 @@
 two or three times apart, which no comparison of results shows.  The limits leave half as much again for noise."""
 import pytest
 
-from cubek_amd import ComputeClient, ElemType, TensorHandleRef
+from cubek_amd import ComputeClient, ElemType, QuantScheme, TensorHandleRef
+from cubek_amd import quantize as qz
 from cubek_amd import reduce as rd
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +62,37 @@ def test_many_short_axes_as_fast_as_one_of_the_same_bytes():
     """[34978, 9, 23] along 9: 54 us with a workgroup for each of its matrices."""
     many, one = micros(max_abs(ElemType.BF16, 9, 23, 0, outer=(34978,)), max_abs(ElemType.BF16, 9, 34978 * 23, 0))
     assert many < 2.5 * one, (many, one)
+
+
+def one_scale(mib, streams):
+    """The time of a quantize with one scale of a bf16 tensor on each stream, until all of them have ended."""
+    import time
+
+    import torch
+
+    h, scheme, calls = TensorHandleRef.from_torch, QuantScheme.default(), []
+    for s in streams:
+        x = torch.empty(mib << 19, dtype=torch.bfloat16, device="cuda").normal_()
+        codes = torch.empty(scheme.packed_shape(x.shape), dtype=torch.int32, device="cuda")
+        scale, ws = torch.empty(1, device="cuda"), torch.empty(1024, dtype=torch.uint8, device="cuda")
+        calls.append((s, h(x), h(codes), h(scale), ws, (x, codes, scale)))
+
+    def wall():
+        torch.cuda.synchronize()
+        begin = time.perf_counter()
+        for _ in range(10):
+            for s, x, codes, scale, ws, _ in calls:
+                with torch.cuda.stream(s):
+                    qz.launch_dynamic(ComputeClient.current(), x, codes, scale, scheme, ElemType.BF16, ws.data_ptr(), 1024)
+        torch.cuda.synchronize()
+        return (time.perf_counter() - begin) / 10
+
+    return min(wall() for _ in range(4))
+
+
+def test_four_times_the_tensor_takes_about_four_times_as_long():
+    """One scale for 1 GiB and for 4 GiB: 430 and 1770 us; 445 and 2800 where workgroups gave up waiting for one another."""
+    import torch
+
+    large, small = one_scale(4096, [torch.cuda.Stream()]), one_scale(1024, [torch.cuda.Stream()])
+    assert large < 5 * small, (large, small)

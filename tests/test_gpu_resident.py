@@ -246,3 +246,30 @@ def test_workgroups_that_work_out_the_shares_of_others(waits, kind, elem, value,
                     given = call.scale.to(call.x.dtype)
                     qz.launch_ref(ComputeClient.current(), H(call.x[tail]), H(call.codes[tail]), H(given), H(torch.empty_like(call.scale)), call.scheme, elem)
                 call.check((chunks, grace, patience, slots is None))
+
+
+def one_read(call):
+    """Whether a launch leaves the workspace alone: two passes write the workgroups' abs-maxima to it."""
+    call.ws.fill_(0x5A)
+    call.fused()
+    call.torch.cuda.synchronize()
+    return bool((call.ws == 0x5A).all())
+
+
+def test_sizes_of_one_read():
+    """Both sides of every line between one read and two passes (their results are the same)."""
+    import torch
+
+    def reads_once(elem, value, chunks):
+        per = 4 if elem == ElemType.F32 else 8
+        call = Call(torch, torch.empty(chunks * per, dtype=dtype_of(torch, elem), device="cuda").normal_(), elem, scheme_of(value))
+        call.fused()  # from here on the stream is one of the last two
+        return one_read(call)
+
+    mib = 1 << 16
+    assert reads_once(ElemType.BF16, QuantValue.Q8S, 4) and reads_once(ElemType.BF16, QuantValue.Q8S, 16 * mib)
+    assert not reads_once(ElemType.BF16, QuantValue.Q8S, 16 * mib + 4) and not reads_once(ElemType.BF16, QuantValue.Q8S, 48 * mib - 4)
+    assert reads_once(ElemType.BF16, QuantValue.Q8S, 48 * mib) and reads_once(ElemType.F16, QuantValue.Q8S, 448 * mib)
+    assert not reads_once(ElemType.BF16, QuantValue.Q8S, 448 * mib + 4) and reads_once(ElemType.F32, QuantValue.Q8S, 448 * mib + 4)
+    assert not reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib - 4) and reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib)
+    assert reads_once(ElemType.BF16, QuantValue.Q4S, 768 * mib) and not reads_once(ElemType.F32, QuantValue.Q4S, 768 * mib + 8)

@@ -133,3 +133,20 @@ def test_reductions_along_an_outer_axis_take_the_faster_way(answer):
     got = answer([f"{reduce_way(*case)} == ReduceWay::{way}" for case, way in REDUCE.items()])
     wrong = [case for case, right in zip(REDUCE, got) if not right]
     assert not wrong
+
+
+MIB = 1 << 16  # chunks
+# (chunks, bits, bytes of a float, captured): whether one read of the tensor is the faster way
+ONE_READ = {
+    (4, 8, 2, False): True, (16 * MIB, 8, 2, False): True, (16 * MIB + 4, 8, 2, False): False, (48 * MIB - 4, 8, 2, False): False,
+    (48 * MIB, 8, 2, False): True, (384 * MIB, 8, 2, False): True, (512 * MIB, 8, 2, False): False, (4096 * MIB, 8, 2, False): False,
+    (48 * MIB, 4, 2, False): False, (56 * MIB - 4, 4, 2, False): False, (56 * MIB, 4, 2, False): True, (640 * MIB, 4, 2, False): True, (1024 * MIB, 4, 2, False): False,
+    (48 * MIB, 8, 4, False): True, (640 * MIB, 8, 4, False): True, (2048 * MIB, 8, 4, False): False,
+    (4, 8, 2, True): False, (16 * MIB, 8, 2, True): False, (60 * MIB - 4, 8, 2, True): False, (60 * MIB, 8, 2, True): True, (512 * MIB, 8, 2, True): False,
+    (96 * MIB - 4, 4, 2, True): False, (96 * MIB, 4, 2, True): True, (96 * MIB, 2, 4, True): True, (2048 * MIB, 2, 4, True): False,
+}
+
+
+def test_one_scale_is_read_once_where_that_is_faster(answer):
+    got = answer([f"quantize_stays_resident({chunks}ull, {bits}, {size}, {str(captured).lower()})" for chunks, bits, size, captured in ONE_READ])
+    assert got == [int(once) for once in ONE_READ.values()], dict(zip(ONE_READ, got))
