@@ -365,6 +365,37 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_resident_kernel(Resident
         r.run();
 }
 
+// Whether `stream` is one of the last two that asked on this device.  Launches on two streams mostly take turns, but three or more at
+// once each get a part of the compute units, and a workgroup here holds one while it waits: bf16 to 8 bits on 2, 3, 4
+// streams, two passes and one, us a launch: 64 MiB 24.2 and 21.0, 25.2 and 37.6, 27.7 and 72; 128 MiB 53 and 38, 58 and 61, 58 and
+// 77; 256 MiB 115 and 90, 118 and 142, 120 and 172; 16 MiB on four 7.3 and 13.4.
+inline bool streams_are_few(int device, hipStream_t stream) {
+    struct Recent {
+        std::atomic<uintptr_t> streams[2]{~uintptr_t{0}, ~uintptr_t{0}};  // none yet
+    };
+    static Recent recent[16];
+    auto& [first, second] = recent[device % 16].streams;
+    const uintptr_t s = reinterpret_cast<uintptr_t>(stream);
+    const uintptr_t last = first.load(std::memory_order_relaxed), one_before = second.load(std::memory_order_relaxed);
+    if (s == last || s == one_before) return true;
+    first.store(s, std::memory_order_relaxed);
+    second.store(last, std::memory_order_relaxed);
+    return one_before == ~uintptr_t{0};
+}
+
+// Whether `stream` may use a compute unit for each workgroup.  With a mask of 128 or 200 of them, two passes and one, us: 64 MiB 33 and
+// 61, 28 and 61; 256 MiB 136 and 190, 128 and 187.
+inline bool has_every_unit(hipStream_t stream) {
+    uint32_t mask[kGroups / 32] = {};
+    if (hipExtStreamGetCUMask(stream, kGroups / 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    uint32_t units = 0;
+    for (uint32_t m : mask) units += static_cast<uint32_t>(__builtin_popcount(m));
+    return units == 0 || units >= kGroups;  // no bit: no mask
+}
+
 // The number of a launch of several workgroups; not 0.
 inline uint32_t next_number(int device) {
     static std::atomic<uint32_t> counts[16];
@@ -424,8 +455,9 @@ ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, con
     if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, float_bytes, false)) return ResidentWay::kNone;
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        units < static_cast<int>(resident::kGroups))
+        units < static_cast<int>(resident::kGroups) || !resident::streams_are_few(device, stream))
         return ResidentWay::kNone;
+    if (f.num_chunks > resident::kSome * resident::kThreads * resident::kGroups && !resident::has_every_unit(stream)) return ResidentWay::kNone;
     hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
     if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return ResidentWay::kNumbered;
     (void)hipGetLastError();  // the default stream during another one's capture: an error, for the launch to report

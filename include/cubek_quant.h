@@ -21,7 +21,8 @@
  *   - calls are re-entrant and thread safe.  The library's state is the per-thread code behind
  *     cq_last_hip_error(); one array per GPU inside the library's device code (128 KiB) through which the
  *     workgroups of a launch exchange abs-maxima, with a count of such launches (launches at once, on any
- *     streams, do not disturb one another's results); and, for cq_quantize_dynamic_static only, one scratch
+ *     streams, do not disturb one another's results) and the last two streams that made such a launch or would
+ *     have (on a third one the call takes two launches: the same results, and faster there); and, for cq_quantize_dynamic_static only, one scratch
  *     array per GPU, shared by all calls of that entry point on that GPU (see there).
  */
 #ifndef CUBEK_QUANT_H

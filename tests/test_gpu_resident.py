@@ -81,17 +81,17 @@ def test_small_sizes(elem, value, store):
 
 
 def test_many_small_launches():
-    """More launches than there are regions of slots, on four streams, each with its workspace; then
+    """More launches than there are regions of slots, on two streams, each with its workspace; then
     captured ones, replayed on new values between launches outside the graph."""
     import torch
 
     scheme = scheme_of(QuantValue.Q8S)
     calls = [Call(torch, values(torch, 8 * (512 * (3 + i) + 4), ElemType.BF16, i) * (i + 1), ElemType.BF16, scheme) for i in range(100)]
-    streams = [torch.cuda.Stream() for _ in range(4)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
     torch.cuda.synchronize()
     for _ in range(2):
         for i, call in enumerate(calls):
-            with torch.cuda.stream(streams[i % 4]):
+            with torch.cuda.stream(streams[i % 2]):
                 call.fused()
     torch.cuda.synchronize()
     for i, call in enumerate(calls):
@@ -273,3 +273,35 @@ def test_sizes_of_one_read():
     assert not reads_once(ElemType.BF16, QuantValue.Q8S, 448 * mib + 4) and reads_once(ElemType.F32, QuantValue.Q8S, 448 * mib + 4)
     assert not reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib - 4) and reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib)
     assert reads_once(ElemType.BF16, QuantValue.Q4S, 768 * mib) and not reads_once(ElemType.F32, QuantValue.Q4S, 768 * mib + 8)
+
+
+def test_two_passes_on_a_third_stream_and_on_part_of_the_compute_units():
+    import torch
+
+    call = Call(torch, values(torch, (48 << 16) * 8, ElemType.BF16, 1), ElemType.BF16, scheme_of(QuantValue.Q8S))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+
+    def on(i):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[i]):
+            return one_read(call)
+
+    on(0), on(1)
+    assert [on(i) for i in (0, 1, 0, 1)] == [True] * 4
+    assert not on(2) and on(2) and on(1) and not on(0)
+    call.check("streams")
+
+    hip = ctypes.CDLL("libamdhip64.so")
+    half, stream = (ctypes.c_uint32 * 8)(*[0xffffffff] * 4 + [0] * 4), ctypes.c_void_p()
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(stream), 8, half) == 0
+    masked = torch.cuda.ExternalStream(stream.value)
+    for _ in range(2):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(masked):
+            assert not one_read(call)
+    call.check("mask")
+    small = Call(torch, values(torch, 8 * 512 * 100, ElemType.BF16, 2), ElemType.BF16, scheme_of(QuantValue.Q8S))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(masked):
+        assert one_read(small)
+    small.check("mask, small")
