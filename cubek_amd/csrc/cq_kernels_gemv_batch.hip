@@ -27,6 +27,7 @@
 
 #include "../../include/cubek_quant_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 
 namespace cq {
 namespace {
@@ -333,39 +334,16 @@ void launch_shape(hipStream_t s, const GemvArgs& a) {
                        static_cast<uint32_t>(a.x_stride * 2), a.y_stride);
 }
 
-// How many row groups share a workgroup's x, and how many waves share a row.  x comes from the L2 once per workgroup, so
-// row groups together save L2 traffic; a launch wants a workgroup per compute unit and eight waves in each; and since
-// the arithmetic bounds it, it ends with the compute unit that has the most row groups: with 600 of them, 1 x 4 leaves at most
-// three on one, 2 x 4 four.  Measured on MI355X, us, kG x kS:
-// * up to 256 groups, one to a compute unit: 1 x 8 as long as its LDS fits one (1 x 4, 1 x 8: e4m3 bytes, 112 groups, 9088 columns,
-//   16 vectors 16.5, 11.7; 4 bits, 193 groups, 12288 columns, 12 vectors 13.6, 11.9), but not for the one round that it saves of 9 to
-//   12 stages where it leaves a compute unit one workgroup (117 groups, 91 units, 8 vectors 5.6, 5.9).
-// * up to 512: 1 x 8 while two workgroups of it fit a compute unit's LDS, 80 KiB each; past that 1 x 4, but 2 x 4 for the widest x
-//   (1 x 4, 2 x 4: 4 bits, 503 groups, 16 vectors 10.2, 7.4; 494 groups, 5 vectors 26.8, 29.2).
-// * up to 1024: 4 x 2 for a wide x (2 x 4, 4 x 2: 4 bits, 990 groups, 16 vectors 9.1, 6.6; 661 groups, 12 vectors 9.2, 7.0), else 1 x 4 up to
-//   768 (2 x 4, 1 x 4: 589 groups, 3 vectors 35.5, 28.9; 727 groups, 4 vectors 25.7, 22.1), 2 x 4 above (896 groups, 8 vectors 11.5, 12.7).
-// * up to 1536: 1 x 4 for a narrow x, 2 x 4 for a middling one (4 x 2, 2 x 4, 1 x 4: 1416 groups, 2 vectors 79.7, 62.0, 58.4; 8 bits, 1306
-//   groups, 16 vectors 155, 132, 146), not for rows of a few stages (1274 groups, 44 units 8.6, 9.2, 9.2) nor for e4m3 and e5m2 bytes,
-//   which wait for memory (1200 groups, 7 vectors 29.4, 32.6, 34.7).
-// * else 4 x 2 (4-bit bf16 [28672, 8192], 16 vectors 4 x 2, 2 x 4, 1 x 4 37.7, 49.6, 64.5).
 template <dev::Float kF, class FS, int kCode>
 void launch_code(hipStream_t s, const GemvArgs& a) {
-    const uint32_t groups = (a.rows + 15) / 16, x = x_bytes<kCode>(a.vectors), lds_of_eight = 2 * 8 * (x + kWaveBytes);
-    const bool wide = x >= 6 * 1024, long_rows = a.cols / values_per_unit(kCode) >= 6 * kU, bytes = kCode == kCodeE4M3 || kCode == kCodeE5M2;
-    const uint32_t stages = (a.cols / values_per_unit(kCode) + kU - 1) / kU;
-    const bool eight = stages <= 8 || stages > 12 || lds_of_eight <= 80 * 1024;
-    if (groups <= 256 ? eight && lds_of_eight <= 160 * 1024 : groups <= 512 && lds_of_eight <= 80 * 1024)
-        launch_shape<kF, FS, kCode, 1, 8>(s, a);
-    else if (groups <= 256)
-        launch_shape<kF, FS, kCode, 1, 4>(s, a);
-    else if (groups <= 512)
-        lds_of_eight > 160 * 1024 ? launch_shape<kF, FS, kCode, 2, 4>(s, a) : launch_shape<kF, FS, kCode, 1, 4>(s, a);
-    else if (groups <= 1024 && !wide)
-        groups <= 768 ? launch_shape<kF, FS, kCode, 1, 4>(s, a) : launch_shape<kF, FS, kCode, 2, 4>(s, a);
-    else if (groups > 1024 && groups <= 1536 && !wide && long_rows && !bytes)
-        x <= 2 * 1024 ? launch_shape<kF, FS, kCode, 1, 4>(s, a) : launch_shape<kF, FS, kCode, 2, 4>(s, a);
-    else
-        launch_shape<kF, FS, kCode, 4, 2>(s, a);
+    const uint32_t units = a.cols / values_per_unit(kCode), x = x_bytes<kCode>(a.vectors);
+    static_assert(kU == 8, "the stages of gemv_batch_shape()");
+    switch (gemv_batch_shape((a.rows + 15) / 16, x, 2 * 8 * (x + kWaveBytes), units, kCode == kCodeE4M3 || kCode == kCodeE5M2)) {
+        case GemvShape::k1x8: return launch_shape<kF, FS, kCode, 1, 8>(s, a);
+        case GemvShape::k1x4: return launch_shape<kF, FS, kCode, 1, 4>(s, a);
+        case GemvShape::k2x4: return launch_shape<kF, FS, kCode, 2, 4>(s, a);
+        case GemvShape::k4x2: return launch_shape<kF, FS, kCode, 4, 2>(s, a);
+    }
 }
 
 template <dev::Float kF, class FS>

@@ -173,4 +173,35 @@ inline ReduceWay reduce_way(const ReduceColumns& c) {
     return one ? ReduceWay::kOneLaunch : ReduceWay::kPlan;
 }
 
+// A product with several vectors (cq_kernels_gemv_batch.hip): how many row groups share a workgroup's x, and how many waves share a
+// row (kG x kS).  x comes from the L2 once per workgroup, so
+// row groups together save L2 traffic; a launch wants a workgroup per compute unit and eight waves in each; and since
+// the arithmetic bounds it, it ends with the compute unit that has the most row groups: with 600 of them, 1 x 4 leaves at most
+// three on one, 2 x 4 four.  Measured on MI355X, us, kG x kS:
+// * up to 256 groups, one to a compute unit: 1 x 8 as long as its LDS fits one (1 x 4, 1 x 8: e4m3 bytes, 112 groups, 9088 columns,
+//   16 vectors 16.5, 11.7; 4 bits, 193 groups, 12288 columns, 12 vectors 13.6, 11.9; six stages 115 groups, 5 vectors 3.95, 3.69), but where
+//   it leaves a compute unit one workgroup not for up to four stages, which are one round either way (4 bits, 148 groups, 10 units, 5 vectors
+//   3.16, 3.52; 8 bits, 226 groups, 32 units, 12 vectors 2.92, 3.24), nor for the one round that it saves of 9 to 12 (117 groups, 91 units, 8
+//   vectors 5.6, 5.9).
+// * up to 512: 1 x 8 while two workgroups of it fit a compute unit's LDS, 80 KiB each; past that 1 x 4, but 2 x 4 for the widest x
+//   (1 x 4, 2 x 4: 4 bits, 503 groups, 16 vectors 10.2, 7.4; 494 groups, 5 vectors 26.8, 29.2).
+// * up to 1024: 4 x 2 for a wide x (2 x 4, 4 x 2: 4 bits, 990 groups, 16 vectors 9.1, 6.6; 661 groups, 12 vectors 9.2, 7.0), else 1 x 4 up to
+//   768 (2 x 4, 1 x 4: 589 groups, 3 vectors 35.5, 28.9; 727 groups, 4 vectors 25.7, 22.1), 2 x 4 above (896 groups, 8 vectors 11.5, 12.7).
+// * up to 1536: 1 x 4 for a narrow x, 2 x 4 for a middling one (4 x 2, 2 x 4, 1 x 4: 1416 groups, 2 vectors 79.7, 62.0, 58.4; 8 bits, 1306
+//   groups, 16 vectors 155, 132, 146), not for rows of a few stages (1274 groups, 44 units 8.6, 9.2, 9.2) nor for e4m3 and e5m2 bytes,
+//   which wait for memory (1200 groups, 7 vectors 29.4, 32.6, 34.7).
+// * else 4 x 2 (4-bit bf16 [28672, 8192], 16 vectors 4 x 2, 2 x 4, 1 x 4 37.7, 49.6, 64.5).
+enum class GemvShape { k1x8, k1x4, k2x4, k4x2 };
+// `x`: bytes of a stage of x; lds_of_eight: of a workgroup of 1 x 8; `units` of a row, eight to a stage; `bytes`: e4m3 and e5m2
+inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_eight, uint32_t units, bool bytes) {
+    const bool wide = x >= 6 * 1024;
+    const uint32_t stages = (units + 7) / 8;
+    const bool eight = (stages > 4 && stages <= 8) || stages > 12 || lds_of_eight <= 80 * 1024;
+    if (groups <= 256) return eight && lds_of_eight <= 160 * 1024 ? GemvShape::k1x8 : GemvShape::k1x4;
+    if (groups <= 512) return lds_of_eight <= 80 * 1024 ? GemvShape::k1x8 : lds_of_eight > 160 * 1024 ? GemvShape::k2x4 : GemvShape::k1x4;
+    if (groups <= 1024 && !wide) return groups <= 768 ? GemvShape::k1x4 : GemvShape::k2x4;
+    if (groups > 1024 && groups <= 1536 && !wide && units >= 48 && !bytes) return x <= 2 * 1024 ? GemvShape::k1x4 : GemvShape::k2x4;
+    return GemvShape::k4x2;
+}
+
 }  // namespace cq

@@ -150,3 +150,25 @@ ONE_READ = {
 def test_one_scale_is_read_once_where_that_is_faster(answer):
     got = answer([f"quantize_stays_resident({chunks}ull, {bits}, {size}, {str(captured).lower()})" for chunks, bits, size, captured in ONE_READ])
     assert got == [int(once) for once in ONE_READ.values()], dict(zip(ONE_READ, got))
+
+
+# (row groups, columns, vectors, values in 16 bytes of codes, e4m3 or e5m2): the shape that was the fastest, or within 5 % of it
+GEMV = {
+    # up to four stages of 8 x 16 bytes of codes are one round of four waves
+    (148, 320, 5, 32, False): "k1x4", (160, 512, 5, 32, False): "k1x4", (175, 576, 7, 32, False): "k1x4", (226, 512, 12, 16, False): "k1x4",
+    (171, 384, 16, 16, True): "k1x4", (252, 960, 7, 32, False): "k1x4", (64, 512, 3, 32, False): "k1x8",
+    # five to eight are two rounds of four waves and one of eight
+    (115, 1440, 5, 32, False): "k1x8", (163, 1728, 5, 32, False): "k1x8", (83, 800, 12, 16, False): "k1x8", (46, 1952, 7, 32, False): "k1x8",
+    (117, 2912, 8, 32, False): "k1x4", (145, 3840, 6, 32, False): "k1x8", (112, 9088, 16, 16, True): "k1x8", (193, 12288, 12, 32, False): "k1x8",
+    (896, 4096, 8, 32, False): "k2x4", (1792, 8192, 16, 32, False): "k4x2", (589, 8192, 3, 32, False): "k1x4", (990, 8192, 16, 32, False): "k4x2",
+}
+
+
+def test_products_with_several_vectors_take_the_fastest_shape(answer):
+    def shape(groups, cols, vectors, per_unit, is_bytes):
+        x = (vectors * 2 * 8 * per_unit + 1023) // 1024 * 1024
+        return f"gemv_batch_shape({groups}, {x}, {16 * (x + 2560)}, {cols // per_unit}, {str(is_bytes).lower()})"
+
+    got = answer([f"{shape(*case)} == GemvShape::{want}" for case, want in GEMV.items()])
+    wrong = [case for case, right in zip(GEMV, got) if not right]
+    assert not wrong
