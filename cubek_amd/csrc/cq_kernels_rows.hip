@@ -19,6 +19,7 @@
 //   absmax_rows_kernel        per-tensor abs-max partials over strided rows
 #include "cq_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 
 namespace cq {
 namespace {
@@ -683,18 +684,15 @@ bool blocks_geom(uint32_t per_chunk, uint32_t bits, const RowArgs& a, BlocksGeom
     return tiles < (1ull << 31);
 }
 
-// Whether quantize_block_tiles_kernel takes the launch: its lanes along the row, and how many chunks of a block's column each
-// lane would hold in a workgroup of 256.
 bool block_tiles_geom(uint32_t per_chunk, const RowArgs& a, BlockTilesGeom* g, uint32_t* per_lane) {
     if (a.rank < 2) return false;
-    const uint32_t last = a.rank - 1, br = a.block[last - 1], cpb = a.block[last] / per_chunk;
-    if ((br & (br - 1)) != 0 || (cpb & (cpb - 1)) != 0 || cpb > 64 || a.rows / br > 65535) return false;
+    const uint32_t last = a.rank - 1;
+    const BlockTiles t = block_tiles_of(per_chunk == 4, a.block[last - 1], a.block[last] / per_chunk, a.rows, a.shape[last] / per_chunk);
+    if (t.per_lane == 0) return false;
     g->chunks_per_row = a.shape[last] / per_chunk;
-    g->cpb_log2 = g->tj_log2 = 0;
-    while ((1u << g->cpb_log2) < cpb) g->cpb_log2++;
-    while ((1u << g->tj_log2) < cpb || g->tj_log2 < 4 || (br << g->tj_log2) < kThreads) g->tj_log2++;
-    if (g->tj_log2 > 6 || g->chunks_per_row < (1u << g->tj_log2) || (br << g->tj_log2) > 4096) return false;
-    *per_lane = (br << g->tj_log2) / kThreads;
+    g->cpb_log2 = t.cpb_log2;
+    g->tj_log2 = t.tj_log2;
+    *per_lane = t.per_lane;
     g->pairs = aligned8(a.output);
     for (uint32_t d = 0; d < last; d++) g->pairs = g->pairs && a.vstride[d] % 2 == 0;
     return true;

@@ -204,4 +204,33 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
     return GemvShape::k4x2;
 }
 
+// Blocks over two dimensions, scale computed in the launch: whether quantize_block_tiles_kernel takes it (cq_kernels_rows.hip; per_lane 0:
+// no), its lanes along the row, and how many chunks of a block's column each lane would hold in a workgroup of 256.  Blocks of a few rows are one chunk a lane, and a large launch of those waits for its many
+// small workgroups to be dispatched (1.1 - 1.7 ns each): from kWideTileChunks on their tiles are wider, two or four chunks a lane.
+// quantize_blocks_kernel, one chunk, wider, us, blocks of 8 and 16 rows: bf16 [736, 7808] 6.2, 7.1, 4.0, [8880, 4800] 24.7, 38.9, 20.7, f16
+// [67136, 2048] 74.9, 121, 61.8, f32 [17392, 1728] 28.4, 33.5, 24.3.  Where blocks have four rows, or rows no room for 64 lanes, that is
+// the first of them's: f16 [103208, 320] 28.2, 41.9, bf16 [44832, 768] 26.8, 37.0, f32 [2984, 9344] 25.1, 29.9 (but [7864, 4864]
+// 53, 40); smaller ones of f32 are faster here, [30360, 256] 19.6, 9.0, unless the tiles are less than three quarters full ([310176, 80] 38.8, 43.4).
+constexpr uint64_t kWideTileChunks = 5u << 17;
+struct BlockTiles {
+    uint32_t per_lane, tj_log2, cpb_log2;
+};
+// blocks of `br` rows by `cpb` chunks, `rows` rows of `row_chunks`
+inline BlockTiles block_tiles_of(bool f32, uint32_t br, uint32_t cpb, uint64_t rows, uint32_t row_chunks) {
+    constexpr uint32_t kLanes = 256;
+    constexpr BlockTiles kNo = {0, 0, 0};
+    if (br == 0 || cpb == 0 || (br & (br - 1)) != 0 || (cpb & (cpb - 1)) != 0 || cpb > 64 || rows / br > 65535) return kNo;
+    uint32_t cpb_log2 = 0, tj_log2 = 0;
+    while ((1u << cpb_log2) < cpb) cpb_log2++;
+    while ((1u << tj_log2) < cpb || tj_log2 < 4 || (br << tj_log2) < kLanes) tj_log2++;
+    const uint64_t chunks = rows * row_chunks;
+    if (chunks >= kWideTileChunks && (br << tj_log2) == kLanes)
+        while (tj_log2 < 6 && (br << tj_log2) < 4 * kLanes && row_chunks >= (2u << tj_log2)) tj_log2++;
+    if (tj_log2 > 6 || row_chunks < (1u << tj_log2) || (br << tj_log2) > 4096) return kNo;
+    const uint32_t per_lane = (br << tj_log2) / kLanes;
+    const bool filled = row_chunks * 4 >= ((row_chunks + (1u << tj_log2) - 1) >> tj_log2 << tj_log2) * 3;
+    if (per_lane == 1 && chunks >= (f32 && filled ? 6u << 20 : 3u << 18)) return kNo;
+    return {per_lane, tj_log2, cpb_log2};
+}
+
 }  // namespace cq

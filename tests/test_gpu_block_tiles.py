@@ -68,6 +68,23 @@ def test_blocks_and_widths(elem, value, store):
             compare(torch, x, scheme.with_param(QuantParam(i % 3)), elem, what=(br, bc, cols))
 
 
+@pytest.mark.parametrize("elem", [ElemType.F32, ElemType.BF16], ids=lambda e: e.name)
+def test_large_launches_of_blocks_of_a_few_rows(elem):
+    """Both sides of the size from which their tiles are wider, with a whole and a cut last tile, and without room for wider ones."""
+    import torch
+
+    per = 4 if elem == ElemType.F32 else 8
+    scheme = QuantScheme.default().with_value(QuantValue.Q8S)
+    for br, bc in ((8, 32), (16, 64), (8, 128), (4, 64)):
+        for row_chunks in (64, 256, 224):
+            rows = -(-(5 << 17) // row_chunks // br) * br
+            for n in (rows - br, rows):
+                x = values(torch, (n, row_chunks * per), elem, br + n)
+                compare(torch, x, scheme.with_level(QuantLevel.block([br, bc])), elem, what=(br, bc, n, row_chunks))
+        x = values(torch, (br * (-(-(11 << 20) // 48 // br)), 48 * per), elem, br)
+        compare(torch, x, scheme.with_level(QuantLevel.block([br, 16])), elem, what=(br, 16), tiles=False)
+
+
 @pytest.mark.parametrize("elem", [ElemType.F32, ElemType.BF16, ElemType.F16], ids=lambda e: e.name)
 @pytest.mark.parametrize("value", [QuantValue.Q8S, QuantValue.Q4S], ids=lambda v: v.name)
 def test_layouts(elem, value):

@@ -172,3 +172,19 @@ def test_products_with_several_vectors_take_the_fastest_shape(answer):
     got = answer([f"{shape(*case)} == GemvShape::{want}" for case, want in GEMV.items()])
     wrong = [case for case, right in zip(GEMV, got) if not right]
     assert not wrong
+
+
+# (bytes of a float, rows and columns of a block, rows and columns): chunks per lane of the tile kernel, 0 where another is faster or it cannot
+BLOCK_TILES = {
+    (2, 128, 128, 14336, 4096): 8, (2, 64, 64, 14336, 4096): 4, (2, 32, 32, 2048, 4096): 2, (2, 32, 32, 128, 512): 2, (4, 64, 64, 14336, 4096): 4,
+    (2, 64, 64, 65536, 512): 4, (2, 32, 32, 65536, 288): 2, (2, 24, 32, 2400, 4096): 0, (2, 32, 48, 2048, 4800): 0, (2, 32, 32, 128, 96): 0,
+    # blocks of a few rows: one chunk, wider tiles from 10 MiB on, the general kernel where there is no room for those
+    (2, 8, 128, 744, 1792): 1, (2, 16, 64, 1104, 1408): 1, (2, 8, 128, 5840, 10112): 2, (2, 16, 64, 8512, 1472): 4, (4, 16, 16, 310176, 80): 0,
+    (2, 8, 32, 8880, 4800): 2, (4, 8, 64, 17392, 1728): 2, (2, 8, 32, 103208, 320): 0, (2, 4, 128, 5840, 1024): 1, (2, 4, 128, 44832, 768): 0,
+    (4, 4, 128, 30360, 256): 1, (4, 4, 128, 26088, 4096): 0,
+}
+
+
+def test_blocks_over_two_dimensions_take_the_faster_kernel(answer):
+    got = answer([f"block_tiles_of({str(size == 4).lower()}, {br}, {bc * size // 16}, {rows}, {cols * size // 16}).per_lane" for size, br, bc, rows, cols in BLOCK_TILES])
+    assert got == list(BLOCK_TILES.values()), dict(zip(BLOCK_TILES, got))
