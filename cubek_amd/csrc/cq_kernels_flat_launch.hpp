@@ -5,6 +5,7 @@
 
 #include <type_traits>
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 #include "cq_kernels_flat.hpp"
 
 namespace cq {
@@ -286,13 +287,6 @@ struct RunOffsets {
 // 300 000 chunks 4.5 and 3.4, 5.6 and 4.5, 2.95 and 2.99, 6.3 and 6.1; 2^19 4.85 and 4.26, 6.0 and 5.8, 3.4 and 3.9, 7.4 and
 // 7.5.  One line for all four, where the dequantize has nothing to gain any more.
 constexpr uint64_t kSmallRunChunks = 1u << 18;
-// Lane by lane the same: tiles of one step, a chunk per lane, for launches of fewer chunks.  There a tile of four steps is a few
-// workgroups' serial work, every step with a walk of its own over the levels.  Quantize and dequantize, us, tiles of several steps
-// and of one: f16 [16, 8, 3, 128] behind permuted dimensions 8.3 and 5.2, 120 tokens 9.5 and 6.7, 250 (512 000 chunks) 10.4 and 9.7,
-// 500 14.3 and 14.2; 4 bits of bf16 [16, 8, 500, 80] (640 000) 13.5 and 12.4, 1200 tokens 19.2 and 19.4, [20, 4, 980, 128] 14.5 and
-// 15.0; runs of 4 bits, blocks of 16, [1024, 1024] 7.4 and 5.0, [4096, 1024] 9.5 and 8.0; of 8 bits, blocks of 24, [2048, 1536] 8.3
-// and 8.1, [4096, 1536] (786 432) 11.3 and 11.6.
-constexpr uint64_t kSmallLaneChunks = 3u << 18;
 template <class WholeFn, class LanesFn>
 hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole, LanesFn lanes) {
     const uint64_t tile = static_cast<uint64_t>(kThreads) * unroll;
@@ -300,7 +294,7 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
     const int group = group_of(f_dtype, a.block);
     hipError_t e = hipSuccess;
     if (a.lanes.levels > 0) {
-        const bool one = a.rows * a.num_chunks < kSmallLaneChunks;
+        const bool one = a.rows * a.num_chunks < small_lane_chunks(a.any_group);
         lanes(lane_rows(a, one ? 1 : unroll), 0u, lanes_grid(a, one ? 1 : unroll), RunOffsets{0}, one);
         return hipGetLastError();
     }
@@ -315,7 +309,7 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         if (full < tiles) {
-            const bool one = full == 0 && lr.total_chunks < kSmallLaneChunks;
+            const bool one = full == 0 && lr.total_chunks < small_lane_chunks(a.any_group);
             lanes(lr, full, one ? grid_for(lr.total_chunks, 1) : tiles - full, RunOffsets{0}, one);
             e = hipGetLastError();
         }
@@ -333,7 +327,7 @@ hipError_t launch_flat(const FlatArgs& a, int f_dtype, int unroll, WholeFn whole
     const uint64_t piece = a.any_group == 0 ? (1ull << 30) : (1ull << 30) / (4ull * a.any_group) * (4ull * a.any_group);
     for (uint64_t begin = 0; begin < a.num_chunks; begin += piece) {
         const uint64_t n = a.num_chunks - begin < piece ? a.num_chunks - begin : piece;
-        const bool one = n < kSmallLaneChunks;
+        const bool one = n < small_lane_chunks(a.any_group);
         lanes(lane_rows_of_run(n), 0u, grid_for(n, one ? 1 : unroll), RunOffsets{begin}, one);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }

@@ -233,4 +233,14 @@ inline BlockTiles block_tiles_of(bool f32, uint32_t br, uint32_t cpb, uint64_t r
     return {per_lane, tj_log2, cpb_log2};
 }
 
+// Quantize and dequantize lane by lane (cq_kernels_flat_launch.hpp): tiles of one step, a chunk per lane, for launches of fewer chunks.  There a tile of four steps is a few
+// workgroups' serial work, every step with a walk of its own over the levels.  Quantize and dequantize, us, tiles of several steps
+// and of one: f16 [16, 8, 3, 128] behind permuted dimensions 8.3 and 5.2, 120 tokens 9.5 and 6.7, 250 (512 000 chunks) 10.4 and 9.7,
+// 500 14.3 and 14.2; 4 bits of bf16 [16, 8, 500, 80] (640 000) 13.5 and 12.4, 1200 tokens 19.2 and 19.4, [20, 4, 980, 128] 14.5 and
+// 15.0; runs of 4 bits, blocks of 16, [1024, 1024] 7.4 and 5.0, [4096, 1024] 9.5 and 8.0; of 8 bits, blocks of 24, [2048, 1536] 8.3
+// and 8.1, [4096, 1536] (786 432) 11.3 and 11.6.  Blocks that are no power of two of lanes lose earlier: of 48 f32 565 248 chunks 7.7 and
+// 8.3, f16 479 232 11.4 and 12.1, of 24 f16 639 744 8.6 and 9.5, bf16 314 880 7.3 and 6.5.
+// `any_group`: lanes per block that are no power of two, else 0
+inline uint64_t small_lane_chunks(uint32_t any_group) { return any_group != 0 ? 7u << 16 : 3u << 18; }
+
 }  // namespace cq

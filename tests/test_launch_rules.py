@@ -188,3 +188,11 @@ BLOCK_TILES = {
 def test_blocks_over_two_dimensions_take_the_faster_kernel(answer):
     got = answer([f"block_tiles_of({str(size == 4).lower()}, {br}, {bc * size // 16}, {rows}, {cols * size // 16}).per_lane" for size, br, bc, rows, cols in BLOCK_TILES])
     assert got == list(BLOCK_TILES.values()), dict(zip(BLOCK_TILES, got))
+
+
+def test_lanes_of_one_chunk_where_they_are_faster(answer):
+    """(chunks, lanes per block if no power of two)"""
+    cases = {(512000, 0): True, (640000, 0): True, (776192, 0): True, (819200, 0): False, (314880, 3): True, (393216, 3): True, (479232, 6): False,
+             (565248, 12): False, (639744, 3): False}
+    got = answer([f"{chunks} < small_lane_chunks({group})" for chunks, group in cases])
+    assert got == [int(one) for one in cases.values()], dict(zip(cases, got))
