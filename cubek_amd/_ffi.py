@@ -113,8 +113,8 @@ def calls():
         try:
             from . import _call
         except ImportError as e:
-            raise RuntimeError("native module not built: there is no fallback path. "
-                               "Build it with `make -C cubek_amd/csrc` (needs hipcc and Python's headers).") from e
+            raise RuntimeError("native module not built for this Python: there is no fallback path. "
+                               "Build it with `make -C cubek_amd/csrc PYTHON=...` (needs hipcc and Python's headers).") from e
         from .scheme import QuantScheme
         from .tensor import TensorHandleRef
 

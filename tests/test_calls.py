@@ -1,12 +1,15 @@
 """The package's calls (csrc/py_call.cpp) against the C ABI called with the structs that the handles and the scheme build: the same
 status for every descriptor that is refused before anything touches a GPU, and the same refusals of other Python objects."""
 import ctypes
+import os
+import subprocess
 
 import pytest
 
 from cubek_amd import (ElemType, QuantError, QuantLevel, QuantParam, QuantScheme, QuantStore, QuantValue, TensorHandleRef, ComputeClient,
                        _ffi, contiguous, dequantize, matvec, quantize, reduce)
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 P = 1 << 20  # never read: every call here is refused
 BLOCK = QuantScheme.default().with_value(QuantValue.Q4S).with_level(QuantLevel.block([32]))
 
@@ -89,3 +92,15 @@ def test_other_objects_are_refused():
     # a ctypes pointer and a ctypes integer go for numbers
     got = _ffi.calls().max_abs(ctypes.c_void_p(0), h, h, ctypes.c_uint32(1), ElemType.F16, ctypes.c_void_p(0), ctypes.c_size_t(0))
     assert got == _ffi.ERR_SHAPE_MISMATCH
+
+
+def test_the_module_is_named_after_the_interpreter_it_was_built_for():
+    import sysconfig
+
+    assert os.path.basename(_ffi.calls().__file__) == "_call" + sysconfig.get_config_var("EXT_SUFFIX")
+
+
+def test_the_library_builds_without_python():
+    made = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "cubek_amd", "csrc"), "native", "PYTHON=false"], stdout=subprocess.PIPE,
+                          stderr=subprocess.STDOUT, text=True)
+    assert made.returncode == 0 and "libcubek_quant_hip.so" in made.stdout and "py_call.cpp" not in made.stdout
