@@ -27,7 +27,8 @@ memory     = buffers are dropped between the cases but never handed back to the 
              tensors allocated out of memory that the process had released and mapped again made the larger
              matrix-vector launches 10 % slower (37.1 against 33.5 us) and the other kernels 0-3 %
 
-Prints ONE JSON line on stdout.
+Prints ONE JSON line on stdout, with the step's figures and the roofline in brief; everything that is measured goes to the file
+that --details names (bench_details.json beside this one).
 """
 from __future__ import annotations
 
@@ -961,12 +962,28 @@ def per_tensor_passes(torch):
     return out
 
 
+# What the printed line holds of the result: a line of all of it is 50 KB, which whoever keeps the last few KB of a log cannot parse.
+LINE = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline", "dtype", "data",
+        "config", "pct_hbm_peak", "elements_per_s")
+LINE_ROOFLINE = ("bound", "kernel", "achieved", "peak", "unit", "frac", "traffic", "median_launch_ms", "per_config", "min_frac_cfg3_5")
+
+
+def one_line(result) -> str:
+    line = {key: result[key] for key in LINE}
+    for name, keys in (("roofline", LINE_ROOFLINE), ("roofline_dequantize", ("achieved", "frac", "median_launch_ms")),
+                       ("first_call_ms", ("quantize_dynamic", "dequantize")), ("cpu_baseline", ("value", "unit", "cores"))):
+        if name in result:
+            line[name] = {key: result[name][key] for key in keys if key in result[name]}
+    return json.dumps(line)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=50)
     ap.add_argument("--warmup", type=int, default=10)
     ap.add_argument("--workload", default="cfg5", choices=sorted(WORKLOADS))
+    ap.add_argument("--details", default=os.path.join(ROOT, "bench_details.json"), help="file for everything that is measured")
     ap.add_argument("--no-sweep", action="store_true", help="skip the per-config table")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--adjacent-only", action="store_true",
@@ -1171,7 +1188,12 @@ def main():
             row[k]["frac_hbm_peak"] for row in table if row["workload"] in ("cfg3", "cfg4", "cfg5") for k in short)
         result["adjacent_kernels"] = adjacent_kernels(torch) + corner_layouts(torch) + per_tensor_passes(torch) + packed_gemv(torch)
 
-    print(json.dumps(result))
+    print(one_line(result))
+    try:
+        with open(args.details, "w") as f:
+            json.dump(result, f, indent=1)
+    except OSError as e:
+        print(f"details not written: {e}", file=sys.stderr)
 
 
 if __name__ == "__main__":

@@ -45,3 +45,26 @@ def test_bench_probe_library_loads():
                                       ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_uint32]
     assert L.cq_probe_transposed(0, 0, 0, None, None, None, None, 100, 256) == -1   # rows not in whole tiles
     assert L.cq_probe_transposed(1, 1, 1, None, None, None, None, 128, 0) == -1     # no columns
+
+
+def test_the_printed_line_is_short_and_whole():
+    """Everything that is measured goes to a file; the line holds the contract's fields and the roofline in brief."""
+    import json
+
+    import bench
+
+    fractions = {f"cfg{i}": {"dynamic": 0.7654, "given": 0.7654, "dequantize": 0.7654} for i in range(1, 6)}
+    roofline = dict(bound="hbm", kernel="quantize_flat_kernel (fused abs-max+scale+quantize+pack)", achieved=6536.3, peak=8000.0, unit="GB/s", frac=0.8171,
+                    traffic=616710144, median_launch_ms=0.0943, per_config=fractions, min_frac_cfg3_5=0.7543, in_step={"note": "x" * 300})
+    result = dict(metric="quant/dequant GB/s (bytes read+written) and % of MI355X HBM peak, 1 GPU", value=6991.5, unit="GB/s", n_gpus=1, steps=20, warmup=5,
+                  ms_per_step=0.1764, higher_is_better=True, scaling="weak", vs_baseline=None, dtype="bf16", data="synthetic",
+                  config=dict(workload="cfg5: " + "x" * 120, shape=[28672, 8192], block=32, value="E2M1", store="U32", param="F32",
+                              algorithmic_bytes_per_step=1233125376), pct_hbm_peak=87.4, elements_per_s=2663049705215, value_note="x" * 500,
+                  roofline=roofline, roofline_dequantize=roofline, first_call_ms={"quantize_dynamic": 1.8, "dequantize": 1.0, "library_bytes": 1},
+                  cpu_baseline={"value": 5.29, "unit": "GB/s", "cores": 16, "what": "x" * 200}, per_config=[{"x": "y" * 1000}] * 5)
+    line = bench.one_line(result)
+    assert len(line) < 1800 and "\n" not in line
+    got = json.loads(line)
+    for key in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline", "dtype", "data", "config"):
+        assert got[key] == result[key]
+    assert got["roofline"]["frac"] == 0.8171 and got["cpu_baseline"]["value"] == 5.29
