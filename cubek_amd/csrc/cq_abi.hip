@@ -1200,8 +1200,8 @@ static cq_status quantize_dynamic(cq_stream_t stream, const cq_tensor* input, co
         a.param_dtype = pd;
         a.encoding = flat_encoding(scheme);
         a.range = p.range;
-        const cq::ResidentWay way = wraps || g_probe.on ? cq::ResidentWay::kNone : cq::quantize_resident(stream, static_cast<int>(p.bits), static_cast<int>(dtype_size(input_dtype)), a);
-        if (way != cq::ResidentWay::kNone) {
+        const cq::ResidentWay way = wraps || g_probe.on ? cq::ResidentWay{} : cq::quantize_resident(stream, static_cast<int>(p.bits), static_cast<int>(dtype_size(input_dtype)), a);
+        if (way.take) {
             st = CQ_RUN(cq::flat_family(a, input_dtype), cq::launch_quantize_resident(stream, way, input_dtype, static_cast<int>(p.bits), a, p.n, workspace));
         } else {
             uint32_t num_partials = 0;

@@ -91,9 +91,12 @@ constexpr uint32_t kMaxPartials = 256;
 hipError_t launch_absmax_partials(hipStream_t s, int dtype, const void* input, uint64_t num_elems,
                                   float* partials, uint32_t* num_partials);
 // One scale per tensor in one read of it (cq_kernels_resident.hpp): abs-max of `num_elems` elements, codes of a.num_chunks
-// chunks, out_scale[0].  quantize_resident(): whether it is the faster way, and whether `slots` (kMaxPartials words of
-// workspace) are needed, as in a captured launch.
-enum class ResidentWay { kNone, kNumbered, kCaptured };
+// chunks, out_scale[0].  quantize_resident(): whether it is the faster way, and how: captured launches need `slots`
+// (kMaxPartials words of workspace), others are numbered per device.
+struct ResidentWay {
+    bool take = false, captured = false;
+    int device = 0;
+};
 ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, const FlatArgs& a);
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& a, uint64_t num_elems, void* slots);
 // Per-tensor scale from the partials: out_dtype(f_dtype(2*absmax/(hi-lo))) stored at out[0].

@@ -39,7 +39,7 @@ constexpr int kThreads = 512;
 constexpr uint32_t kGroups = 256;  // most workgroups = slots
 static_assert(kGroups <= kMaxPartials, "a captured launch's slots are the caller's workspace");
 constexpr uint32_t kUnset = 0xffffffffu, kStarted = 0xfffffffeu;  // no abs-maxima: NaN elements are ignored
-constexpr uint32_t kGrace = 8, kGraceOfSmall = 32, kPatience = 1024, kBySize = 0xffffffffu;  // polls
+constexpr uint32_t kGrace = 8, kGraceOfSmall = 32, kPatience = 1024, kBySize = 0xffffu;  // polls
 typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
 constexpr uint32_t kPerVector = 8;  // chunks
 
@@ -50,18 +50,18 @@ static __device__ uint64_t g_slots[kRegions * kGroups];
 
 __global__ __launch_bounds__(kGroups) void unset_slots_kernel(uint32_t* __restrict__ slots) { slots[threadIdx.x] = kUnset; }
 
-struct ResidentArgs {
+struct ResidentArgs {  // the first 16 words come in registers: what is read while others wait
     const void* in;
     void* out;
     uint32_t* slots;     // of a captured launch
     void* scale_out;
     uint64_t chunks;     // whole chunks that the launch quantizes
-    uint64_t num_elems;  // elements of the tensor: the abs-max covers those behind the chunks too
+    uint32_t tail;       // elements behind them, which the abs-max covers too
     uint32_t groups;     // workgroups, a power of two
     uint32_t rounds;     // steps of the busiest one
     uint32_t streamed;   // the first of them, read twice
     uint32_t number;     // of the launch; 0: a captured one, with slots in the workspace
-    uint32_t grace = kBySize, patience = kPatience;
+    uint16_t grace, patience;
     int param_dtype;
     QuantParams qp;
 };
@@ -125,8 +125,7 @@ struct Resident {
     }
     // the elements behind the last chunk: share 0 has them
     __device__ __forceinline__ float tail_absmax(uint32_t group, float acc) const {
-        const uint64_t e = a.chunks * kN + threadIdx.x;
-        if (group == 0 && e < a.num_elems) acc = fmaxf(acc, fabsf(F::load(a.in, e)));
+        if (group == 0 && threadIdx.x < a.tail) acc = fmaxf(acc, fabsf(F::load(a.in, a.chunks * kN + threadIdx.x)));
         return acc;
     }
     // another workgroup's share, a few loads at a time: the registers are full
@@ -289,9 +288,11 @@ struct Resident {
     }
     __device__ __forceinline__ void run() const {
         __shared__ u32x4 lds[kInLds][kThreads];
-        publish(blockIdx.x, kStarted);
         float amax = 0.0f;
-        if (a.streamed) amax = streamed_absmax(blockIdx.x, a.streamed, amax);
+        if (a.streamed) {
+            publish(blockIdx.x, kStarted);
+            amax = streamed_absmax(blockIdx.x, a.streamed, amax);
+        }
         amax = tail_absmax(blockIdx.x, amax);
         const Window w(a, a.streamed, kResident);
         const uint32_t held = a.rounds - a.streamed;  // of the kResident chunks: the others read as zeros, and are skipped
@@ -330,6 +331,7 @@ struct Resident {
                 }
             }
         }
+        if (!a.streamed) publish(blockIdx.x, kStarted);  // behind the loads, so that none of them waits for it
 #pragma unroll
         for (uint32_t u = 0; u < kInRegisters; u += 4) {
             if (u < held) {
@@ -406,7 +408,8 @@ inline uint32_t next_number(int device) {
 }
 
 template <class F, int kBits, int kEnc>
-hipError_t launch(hipStream_t s, ResidentWay way, ResidentArgs a) {
+hipError_t launch(hipStream_t s, ResidentWay way, ResidentArgs a, uint64_t num_elems) {
+    a.tail = static_cast<uint32_t>(num_elems - a.chunks * F::kPerChunk);
     const uint64_t steps = (a.chunks + kThreads - 1) / kThreads;
     a.groups = 1;
     if (steps > kSome)  // up to there a workgroup alone has nothing to wait for
@@ -416,13 +419,10 @@ hipError_t launch(hipStream_t s, ResidentWay way, ResidentArgs a) {
     a.streamed = a.rounds > kMost ? a.rounds - kMost : 0;
     if (a.grace == kBySize) a.grace = a.rounds > kSome ? kGrace : kGraceOfSmall;
     if (a.groups > 1) {
-        int device = 0;
-        if (way == ResidentWay::kCaptured)
+        if (way.captured)
             hipLaunchKernelGGL(unset_slots_kernel, dim3(1), dim3(kGroups), 0, s, a.slots);
-        else if (const hipError_t e = hipGetDevice(&device); e != hipSuccess)
-            return e;
         else
-            a.number = next_number(device);
+            a.number = next_number(way.device);
     }
     const auto kernel = a.rounds <= kFew    ? quantize_resident_kernel<F, kBits, kEnc, kFew, 0>
                         : a.rounds <= kSome ? quantize_resident_kernel<F, kBits, kEnc, kSome, 0>
@@ -432,18 +432,18 @@ hipError_t launch(hipStream_t s, ResidentWay way, ResidentArgs a) {
 }
 
 template <class F>
-hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encoding, const ResidentArgs& a) {
+hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encoding, const ResidentArgs& a, uint64_t num_elems) {
     switch (encoding) {
         case kEncInt:
             switch (bits) {
-                case 2: return launch<F, 2, kEncInt>(s, way, a);
-                case 4: return launch<F, 4, kEncInt>(s, way, a);
-                case 8: return launch<F, 8, kEncInt>(s, way, a);
+                case 2: return launch<F, 2, kEncInt>(s, way, a, num_elems);
+                case 4: return launch<F, 4, kEncInt>(s, way, a, num_elems);
+                case 8: return launch<F, 8, kEncInt>(s, way, a, num_elems);
             }
             break;
-        case kEncE4M3: return launch<F, 8, kEncE4M3>(s, way, a);
-        case kEncE5M2: return launch<F, 8, kEncE5M2>(s, way, a);
-        case kEncE2M1: return launch<F, 4, kEncE2M1>(s, way, a);
+        case kEncE4M3: return launch<F, 8, kEncE4M3>(s, way, a, num_elems);
+        case kEncE5M2: return launch<F, 8, kEncE5M2>(s, way, a, num_elems);
+        case kEncE2M1: return launch<F, 4, kEncE2M1>(s, way, a, num_elems);
     }
     return hipErrorInvalidValue;
 }
@@ -452,16 +452,16 @@ hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encodin
 
 ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, const FlatArgs& f) {
     const bool captured_too = quantize_stays_resident(f.num_chunks, bits, float_bytes, true);
-    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, float_bytes, false)) return ResidentWay::kNone;
+    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, float_bytes, false)) return {};
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         units < static_cast<int>(resident::kGroups) || !resident::streams_are_few(device, stream))
-        return ResidentWay::kNone;
-    if (f.num_chunks > resident::kSome * resident::kThreads * resident::kGroups && !resident::has_every_unit(stream)) return ResidentWay::kNone;
+        return {};
+    if (f.num_chunks > resident::kSome * resident::kThreads * resident::kGroups && !resident::has_every_unit(stream)) return {};
     hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
-    if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return ResidentWay::kNumbered;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return {true, false, device};
     (void)hipGetLastError();  // the default stream during another one's capture: an error, for the launch to report
-    return captured_too ? ResidentWay::kCaptured : ResidentWay::kNone;
+    return {captured_too, true, device};
 }
 
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {
@@ -471,13 +471,14 @@ hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, i
     a.slots = static_cast<uint32_t*>(slots);
     a.scale_out = f.scale_out;
     a.chunks = f.num_chunks;
-    a.num_elems = num_elems;
+    a.grace = resident::kBySize;
+    a.patience = resident::kPatience;
     a.param_dtype = f.param_dtype;
     a.qp = quant_params(f.range);
     switch (dtype) {
-        case CQ_F32: return resident::launch_encoding<F32>(s, way, bits, f.encoding, a);
-        case CQ_BF16: return resident::launch_encoding<BF16>(s, way, bits, f.encoding, a);
-        case CQ_F16: return resident::launch_encoding<F16>(s, way, bits, f.encoding, a);
+        case CQ_F32: return resident::launch_encoding<F32>(s, way, bits, f.encoding, a, num_elems);
+        case CQ_BF16: return resident::launch_encoding<BF16>(s, way, bits, f.encoding, a, num_elems);
+        case CQ_F16: return resident::launch_encoding<F16>(s, way, bits, f.encoding, a, num_elems);
         default: return hipErrorInvalidValue;
     }
 }

@@ -13,12 +13,11 @@ extern "C" int cq_test_resident(int kind, void* stream, const void* in, void* ou
     a.slots = static_cast<uint32_t*>(slots);
     a.scale_out = scale;
     a.chunks = chunks;
-    a.num_elems = num_elems;
     a.param_dtype = CQ_F32;
-    a.grace = grace;
-    a.patience = patience;
+    a.grace = static_cast<uint16_t>(grace);
+    a.patience = static_cast<uint16_t>(patience);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const ResidentWay way = slots == nullptr ? ResidentWay::kNumbered : ResidentWay::kCaptured;
+    const ResidentWay way{true, slots != nullptr, 0};
     Range range{};
     switch (kind) {
         case 0: range.lo = -127.0f, range.hi = 127.0f; break;
@@ -28,8 +27,8 @@ extern "C" int cq_test_resident(int kind, void* stream, const void* in, void* ou
     }
     a.qp = quant_params(range);
     switch (kind) {
-        case 0: return resident::launch<BF16, 8, kEncInt>(s, way, a);
-        case 1: return resident::launch<F32, 4, kEncInt>(s, way, a);
-        default: return resident::launch<F16, 8, kEncE4M3>(s, way, a);
+        case 0: return resident::launch<BF16, 8, kEncInt>(s, way, a, num_elems);
+        case 1: return resident::launch<F32, 4, kEncInt>(s, way, a, num_elems);
+        default: return resident::launch<F16, 8, kEncE4M3>(s, way, a, num_elems);
     }
 }
