@@ -207,9 +207,9 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
 // Blocks over two dimensions, scale computed in the launch: whether quantize_block_tiles_kernel takes it (cq_kernels_rows.hip; per_lane 0:
 // no), its lanes along the row, and how many chunks of a block's column each lane would hold in a workgroup of 256.  Blocks of a few rows are one chunk a lane, and a large launch of those waits for its many
 // small workgroups to be dispatched (1.1 - 1.7 ns each): from kWideTileChunks on their tiles are wider, two or four chunks a lane.
-// quantize_blocks_kernel, one chunk, wider, us, blocks of 8 and 16 rows: bf16 [736, 7808] 6.2, 7.1, 4.0, [8880, 4800] 24.7, 38.9, 20.7, f16
-// [67136, 2048] 74.9, 121, 61.8, f32 [17392, 1728] 28.4, 33.5, 24.3.  Where blocks have four rows, or rows no room for 64 lanes, that is
-// the first of them's: f16 [103208, 320] 28.2, 41.9, bf16 [44832, 768] 26.8, 37.0, f32 [2984, 9344] 25.1, 29.9 (but [7864, 4864]
+// quantize_blocks_kernel, one chunk, wider, us: 8 x 128 bf16 [736, 7808] 6.2, 7.2, 3.9, 8 x 32 [8880, 4800] 24.3, 37.2, 20.0, 16 x 64 f16
+// [67136, 2048] 73.7, 112, 61.6, f32 [17392, 1728] 29.2, 33.0, 23.9.  Where blocks have four rows, or rows no room for 64 lanes, that is
+// the first of them's: 8 x 32 f16 [103208, 320] 29.2, 42.9, 4 x 128 bf16 [44832, 768] 26.9, 38.1, f32 [2984, 9344] 25.1, 29.9 (but [7864, 4864]
 // 53, 40); smaller ones of f32 are faster here, [30360, 256] 19.6, 9.0, unless the tiles are less than three quarters full ([310176, 80] 38.8, 43.4).
 constexpr uint64_t kWideTileChunks = 5u << 17;
 struct BlockTiles {

@@ -1,4 +1,4 @@
-"""The lane-wise kernels by the size of a launch: one chunk per lane below kSmallLaneChunks (cq_kernels_flat_launch.hpp), several from
+"""The lane-wise kernels by the size of a launch: one chunk per lane below small_lane_chunks() (cq_launch_rules.hpp), several from
 there on.  The other tests hold small launches against the oracle; here a large launch has to give, bit for bit, what small
 ones give on its parts, and small ones what the kernels over contiguous runs give."""
 import pytest
