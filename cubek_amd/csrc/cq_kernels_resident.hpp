@@ -451,17 +451,20 @@ hipError_t launch_encoding(hipStream_t s, ResidentWay way, int bits, int encodin
 }  // namespace resident
 
 ResidentWay quantize_resident(hipStream_t stream, int bits, int float_bytes, const FlatArgs& f) {
-    const bool captured_too = quantize_stays_resident(f.num_chunks, bits, float_bytes, true);
-    if (!captured_too && !quantize_stays_resident(f.num_chunks, bits, float_bytes, false)) return {};
+    const bool numbered = quantize_stays_resident(f.num_chunks, bits, float_bytes, false);
+    const bool captured = quantize_stays_resident(f.num_chunks, bits, float_bytes, true);
+    if (!numbered && !captured) return {};
     int device = 0, units = 0;  // a partition of the GPU with fewer compute units would run the workgroups in turns
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        units < static_cast<int>(resident::kGroups) || !resident::streams_are_few(device, stream))
+        units < static_cast<int>(resident::kGroups))
         return {};
-    if (f.num_chunks > resident::kSome * resident::kThreads * resident::kGroups && !resident::has_every_unit(stream)) return {};
     hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
-    if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) return {true, false, device};
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone) {
+        const bool large = f.num_chunks > resident::kSome * resident::kThreads * resident::kGroups;
+        return {numbered && resident::streams_are_few(device, stream) && !(large && !resident::has_every_unit(stream)), false, device};
+    }
     (void)hipGetLastError();  // the default stream during another one's capture: an error, for the launch to report
-    return {captured_too, true, device};
+    return {captured, true, device};  // replays may be on any stream
 }
 
 hipError_t launch_quantize_resident(hipStream_t s, ResidentWay way, int dtype, int bits, const FlatArgs& f, uint64_t num_elems, void* slots) {

@@ -75,17 +75,23 @@ inline bool repack_stays(uint64_t bytes, bool whole_lines) {
 // 11.4 -> 11.7, 48 MiB 17.4 -> 15.7; 4 bits of bf16 16 MiB 8.6 -> 8.2, 24 MiB 10.8 -> 11.1, 48 MiB 17.8 -> 17.9, 60 MiB 22.1 -> 21.4;
 // e4m3 of f16 48 MiB 20.3 -> 20.1.
 //
-// Captured launches need one more in front, which marks their slots: from 60 MiB on (8 bits of bf16 48 MiB 23.3 -> 23.4,
-// 64 MiB 30.9 -> 27.0, of f32 64 MiB 26.1 -> 24.6), narrower codes from 96 MiB on (4 bits of bf16 64 MiB 27.1 -> 27.7, 128 MiB 52.9
-// -> 48.5, 2 bits of bf16 100 MiB 37.5 -> 37.4, of f32 100 MiB 35.5 -> 32.7, e2m1 of bf16 100 MiB 41.3 -> 35.7).
+// Two bits of 16-bit floats have the least to write and lose until 128 MiB: bf16 56 MiB 20.0 -> 21.8, 80 MiB 26.9 -> 28.5, 112 MiB even, 128
+// MiB 0.97 of the two.
+//
+// Captured launches need one more in front, which marks their slots: of 8 bits from 72 MiB on for 16-bit floats (f16 to e4m3 64 MiB 24.9 ->
+// 26.3, 72 MiB 1.02 of the two; bf16 72 MiB 0.92), from 60 for f32 (64 MiB 26.1 -> 24.6), of narrower codes from 120 MiB (f16, 4 bits 100
+// MiB 34.7 -> 36.2, 120 MiB 0.99) and 96 for f32 (2 bits 100 MiB 35.5 -> 32.7), not for two bits of 16-bit floats (f16 200 MiB 63.7 -> 68.0).
 //
 // What is beyond the chip's 128 MiB is read twice here too, by fewer waves than the two passes have, which cost more than the one read
-// saves from 448 MiB on with a byte of codes for two of a tensor, from 768 MiB with one for four (8 bits of bf16 384 MiB 174 -> 154, 512 MiB 208 ->
-// 211, 4 GiB 1770 -> 1990; of f32 512 MiB 201 -> 171, 1 GiB 378 -> 377; 4 bits of bf16 512 MiB 201 -> 178, 1 GiB 380 -> 387).
+// saves: past 384 MiB (captured 448) with a byte of codes for two of a tensor, past 768 MiB with one for four (8 bits of bf16 384 MiB 174 ->
+// 154, 400 MiB 1.01 of the two, captured 448 MiB 177 -> 169, 4 GiB 1770 -> 1990; of f32 512 MiB 201 -> 171, 1 GiB 378 -> 377; 4 bits of bf16
+// 512 MiB 201 -> 178, 1 GiB 380 -> 387).
 inline bool quantize_stays_resident(uint64_t chunks, int bits, int float_bytes, bool captured) {
-    if (chunks > (bits == 8 && float_bytes == 2 ? 448ull << 16 : 768ull << 16)) return false;
-    if (captured) return chunks >= (bits == 8 ? 60ull << 16 : 96ull << 16);
-    return chunks <= 16ull << 16 || chunks >= (bits == 8 ? 48ull << 16 : 56ull << 16);
+    constexpr uint64_t kMiB = 1 << 16;
+    const bool f32 = float_bytes == 4;
+    if (chunks > (bits == 8 && !f32 ? (captured ? 448 : 384) : 768) * kMiB) return false;
+    if (captured) return bits == 8 ? chunks >= (f32 ? 60 : 72) * kMiB : f32 ? chunks >= 96 * kMiB : bits == 4 && chunks >= 120 * kMiB;
+    return chunks <= 16 * kMiB || chunks >= (bits == 8 ? 48 : bits == 2 && !f32 ? 128 : 56) * kMiB;
 }
 
 inline uint32_t pow2_at_least(uint64_t v, uint32_t cap) {

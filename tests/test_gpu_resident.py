@@ -115,7 +115,7 @@ def test_many_small_launches():
 
 KINDS = [(QuantValue.Q8S, QuantStore.U32, 60), (QuantValue.Q8F, QuantStore.U32, 61), (QuantValue.E4M3, QuantStore.Native, 64),
          (QuantValue.E5M2, QuantStore.Native, 65), (QuantValue.Q8S, QuantStore.Native, 48 + 13), (QuantValue.Q4S, QuantStore.U32, 96),
-         (QuantValue.Q4F, QuantStore.U32, 113), (QuantValue.Q2S, QuantStore.U32, 97), (QuantValue.E2M1, QuantStore.Native, 96),
+         (QuantValue.Q4F, QuantStore.U32, 113), (QuantValue.Q2S, QuantStore.U32, 129), (QuantValue.E2M1, QuantStore.Native, 96),
          (QuantValue.E2M1_OCP, QuantStore.U32, 96)]
 
 
@@ -188,7 +188,7 @@ def test_streams_and_graphs():
     one that has not started), and a captured launch replayed on new values."""
     import torch
 
-    n = (64 << 16) * 8
+    n = (80 << 16) * 8
     scheme = scheme_of(QuantValue.Q8S)
     calls = [Call(torch, values(torch, n + 8 * 64 * i, ElemType.BF16, i), ElemType.BF16, scheme) for i in range(4)]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
@@ -269,9 +269,10 @@ def test_sizes_of_one_read():
     mib = 1 << 16
     assert reads_once(ElemType.BF16, QuantValue.Q8S, 4) and reads_once(ElemType.BF16, QuantValue.Q8S, 16 * mib)
     assert not reads_once(ElemType.BF16, QuantValue.Q8S, 16 * mib + 4) and not reads_once(ElemType.BF16, QuantValue.Q8S, 48 * mib - 4)
-    assert reads_once(ElemType.BF16, QuantValue.Q8S, 48 * mib) and reads_once(ElemType.F16, QuantValue.Q8S, 448 * mib)
-    assert not reads_once(ElemType.BF16, QuantValue.Q8S, 448 * mib + 4) and reads_once(ElemType.F32, QuantValue.Q8S, 448 * mib + 4)
+    assert reads_once(ElemType.BF16, QuantValue.Q8S, 48 * mib) and reads_once(ElemType.F16, QuantValue.Q8S, 384 * mib)
+    assert not reads_once(ElemType.BF16, QuantValue.Q8S, 384 * mib + 4) and reads_once(ElemType.F32, QuantValue.Q8S, 384 * mib + 4)
     assert not reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib - 4) and reads_once(ElemType.BF16, QuantValue.Q4S, 56 * mib)
+    assert not reads_once(ElemType.F16, QuantValue.Q2S, 128 * mib - 4) and reads_once(ElemType.F16, QuantValue.Q2S, 128 * mib)
     assert reads_once(ElemType.BF16, QuantValue.Q4S, 768 * mib) and not reads_once(ElemType.F32, QuantValue.Q4S, 768 * mib + 8)
 
 
@@ -305,3 +306,27 @@ def test_two_passes_on_a_third_stream_and_on_part_of_the_compute_units():
     with torch.cuda.stream(masked):
         assert one_read(small)
     small.check("mask, small")
+
+
+def test_captured_launches_on_any_stream():
+    """The fourth stream's capture is one read too (its slots are the workspace's): the share of the largest value is the slot that
+    holds it after a replay."""
+    import torch
+
+    call = Call(torch, values(torch, (72 << 16) * 8, ElemType.BF16, 3), ElemType.BF16, scheme_of(QuantValue.Q8S))
+    call.x[8 * 512 * 37 + 5] = -0.75  # step 37: the share of workgroup 37
+    graphs = []
+    for _ in range(4):
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call.fused()
+        graphs.append(graph)
+    for graph in graphs:
+        call.codes.zero_()
+        call.ws.fill_(0x5A)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        slots = call.ws.view(torch.float32)
+        assert slots[37].item() == 0.75 and slots.argmax().item() == 37
+        call.check("captured")

@@ -139,11 +139,13 @@ MIB = 1 << 16  # chunks
 # (chunks, bits, bytes of a float, captured): whether one read of the tensor is the faster way
 ONE_READ = {
     (4, 8, 2, False): True, (16 * MIB, 8, 2, False): True, (16 * MIB + 4, 8, 2, False): False, (48 * MIB - 4, 8, 2, False): False,
-    (48 * MIB, 8, 2, False): True, (384 * MIB, 8, 2, False): True, (512 * MIB, 8, 2, False): False, (4096 * MIB, 8, 2, False): False,
+    (48 * MIB, 8, 2, False): True, (384 * MIB, 8, 2, False): True, (400 * MIB, 8, 2, False): False, (4096 * MIB, 8, 2, False): False,
     (48 * MIB, 4, 2, False): False, (56 * MIB - 4, 4, 2, False): False, (56 * MIB, 4, 2, False): True, (640 * MIB, 4, 2, False): True, (1024 * MIB, 4, 2, False): False,
+    (16 * MIB, 2, 2, False): True, (56 * MIB, 2, 2, False): False, (80 * MIB, 2, 2, False): False, (128 * MIB, 2, 2, False): True, (56 * MIB, 2, 4, False): True,
     (48 * MIB, 8, 4, False): True, (640 * MIB, 8, 4, False): True, (2048 * MIB, 8, 4, False): False,
-    (4, 8, 2, True): False, (16 * MIB, 8, 2, True): False, (60 * MIB - 4, 8, 2, True): False, (60 * MIB, 8, 2, True): True, (512 * MIB, 8, 2, True): False,
-    (96 * MIB - 4, 4, 2, True): False, (96 * MIB, 4, 2, True): True, (96 * MIB, 2, 4, True): True, (2048 * MIB, 2, 4, True): False,
+    (4, 8, 2, True): False, (16 * MIB, 8, 2, True): False, (64 * MIB, 8, 2, True): False, (72 * MIB, 8, 2, True): True, (60 * MIB - 4, 8, 4, True): False,
+    (60 * MIB, 8, 4, True): True, (440 * MIB, 8, 2, True): True, (512 * MIB, 8, 2, True): False, (100 * MIB, 4, 2, True): False, (120 * MIB, 4, 2, True): True,
+    (200 * MIB, 2, 2, True): False, (96 * MIB - 4, 4, 4, True): False, (96 * MIB, 4, 4, True): True, (96 * MIB, 2, 4, True): True, (2048 * MIB, 2, 4, True): False,
 }
 
 
