@@ -22,8 +22,8 @@
 //
 // Bound by its phases one after the other.  bf16 128 MiB to 8 bits, 38 us: 2 of the launch, the read 19.5 (6.9 TB/s), 4
 // from the first published maximum to the last one seen, the arithmetic 11.5, which the stores overlap with.  Two passes -> one,
-// us: bf16 8 bits 32 KiB 5.6 -> 4.2, 1 MiB 5.9 -> 5.1, 4 MiB 6.3 -> 5.5, 16 MiB 8.7 -> 8.1, 64 MiB 25.0 -> 21.7, 112 MiB 50.6 -> 34.4,
-// 128 MiB 58.6 -> 38.0, 192 MiB 86.3 -> 66.5; f32 8 bits 64 MiB 22.3 -> 19.5, 128 MiB 45.4 -> 33.9; f16 to e4m3 128 MiB 60.1 -> 45.2.
+// us, calls on rotated buffers: bf16 8 bits 1 MiB 6.0 -> 4.6, 4 MiB 6.0 -> 5.2, 16 MiB 8.6 -> 7.8, 48 MiB 22.8 -> 17.8, 64 MiB 30.1 -> 22.2,
+// 128 MiB 58.8 -> 38.2, 192 MiB 86.1 -> 65.5; f32 8 bits 64 MiB 22.3 -> 19.5, 128 MiB 49.8 -> 34.8; f16 to e4m3 128 MiB 60.1 -> 45.2.
 #pragma once
 
 #include <atomic>
