@@ -12,7 +12,7 @@ template <class F, int kGroup>
 hipError_t scales_launch(hipStream_t s, const FlatArgs& a) {
     dim3 block(kThreads);
     if (a.lanes.levels > 0) {
-        const bool one = a.rows * a.num_chunks < small_lane_chunks(a.any_group);
+        const bool one = a.rows * a.num_chunks < kSmallLaneScaleChunks;
         const auto kernel = one ? scales_flat_lanes_kernel<F, kGroupRt, 1, kThreads> : scales_flat_lanes_kernel<F, kGroupRt, kUnrollQ, kThreads>;
         hipLaunchKernelGGL(kernel, dim3(lanes_grid(a, one ? 1 : kUnrollQ)), block, 0, s,
                            static_cast<const u32x4*>(a.input), a.scale_out, quant_params(a.range), with_group(lane_rows(a), kGroup));

@@ -198,3 +198,5 @@ def test_lanes_of_one_chunk_where_they_are_faster(answer):
              (565248, 12): False, (639744, 3): False}
     got = answer([f"{chunks} < small_lane_chunks({group})" for chunks, group in cases])
     assert got == [int(one) for one in cases.values()], dict(zip(cases, got))
+    scales = {409600: True, 502000: True, 598016: False, 778240: False}
+    assert answer([f"{chunks} < kSmallLaneScaleChunks" for chunks in scales]) == [int(one) for one in scales.values()]
