@@ -294,6 +294,7 @@ struct GemvArgs {
     uint64_t x_stride, y_stride;
     bool x_aligned16, words_aligned16;
 };
+struct QuadsSplit;  // cq_launch_rules.hpp
 bool gemv_streams(const GemvArgs& a);  // the launch takes the streaming kernel
 uint32_t gemv_vectors_per_launch(const GemvArgs& a, uint32_t remaining);
 hipError_t gemv_stream_f32_scales(hipStream_t s, const GemvArgs& a);    // the streaming kernels, by object
@@ -306,6 +307,12 @@ hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_quads_bf16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);       // one to four vectors
+hipError_t gemv_quads_bf16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
+hipError_t gemv_quads_bf16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
+hipError_t gemv_quads_f16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
+hipError_t gemv_quads_f16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
+hipError_t gemv_quads_f16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
 hipError_t launch_gemv_quantized(hipStream_t s, const GemvArgs& a);
 
 }  // namespace cq

@@ -16,6 +16,7 @@
 
 #include "../../include/cubek_quant_device.hpp"
 #include "cq_internal.hpp"
+#include "cq_launch_rules.hpp"
 
 namespace cq {
 namespace {
@@ -495,7 +496,25 @@ hipError_t gemv_batch(hipStream_t s, const GemvArgs& a) {
     return a.param_dtype == CQ_F32 ? gemv_batch_f16_f32(s, a) : a.param_dtype == CQ_F16 ? gemv_batch_f16_f16(s, a) : gemv_batch_f16_bf16(s, a);
 }
 
+hipError_t gemv_quads(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) {
+    if (a.dtype == CQ_BF16)
+        return a.param_dtype == CQ_F32 ? gemv_quads_bf16_f32(s, a, q) : a.param_dtype == CQ_F16 ? gemv_quads_bf16_f16(s, a, q) : gemv_quads_bf16_bf16(s, a, q);
+    return a.param_dtype == CQ_F32 ? gemv_quads_f16_f32(s, a, q) : a.param_dtype == CQ_F16 ? gemv_quads_f16_f16(s, a, q) : gemv_quads_f16_bf16(s, a, q);
+}
+
+// Whether the distances inside four or sixteen rows (and between the vectors) fit the 32 bits that the kernels on the matrix cores keep
+// them in, and x its type: all but f32, and no 2-bit fields.
+bool matrix_cores_serve(const GemvArgs& a) {
+    return gemv_streams(a) && a.bits != 2 && a.dtype != CQ_F32 && a.rows < (1u << 31) && a.word_pitch < (1u << 25) &&
+           a.scale_stride_row < (1u << 25) && (a.vectors == 1 || ((a.x_stride * 2) % 16 == 0 && a.x_stride < (1u << 26)));
+}
+
 hipError_t launch_one(hipStream_t s, const GemvArgs& a) {
+    if (a.vectors <= 4 && matrix_cores_serve(a)) {
+        const uint32_t values = 128 / a.bits;
+        const QuadsSplit q = quads_split(a.rows, a.cols / values, values, a.vectors, a.bits == 4 && a.native == 0, a.dtype == CQ_F16, a.native == 1 || a.native == 2);
+        if (q.grid != 0) return gemv_quads(s, a, q);
+    }
     if (a.vectors > 1) return gemv_batch(s, a);
     if (gemv_streams(a)) {
         if (a.dtype == CQ_F32) return gemv_stream_f32_x(s, a);
@@ -523,10 +542,11 @@ uint32_t dtype_bytes(int dtype) { return dtype == CQ_F32 ? 4u : 2u; }
 
 // How many of the remaining vectors the next launch takes: up to sixteen at once on the matrix cores where the streaming
 // kernel's layouts come with x in a 16-bit type (all but the 2-bit fields), every vector starts on a 16-byte boundary and
-// the distances inside sixteen rows (and between the vectors) fit the 32 bits the kernel keeps them in; else one.
+// the distances fit; else one.
 uint32_t gemv_vectors_per_launch(const GemvArgs& a, uint32_t remaining) {
-    if (remaining < 2 || !gemv_streams(a) || (a.x_stride * 2) % 16 != 0 || a.bits == 2 || a.dtype == CQ_F32) return 1;
-    if (a.rows >= (1u << 31) || a.word_pitch >= (1u << 25) || a.scale_stride_row >= (1u << 25) || a.x_stride >= (1u << 26)) return 1;
+    GemvArgs b = a;
+    b.vectors = remaining;
+    if (remaining < 2 || !matrix_cores_serve(b)) return 1;
     return remaining < 16 ? remaining : 16;
 }
 

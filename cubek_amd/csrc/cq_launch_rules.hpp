@@ -210,6 +210,63 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
     return GemvShape::k4x2;
 }
 
+// A product with one to four vectors by gemv_quads_kernel (cq_kernels_gemv_quads.hip), whose workgroups, one per compute unit, take four
+// rows a wave from x in LDS: whether it does, its workgroups and waves, and how many waves share four rows.  With `work`, the most steps (16
+// units of four rows) that a workgroup has, us before (gemv_stream_kernel, gemv_batch_kernel) -> with it:
+// * Several vectors: against the units that the busiest compute unit goes through there, in groups of 16 rows and stages of eight units.  Under
+//   0.7 of them always ([1163, 23392] 8 bits, 2 vectors 26.4 -> 12.5, [4444, 10272] 4 bits of bf16, 4 16.1 -> 11.6, [4115, 5120] 7.7 -> 7.1;
+//   0.79 [2856, 4864] 5.7 -> 5.9, level [3454, 1920] 4.1 -> 4.3), from work 64 on under 0.92 ([14336, 4096] 0.88, 8 bits 14.4 -> 13.3,
+//   e4m3 13.6 -> 12.4; level [16384, 5120] 8 bits 17.0 -> 18.2, [15872, 1280] e4m3 6.1 -> 6.6), and where fields of 4 bits fill the chip (from work 128, of
+//   f16 from 64) as long as it is any less ([23373, 10080] 0.96 40.4 -> 38.1, [21782, 7552] 26.3 -> 22.9; at work 112 0.88 [14336, 4096] 10.2 -> 10.5).
+// * One vector, 4 bits of f16: always, the digits pair up without being shifted together (x is permuted on its way into LDS;
+//   [18484, 6912] 23.3 -> 17.5, [7455, 2240] 7.3 -> 5.7).  e4m3 and e5m2 bytes, which leave time beside the arithmetic: from work 64 on ([9472,
+//   18176] 34.5 -> 31.7, [4352, 24448] 28.9 -> 22.8; [5888, 1664] 5.3 -> 5.7).
+// * Else one vector is bound by the same instructions either way, and it takes the launch where the other's strips of 64 units and workgroups
+//   of 8 or 16 rows are filled badly: four-row steps of 16 units under 0.72 of what its busiest compute unit goes through ([4524, 16512] 18.2
+//   -> 14.6, [1024, 28672] 14.9 -> 8.4, [25471, 2240] 14.4 -> 11.8, [2675, 4672] 6.1 -> 5.6; 0.77 [6867, 3584] 6.7 -> 7.3), not in the
+//   smallest launches ([3011, 1408] 3.8 -> 4.0).
+// Eight waves where there is little for sixteen to do: work 28 [7455, 2240] f16 5.7, 6.1 of 16; 64 [16115, 1920] 7.9, 7.3; 96 [4352, 24448]
+// 30, 22.8.  Shares of four rows are the fewest steps for the busiest wave, a quarter of one for each sum of its lanes.
+struct QuadsSplit {
+    uint32_t grid, waves, shares_log2, lds;  // grid 0: the other kernels
+};
+// rows of `units` units of `values` values; `fields4`: fields of 4 bits; `f16`: x is; `bytes`: e4m3 and e5m2
+inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, uint32_t vectors, bool fields4, bool f16, bool bytes) {
+    constexpr uint32_t kComputeUnits = 256, kMostQuads = 64, kMostLds = 160 * 1024;
+    constexpr QuadsSplit kNo = {0, 0, 0, 0};
+    const uint64_t x_bytes = (static_cast<uint64_t>(units) + 15) / 16 * 16 * values * 2 * (vectors > 2 ? 4 : vectors);
+    if (vectors > 4 || x_bytes > kMostLds) return kNo;
+    const uint32_t quads = rows / 4 + (rows % 4 != 0), steps = (units + 15) / 16;
+    QuadsSplit q = {quads < kComputeUnits ? quads : kComputeUnits, 16, 0, 0};
+    while ((quads + q.grid - 1) / q.grid > kMostQuads) q.grid *= 2;
+    const uint32_t each = (quads + q.grid - 1) / q.grid;
+    const uint64_t work = static_cast<uint64_t>(quads + kComputeUnits - 1) / kComputeUnits * steps;
+    if (vectors > 1) {
+        const uint32_t stage = (vectors * 16 * values + 1023) / 1024 * 1024, groups = rows / 16 + (rows % 16 != 0);
+        const GemvShape shape = gemv_batch_shape(groups, stage, 16 * (stage + 2560), units, bytes);
+        const uint32_t together = shape == GemvShape::k4x2 ? 4 : shape == GemvShape::k2x4 ? 2 : 1;
+        const uint64_t busiest = static_cast<uint64_t>((groups + together - 1) / together + kComputeUnits - 1) / kComputeUnits * together * 16 * ((units + 7) / 8) * 8;
+        const uint32_t most = work < 64 ? 70 : !fields4 ? 92 : f16 || work >= 128 ? 99 : 85;
+        if (work * 64 * 100 >= busiest * most) return kNo;
+    } else if (bytes) {
+        if (work < 64) return kNo;
+    } else if (!(fields4 && f16)) {
+        const uint32_t group = static_cast<uint64_t>(units) * values >= 16384 ? 16 : 8, groups = rows / group + (rows % group != 0);
+        const uint64_t stream = static_cast<uint64_t>((units + 63) / 64) * 64 * group * ((groups + kComputeUnits - 1) / kComputeUnits);
+        if (work < 24 || work * 64 * 25 >= stream * 18) return kNo;
+    }
+    if (work < (vectors > 1 ? 32 : 48)) q.waves = 8;
+    uint64_t least = ~0ull;
+    for (uint32_t l = 0; (1u << l) <= q.waves; l++) {
+        const uint64_t slots = q.waves >> l, cost = (each + slots - 1) / slots * (4 * ((static_cast<uint64_t>(steps) + (1u << l) - 1) >> l) + 1);
+        if (cost < least) q.shares_log2 = l, least = cost;
+    }
+    const uint64_t lds = x_bytes + (each << q.shares_log2) * 64;
+    if (lds > kMostLds) return kNo;
+    q.lds = static_cast<uint32_t>(lds);
+    return q;
+}
+
 // Blocks over two dimensions, scale computed in the launch: whether quantize_block_tiles_kernel takes it (cq_kernels_rows.hip; per_lane 0:
 // no), its lanes along the row, and how many chunks of a block's column each lane would hold in a workgroup of 256.  Blocks of a few rows are one chunk a lane, and a large launch of those waits for its many
 // small workgroups to be dispatched (1.1 - 1.7 ns each): from kWideTileChunks on their tiles are wider, two or four chunks a lane.

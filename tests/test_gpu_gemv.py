@@ -153,6 +153,34 @@ def test_gemv_on_the_matrix_cores(oracle, case, vectors):
     check_case(oracle, case, 3 + vectors, vectors=vectors)
 
 
+# Four rows a wave (gemv_quads_kernel): rows that end inside four and workgroups with one more than others, columns that end inside a
+# step of sixteen units or a unit behind one, fewer steps than waves share a row and some waves without, more than 64 times four rows to a compute
+# unit, blocks over rows, every slot count of x (one, two, four; three vectors in four), x longer than two pieces a thread.  (Tolerance:
+# as above; a share's sums are at most as many additions in a row.)
+QUADS_CASES = [
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F16, 1, 32, None, 1, False),
+    (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 1027, 544, None, 1, False),        # a unit behind a step
+    (ElemType.F16, QuantValue.E2M1, [128], QuantParam.F32, 70, 4224, 532, 1, False),        # pitched, shares of unequal steps
+    (ElemType.F16, QuantValue.Q4S, [64], QuantParam.BF16, 65541, 64, None, 1, False),       # more workgroups than compute units
+    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 1026, 28672, None, 1, False),
+    (ElemType.BF16, QuantValue.Q8S, [6, 32], QuantParam.F32, 1026, 12800, None, 1, False),  # blocks of six rows
+    (ElemType.F16, QuantValue.E4M3, [32], QuantParam.F32, 1030, 16384, None, 1, True),
+    (ElemType.BF16, QuantValue.E5M2, None, QuantParam.F32, 2, 16400, None, 1, True),        # one scale
+    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.BF16, 7, 96, None, 2, False),
+    (ElemType.F16, QuantValue.Q8S, [16], QuantParam.F16, 1031, 1296, None, 2, False),       # a scale per unit
+    (ElemType.BF16, QuantValue.E2M1, [64], QuantParam.F32, 1050, 8256, None, 3, True),
+    (ElemType.BF16, QuantValue.E4M3, [32, 32], QuantParam.F32, 1056, 2080, None, 4, True),
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 4444, 1056, None, 4, False),
+    (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 9, 19424, None, 4, False),         # nearly all of the LDS
+    (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 9, 20512, None, 4, False),         # ... and more than there is
+]
+
+
+@pytest.mark.parametrize("case", QUADS_CASES, ids=lambda c: _id(c[:7]) + f"-{c[7]}")
+def test_gemv_of_four_rows_a_wave(oracle, case):
+    check_case(oracle, case[:7], case[4] + case[7], native=case[8], vectors=case[7])
+
+
 # Every split of a workgroup (four, two or one group of 16 rows; rows on two, four or eight waves): rows that end inside a
 # group and leave a workgroup's other groups empty, columns that end inside a stage of eight units or have fewer stages
 # than waves, every width of codes and type of scales, as many vectors as one launch takes and one more.  (Tolerance: as

@@ -176,6 +176,37 @@ def test_products_with_several_vectors_take_the_fastest_shape(answer):
     assert not wrong
 
 
+# (rows, columns, vectors, values in 16 bytes of codes, 4-bit fields, x in f16, e4m3 or e5m2): waves of the kernel of four rows a wave, 0 where
+# another is faster, or within 5 % of it
+QUADS = {
+    (28672, 8192, 1, 32, True, False, False): 0, (4524, 16512, 1, 32, True, False, False): 16, (1024, 28672, 1, 32, True, False, False): 16,
+    (6867, 3584, 1, 32, True, False, False): 0, (3011, 1408, 1, 32, True, False, False): 0, (25471, 2240, 1, 32, True, False, False): 16,
+    (7455, 2240, 1, 32, True, True, False): 8, (18484, 6912, 1, 32, True, True, False): 16, (5888, 1664, 1, 16, False, False, True): 0,
+    (9472, 18176, 1, 16, False, False, True): 16, (1163, 23392, 2, 16, False, False, False): 16, (1486, 4288, 2, 32, True, False, False): 8,
+    (3454, 1920, 2, 32, True, False, False): 0, (16384, 5120, 4, 16, False, False, False): 0, (14336, 4096, 4, 16, False, False, True): 16,
+    (14336, 4096, 2, 32, True, False, False): 0, (23373, 10080, 4, 32, True, False, False): 16, (1024, 28672, 4, 32, True, False, False): 0,
+    (14336, 4096, 5, 32, True, True, False): 0,
+}
+
+
+def quads_split(rows, cols, vectors, per_unit, *flags):
+    return f"quads_split({rows}u, {cols // per_unit}u, {per_unit}, {vectors}, {', '.join(str(flag).lower() for flag in flags)})"
+
+
+def test_products_take_four_rows_a_wave_where_that_is_faster(answer):
+    got = answer([f"{quads_split(*case)}.waves" for case in QUADS])
+    assert got == list(QUADS.values()), dict(zip(QUADS, got))
+
+
+def test_four_rows_a_wave_fit_what_the_kernel_keeps(answer):
+    """Quads per workgroup in 8 bits, what is left over in 24, x and the sums in the shared memory of a compute unit, workgroups no more than quads."""
+    cases = [(rows, cols, vectors, 32, True, True, False) for rows in (1, 4, 5, 1023, 65536, 65541, 1 << 22, (1 << 31) - 1)
+             for cols in (32, 544, 19424, 38880) for vectors in (1, 2, 3, 4)]
+    got = answer([f"[] {{ const QuadsSplit q = {quads_split(*case)}; const uint32_t quads = ({case[0]}u + 3) / 4; return q.grid == 0 ? 2 : q.grid <= quads && "
+                  f"(quads + q.grid - 1) / q.grid <= 64 && quads % q.grid < (1u << 24) && (1u << q.shares_log2) <= q.waves && q.lds <= 160 * 1024; }}()" for case in cases])
+    assert 0 not in got and got.count(1) > 40, dict(zip(cases, got))
+
+
 # (bytes of a float, rows and columns of a block, rows and columns): chunks per lane of the tile kernel, 0 where another is faster or it cannot
 BLOCK_TILES = {
     (2, 128, 128, 14336, 4096): 8, (2, 64, 64, 14336, 4096): 4, (2, 32, 32, 2048, 4096): 2, (2, 32, 32, 128, 512): 2, (4, 64, 64, 14336, 4096): 4,
