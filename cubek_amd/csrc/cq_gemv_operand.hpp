@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/cubek_quant_device.hpp"
 #include "cq_internal.hpp"
 
@@ -20,43 +22,50 @@ constexpr int kCodeE4M3 = 100, kCodeE5M2 = 101, kCodeE2M1x2 = 102;  // the nativ
 
 constexpr uint32_t values_per_unit(int code) { return code <= 8 ? 128u / static_cast<uint32_t>(code) : (code == kCodeE2M1x2 ? 32u : 16u); }
 
-// The 4-bit fields of f16 tensors pair up as (0, 4), (1, 5), (2, 6), (3, 7): one mask plants two digits in two
-// halves, without shifting them together; x is brought into the same order.
+// The 4-bit fields of f16 tensors come out of a word's bytes as (0, 2), (4, 6), (1, 3), (5, 7).  Where x is laid out by the kernel it is brought
+// into the same order (`crossed`), else the bytes are put in order first, half the work of reordering x in every step.
 template <dev::Float kF, int kCode>
-constexpr bool kCrossPairs = kF == dev::Float::F16 && kCode == 4;
+constexpr bool kPairsCross = kF == dev::Float::F16 && kCode == 4;
+__device__ __forceinline__ u32x4 crossed(u32x4 p) {
+    return u32x4{__builtin_amdgcn_perm(p[1], p[0], 0x05040100u), __builtin_amdgcn_perm(p[3], p[2], 0x05040100u),
+                 __builtin_amdgcn_perm(p[1], p[0], 0x07060302u), __builtin_amdgcn_perm(p[3], p[2], 0x07060302u)};
+}
 
-// Eight consecutive values (kVals of a unit / 8 such groups) of a lane's unit as the matrix instruction takes them.
-template <dev::Float kF, int kCode, bool kShort>
+// Scales of less than this size take the short dequantization (their bits as a number, sign apart): where digit * s - bias * s
+// is exact.  A sum does not see the sign of a zero product, so unlike a stored value zero and negative scales may go that way.
+template <dev::Float kF, int kCode>
+constexpr uint32_t kShortBelow = kPairsCross<kF, kCode> ? 0x45800000u : 0x71800000u;  // 4096, so that 8 * s is a number of f16; 2^100
+
+// Eight consecutive values (kVals of a unit / 8 such groups) of a lane's unit as the matrix instruction takes them; kCrossed: in the
+// order of crossed().
+//
+// 4 bits of f16: a byte 0x0d read as an e4m3 number is d * 2^-9 for every d in 0..15, so one conversion gives two digits and one packed FMA
+// their values, rounded once: 44 cycles of VALU for eight, 50 by digits planted under the exponent of 1024, which take a
+// subtraction and a product.
+template <dev::Float kF, int kCode, bool kShort, bool kCrossed = false>
 __device__ __forceinline__ u32x4 operand(const u32x4& unit, uint32_t m, float scale) {
+    static_assert(!kCrossed || kPairsCross<kF, kCode>, "other pairs come in order");
     uint32_t p[8];
-    if constexpr (kCrossPairs<kF, kCode> && kShort) {
+    if constexpr (kPairsCross<kF, kCode> && kShort) {
         const uint32_t w = unit[m];
         const _Float16 sh = static_cast<_Float16>(scale);
-        const f16x2 s2 = {sh, sh};
-        const f16x2 off0 = {static_cast<_Float16>(-1032.0f), static_cast<_Float16>(-1032.0f)};
-        const f16x2 off1 = {static_cast<_Float16>(-72.0f), static_cast<_Float16>(-72.0f)};
-        const f16x2 sixteenth = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t v = h ? w >> 8 : w;
-            const uint32_t a = (v & 0x000f000fu) ^ 0x64086408u;  // 1024 + digit
-            const uint32_t b = (v & 0x00f000f0u) ^ 0x64806480u;  // 1024 + 16 * digit
-            const f16x2 qa = __builtin_bit_cast(f16x2, a) + off0;                                            // exact
-            const f16x2 qb = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, b), sixteenth, off1);      // exact
-            p[2 * h] = __builtin_bit_cast(uint32_t, s2 * qa);
-            p[2 * h + 1] = __builtin_bit_cast(uint32_t, s2 * qb);
+        const f16x2 s2 = {sh, sh}, bias = s2 * f16x2{static_cast<_Float16>(-8.0f), static_cast<_Float16>(-8.0f)};  // exact
+        uint32_t first = (w & 0x0f0f0f0fu) ^ 0x08080808u, second = ((w >> 4) & 0x0f0f0f0fu) ^ 0x08080808u;  // digits 0, 2, 4, 6; 1, 3, 5, 7
+        if constexpr (!kCrossed) {
+            const uint32_t even = first, odd = second;
+            first = __builtin_amdgcn_perm(odd, even, 0x05010400u), second = __builtin_amdgcn_perm(odd, even, 0x07030602u);
         }
-        return u32x4{p[0], p[1], p[2], p[3]};
+        const auto values = [&](uint32_t digits, auto high) {
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(digits, 512.0f, high.value)), s2, bias));
+        };
+        return u32x4{values(first, std::false_type{}), values(first, std::true_type{}), values(second, std::false_type{}), values(second, std::true_type{})};
     } else if constexpr (kCode == 4) {
         if constexpr (kShort)
             dev::dequantize_symmetric_packed_value_pairs_tame<kF, 4>(unit[m], scale, p);
         else
             dev::dequantize_symmetric_packed_value_pairs<kF, 4>(unit[m], scale, p);
-        if constexpr (kCrossPairs<kF, kCode>)
-            return u32x4{__builtin_amdgcn_perm(p[2], p[0], 0x05040100u), __builtin_amdgcn_perm(p[2], p[0], 0x07060302u),
-                         __builtin_amdgcn_perm(p[3], p[1], 0x05040100u), __builtin_amdgcn_perm(p[3], p[1], 0x07060302u)};
-        else
-            return u32x4{p[0], p[1], p[2], p[3]};
+        const u32x4 in_order = {p[0], p[1], p[2], p[3]};
+        return kCrossed ? crossed(in_order) : in_order;
     } else if constexpr (kCode == 8) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {

@@ -171,18 +171,6 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
                 for (uint32_t m = 0; m < kM; m++) xb[q][m] = past ? u32x4{0, 0, 0, 0} : xb[q][m];
             }
         }
-        if constexpr (kCrossPairs<kF, kCode>) {
-#pragma unroll
-            for (uint32_t q = 0; q < kQ; q++)
-#pragma unroll
-                for (uint32_t m = 0; m < kM; m++) {
-                    const u32x4 p = xb[q][m];
-                    xb[q][m] = u32x4{__builtin_amdgcn_perm(p[2], p[0], 0x05040100u), __builtin_amdgcn_perm(p[2], p[0], 0x07060302u),
-                                     __builtin_amdgcn_perm(p[3], p[1], 0x05040100u), __builtin_amdgcn_perm(p[3], p[1], 0x07060302u)};
-                }
-        }
-        // The short dequantization serves every scale below 2^100: a sum does not see the sign of a zero product, so unlike
-        // a stored value zero and negative scales may go this way, and digit * s - bias * s is exact down to the denormals.
         float sc[kQ];
         uint32_t largest = 0;
 #pragma unroll
@@ -190,7 +178,7 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
             sc[q] = dev::round_to<kF>(dev::widen(stored[q]));
             if (kPacked) largest = max(largest, __builtin_bit_cast(uint32_t, sc[q]) & 0x7fffffffu);
         }
-        if (!kPacked || __builtin_amdgcn_ballot_w64(largest >= 0x71800000u) == 0) {  // ordinary scales all are
+        if (!kPacked || __builtin_amdgcn_ballot_w64(largest >= kShortBelow<kF, kCode>) == 0) {  // ordinary scales all are
 #pragma unroll
             for (uint32_t q = 0; q < kQ; q++)
 #pragma unroll

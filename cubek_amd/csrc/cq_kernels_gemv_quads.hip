@@ -82,9 +82,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_quads_kernel(
     const auto x_to = [&](uint32_t at, u32x4 val) {
         const uint32_t v = __umulhi(at, pieces_inverse), p = at - v * pieces, u = p / kM, m = p % kM;
         if (u >= units_per_row) val = u32x4{0, 0, 0, 0};
-        if constexpr (kCrossPairs<kF, kCode>)
-            val = u32x4{__builtin_amdgcn_perm(val[2], val[0], 0x05040100u), __builtin_amdgcn_perm(val[2], val[0], 0x07060302u),
-                        __builtin_amdgcn_perm(val[3], val[1], 0x05040100u), __builtin_amdgcn_perm(val[3], val[1], 0x07060302u)};
+        if constexpr (kPairsCross<kF, kCode>) val = crossed(val);
         const uint32_t at_lds = (((u >> 4) * kM + m) << (4u + slots_log2)) + ((((u & 15u) << slots_log2) + v + m * rot) & ring);
         *reinterpret_cast<u32x4*>(lds + at_lds * 16u) = val;
     };
@@ -156,12 +154,12 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_quads_kernel(
         }
         const char* const x_step = lds + work_step * step_bytes;
         const float s = dev::round_to<kF>(dev::widen(stored));
-        // The short dequantization serves every scale below 2^100 (gemv_batch_kernel says why); ordinary scales all are.
-        if (!kPacked || __builtin_amdgcn_ballot_w64((bits_of(s) & 0x7fffffffu) >= 0x71800000u) == 0) {
+        // ordinary scales all take the short dequantization
+        if (!kPacked || __builtin_amdgcn_ballot_w64((bits_of(s) & 0x7fffffffu) >= kShortBelow<kF, kCode>) == 0) {
 #pragma unroll
             for (uint32_t m = 0; m < kM; m++) {
                 const u32x4 xb = *reinterpret_cast<const u32x4*>(x_step + x_lane[m]);
-                const u32x4 p = operand<kF, kCode, true>(w, m, s);
+                const u32x4 p = operand<kF, kCode, true, kPairsCross<kF, kCode>>(w, m, s);
                 acc[0] = mfma4<kF>(p[0], p[1], xb[0], xb[1], acc[0]);
                 acc[1] = mfma4<kF>(p[2], p[3], xb[2], xb[3], acc[1]);
             }
@@ -177,7 +175,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_quads_kernel(
                         x_at = x_lane[t];
                     }
                 const u32x4 xb = *reinterpret_cast<const u32x4*>(x_step + x_at);
-                const u32x4 p = operand<kF, kCode, false>(word, 0, s);
+                const u32x4 p = operand<kF, kCode, false, kPairsCross<kF, kCode>>(word, 0, s);
                 acc[0] = mfma4<kF>(p[0], p[1], xb[0], xb[1], acc[0]);
                 acc[0] = mfma4<kF>(p[2], p[3], xb[2], xb[3], acc[0]);
             }

@@ -368,6 +368,7 @@ SCALE_CASES = {
     "bf16": [-0.01, 0.0, -0.0, 1e-36, -3.0, 2.0 ** -110, 3000.0, -1e-30, 1e-39, 2.0 ** 99, -(2.0 ** 99)],
     "bf16-large": [-0.01, 0.0, 2.0 ** 100, -(2.0 ** 101), 2.0 ** 110],
     "f16": [-0.01, 0.0, -0.0, 1e-36, -3.0, 1e-7, -6e-8, 400.0, 2.0 ** -110],
+    "f16-edge": [4092.0, -4092.0, 4096.0, -4096.0, 8188.0, -8188.0, 6e-8, -6e-8],   # both sides of where the short way of 4 bits ends
     "f16-infinite": [1e6, 65520.0, np.inf],   # infinite once they are f16
     "bf16-infinite": [np.inf],
 }
@@ -395,6 +396,8 @@ def test_gemv_of_a_batch_scales_of_every_kind(oracle, kind, value, vectors):
         codes &= 0xBF   # no NaN, and 1.9 at most
     scales = rng.uniform(0.001, 0.02, (rows, cols // 32)).astype(np.float32)
     odd = np.array(SCALE_CASES[kind], np.float32)
+    if kind == "f16-edge" and value == QuantValue.Q8S:
+        odd /= 16  # 128 * 512 would not be a number of f16
     xb = oracle.to_bits(rng.normal(0, 1, (vectors, cols)).astype(np.float32), elem).reshape(vectors, cols)
     if infinite:
         for k, (row, block) in enumerate(((2, 0), (17, 20), (40, cols // 32 - 1), (82, 7))):
