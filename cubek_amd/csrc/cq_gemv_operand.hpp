@@ -1,4 +1,4 @@
-// What the kernels of the products with quantized weights on the matrix cores share (cq_kernels_gemv_quads.hip,
+// What the kernels of the products with quantized weights on the matrix cores share (cq_kernels_gemv_quads.hpp,
 // cq_kernels_gemv_batch.hip): codes to operands of the matrix instructions, and the store of y.
 #pragma once
 
@@ -84,6 +84,12 @@ __device__ __forceinline__ u32x4 operand(const u32x4& unit, uint32_t m, float sc
         dev::dequantize_symmetric_native_value_pairs<kF, kNative>(unit[2 * m + 1], scale, p + 2);
         return u32x4{p[0], p[1], p[2], p[3]};
     }
+}
+
+inline uint32_t log2_of(uint32_t v) {
+    uint32_t l = 0;
+    while ((1u << l) < v) l++;
+    return l;
 }
 
 __device__ __forceinline__ void store_y(int dtype, void* y, uint64_t i, float v) {

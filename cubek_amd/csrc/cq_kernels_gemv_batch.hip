@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include "cq_gemv_operand.hpp"
+#include "cq_kernels_gemv_quads.hpp"
 #include "cq_launch_rules.hpp"
 
 namespace cq {
@@ -228,12 +229,6 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
         if (i < vectors && !idle && row0 + 4u * g + r < rows) store_y(y_dtype, y, i * y_stride + row0 + 4u * g + r, sum[r]);
 }
 
-uint32_t log2_of(uint32_t v) {
-    uint32_t l = 0;
-    while ((1u << l) < v) l++;
-    return l;
-}
-
 template <dev::Float kF, class FS, int kCode, int kG, int kS>
 void launch_shape(hipStream_t s, const GemvArgs& a) {
     constexpr uint32_t kVals = values_per_unit(kCode);
@@ -278,21 +273,27 @@ hipError_t launch_codes(hipStream_t s, const GemvArgs& a) {
 // code of the kind it uses.
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 0
 hipError_t gemv_batch_bf16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, float>(s, a); }
+hipError_t gemv_quads_bf16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, float>(s, a, q); }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 1
 hipError_t gemv_batch_bf16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, __bf16>(s, a); }
+hipError_t gemv_quads_bf16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, __bf16>(s, a, q); }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 2
 hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, _Float16>(s, a); }
+hipError_t gemv_quads_bf16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, _Float16>(s, a, q); }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 3
 hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, float>(s, a); }
+hipError_t gemv_quads_f16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, float>(s, a, q); }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 4
 hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, __bf16>(s, a); }
+hipError_t gemv_quads_f16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, __bf16>(s, a, q); }
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 5
 hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, _Float16>(s, a); }
+hipError_t gemv_quads_f16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, _Float16>(s, a, q); }
 #endif
 
 }  // namespace cq
