@@ -394,6 +394,7 @@ void launch_stream_waves(hipStream_t s, const GemvArgs& a) {
                        a.word_pitch, static_cast<uint32_t>(a.scale_stride_row), static_cast<uint32_t>(a.scale_stride_col));
 }
 
+// One vector of x in a 16-bit type comes here only where quads_split() does not take it.
 // Two rows per wave, two strips in flight, four waves (eight rows) per workgroup; eight waves from 16384 columns
 // on, where the 32 KiB and more of x that every workgroup stages weigh more than the smaller workgroup gains.
 // Measured on MI355X (rows / waves / strips in flight; 4-bit weights [14336, 4096], [28672, 8192], [4096, 11008],

@@ -16,12 +16,13 @@
 // dequantization, 0.5 for the rest; at 4 cycles each they issue for more than half of the time ([28672, 8192], blocks of 32:
 // 34 us for 4 vectors, 38 us for 16; a read of the bytes 21 us), the matrix instructions for a tenth beside them.  With 8
 // bits and e4m3 bytes ([28672, 8192] 8 bits, 16 vectors 57 us), and in launches of a few rounds ([14336, 4096] f16, 8 vectors
-// 11 us), they issue for 35 - 43 %, and the waves spend about half of theirs waiting for a stage; few rows ([1024, 28672],
+// 10 us), they issue for 35 - 43 %, and the waves spend about half of theirs waiting for a stage; few rows ([1024, 28672],
 // 64 workgroups, 28 us) are a chain of stages on a quarter of the chip.
 //
-// Against the kernels of two to four vectors a launch before it, us: [28672, 8192] 4 bits bf16 2 vectors 35.0 -> 34.1, 16
+// Products of up to four vectors go through it only where its groups of 16 rows fill the chip (quads_split()).  Against the kernels of
+// two to four vectors a launch before it, us: [28672, 8192] 4 bits bf16 2 vectors 35.0 -> 34.1, 16
 // vectors 140 -> 39, f16 2 vectors 54 -> 31, 8 bits 57 -> 51, e4m3 56 -> 50; [14336, 4096] bf16 2 vectors 12.5 -> 11.7, f16
-// blocks of 128 20.0 -> 10.5; [1024, 28672] 2 vectors 30 -> 17.8, 16 vectors 141 -> 28.6.  The one size that lost is
+// blocks of 128 20.0 -> 10.5 (9.95 since its codes are put in order instead of x); [1024, 28672] 2 vectors 30 -> 17.8, 16 vectors 141 -> 28.6.  The one size that lost is
 // [8192, 28672] in e4m3 bytes with 3 vectors, 54.2 -> 56.5.
 #include <hip/hip_runtime.h>
 
