@@ -252,6 +252,14 @@ __device__ __forceinline__ void dequantize_symmetric_packed_value_pairs_tame(uin
 #pragma unroll
         for (int i = 0; i < kN / 2; i++) {
             // values 2i and 2i+1: their digits into the low mantissa bits of two halves holding 1024.0
+            // (8 bits: bytes are digits already, and 0x64 is the exponent's byte; products with [14336, 4096] 13.4 -> 12.7 us, which were
+            // shifted and joined by four more operations)
+            if constexpr (kBits == 8) {
+                const uint32_t planted = __builtin_amdgcn_perm(0x64646464u, digits, i == 0 ? 0x04010400u : 0x04030402u);
+                const f16x2 code = __builtin_bit_cast(f16x2, planted) + off2;  // exact
+                out[i] = __builtin_bit_cast(uint32_t, s2 * code);              // v_pk_mul_f16, one rounding
+                continue;
+            }
             const uint32_t lo = (digits >> (2 * i * kBits)) & kDigit;
             const uint32_t hi = (digits >> ((2 * i + 1) * kBits)) & kDigit;
             const uint32_t planted = 0x64006400u | lo | (hi << 16);
