@@ -109,6 +109,10 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
         x_piece[n] = (in & ~15u) | ((in - v) & 15u);
         x_at[n] = v * x_stride_bytes;
     }
+    // Rows that do not start on lines of 128 bytes: a stage reads parts of lines, whose rest the next one wants from the caches (streaming ->
+    // plain loads, us: f16 4 bits [2788, 4256] 5 vectors 6.4 -> 5.6, [3590, 14752] 16 19.4 -> 17.6, 8 bits [20000, 6752] 8 44.0 -> 40.8; whole lines
+    // [28672, 8192] 8 bits 16 54.7 -> 59.2, 4 bits 36.9 -> 38.9, [14336, 4096] f16 8 10.1 -> 9.7).
+    const bool whole_lines = ((reinterpret_cast<uintptr_t>(words) | row_bytes) & 127u) == 0;
     const auto load = [&](uint32_t stage, uint32_t into) {
         const uint32_t unit0 = stage * kU, block0 = unit0 >> units_per_block_log2;
         const bool partial = unit0 + kU > units_per_row;  // wave-uniform: units past the end are the last one again
@@ -119,8 +123,11 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
 #pragma unroll
         for (uint32_t t = 0; t < kCodeLoads; t++) {
             const uint32_t unit = partial ? min(code_unit[t], last_unit) : code_unit[t];
-            __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u)), CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0,
-                                             2 /* nt */);
+            const u32x4* const p = reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u));
+            if (whole_lines)
+                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 2 /* nt */);
+            else
+                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 0);
         }
         const uint32_t slot = partial ? min(scale_slot, last_block) : scale_slot;
 #pragma unroll
