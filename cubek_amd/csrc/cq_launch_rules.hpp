@@ -215,7 +215,8 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
 // units of four rows) that a workgroup has, us before (gemv_stream_kernel, gemv_batch_kernel) -> with it:
 // * Several vectors: against the units that the busiest compute unit goes through there, in groups of 16 rows and stages of eight units.  Under
 //   0.7 of them always ([1163, 23392] 8 bits, 2 vectors 26.4 -> 12.5, [4444, 10272] 4 bits of bf16, 4 16.1 -> 11.6, [4115, 5120] 7.7 -> 7.1;
-//   0.79 [2856, 4864] 5.7 -> 5.9, level [3454, 1920] 4.1 -> 4.3), from work 64 on under 0.92 ([14336, 4096] 0.88, 8 bits 14.4 -> 13.3,
+//   0.79 [2856, 4864] 5.7 -> 5.9, level [3454, 1920] 4.1 -> 4.3), from work 64 on under 0.8 ([9559, 1952] f16 8 bits, 3 vectors
+//   0.83 6.75 -> 7.45), from 128 on under 0.92 ([14336, 4096] 0.88, 8 bits 14.4 -> 13.3,
 //   e4m3 13.6 -> 12.4; level [16384, 5120] 8 bits 17.0 -> 18.2, [15872, 1280] e4m3 6.1 -> 6.6), and where fields of 4 bits fill the chip (from work 128, of
 //   f16 from 64) as long as it is any less ([23373, 10080] 0.96 40.4 -> 38.1, [21782, 7552] 26.3 -> 22.9; at work 112 0.88 [14336, 4096] 10.2 -> 10.5).
 // * One vector, 4 bits of f16: always, the digits pair up without being shifted together (x is permuted on its way into LDS;
@@ -246,7 +247,7 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const GemvShape shape = gemv_batch_shape(groups, stage, 16 * (stage + 2560), units, bytes);
         const uint32_t together = shape == GemvShape::k4x2 ? 4 : shape == GemvShape::k2x4 ? 2 : 1;
         const uint64_t busiest = static_cast<uint64_t>((groups + together - 1) / together + kComputeUnits - 1) / kComputeUnits * together * 16 * ((units + 7) / 8) * 8;
-        const uint32_t most = work < 64 ? 70 : !fields4 ? 92 : f16 || work >= 128 ? 99 : 85;
+        const uint32_t most = work < 64 ? 70 : !fields4 ? (work < 128 ? 80 : 92) : f16 || work >= 128 ? 99 : 85;
         if (work * 64 * 100 >= busiest * most) return kNo;
     } else if (bytes) {
         if (work < 64) return kNo;

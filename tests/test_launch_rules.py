@@ -185,7 +185,7 @@ QUADS = {
     (9472, 18176, 1, 16, False, False, True): 16, (1163, 23392, 2, 16, False, False, False): 16, (1486, 4288, 2, 32, True, False, False): 8,
     (3454, 1920, 2, 32, True, False, False): 0, (16384, 5120, 4, 16, False, False, False): 0, (14336, 4096, 4, 16, False, False, True): 16,
     (14336, 4096, 2, 32, True, False, False): 0, (23373, 10080, 4, 32, True, False, False): 16, (1024, 28672, 4, 32, True, False, False): 0,
-    (14336, 4096, 5, 32, True, True, False): 0,
+    (14336, 4096, 5, 32, True, True, False): 0, (9559, 1952, 3, 16, False, True, False): 0, (19328, 1280, 4, 16, False, False, True): 16,
 }
 
 
