@@ -57,7 +57,13 @@ __host__ __device__ constexpr uint32_t x_bytes(uint32_t vectors) {
 
 // kG groups of 16 rows per workgroup times kS shares of the row's stages (every kS-th one): kG * kS waves.  The waves
 // of a share use its x together; the shares' sums meet in LDS at the end.
-template <dev::Float kF, class FS, int kCode, int kG, int kS>
+//
+// kWholeLines: the rows start on lines of 128 bytes, and the codes, of which a stage takes whole lines, are streamed past the caches.  Rows that do
+// not: a stage reads parts of lines, whose rest the next one wants from the caches (streaming -> plain loads, us: f16 4 bits [2788, 4256] 5 vectors
+// 6.4 -> 5.6, [3590, 14752] 16 19.4 -> 17.6, 8 bits [20000, 6752] 8 44.0 -> 40.8; whole lines [28672, 8192] 8 bits 16 54.7 -> 59.2, 4 bits 36.9 -> 38.9,
+// [14336, 4096] f16 8 10.1 -> 9.7).  A kernel of its own for each: with both behind a branch in every stage whole lines lost 1 - 5 %
+// (4 bits [8192, 28672] 2 vectors 30.8 -> 32.0, e4m3 [12288, 11904] 4 26.7 -> 28.0, 4 bits [14439, 4352] 16 13.2 -> 13.6).
+template <dev::Float kF, class FS, int kCode, int kG, int kS, bool kWholeLines>
 __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
     const char* __restrict__ words, const char* __restrict__ scales, const char* __restrict__ x, void* __restrict__ y, int y_dtype,
     uint32_t rows, uint32_t units_per_row, uint32_t units_per_block_log2, uint32_t block_rows, uint64_t row_bytes,
@@ -109,10 +115,6 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
         x_piece[n] = (in & ~15u) | ((in - v) & 15u);
         x_at[n] = v * x_stride_bytes;
     }
-    // Rows that do not start on lines of 128 bytes: a stage reads parts of lines, whose rest the next one wants from the caches (streaming ->
-    // plain loads, us: f16 4 bits [2788, 4256] 5 vectors 6.4 -> 5.6, [3590, 14752] 16 19.4 -> 17.6, 8 bits [20000, 6752] 8 44.0 -> 40.8; whole lines
-    // [28672, 8192] 8 bits 16 54.7 -> 59.2, 4 bits 36.9 -> 38.9, [14336, 4096] f16 8 10.1 -> 9.7).
-    const bool whole_lines = ((reinterpret_cast<uintptr_t>(words) | row_bytes) & 127u) == 0;
     const auto load = [&](uint32_t stage, uint32_t into) {
         const uint32_t unit0 = stage * kU, block0 = unit0 >> units_per_block_log2;
         const bool partial = unit0 + kU > units_per_row;  // wave-uniform: units past the end are the last one again
@@ -123,11 +125,8 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
 #pragma unroll
         for (uint32_t t = 0; t < kCodeLoads; t++) {
             const uint32_t unit = partial ? min(code_unit[t], last_unit) : code_unit[t];
-            const u32x4* const p = reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u));
-            if (whole_lines)
-                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 2 /* nt */);
-            else
-                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u)), CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0,
+                                             kWholeLines ? 2 /* nt */ : 0);
         }
         const uint32_t slot = partial ? min(scale_slot, last_block) : scale_slot;
 #pragma unroll
@@ -237,15 +236,23 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
         if (i < vectors && !idle && row0 + 4u * g + r < rows) store_y(y_dtype, y, i * y_stride + row0 + 4u * g + r, sum[r]);
 }
 
-template <dev::Float kF, class FS, int kCode, int kG, int kS>
-void launch_shape(hipStream_t s, const GemvArgs& a) {
+template <dev::Float kF, class FS, int kCode, int kG, int kS, bool kWholeLines>
+void launch_lines(hipStream_t s, const GemvArgs& a) {
     constexpr uint32_t kVals = values_per_unit(kCode);
-    hipLaunchKernelGGL((gemv_batch_kernel<kF, FS, kCode, kG, kS>), dim3((a.rows + 16 * kG - 1) / (16 * kG)),
+    hipLaunchKernelGGL((gemv_batch_kernel<kF, FS, kCode, kG, kS, kWholeLines>), dim3((a.rows + 16 * kG - 1) / (16 * kG)),
                        dim3(64 * kG * kS), 2 * (kS * x_bytes<kCode>(a.vectors) + kG * kS * kWaveBytes), s,
                        static_cast<const char*>(a.words), static_cast<const char*>(a.scales), static_cast<const char*>(a.x), a.y, a.y_dtype,
                        a.rows, a.cols / kVals, a.block_rows == 0 ? 31u : log2_of(a.block_cols / kVals), a.block_rows == 0 ? 1u : a.block_rows,
                        a.word_pitch * 4, a.scale_stride_row * sizeof(FS), static_cast<uint32_t>(a.scale_stride_col * sizeof(FS)), a.vectors,
                        static_cast<uint32_t>(a.x_stride * 2), a.y_stride);
+}
+
+template <dev::Float kF, class FS, int kCode, int kG, int kS>
+void launch_shape(hipStream_t s, const GemvArgs& a) {
+    if (((reinterpret_cast<uintptr_t>(a.words) | (a.word_pitch * 4)) & 127u) == 0)
+        launch_lines<kF, FS, kCode, kG, kS, true>(s, a);
+    else
+        launch_lines<kF, FS, kCode, kG, kS, false>(s, a);
 }
 
 template <dev::Float kF, class FS, int kCode>
