@@ -215,19 +215,34 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
 // units of four rows) that a workgroup has, us before (gemv_stream_kernel, gemv_batch_kernel) -> with it:
 // * Several vectors: against the units that the busiest compute unit goes through there, in groups of 16 rows and stages of eight units.  Under
 //   0.7 of them always ([1163, 23392] 8 bits, 2 vectors 26.4 -> 12.5, [4444, 10272] 4 bits of bf16, 4 16.1 -> 11.6, [4115, 5120] 7.7 -> 7.1;
-//   0.79 [2856, 4864] 5.7 -> 5.9, level [3454, 1920] 4.1 -> 4.3), from work 64 on under 0.8 ([9559, 1952] f16 8 bits, 3 vectors
+//   0.79 [2856, 4864] 5.7 -> 5.9, 0.83 [3454, 1920] 4.05 -> 4.18), from work 64 on under 0.8 ([9559, 1952] f16 8 bits, 3 vectors
 //   0.83 6.75 -> 7.45), from 128 on under 0.92 ([14336, 4096] 0.88, 8 bits 14.4 -> 13.3,
-//   e4m3 13.6 -> 12.4; level [16384, 5120] 8 bits 17.0 -> 18.2, [15872, 1280] e4m3 6.1 -> 6.6), and where fields of 4 bits fill the chip (from work 128, of
+//   e4m3 13.6 -> 12.4; 1.0 [16384, 5120] 8 bits 17.0 -> 18.2, [15872, 1280] e4m3 6.1 -> 6.6), and where fields of 4 bits fill the chip (from work 128, of
 //   f16 from 64) as long as it is any less ([23373, 10080] 0.96 40.4 -> 38.1, [21782, 7552] 26.3 -> 22.9; at work 112 0.88 [14336, 4096] 10.2 -> 10.5).
-// * One vector, 4 bits of f16: always, the digits pair up without being shifted together (x is permuted on its way into LDS;
-//   [18484, 6912] 23.3 -> 17.5, [7455, 2240] 7.3 -> 5.7).  e4m3 and e5m2 bytes, which leave time beside the arithmetic: from work 64 on ([9472,
-//   18176] 34.5 -> 31.7, [4352, 24448] 28.9 -> 22.8; [5888, 1664] 5.3 -> 5.7).
+//   Not where waves are left without rows that the other has a round of for each: 4 bits, two four-row groups of three or four steps
+//   on a compute unit (2 vectors [1693, 1920] 3.68 -> 3.83, 4 [1362, 1920] 3.68 -> 3.90; two steps [1024, 2048] 3.66 -> 3.36, five [1085, 2080] 4.31 -> 3.88), and
+//   short rows of 8 bits in five groups of four rows for eight waves or pairs of waves ([5120, 1024] 2 vectors 4.33 -> 4.58, e4m3 3.98 -> 4.50,
+//   [4608, 3456] 3 6.85 -> 7.65; 8 bits [5120, 3072] 4 7.15 -> 6.68, e4m3 [4736, 5504] 3 8.94 -> 8.34).
+// * One vector, 4 bits of f16: the digits pair up without being shifted together (x is permuted on its way into LDS;
+//   [18484, 6912] 23.3 -> 17.5, [7455, 2240] 7.3 -> 5.7), except in the smallest launches that fill the other's strips as well ([1514, 1280] 3.21 -> 3.42,
+//   [1814, 1792] 3.35 -> 3.70; work 9 [2347, 1408] 3.85 -> 3.64, 12 [3425, 1344] 4.13 -> 3.74).
+// * One vector of e4m3 and e5m2 bytes, which leave time beside the arithmetic: from work 64 on ([9472, 18176] 32.6 -> 30.2, [4352, 24448] 28.9 ->
+//   22.8; [5888, 1664] 5.3 -> 5.7), but up to 128 not with three to six groups of four rows on a compute unit, whose waves, two to four to a group, start and
+//   end more often than they step ([4736, 4352] 7.46 -> 8.23, [5120, 4096] 6.60 -> 7.37, [3968, 4992] 6.27 -> 6.79; two [2048, 14592] 1.17 and eight [8576, 3328] 1.07
+//   times as fast).  The waves go through their rows in step, so they ask the same channels of memory at a time where those rows lie apart by
+//   the wrong distances: a compute unit's share a multiple of 2^18 bytes ([8192, 8192] 14.5 -> 15.3, [16384, 8192] 24.7 -> 27.2, [24576, 8192] 35.0 -> 42.3),
+//   and others ([14336, 11008] 31.1 -> 34.7, [28672, 10624] 51 -> 55; [28672, 10496] 52 -> 50, [20480, 11008] 42.5 -> 38.4).  From work 512 on, where the other
+//   kernel is near memory's rate, only where that one's strips and workgroups are filled badly ([5120, 28672] 32.5 -> 26.5, [6144, 24576] 29.1 -> 26.5).
 // * Else one vector is bound by the same instructions either way, and it takes the launch where the other's strips of 64 units and workgroups
 //   of 8 or 16 rows are filled badly: four-row steps of 16 units under 0.72 of what its busiest compute unit goes through ([4524, 16512] 18.2
 //   -> 14.6, [1024, 28672] 14.9 -> 8.4, [25471, 2240] 14.4 -> 11.8, [2675, 4672] 6.1 -> 5.6; 0.77 [6867, 3584] 6.7 -> 7.3), not in the
-//   smallest launches ([3011, 1408] 3.8 -> 4.0).
+//   smallest launches ([3011, 1408] 3.8 -> 4.0); 8 bits and e2m1 bytes, with fewer steps in a row, under 0.55 up to work 48 (0.62 [2774, 2432] 5.05 -> 5.30, 0.66
+//   [2583, 3360] 5.38 -> 5.63, e2m1 0.62 [4120, 4320] 6.49 -> 6.71; 0.5 [1024, 8192] 6.49 -> 5.28).
 // Eight waves where there is little for sixteen to do: work 28 [7455, 2240] f16 5.7, 6.1 of 16; 64 [16115, 1920] 7.9, 7.3; 96 [4352, 24448]
 // 30, 22.8.  Shares of four rows are the fewest steps for the busiest wave, a quarter of one for each sum of its lanes.
+//
+// Over 2730 launches from [1024, 1024] to [28672, 28672] that it takes it is 1.17 times as fast as the others on the mean; 3 % are more than 2.5 % slower, three
+// or four vectors on three groups of four long rows the most (e2m1 bytes [2588, 14272] 9.4 -> 11.0, 4 bits [3072, 14336] 10.6 -> 11.4; e4m3 [14336, 14336] 34.4 -> 37.6).
 struct QuadsSplit {
     uint32_t grid, waves, shares_log2, lds;  // grid 0: the other kernels
 };
@@ -249,12 +264,19 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const uint64_t busiest = static_cast<uint64_t>((groups + together - 1) / together + kComputeUnits - 1) / kComputeUnits * together * 16 * ((units + 7) / 8) * 8;
         const uint32_t most = work < 64 ? 70 : !fields4 ? (work < 128 ? 80 : 92) : f16 || work >= 128 ? 99 : 85;
         if (work * 64 * 100 >= busiest * most) return kNo;
-    } else if (bytes) {
-        if (work < 64) return kNo;
-    } else if (!(fields4 && f16)) {
+        if (values == 32 ? each > 1 && steps > 2 && work <= 8 : each == 5 && work < (bytes ? 96 : 48)) return kNo;
+    } else {
         const uint32_t group = static_cast<uint64_t>(units) * values >= 16384 ? 16 : 8, groups = rows / group + (rows % group != 0);
         const uint64_t stream = static_cast<uint64_t>((units + 63) / 64) * 64 * group * ((groups + kComputeUnits - 1) / kComputeUnits);
-        if (work < 24 || work * 64 * 25 >= stream * 18) return kNo;
+        const auto at_least = [&](uint32_t percent) { return work * 64 * 100 >= stream * percent; };  // ... of what the other goes through
+        if (bytes) {
+            const bool apart_by_2_18 = static_cast<uint64_t>(rows) * units % (1u << 22) == 0;  // 256 shares of units of 16 bytes
+            if (work < 64 || (work < 128 && each > 2 && each <= 6) || ((work >= 512 || apart_by_2_18) && at_least(85))) return kNo;
+        } else if (fields4 && f16) {
+            if (work <= 8 && at_least(72)) return kNo;
+        } else {
+            if (work < 24 || at_least(72) || (!fields4 && work < 48 && at_least(55))) return kNo;
+        }
     }
     if (work < (vectors > 1 ? 32 : 48)) q.waves = 8;
     uint64_t least = ~0ull;

@@ -186,6 +186,19 @@ QUADS = {
     (3454, 1920, 2, 32, True, False, False): 0, (16384, 5120, 4, 16, False, False, False): 0, (14336, 4096, 4, 16, False, False, True): 16,
     (14336, 4096, 2, 32, True, False, False): 0, (23373, 10080, 4, 32, True, False, False): 16, (1024, 28672, 4, 32, True, False, False): 0,
     (14336, 4096, 5, 32, True, True, False): 0, (9559, 1952, 3, 16, False, True, False): 0, (19328, 1280, 4, 16, False, False, True): 16,
+    # several vectors, and waves without rows: two groups of four rows in three or four steps, five groups of short rows
+    (1693, 1920, 2, 32, True, False, False): 0, (1362, 1920, 4, 32, True, True, False): 0, (1439, 1664, 4, 32, False, True, False): 0, (1085, 2080, 2, 32, True, False, False): 8,
+    (1024, 2048, 4, 32, True, False, False): 8, (5120, 1024, 2, 16, False, False, False): 0, (5120, 1024, 4, 16, False, True, True): 0, (4608, 3456, 3, 16, False, False, True): 0,
+    (5120, 3072, 4, 16, False, False, False): 16, (4736, 5504, 3, 16, False, False, True): 16,
+    # one vector of 4 bits of f16 in the smallest launches
+    (1514, 1280, 1, 32, True, True, False): 0, (1814, 1792, 1, 32, True, True, False): 0, (2347, 1408, 1, 32, True, True, False): 8, (3425, 1344, 1, 32, True, True, False): 8,
+    # ... of bytes: few groups of four rows, shares 2^18 bytes apart, large weights
+    (4096, 4096, 1, 16, False, False, True): 0, (4736, 4352, 1, 16, False, True, True): 0, (2048, 14336, 1, 16, False, False, True): 16, (8576, 3328, 1, 16, False, False, True): 16,
+    (8192, 8192, 1, 16, False, False, True): 0, (16384, 4096, 1, 16, False, True, True): 0, (8192, 11008, 1, 16, False, False, True): 16, (24576, 8192, 1, 16, False, False, True): 0,
+    (14336, 11008, 1, 16, False, True, True): 0, (28672, 10624, 1, 16, False, False, True): 0, (5120, 28672, 1, 16, False, False, True): 16, (6144, 24576, 1, 16, False, True, True): 16,
+    # ... of 8 bits and e2m1 bytes in short launches
+    (2774, 2432, 1, 16, False, False, False): 0, (2583, 3360, 1, 16, False, False, False): 0, (4120, 4320, 1, 32, False, False, False): 0, (1024, 8192, 1, 16, False, True, False): 8,
+    (2614, 5440, 1, 16, False, False, False): 16,
 }
 
 
