@@ -318,8 +318,7 @@ __global__ __launch_bounds__(kThreads) void reduce_cols_kernel(const u32x4* __re
 // ---- columns, few outputs: one workgroup per (outer, column tile, slice of L) ----------
 // Lanes form a [kT / kCW row phases][kCW chunk columns] grid.  FIn is the type read
 // (F32 when folding partials), FOut the type of the final result.  kAhead: the next loads go out before the previous ones are
-// folded; a long axis is faster without, where the tiles of a row stay closer together (bf16 [4093, 11008] 18.0 -> 18.7 us, [3726,
-// 16384] 22.2 -> 24.2; [1041, 9088] 6.3 -> 5.9, [600, 8448] 5.2 -> 4.7, [752, 19680] 8.65 -> 8.3, [1281, 17536] level).
+// folded (reduce_loads_ahead() says where).
 enum TileOut { kTileFinalPacked = 0, kTilePartial = 1, kTileFinalChecked = 2 };
 
 template <class FIn, class FOut, int kCW, int kT, int kMode, bool kRagged, bool kAhead>
@@ -712,15 +711,15 @@ ReducePlan plan_reduce(uint64_t outer, uint64_t len, uint64_t inner, uint64_t kN
     return p;
 }
 
-// kWidest: of the tiles that the caller asks for
-template <class FIn, class FOut, int kT, int kMode, int kWidest = kWave, bool kAhead = false>
+// kWidest, kNarrowest: of the tiles that the caller asks for
+template <class FIn, class FOut, int kT, int kMode, int kWidest = kWave, bool kAhead = false, int kNarrowest = 1>
 void launch_tile(hipStream_t s, bool ragged, uint32_t cw, uint64_t jobs, const void* in, void* out, uint64_t len,
                  uint64_t inner, uint32_t col_tiles, uint32_t slices, uint64_t pitch, uint64_t count) {
     auto src = static_cast<const u32x4*>(in);
     dim3 grid(static_cast<uint32_t>(jobs));
     switch (cw * 2 + (ragged ? 1 : 0)) {
 #define CQ_TILE(W, R) hipLaunchKernelGGL((reduce_tile_kernel<FIn, FOut, W, kT, kMode, R, kAhead>), grid, dim3(kT), 0, s, src, out, len, inner, col_tiles, slices, pitch, count)
-#define CQ_CASE(W) case W * 2: if constexpr (W <= kWidest) CQ_TILE(W, false); break; case W * 2 + 1: if constexpr (W <= kWidest && kMode != kTileFinalChecked) CQ_TILE(W, true); break;
+#define CQ_CASE(W) case W * 2: if constexpr (W >= kNarrowest && W <= kWidest) CQ_TILE(W, false); break; case W * 2 + 1: if constexpr (W >= kNarrowest && W <= kWidest && kMode != kTileFinalChecked && !kAhead) CQ_TILE(W, true); break;
         CQ_CASE(1) CQ_CASE(2) CQ_CASE(4) CQ_CASE(8) CQ_CASE(16) CQ_CASE(32) CQ_CASE(64)
 #undef CQ_CASE
 #undef CQ_TILE
@@ -897,8 +896,8 @@ hipError_t reduce_dispatch(hipStream_t s, const ReduceArgs& a) {
                 const uint32_t col_tiles = static_cast<uint32_t>(tile.col_tiles);
                 if (a.len <= 128)
                     launch_tile<F, F, 256, kTileFinalPacked>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
-                else if (a.len <= 1536)
-                    launch_tile<F, F, 512, kTileFinalPacked, kWidestReduceTile, true>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
+                else if (reduce_loads_ahead(c, tile))
+                    launch_tile<F, F, 512, kTileFinalPacked, kWidestReduceTile, true, 8>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
                 else
                     launch_tile<F, F, 512, kTileFinalPacked, kWidestReduceTile>(s, p.ragged, tile.cw, a.outer * tile.col_tiles, a.input, a.output, a.len, a.inner, col_tiles, 1u, 0, 0);
                 return hipGetLastError();

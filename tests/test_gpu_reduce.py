@@ -73,8 +73,12 @@ def test_reduce_short_rows_and_small_outer_axes(gpu, oracle, elem):
     n = 4 if elem == ElemType.F32 else 8
     cases = [((rows, chunks * n), 1) for rows, chunks in ((70, 3), (129, 5), (1, 6), (33, 41), (257, 61), (20000, 17), (9, 130), (300, 511),
                                                           (40000, 67), (31, 513))]
-    # one launch of tiles: an odd and an even number of trips of 512 rows, whole and with a remainder, and an axis past those that load ahead
+    # one launch of tiles of four columns: one to four trips of 512 rows, whole and with a remainder
     cases += [((length, 24 * n), 0) for length in (129, 512, 513, 1024, 1025, 1536, 1537)]
+    # ... that load ahead: eight columns (trips of 256 rows) and sixteen (of 128), odd and even numbers of trips, whole and with a remainder, a row that
+    # shares its lines, and axes past them
+    cases += [((length, 832 * n), 0) for length in (257, 512, 513, 1025, 1536, 1537)] + [((length, 2208 * n), 0) for length in (129, 256, 385, 641)]
+    cases += [((length, 2202 * n), 0) for length in (300, 512, 513)]
     cases += [((length, chunks * n), 0) for length, chunks in ((1024, 300), (1025, 300), (37, 257), (1000, 5), (513, 2), (1023, 1))]
     cases += [((3, 600, 33 * n), 1)]
     # slices of whole loops of rows: a last slice of one row, of less than a loop, of a whole one; several outer entries
