@@ -138,9 +138,10 @@ def test_reductions_along_an_outer_axis_take_the_faster_way(answer):
 # (outer, length, inner, bytes of an element, ragged): whether loading ahead was the faster way in one launch, or within 3 % of it
 LOADS_AHEAD = {
     (1, 1041, 9088, 2, False): True, (1, 600, 8448, 2, False): True, (1, 752, 19680, 2, False): True, (1, 457, 21968, 2, False): True, (1, 250, 19368, 2, False): True,
-    (1, 1005, 3968, 4, False): True, (2, 405, 5760, 2, False): True, (5, 446, 7552, 4, False): True,
+    (1, 1005, 3968, 4, False): True, (2, 405, 5760, 2, False): True, (5, 446, 7552, 4, False): True, (1, 602, 32768, 2, False): True,
+    (1, 602, 32896, 2, False): False, (2, 655, 17728, 2, False): False,
     (1, 558, 9249, 2, True): False, (5, 738, 3761, 2, True): False, (1, 509, 10464, 2, False): False, (1, 1116, 2307, 2, True): False, (1, 1134, 115, 4, True): False,
-    (1, 1154, 512, 2, False): False, (1, 1134, 16384, 2, False): False, (1, 1082, 11776, 2, False): False, (5, 216, 30208, 2, False): False, (1, 250, 9728, 2, False): False,
+    (1, 1154, 512, 2, False): False, (1, 1134, 16384, 2, False): False, (1, 1082, 11776, 2, False): False, (5, 138, 25216, 2, False): False, (1, 250, 9728, 2, False): False,
     (1, 4093, 11008, 2, False): False, (1, 3726, 16384, 2, False): False,
 }
 
