@@ -301,12 +301,19 @@ hipError_t gemv_stream_f32_scales(hipStream_t s, const GemvArgs& a);    // the s
 hipError_t gemv_stream_16bit_scales(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_stream_wide(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_stream_f32_x(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_batch_bf16_f32(hipStream_t s, const GemvArgs& a);       // two to sixteen vectors, by type of x and of the scales
-hipError_t gemv_batch_bf16_bf16(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a);
-hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a);
+// two to sixteen vectors, by type of x and of the scales; rows of whole lines of 128 bytes, and others
+hipError_t gemv_batch_lines_bf16_f32(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_bf16_f32(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_lines_bf16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_bf16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_lines_bf16_f16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_bf16_f16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_lines_f16_f32(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_f16_f32(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_lines_f16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_f16_bf16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_lines_f16_f16(hipStream_t s, const GemvArgs& a);
+hipError_t gemv_batch_parts_f16_f16(hipStream_t s, const GemvArgs& a);
 hipError_t gemv_quads_bf16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);       // one to four vectors
 hipError_t gemv_quads_bf16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);
 hipError_t gemv_quads_bf16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q);

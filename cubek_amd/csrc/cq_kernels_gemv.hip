@@ -492,9 +492,13 @@ bool gemv_streams(const GemvArgs& a) {
 namespace {
 
 hipError_t gemv_batch(hipStream_t s, const GemvArgs& a) {
+    const bool lines = ((reinterpret_cast<uintptr_t>(a.words) | (a.word_pitch * 4)) & 127u) == 0, f32 = a.param_dtype == CQ_F32, f16 = a.param_dtype == CQ_F16;
+    const auto of = [&](hipError_t (*by_f32)(hipStream_t, const GemvArgs&), hipError_t (*by_f16)(hipStream_t, const GemvArgs&), hipError_t (*by_bf16)(hipStream_t, const GemvArgs&)) {
+        return (f32 ? by_f32 : f16 ? by_f16 : by_bf16)(s, a);
+    };
     if (a.dtype == CQ_BF16)
-        return a.param_dtype == CQ_F32 ? gemv_batch_bf16_f32(s, a) : a.param_dtype == CQ_F16 ? gemv_batch_bf16_f16(s, a) : gemv_batch_bf16_bf16(s, a);
-    return a.param_dtype == CQ_F32 ? gemv_batch_f16_f32(s, a) : a.param_dtype == CQ_F16 ? gemv_batch_f16_f16(s, a) : gemv_batch_f16_bf16(s, a);
+        return lines ? of(gemv_batch_lines_bf16_f32, gemv_batch_lines_bf16_f16, gemv_batch_lines_bf16_bf16) : of(gemv_batch_parts_bf16_f32, gemv_batch_parts_bf16_f16, gemv_batch_parts_bf16_bf16);
+    return lines ? of(gemv_batch_lines_f16_f32, gemv_batch_lines_f16_f16, gemv_batch_lines_f16_bf16) : of(gemv_batch_parts_f16_f32, gemv_batch_parts_f16_f16, gemv_batch_parts_f16_bf16);
 }
 
 hipError_t gemv_quads(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) {

@@ -27,7 +27,6 @@
 #include <hip/hip_runtime.h>
 
 #include "cq_gemv_operand.hpp"
-#include "cq_kernels_gemv_quads.hpp"
 #include "cq_launch_rules.hpp"
 
 namespace cq {
@@ -237,7 +236,7 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
 }
 
 template <dev::Float kF, class FS, int kCode, int kG, int kS, bool kWholeLines>
-void launch_lines(hipStream_t s, const GemvArgs& a) {
+void launch_shape(hipStream_t s, const GemvArgs& a) {
     constexpr uint32_t kVals = values_per_unit(kCode);
     hipLaunchKernelGGL((gemv_batch_kernel<kF, FS, kCode, kG, kS, kWholeLines>), dim3((a.rows + 16 * kG - 1) / (16 * kG)),
                        dim3(64 * kG * kS), 2 * (kS * x_bytes<kCode>(a.vectors) + kG * kS * kWaveBytes), s,
@@ -247,68 +246,70 @@ void launch_lines(hipStream_t s, const GemvArgs& a) {
                        static_cast<uint32_t>(a.x_stride * 2), a.y_stride);
 }
 
-template <dev::Float kF, class FS, int kCode, int kG, int kS>
-void launch_shape(hipStream_t s, const GemvArgs& a) {
-    if (((reinterpret_cast<uintptr_t>(a.words) | (a.word_pitch * 4)) & 127u) == 0)
-        launch_lines<kF, FS, kCode, kG, kS, true>(s, a);
-    else
-        launch_lines<kF, FS, kCode, kG, kS, false>(s, a);
-}
-
-template <dev::Float kF, class FS, int kCode>
+template <dev::Float kF, class FS, int kCode, bool kWholeLines>
 void launch_code(hipStream_t s, const GemvArgs& a) {
     const uint32_t units = a.cols / values_per_unit(kCode), x = x_bytes<kCode>(a.vectors);
     static_assert(kU == 8, "the stages of gemv_batch_shape()");
     switch (gemv_batch_shape((a.rows + 15) / 16, x, 2 * 8 * (x + kWaveBytes), units, kCode == kCodeE4M3 || kCode == kCodeE5M2)) {
-        case GemvShape::k1x8: return launch_shape<kF, FS, kCode, 1, 8>(s, a);
-        case GemvShape::k1x4: return launch_shape<kF, FS, kCode, 1, 4>(s, a);
-        case GemvShape::k2x4: return launch_shape<kF, FS, kCode, 2, 4>(s, a);
-        case GemvShape::k4x2: return launch_shape<kF, FS, kCode, 4, 2>(s, a);
+        case GemvShape::k1x8: return launch_shape<kF, FS, kCode, 1, 8, kWholeLines>(s, a);
+        case GemvShape::k1x4: return launch_shape<kF, FS, kCode, 1, 4, kWholeLines>(s, a);
+        case GemvShape::k2x4: return launch_shape<kF, FS, kCode, 2, 4, kWholeLines>(s, a);
+        case GemvShape::k4x2: return launch_shape<kF, FS, kCode, 4, 2, kWholeLines>(s, a);
     }
 }
 
-template <dev::Float kF, class FS>
+template <dev::Float kF, class FS, bool kWholeLines>
 hipError_t launch_codes(hipStream_t s, const GemvArgs& a) {
     if (a.native == 1)
-        launch_code<kF, FS, kCodeE4M3>(s, a);
+        launch_code<kF, FS, kCodeE4M3, kWholeLines>(s, a);
     else if (a.native == 2)
-        launch_code<kF, FS, kCodeE5M2>(s, a);
+        launch_code<kF, FS, kCodeE5M2, kWholeLines>(s, a);
     else if (a.native == 3)
-        launch_code<kF, FS, kCodeE2M1x2>(s, a);
+        launch_code<kF, FS, kCodeE2M1x2, kWholeLines>(s, a);
     else if (a.bits == 4)
-        launch_code<kF, FS, 4>(s, a);
+        launch_code<kF, FS, 4, kWholeLines>(s, a);
     else
-        launch_code<kF, FS, 8>(s, a);
+        launch_code<kF, FS, 8, kWholeLines>(s, a);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// One object per type of x and of the scales (CQ_GEMV_PART names the one being compiled), so that a process loads the
-// code of the kind it uses.
+// One object per type of x and of the scales (CQ_GEMV_PART names the one being compiled) and for either kind of rows
+// (CQ_GEMV_LINES), so that a process loads the code of the kind it uses.
+#if !defined(CQ_GEMV_LINES) || CQ_GEMV_LINES == 1
+#define CQ_GEMV_BATCH_LINES(NAME, F, FS) hipError_t gemv_batch_lines_##NAME(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F, FS, true>(s, a); }
+#else
+#define CQ_GEMV_BATCH_LINES(NAME, F, FS)
+#endif
+#if !defined(CQ_GEMV_LINES) || CQ_GEMV_LINES == 0
+#define CQ_GEMV_BATCH_PARTS(NAME, F, FS) hipError_t gemv_batch_parts_##NAME(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F, FS, false>(s, a); }
+#else
+#define CQ_GEMV_BATCH_PARTS(NAME, F, FS)
+#endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 0
-hipError_t gemv_batch_bf16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, float>(s, a); }
-hipError_t gemv_quads_bf16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, float>(s, a, q); }
+CQ_GEMV_BATCH_LINES(bf16_f32, BF16, float)
+CQ_GEMV_BATCH_PARTS(bf16_f32, BF16, float)
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 1
-hipError_t gemv_batch_bf16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, __bf16>(s, a); }
-hipError_t gemv_quads_bf16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, __bf16>(s, a, q); }
+CQ_GEMV_BATCH_LINES(bf16_bf16, BF16, __bf16)
+CQ_GEMV_BATCH_PARTS(bf16_bf16, BF16, __bf16)
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 2
-hipError_t gemv_batch_bf16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::BF16, _Float16>(s, a); }
-hipError_t gemv_quads_bf16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::BF16, _Float16>(s, a, q); }
+CQ_GEMV_BATCH_LINES(bf16_f16, BF16, _Float16)
+CQ_GEMV_BATCH_PARTS(bf16_f16, BF16, _Float16)
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 3
-hipError_t gemv_batch_f16_f32(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, float>(s, a); }
-hipError_t gemv_quads_f16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, float>(s, a, q); }
+CQ_GEMV_BATCH_LINES(f16_f32, F16, float)
+CQ_GEMV_BATCH_PARTS(f16_f32, F16, float)
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 4
-hipError_t gemv_batch_f16_bf16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, __bf16>(s, a); }
-hipError_t gemv_quads_f16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, __bf16>(s, a, q); }
+CQ_GEMV_BATCH_LINES(f16_bf16, F16, __bf16)
+CQ_GEMV_BATCH_PARTS(f16_bf16, F16, __bf16)
 #endif
 #if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 5
-hipError_t gemv_batch_f16_f16(hipStream_t s, const GemvArgs& a) { return launch_codes<dev::Float::F16, _Float16>(s, a); }
-hipError_t gemv_quads_f16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return quads::launch_codes<dev::Float::F16, _Float16>(s, a, q); }
+CQ_GEMV_BATCH_LINES(f16_f16, F16, _Float16)
+CQ_GEMV_BATCH_PARTS(f16_f16, F16, _Float16)
 #endif
 
 }  // namespace cq

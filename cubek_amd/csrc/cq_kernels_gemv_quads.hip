@@ -14,8 +14,6 @@
 // the four cycles a unit of VALU takes, a v_cvt_pk, v_perm or packed f16 operation has four, an f32 FMA three, a shift or product 2.5;
 // a 4 x 4 x 4 matrix instruction takes nine of the same unit, so one vector costs what v_dot2 does and four cost no more), by memory and the
 // one start-up elsewhere.  Two steps ahead: three and four hold more registers than they hide (31.1, 31.9 against 30.2 us).
-#pragma once
-
 #include <hip/hip_runtime.h>
 
 #include "cq_gemv_operand.hpp"
@@ -23,7 +21,6 @@
 
 namespace cq {
 namespace {
-namespace quads {
 
 // D (4 x 4 per block) += A (4 x 4) * B (4 x 4), sixteen blocks side by side: lane (i, b) = (lane % 4, lane / 4) holds row i of
 // A and column i of B of block b, four values each, and column i of D in four registers.
@@ -283,6 +280,27 @@ hipError_t launch_codes(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) {
     return hipGetLastError();
 }
 
-}  // namespace quads
 }  // namespace
+
+// One object per type of x and of the scales (CQ_GEMV_PART names the one being compiled), so that a process loads the
+// code of the kind it uses.
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 0
+hipError_t gemv_quads_bf16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::BF16, float>(s, a, q); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 1
+hipError_t gemv_quads_bf16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::BF16, __bf16>(s, a, q); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 2
+hipError_t gemv_quads_bf16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::BF16, _Float16>(s, a, q); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 3
+hipError_t gemv_quads_f16_f32(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::F16, float>(s, a, q); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 4
+hipError_t gemv_quads_f16_bf16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::F16, __bf16>(s, a, q); }
+#endif
+#if !defined(CQ_GEMV_PART) || CQ_GEMV_PART == 5
+hipError_t gemv_quads_f16_f16(hipStream_t s, const GemvArgs& a, const QuadsSplit& q) { return launch_codes<dev::Float::F16, _Float16>(s, a, q); }
+#endif
+
 }  // namespace cq

@@ -225,7 +225,7 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
     return GemvShape::k4x2;
 }
 
-// A product with one to four vectors by gemv_quads_kernel (cq_kernels_gemv_quads.hpp), whose workgroups, one per compute unit, take four
+// A product with one to four vectors by gemv_quads_kernel (cq_kernels_gemv_quads.hip), whose workgroups, one per compute unit, take four
 // rows a wave from x in LDS: whether it does, its workgroups and waves, and how many waves share four rows.  With `work`, the most steps (16
 // units of four rows) that a workgroup has, us before (gemv_stream_kernel, gemv_batch_kernel) -> with it:
 // * Several vectors: against the units that the busiest compute unit goes through there, in groups of 16 rows and stages of eight units.  Under
