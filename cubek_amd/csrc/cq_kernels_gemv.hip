@@ -492,7 +492,8 @@ bool gemv_streams(const GemvArgs& a) {
 namespace {
 
 hipError_t gemv_batch(hipStream_t s, const GemvArgs& a) {
-    const bool lines = ((reinterpret_cast<uintptr_t>(a.words) | (a.word_pitch * 4)) & 127u) == 0, f32 = a.param_dtype == CQ_F32, f16 = a.param_dtype == CQ_F16;
+    const bool whole_lines = ((reinterpret_cast<uintptr_t>(a.words) | (a.word_pitch * 4)) & 127u) == 0;
+    const bool lines = gemv_batch_streams(whole_lines, (a.rows + 15) / 16, a.cols / 8ull * a.bits, a.vectors), f32 = a.param_dtype == CQ_F32, f16 = a.param_dtype == CQ_F16;
     const auto of = [&](hipError_t (*by_f32)(hipStream_t, const GemvArgs&), hipError_t (*by_f16)(hipStream_t, const GemvArgs&), hipError_t (*by_bf16)(hipStream_t, const GemvArgs&)) {
         return (f32 ? by_f32 : f16 ? by_f16 : by_bf16)(s, a);
     };

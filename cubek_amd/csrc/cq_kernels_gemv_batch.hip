@@ -60,8 +60,10 @@ __host__ __device__ constexpr uint32_t x_bytes(uint32_t vectors) {
 // kWholeLines: the rows start on lines of 128 bytes, and the codes, of which a stage takes whole lines, are streamed past the caches.  Rows that do
 // not: a stage reads parts of lines, whose rest the next one wants from the caches (streaming -> plain loads, us: f16 4 bits [2788, 4256] 5 vectors
 // 6.4 -> 5.6, [3590, 14752] 16 19.4 -> 17.6, 8 bits [20000, 6752] 8 44.0 -> 40.8; whole lines [28672, 8192] 8 bits 16 54.7 -> 59.2, 4 bits 36.9 -> 38.9,
-// [14336, 4096] f16 8 10.1 -> 9.7).  A kernel of its own for each: with both behind a branch in every stage whole lines lost 1 - 5 %
-// (4 bits [8192, 28672] 2 vectors 30.8 -> 32.0, e4m3 [12288, 11904] 4 26.7 -> 28.0, 4 bits [14439, 4352] 16 13.2 -> 13.6).
+// [14336, 4096] f16 8 10.1 -> 9.7).  gemv_batch_streams() names the rows of parts that stream all the same.  A kernel of its own for each: with both
+// behind a branch in every stage whole lines lost 1 - 5 % (4 bits [8192, 28672] 2 vectors 30.8 -> 32.0, e4m3 [12288, 11904] 4 26.7 -> 28.0, 4 bits
+// [14439, 4352] 16 13.2 -> 13.6) and parts of lines 2 %; but in 4 x 2 parts of lines are 2 - 4 % slower without it (1536 groups and more, on
+// the mean of 148 products; [19104, 8128] 8 bits 16 54.5 -> 57.2), whose waves it keeps closer together, and there it stays.
 template <dev::Float kF, class FS, int kCode, int kG, int kS, bool kWholeLines>
 __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
     const char* __restrict__ words, const char* __restrict__ scales, const char* __restrict__ x, void* __restrict__ y, int y_dtype,
@@ -114,6 +116,7 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
         x_piece[n] = (in & ~15u) | ((in - v) & 15u);
         x_at[n] = v * x_stride_bytes;
     }
+    [[maybe_unused]] const bool whole_lines = ((reinterpret_cast<uintptr_t>(words) | row_bytes) & 127u) == 0;
     const auto load = [&](uint32_t stage, uint32_t into) {
         const uint32_t unit0 = stage * kU, block0 = unit0 >> units_per_block_log2;
         const bool partial = unit0 + kU > units_per_row;  // wave-uniform: units past the end are the last one again
@@ -124,8 +127,11 @@ __global__ __launch_bounds__(64 * kG * kS, 4) void gemv_batch_kernel(
 #pragma unroll
         for (uint32_t t = 0; t < kCodeLoads; t++) {
             const uint32_t unit = partial ? min(code_unit[t], last_unit) : code_unit[t];
-            __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u)), CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0,
-                                             kWholeLines ? 2 /* nt */ : 0);
+            const u32x4* const p = reinterpret_cast<const u32x4*>(wfrom + (code_row[t] + unit * 16u));
+            if (kWholeLines || (kG == 4 && whole_lines))
+                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 2 /* nt */);
+            else
+                __builtin_amdgcn_global_load_lds(p, CQ_LDS_PTR(code_img + into + t * 1024u), 16, 0, 0);
         }
         const uint32_t slot = partial ? min(scale_slot, last_block) : scale_slot;
 #pragma unroll

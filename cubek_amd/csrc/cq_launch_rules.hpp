@@ -225,6 +225,15 @@ inline GemvShape gemv_batch_shape(uint32_t groups, uint32_t x, uint32_t lds_of_e
     return GemvShape::k4x2;
 }
 
+// Whether such a product streams its codes past the caches: rows of whole lines of 128 bytes, and long rows of parts of them for twelve vectors and more where
+// most compute units have one workgroup: its eight waves read a row's stages side by side, so that the parts of a line are asked for together, and x
+// takes more of the caches (plain loads -> streaming, us, 16 vectors: 8 bits [3507, 10944] 19.4 -> 16.7, [3449, 16736] 28.2 -> 24.8, e2m1 bytes [3522,
+// 22400] 30.0 -> 25.8; on the mean of 16 products 1.06 times as fast, of 34 with fewer vectors level, of rows of 7 to 9 kB or less 0.95, of up to 160
+// groups 0.94).
+inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_bytes, uint32_t vectors) {
+    return whole_lines || (groups > 176 && groups <= 256 && row_bytes >= 9000 && vectors >= 12);
+}
+
 // A product with one to four vectors by gemv_quads_kernel (cq_kernels_gemv_quads.hip), whose workgroups, one per compute unit, take four
 // rows a wave from x in LDS: whether it does, its workgroups and waves, and how many waves share four rows.  With `work`, the most steps (16
 // units of four rows) that a workgroup has, us before (gemv_stream_kernel, gemv_batch_kernel) -> with it:

@@ -193,6 +193,14 @@ def test_products_with_several_vectors_take_the_fastest_shape(answer):
     assert not wrong
 
 
+def test_products_with_several_vectors_stream_their_codes_where_that_is_faster(answer):
+    # (whole lines, rows, bytes of a row, vectors): streaming was the faster way, or within 3 % of it
+    cases = {(True, 28672, 4096, 16): True, (False, 3507, 10944, 16): True, (False, 3449, 16736, 16): True, (False, 3855, 14496, 14): True,
+             (False, 2788, 2128, 5): False, (False, 3590, 7376, 16): False, (False, 20000, 6752, 8): False, (False, 2744, 12096, 16): False, (False, 3873, 14496, 5): False}
+    got = answer([f"gemv_batch_streams({str(lines).lower()}, {-(-rows // 16)}, {row_bytes}, {vectors})" for lines, rows, row_bytes, vectors in cases])
+    assert got == [int(streams) for streams in cases.values()], dict(zip(cases, got))
+
+
 # (rows, columns, vectors, values in 16 bytes of codes, 4-bit fields, x in f16, e4m3 or e5m2): waves of the kernel of four rows a wave, 0 where
 # another is faster, or within 5 % of it
 QUADS = {
