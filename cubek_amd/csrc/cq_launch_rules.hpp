@@ -247,9 +247,17 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 //   on a compute unit (2 vectors [1693, 1920] 3.68 -> 3.83, 4 [1362, 1920] 3.68 -> 3.90; two steps [1024, 2048] 3.66 -> 3.36, five [1085, 2080] 4.31 -> 3.88), and
 //   short rows of 8 bits in five groups of four rows for eight waves or pairs of waves ([5120, 1024] 2 vectors 4.33 -> 4.58, e4m3 3.98 -> 4.50,
 //   [4608, 3456] 3 6.85 -> 7.65; 8 bits [5120, 3072] 4 7.15 -> 6.68, e4m3 [4736, 5504] 3 8.94 -> 8.34).
+//   Rows of whole lines, which gemv_batch_kernel streams: 4 bits of bf16 and e2m1 bytes gain 1.05 times on the mean where others gain 1.15, and
+//   lose on two groups of up to eight steps (e2m1 bytes [2048, 4096] 4.80 -> 5.17), more of up to six ([5120, 2048] 3 4.87 -> 5.21, [19754, 1024] 6.51 -> 6.97), of fields
+//   on three groups of long rows and nine and more ([2863, 14080] 4 10.2 -> 11.3, [9435, 5120] 3 10.3 -> 11.0; six groups 1.04 times as fast), and from work 128 on
+//   where four-row groups fill rounds of sixteen waves badly, 14, 15, 18, 28 ([14336, 8192] 4 18.6 -> 19.9, [14336, 14336] 28.1 -> 30.1, [18326, 7168] 20.1 -> 22.5,
+//   [28672, 11008] 41.6 -> 43.9; [11008, 11008] 1.04 and [28672, 8192] 1.05 times as fast).
+//   e4m3 and e5m2, where the other is nearer to memory's rate: not in two groups of four steps ([2048, 1024] 3.53 -> 3.82), from 0.8 of the units on not for very short
+//   and very long rows ([28672, 2048] 12.3 -> 13.2, [14336, 14336] 34.8 -> 37.4; [28672, 4096] 1.15, [28672, 11008] 1.25 times as fast) nor where a wave or two have four rows
+//   ([25344, 1664] 10.5 -> 11.4, [6784, 7040] 11.3 -> 12.2): all waves in other rows ask the same channels.
 // * One vector, 4 bits of f16: the digits pair up without being shifted together (x is permuted on its way into LDS;
 //   [18484, 6912] 23.3 -> 17.5, [7455, 2240] 7.3 -> 5.7), except in the smallest launches that fill the other's strips as well ([1514, 1280] 3.21 -> 3.42,
-//   [1814, 1792] 3.35 -> 3.70; work 9 [2347, 1408] 3.85 -> 3.64, 12 [3425, 1344] 4.13 -> 3.74).
+//   [1814, 1792] 3.35 -> 3.70; work 9 [2347, 1408] 3.85 -> 3.64, 12 [3425, 1344] 4.13 -> 3.74) or have four steps ([1024, 2048] 3.43 -> 3.64; eight [1024, 4096] 1.04).
 // * One vector of e4m3 and e5m2 bytes, which leave time beside the arithmetic: from work 64 on ([9472, 18176] 32.6 -> 30.2, [4352, 24448] 28.9 ->
 //   22.8; [5888, 1664] 5.3 -> 5.7), but up to 128 not with three to six groups of four rows on a compute unit, whose waves, two to four to a group, start and
 //   end more often than they step ([4736, 4352] 7.46 -> 8.23, [5120, 4096] 6.60 -> 7.37, [3968, 4992] 6.27 -> 6.79; two [2048, 14592] 1.17 and eight [8576, 3328] 1.07
@@ -262,11 +270,13 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 //   -> 14.6, [1024, 28672] 14.9 -> 8.4, [25471, 2240] 14.4 -> 11.8, [2675, 4672] 6.1 -> 5.6; 0.77 [6867, 3584] 6.7 -> 7.3), not in the
 //   smallest launches ([3011, 1408] 3.8 -> 4.0); 8 bits and e2m1 bytes, with fewer steps in a row, under 0.55 up to work 48 (0.62 [2774, 2432] 5.05 -> 5.30, 0.66
 //   [2583, 3360] 5.38 -> 5.63, e2m1 0.62 [4120, 4320] 6.49 -> 6.71; 0.5 [1024, 8192] 6.49 -> 5.28).
+//   Of eight waves with a group each not for five groups or nine, of bf16 ([4708, 1152] 8 bits 4.62 -> 5.21, [4959, 3072] 4 bits 5.59 -> 6.13; seven 1.07, ten
+//   1.03 times as fast).
 // Eight waves where there is little for sixteen to do: work 28 [7455, 2240] f16 5.7, 6.1 of 16; 64 [16115, 1920] 7.9, 7.3; 96 [4352, 24448]
 // 30, 22.8.  Shares of four rows are the fewest steps for the busiest wave, a quarter of one for each sum of its lanes.
 //
-// Over 2730 launches from [1024, 1024] to [28672, 28672] that it takes it is 1.17 times as fast as the others on the mean; 3 % are more than 2.5 % slower, three
-// or four vectors on three groups of four long rows the most (e2m1 bytes [2588, 14272] 9.4 -> 11.0, 4 bits [3072, 14336] 10.6 -> 11.4; e4m3 [14336, 14336] 34.4 -> 37.6).
+// Over 2500 launches from [1024, 1024] to [28672, 28672] that it takes it is 1.17 times as fast as the others on the mean; 2 % are more than 2.5 % slower, e4m3 the
+// most ([13568, 9984] 4 vectors 24.8 -> 27.3, one [4224, 6656] 9.1 -> 10.0).
 struct QuadsSplit {
     uint32_t grid, waves, shares_log2, lds;  // grid 0: the other kernels
 };
@@ -281,6 +291,8 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
     while ((quads + q.grid - 1) / q.grid > kMostQuads) q.grid *= 2;
     const uint32_t each = (quads + q.grid - 1) / q.grid;
     const uint64_t work = static_cast<uint64_t>(quads + kComputeUnits - 1) / kComputeUnits * steps;
+    const bool lines = units % 8 == 0;  // rows of whole lines of 128 bytes
+    bool full = false;                  // the other kernels go through little more
     if (vectors > 1) {
         const uint32_t stage = (vectors * 16 * values + 1023) / 1024 * 1024, groups = rows / 16 + (rows % 16 != 0);
         const GemvShape shape = gemv_batch_shape(groups, stage, 16 * (stage + 2560), units, bytes);
@@ -288,7 +300,17 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const uint64_t busiest = static_cast<uint64_t>((groups + together - 1) / together + kComputeUnits - 1) / kComputeUnits * together * 16 * ((units + 7) / 8) * 8;
         const uint32_t most = work < 64 ? 70 : !fields4 ? (work < 128 ? 80 : 92) : f16 || work >= 128 ? 99 : 85;
         if (work * 64 * 100 >= busiest * most) return kNo;
-        if (values == 32 ? each > 1 && steps > 2 && work <= 8 : each == 5 && work < (bytes ? 96 : 48)) return kNo;
+        const auto at_least = [&](uint32_t percent) { return work * 64 * 100 >= busiest * percent; };  // ... of what the other goes through
+        if (values == 32) {
+            if (each > 1 && steps > 2 && work <= 8) return kNo;
+            if (lines && !(fields4 && f16) && (each == 2 ? steps <= 8 : each >= 5 && steps <= 6 && work < 64)) return kNo;
+            if (lines && fields4 && !f16 && work >= 64 && work < 128 && at_least(75) && (each >= 9 || (each == 3 && steps < 32))) return kNo;
+            if (lines && !(fields4 && f16) && work >= 128 && at_least(85) && (each == 14 || each == 15 || (at_least(89) && each > 15 && (each < 20 || each >= 28)))) return kNo;
+        } else if (each == 5 && work < (bytes ? 96 : 48)) {
+            return kNo;
+        }
+        full = at_least(80);
+        if (bytes && ((each == 2 && steps == 4) || (full && !at_least(90) && (steps < 10 || steps >= 50)))) return kNo;
     } else {
         const uint32_t group = static_cast<uint64_t>(units) * values >= 16384 ? 16 : 8, groups = rows / group + (rows % group != 0);
         const uint64_t stream = static_cast<uint64_t>((units + 63) / 64) * 64 * group * ((groups + kComputeUnits - 1) / kComputeUnits);
@@ -297,7 +319,7 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
             const bool apart_by_2_18 = static_cast<uint64_t>(rows) * units % (1u << 22) == 0;  // 256 shares of units of 16 bytes
             if (work < 64 || (work < 128 && each > 2 && each <= 6) || ((work >= 512 || apart_by_2_18) && at_least(85))) return kNo;
         } else if (fields4 && f16) {
-            if (work <= 8 && at_least(72)) return kNo;
+            if (work <= 8 && (at_least(72) || (each == 1 && steps <= 4))) return kNo;
         } else {
             if (work < 24 || at_least(72) || (!fields4 && work < 48 && at_least(55))) return kNo;
         }
@@ -308,6 +330,7 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const uint64_t slots = q.waves >> l, cost = (each + slots - 1) / slots * (4 * ((static_cast<uint64_t>(steps) + (1u << l) - 1) >> l) + 1);
         if (cost < least) q.shares_log2 = l, least = cost;
     }
+    if (vectors > 1 ? bytes && (q.shares_log2 == 0 || (q.shares_log2 == 1 && full)) : !bytes && !f16 && q.shares_log2 == 0 && (each == 5 || each == 9)) return kNo;
     const uint64_t lds = x_bytes + (each << q.shares_log2) * 64;
     if (lds > kMostLds) return kNo;
     q.lds = static_cast<uint32_t>(lds);

@@ -215,6 +215,16 @@ QUADS = {
     (1693, 1920, 2, 32, True, False, False): 0, (1362, 1920, 4, 32, True, True, False): 0, (1439, 1664, 4, 32, False, True, False): 0, (1085, 2080, 2, 32, True, False, False): 8,
     (1024, 2048, 4, 32, True, False, False): 8, (5120, 1024, 2, 16, False, False, False): 0, (5120, 1024, 4, 16, False, True, True): 0, (4608, 3456, 3, 16, False, False, True): 0,
     (5120, 3072, 4, 16, False, False, False): 16, (4736, 5504, 3, 16, False, False, True): 16,
+    # ... rows of whole lines: short ones, long ones in three groups, groups that fill rounds of sixteen waves badly
+    (5120, 2048, 3, 32, True, False, False): 0, (5120, 2080, 3, 32, True, False, False): 8, (2048, 4096, 4, 32, False, True, False): 0, (19754, 1024, 3, 32, True, False, False): 0,
+    (2863, 14080, 4, 32, True, False, False): 0, (2863, 14112, 4, 32, True, False, False): 16, (9435, 5120, 3, 32, True, False, False): 0, (14336, 8192, 2, 32, True, False, False): 0,
+    (14336, 8192, 2, 32, True, True, False): 16, (18326, 7168, 2, 32, True, False, False): 0, (28672, 11008, 3, 32, True, False, False): 0, (28672, 8192, 4, 32, True, False, False): 16,
+    (11008, 11008, 2, 32, True, False, False): 16,
+    # ... of bytes: near memory's rate
+    (2048, 1024, 4, 16, False, True, True): 0, (28672, 2048, 3, 16, False, True, True): 0, (28672, 4096, 3, 16, False, True, True): 16, (14336, 14336, 4, 16, False, False, True): 0,
+    (28672, 11008, 2, 16, False, False, True): 16, (25344, 1664, 4, 16, False, False, True): 0, (6784, 7040, 3, 16, False, False, True): 0,
+    # one vector: eight waves with five groups
+    (4708, 1152, 1, 16, False, False, False): 0, (4959, 3072, 1, 32, True, False, False): 0, (1024, 2048, 1, 32, True, True, False): 0, (1024, 4096, 1, 32, True, True, False): 8,
     # one vector of 4 bits of f16 in the smallest launches
     (1514, 1280, 1, 32, True, True, False): 0, (1814, 1792, 1, 32, True, True, False): 0, (2347, 1408, 1, 32, True, True, False): 8, (3425, 1344, 1, 32, True, True, False): 8,
     # ... of bytes: few groups of four rows, shares 2^18 bytes apart, large weights
