@@ -1,4 +1,4 @@
-// What the kernels of the products with quantized weights on the matrix cores share (cq_kernels_gemv_quads.hip,
+// What the kernels of the products with quantized weights share (cq_kernels_gemv.hip, cq_kernels_gemv_quads.hip,
 // cq_kernels_gemv_batch.hip): codes to operands of the matrix instructions, and the store of y.
 #pragma once
 

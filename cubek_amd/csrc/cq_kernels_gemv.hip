@@ -14,16 +14,11 @@
 // weight for 4-bit codes with f32 scales on blocks of 32); x and y are negligible.  The roofline is HBM.
 #include <hip/hip_runtime.h>
 
-#include "../../include/cubek_quant_device.hpp"
-#include "cq_internal.hpp"
+#include "cq_gemv_operand.hpp"
 #include "cq_launch_rules.hpp"
 
 namespace cq {
 namespace {
-
-namespace dev = cubek_quant::device;
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <dev::Float kF>
 struct Elem;
@@ -41,7 +36,6 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float acc) {
         typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
         return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), acc, false);
     } else {
-        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
         return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), acc, false);
     }
 }
@@ -70,15 +64,6 @@ __device__ __forceinline__ float wave_sum_to_lane63(float v) {
     return v;
 }
 
-__device__ __forceinline__ void store_y(int dtype, void* y, uint64_t i, float v) {
-    if (dtype == CQ_F32)
-        static_cast<float*>(y)[i] = v;
-    else if (dtype == CQ_F16)
-        static_cast<_Float16*>(y)[i] = static_cast<_Float16>(v);
-    else
-        static_cast<__bf16*>(y)[i] = static_cast<__bf16>(v);
-}
-
 // ---- streaming kernel: 16-bit float types, blocks along the row ---------------------------------------
 // A lane's unit is one 16-byte load of codes: four words, 64 values of 2 bits, 32 of 4 or 16 of 8, under one scale
 // (f32, f16 or bf16; blocks of 1, 2, 4, ... units along the row and any number of rows, or one scale for the
@@ -94,9 +79,8 @@ __device__ __forceinline__ void store_y(int dtype, void* y, uint64_t i, float v)
 // compiler can count its waits.  Per 4-bit value: half a byte-to-float conversion and one FMA
 // (dequantize_symmetric_packed_value_pairs), half a v_cvt_pk, half a v_dot2.
 // kCode: 2, 4 or 8 for fields of that many bits in the U32 store (and the i8 bytes of the native store, which are
-// the same bits), or one of the native encodings below.
-constexpr int kCodeE4M3 = 100, kCodeE5M2 = 101, kCodeE2M1x2 = 102;
-
+// the same bits), or one of the native encodings.
+//
 // kSegment (rows too long for the LDS): strips of x staged at a time; the workgroup meets at a
 // barrier and stages the next ones when its waves have worked through them (they all do the same work, so nobody
 // waits long).  0: all of x at once.
@@ -364,14 +348,6 @@ hipError_t launch_general_bits(hipStream_t s, const GemvArgs& a, const dev::Scal
 constexpr int kStreamRows = 2, kStreamDepth = 2;
 [[maybe_unused]] constexpr uint32_t kStreamMaxColumns = 32768;  // x of that many columns fills 64 KiB of LDS
 
-uint32_t log2_of(uint32_t v) {
-    uint32_t l = 0;
-    while ((1u << l) < v) l++;
-    return l;
-}
-
-constexpr uint32_t values_per_unit(int code) { return code <= 8 ? 128 / code : (code == kCodeE2M1x2 ? 32 : 16); }
-
 // LDS for x: whole strips, 2 bytes per value
 uint32_t stream_lds_bytes(const GemvArgs& a) {
     const uint32_t vals = 128 / a.bits;
@@ -403,13 +379,15 @@ void launch_stream_waves(hipStream_t s, const GemvArgs& a) {
 // 11.7, 34.5 us.
 constexpr int kWideSegment = 16;  // strips of x at a time where a row has more than kStreamMaxColumns values
 
-// kWide: rows of more than kStreamMaxColumns values, x by segments
+// kWide: rows of more than kStreamMaxColumns values, x by segments.  4 bits of f16: only the smallest launches come here (quads_split()), and pitches
+// that the other kernels do not take, so there is no form of eight waves for rows between 16384 columns and those.
 template <dev::Float kF, class FS, int kBits, bool kWide>
 void launch_stream_bits(hipStream_t s, const GemvArgs& a) {
+    [[maybe_unused]] constexpr bool kEight = !(kF == dev::Float::F16 && kBits == 4);
     if constexpr (kWide)
         launch_stream_waves<kF, FS, kBits, 8, kWideSegment * int(values_per_unit(4)) / int(values_per_unit(kBits)) / (kF == dev::Float::F32 ? 2 : 1)>(s, a);
-    else if (a.cols >= 16384)
-        launch_stream_waves<kF, FS, kBits, 8>(s, a);
+    else if (kEight && a.cols >= 16384)
+        launch_stream_waves<kF, FS, kBits, kEight ? 8 : 4>(s, a);
     else
         launch_stream_waves<kF, FS, kBits, 4>(s, a);
 }
