@@ -12,22 +12,23 @@ from cubek_amd import (ComputeClient, ElemType, QuantLevel, QuantParam, QuantSch
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # elem, value, block, param, rows, cols, word pitch (None: contiguous)     -- the streaming kernel unless noted
+    # elem, value, block, param, rows, cols, word pitch (None: contiguous); 16-bit x of 16384 columns and more, and some of f16 and 4 bits, go to the kernel of
+    # four rows a wave, the others to the streaming kernel unless noted (test_launch_rules.py says which)
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 1000, 4096, None),
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 77, 2048, None),
     (ElemType.BF16, QuantValue.E2M1, [32], QuantParam.F32, 130, 11008, None),     # last strip partly idle
     (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 333, 8192, None),
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 64, 4096, 520),         # pitched rows of words
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 50, 8448, None),        # four strips and an eighth
-    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 21, 16480, None),        # eight waves per workgroup
-    (ElemType.BF16, QuantValue.Q4F, [32], QuantParam.F32, 1, 32768, None),        # one row, the longest it takes
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 21, 16480, None),        # a unit behind a step
+    (ElemType.BF16, QuantValue.Q4F, [32], QuantParam.F32, 1, 32768, None),        # one row
     (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 9, 32, None),           # one block per row
     (ElemType.BF16, QuantValue.E2M1_OCP, [32], QuantParam.F32, 37, 2048, None),   # the extension value: e2m1 nibbles in u32 words
-    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 11, 53248, None),       # rows longer than the LDS holds of x
-    (ElemType.F16, QuantValue.Q8S, [64], QuantParam.F16, 5, 40000, None),         # ... 8-bit codes, two segments
+    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 11, 53248, None),       # x longer than the streaming kernel's LDS
+    (ElemType.F16, QuantValue.Q8S, [64], QuantParam.F16, 5, 40000, None),         # ... 8-bit codes
     (ElemType.F16, QuantValue.Q4S, [128], QuantParam.F16, 33, 4224, None),        # four units under one f16 scale
     (ElemType.BF16, QuantValue.Q8S, [32], QuantParam.F32, 45, 2080, None),        # 8-bit codes, two units per block
-    (ElemType.BF16, QuantValue.Q4F, [64], QuantParam.BF16, 19, 16448, 2060),      # bf16 scales, eight waves, pitched
+    (ElemType.BF16, QuantValue.Q4F, [64], QuantParam.BF16, 19, 16448, 2060),      # bf16 scales, pitched
     (ElemType.F16, QuantValue.Q8F, [16], QuantParam.F32, 70, 1040, None),         # 8-bit codes, a scale per unit
     (ElemType.BF16, QuantValue.Q2S, [64], QuantParam.F32, 52, 4160, None),        # 2-bit codes
     (ElemType.F16, QuantValue.Q2F, [128], QuantParam.F16, 17, 8192, None),        # 2-bit codes, two units per block
@@ -116,7 +117,7 @@ NATIVE_CASES = [
     (ElemType.BF16, QuantValue.E4M3, [32], QuantParam.F32, 77, 4128, None),
     (ElemType.F16, QuantValue.E4M3, [128, 128], QuantParam.F32, 256, 2048, None),   # 128 x 128 weight blocks
     (ElemType.BF16, QuantValue.E5M2, [16], QuantParam.BF16, 30, 2064, 2096),        # a scale per unit, pitched rows
-    (ElemType.F16, QuantValue.E5M2, None, QuantParam.F16, 21, 16400, None),         # per tensor, eight waves
+    (ElemType.F16, QuantValue.E5M2, None, QuantParam.F16, 21, 16400, None),         # per tensor, a unit behind a step
     (ElemType.BF16, QuantValue.E2M1, [32], QuantParam.F32, 53, 8448, None),         # e2m1 pairs, a scale per unit
     (ElemType.F16, QuantValue.E2M1, [64], QuantParam.F16, 18, 1088, None),
     (ElemType.BF16, QuantValue.Q8S, [32], QuantParam.F32, 45, 2080, None),          # i8 bytes: the 8-bit fields
@@ -173,12 +174,38 @@ QUADS_CASES = [
     (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 4444, 1056, None, 4, False),
     (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 9, 19424, None, 4, False),         # nearly all of the LDS
     (ElemType.F16, QuantValue.Q4F, [32], QuantParam.F32, 9, 20512, None, 4, False),         # ... and more than there is
+    (ElemType.F16, QuantValue.Q4S, [64], QuantParam.F16, 1, 2112, None, 1, False),          # one row
+    (ElemType.BF16, QuantValue.Q8S, [6, 32], QuantParam.F32, 1026, 16384, None, 1, False),  # blocks of six rows across groups of four
+    (ElemType.BF16, QuantValue.E4M3, [128, 128], QuantParam.F32, 1152, 14464, None, 1, True),
+    (ElemType.BF16, QuantValue.E2M1, [32], QuantParam.F32, 1030, 28672, None, 1, True),
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 4444, 1376, None, 4, False),       # a last group of its own round
 ]
+# ... of these another kernel takes
+NOT_QUADS = [(1, 32, 1), (1026, 12800, 1), (4444, 1056, 4), (9, 20512, 4)]
 
 
 @pytest.mark.parametrize("case", QUADS_CASES, ids=lambda c: _id(c[:7]) + f"-{c[7]}")
 def test_gemv_of_four_rows_a_wave(oracle, case):
     check_case(oracle, case[:7], case[4] + case[7], native=case[8], vectors=case[7])
+
+
+# The streaming kernel with long rows, which it keeps where they fill its workgroups: eight waves with one piece of x, and x by segments, with a strip that
+# is partly idle and a segment that is cut short.
+STREAM_CASES = [
+    (ElemType.BF16, QuantValue.Q4S, [32], QuantParam.F32, 2309, 18400, None, 1, False),
+    (ElemType.F16, QuantValue.Q8S, [32], QuantParam.F16, 3081, 16416, None, 1, False),
+    (ElemType.BF16, QuantValue.E4M3, [128, 128], QuantParam.BF16, 4096, 16384, None, 1, True),
+    (ElemType.BF16, QuantValue.Q4F, [64], QuantParam.BF16, 11, 90176, None, 1, False),
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 6, 84000, None, 1, False),
+    (ElemType.F16, QuantValue.Q8F, [16], QuantParam.F32, 5, 82000, None, 1, False),
+    (ElemType.BF16, QuantValue.E2M1, [32], QuantParam.F32, 7, 98336, None, 1, True),
+    (ElemType.F16, QuantValue.Q4S, [32], QuantParam.F32, 2, 16416, 1 << 25, 1, False),      # a pitch that the others do not take
+]
+
+
+@pytest.mark.parametrize("case", STREAM_CASES, ids=lambda c: _id(c[:7]))
+def test_gemv_of_long_rows_by_the_streaming_kernel(oracle, case):
+    check_case(oracle, case[:7], case[5], native=case[8])
 
 
 # Every split of a workgroup (four, two or one group of 16 rows; rows on two, four or eight waves): rows that end inside a
@@ -204,9 +231,9 @@ def test_gemv_of_a_batch(oracle, case, vectors):
 
 
 # (rows, cols) on both sides of each line that the split of a launch over row groups and waves is drawn at: 256, 512, 768, 1024 and 1536
-# groups of 16 rows, rows of 8, 12 and 48 units of 32 (4 bits) values and just more
+# groups of 16 rows, rows of 8, 12 and 48 units of 32 (4 bits) values and just more; last, long rows of parts of lines that are streamed all the same (8 bits)
 SPLITS = [(17, 288), (4096, 256), (4096, 288), (1000, 384), (1000, 416), (4097, 416), (8192, 320), (8193, 320), (12288, 320), (12289, 320),
-          (16384, 288), (16385, 1504), (16385, 1536), (24576, 1568), (24577, 1568)]
+          (16384, 288), (16385, 1504), (16385, 1536), (24576, 1568), (24577, 1568), (2833, 9056)]
 
 
 @pytest.mark.parametrize("vectors", [2, 5, 12, 16])
@@ -424,6 +451,70 @@ def test_gemv_of_a_batch_scales_of_every_kind(oracle, kind, value, vectors):
     got = y.cpu().numpy().astype(np.float64)
     finite = np.isfinite(want)
     assert np.array_equal(np.flatnonzero(~finite[0]), [2, 17, 40, 82] if infinite else []) and not np.any(np.isnan(want))
+    assert np.array_equal(got[~finite], want[~finite])
+    err = np.abs(got[finite] - want[finite])
+    assert np.all(err <= 2e-5 * mag[finite] + 1e-30), float(np.max(err / (mag[finite] + 1e-30)))
+
+
+# Steps of sixteen units and a last one of one or two, shared by all waves.  Values of unit deviation for x but where the weights are tiny.
+@pytest.mark.parametrize("vectors", [1, 3])
+@pytest.mark.parametrize("value", [QuantValue.Q4S, QuantValue.Q8S, QuantValue.E4M3, QuantValue.E2M1], ids=lambda v: v.name)
+@pytest.mark.parametrize("kind", ["bf16", "bf16-large", "bf16-subnormal", "bf16-infinite", "f16", "f16-edge", "f16-subnormal", "f16-infinite"])
+def test_gemv_of_four_rows_a_wave_scales_of_every_kind(oracle, kind, value, vectors):
+    """Odd scales in one block in twenty and in a row's last one; all weights subnormal numbers of their type, against x large enough for sums
+    above the tolerance's floor; an infinite scale on codes of one sign against ones in x."""
+    import torch
+
+    rows, cols = 70, 16416
+    elem, ulp, normal = (ElemType.F16, 2.0 ** -24, 2.0 ** -14) if kind.startswith("f16") else (ElemType.BF16, 2.0 ** -133, 2.0 ** -126)
+    infinite, subnormal = kind.endswith("infinite"), kind.endswith("subnormal")
+    native = value in (QuantValue.E4M3, QuantValue.E2M1)
+    scheme = QuantScheme.default().with_value(value).with_level(QuantLevel.block([32]))
+    if native:
+        scheme = scheme.with_store(QuantStore.Native)
+    rng = np.random.default_rng(91 + vectors)
+    bits = {QuantValue.Q8S: 8, QuantValue.E4M3: 8}.get(value, 4)
+    codes = rng.integers(0, 256, (rows, cols * bits // 8), dtype=np.uint8)
+    if value == QuantValue.E4M3:
+        codes &= 0xBF   # no NaN, and 1.9 at most
+    blocks = (rows, cols // 32)
+    x32 = rng.normal(0, 1, (vectors, cols)).astype(np.float32)
+    if subnormal:
+        step = {QuantValue.Q8S: 128, QuantValue.Q4S: 8, QuantValue.E2M1: 6}.get(value, 2)  # the largest code
+        scales = (rng.integers(1, int(normal / ulp / step) + 1, blocks) * ulp).astype(np.float32)
+        x32 *= 100.0 if elem == ElemType.F16 else np.float32(2.0 ** 120)
+    else:
+        scales = rng.uniform(0.001, 0.02, blocks).astype(np.float32)
+        odd = np.array(SCALE_CASES[kind], np.float32)
+        if kind == "f16-edge" and value == QuantValue.Q8S:
+            odd /= 16  # 128 * 512 would not be a number of f16
+        at = rng.random(blocks) < 0.05
+        at[:, -1] |= rng.random(rows) < 0.3
+        if not infinite:
+            scales[at] = rng.choice(odd, int(at.sum()))
+    xb = oracle.to_bits(x32, elem).reshape(vectors, cols)
+    wrong = [2, 17, 40, 69] if infinite else []
+    for k, (row, block) in enumerate(zip(wrong, (0, 300, cols // 32 - 1, 7))):
+        scales[row, block] = odd[k % len(odd)]
+        codes[row, slice(block * 32 * bits // 8, (block + 1) * 32 * bits // 8)] = 0x33 if bits == 4 else 0x38
+        xb[:, block * 32:(block + 1) * 32] = oracle.to_bits(np.ones(32, np.float32), elem)
+    stored = codes if native else codes.view(np.uint32)
+    deq = oracle.from_bits(oracle.dequantize(stored, (rows, cols), scales, elem, scheme), elem).astype(np.float64)
+    if subnormal:
+        assert np.max(np.abs(deq)) <= normal and np.mean(deq != 0) > 0.7
+    x64 = oracle.from_bits(xb, elem).astype(np.float64).reshape(vectors, cols)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want, mag = x64 @ deq.T, np.abs(x64) @ np.abs(deq).T
+    h = TensorHandleRef.from_torch
+    d_stored = torch.from_numpy(stored if native else stored.view(np.int32)).cuda()
+    d_scales, d_x = torch.from_numpy(scales).cuda(), torch.from_numpy(xb.view(np.int16)).cuda()
+    y = torch.zeros((vectors, rows), dtype=torch.float32, device="cuda")
+    h_x, h_y = (h(d_x), h(y)) if vectors > 1 else (h(d_x[0]), h(y[0]))
+    matvec.launch_ref(ComputeClient.current(), h(d_stored), h(d_scales), scheme, h_x, h_y, elem, ElemType.F32)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().astype(np.float64)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.flatnonzero(~finite[0]), wrong) and not np.any(np.isnan(want))
     assert np.array_equal(got[~finite], want[~finite])
     err = np.abs(got[finite] - want[finite])
     assert np.all(err <= 2e-5 * mag[finite] + 1e-30), float(np.max(err / (mag[finite] + 1e-30)))

@@ -246,6 +246,31 @@ def test_products_take_four_rows_a_wave_where_that_is_faster(answer):
     assert got == list(QUADS.values()), dict(zip(QUADS, got))
 
 
+def gemv_route(case, vectors, native):
+    """The kernel of a product that the other tests list: x in 16 bits, fields of 4 or 8 bits, whole units and blocks of a power of two of them."""
+    value, rows, cols = case[1].name, case[4], case[5]
+    per_unit = 16 if value in ("Q8S", "Q8F", "E4M3", "E5M2") else 32
+    return f"{quads_split(rows, cols, vectors, per_unit, per_unit == 32 and not native, case[0].name == 'F16', native and value in ('E4M3', 'E5M2'))}.grid != 0"
+
+
+def test_listed_products_reach_the_kernels_they_are_listed_for(answer):
+    from test_gpu_gemv import CASES, NATIVE_CASES, NOT_QUADS, QUADS_CASES, STREAM_CASES
+
+    got = answer([gemv_route(case, case[7], case[8]) for case in QUADS_CASES])
+    assert [(case[4], case[5], case[7]) for case, quads in zip(QUADS_CASES, got) if not quads] == NOT_QUADS
+    contiguous = [case for case in STREAM_CASES if case[6] is None]
+    assert answer([gemv_route(case, 1, case[8]) for case in contiguous]) == [0] * len(contiguous)
+    # the products with odd scales: every kind of codes, one vector and three
+    odd = [quads_split(70, 16416, vectors, per_unit, *flags) for vectors in (1, 3) for f16 in (False, True)
+           for per_unit, *flags in ((32, True, f16, False), (16, False, f16, False), (16, False, f16, True), (32, False, f16, False))]
+    assert answer([f"{q}.grid != 0" for q in odd]) == [1] * len(odd)
+    # among the others both kernels occur, with either type of x
+    for listed, native in ((CASES, False), (NATIVE_CASES, True)):
+        listed = [case for case in listed if case[0].name != "F32" and not case[1].name.startswith("Q2") and case[5] % 32 == 0 and (case[2] is None or case[2][-1] % 16 == 0)]
+        routes = {(case[0].name, quads) for case, quads in zip(listed, answer([gemv_route(case, 1, native) for case in listed]))}
+        assert routes >= {("F16", 0), ("BF16", 0)} and (native or routes >= {("F16", 1), ("BF16", 1)})
+
+
 def test_four_rows_a_wave_fit_what_the_kernel_keeps(answer):
     """Quads per workgroup in 8 bits, what is left over in 24, x and the sums in the shared memory of a compute unit, workgroups no more than quads."""
     cases = [(rows, cols, vectors, 32, True, True, False) for rows in (1, 4, 5, 1023, 65536, 65541, 1 << 22, (1 << 31) - 1)
