@@ -126,10 +126,10 @@ inline ReduceTile reduce_tile(const ReduceColumns& c) {
 
 // Whether the workgroups of the one launch (512 lanes, four loads a lane in a trip) send out the next trip's loads before the last one's are
 // folded (us, without -> with it): tiles of 16 columns with two to four trips, [404, 23360] 6.3 -> 5.7, [254, 33600] level, and of 8, which read whole lines where
-// rows are whole lines, [829, 6976] 6.1 -> 5.5; half lines lose, [509, 10464] 5.5 -> 5.7.  More trips as long as no compute unit has a second tile, [666, 18112]
-// 7.7 -> 6.9 ([602, 32896], 257 tiles, 9.7 -> 10.3), of 8 columns while every third has none: [1041, 9088] 6.3 -> 5.9 ([1134, 16384] 8.8 -> 9.3, [1082, 11776] 8.35 ->
+// rows are whole lines, [829, 6976] 6.1 -> 5.5; half lines lose, [509, 10464] 5.4 -> 5.5.  More trips as long as no compute unit has a second tile, [666, 18112]
+// 7.7 -> 6.9 ([602, 32896], 257 tiles, 9.7 -> 10.3), of 8 columns while every third has none: [1041, 9088] 6.5 -> 6.2 ([1134, 16384] 8.8 -> 9.3, [1082, 11776] 8.35 ->
 // 8.5).  Not where there is nothing to load ahead, for ragged rows ([558, 9249] 6.95 -> 7.3, [5, 738, 3761] 10.15 -> 10.4), for narrower tiles, whose launches are small
-// ([1116, 2307] 8.25 -> 8.6, f32 [1134, 115] 6.8 -> 7.1), nor past 896 tiles ([5, 138, 25216] 7.6 -> 8.3) or 1536 rows (bf16 [4093, 11008] 18.0 -> 18.7, [3726, 16384]
+// ([1116, 2307] 8.25 -> 8.6, f32 [1134, 115] 5.8 -> 6.1), nor past 896 tiles ([5, 138, 25216] 7.6 -> 8.3) or 1536 rows (bf16 [4093, 11008] 18.0 -> 18.7, [3726, 16384]
 // 22.2 -> 24.2).  Over 1900 launches that it takes 1.03 times as fast on the mean, 0.97 at the least.
 inline bool reduce_loads_ahead(const ReduceColumns& c, const ReduceTile& tile) {
     if (c.ragged || tile.cw < 8 || c.len > 1536) return false;
