@@ -253,7 +253,8 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 //   where four-row groups fill rounds of sixteen waves badly, 14, 15, 18, 28 ([14336, 8192] 4 18.6 -> 19.9, [14336, 14336] 28.1 -> 30.1, [18326, 7168] 20.1 -> 22.5,
 //   [28672, 11008] 41.6 -> 43.9; [11008, 11008] 1.04 and [28672, 8192] 1.05 times as fast).
 //   e4m3 and e5m2, where the other is nearer to memory's rate: not in two groups of four steps ([2048, 1024] 3.53 -> 3.82), from 0.8 of the units on not for very short
-//   and very long rows ([28672, 2048] 12.3 -> 13.2, [14336, 14336] 34.8 -> 37.4; [28672, 4096] 1.15, [28672, 11008] 1.25 times as fast) nor where a wave or two have four rows
+//   and very long rows ([28672, 2048] 12.3 -> 13.2, [14336, 14336] 34.8 -> 37.4; [28672, 4096] 1.15, [28672, 11008] 1.25 times as fast, long ones in eight to
+//   thirteen groups 1.09, [9728, 23936] 46.7 -> 39.8) nor where a wave or two have four rows
 //   ([25344, 1664] 10.5 -> 11.4, [6784, 7040] 11.3 -> 12.2): all waves in other rows ask the same channels.
 // * One vector, 4 bits of f16: the digits pair up without being shifted together (x is permuted on its way into LDS;
 //   [18484, 6912] 23.3 -> 17.5, [7455, 2240] 7.3 -> 5.7), except in the smallest launches that fill the other's strips as well ([1514, 1280] 3.21 -> 3.42,
@@ -261,10 +262,12 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 // * One vector of e4m3 and e5m2 bytes, which leave time beside the arithmetic: from work 64 on ([9472, 18176] 32.6 -> 30.2, [4352, 24448] 28.9 ->
 //   22.8; [5888, 1664] 5.3 -> 5.7), but up to 128 not with three to six groups of four rows on a compute unit, whose waves, two to four to a group, start and
 //   end more often than they step ([4736, 4352] 7.46 -> 8.23, [5120, 4096] 6.60 -> 7.37, [3968, 4992] 6.27 -> 6.79; two [2048, 14592] 1.17 and eight [8576, 3328] 1.07
-//   times as fast).  The waves go through their rows in step, so they ask the same channels of memory at a time where those rows lie apart by
+//   times as fast), and up to 512 not with six or ten in few strips ([9856, 1664] 6.03 -> 7.35, 0.96 and 0.98 times as fast on the mean of 99; nine and eleven 1.03, 1.05).  The waves go through their rows in step, so they ask the same channels of memory at a time where those rows lie apart by
 //   the wrong distances: a compute unit's share a multiple of 2^18 bytes ([8192, 8192] 14.5 -> 15.3, [16384, 8192] 24.7 -> 27.2, [24576, 8192] 35.0 -> 42.3),
 //   and others ([14336, 11008] 31.1 -> 34.7, [28672, 10624] 51 -> 55; [28672, 10496] 52 -> 50, [20480, 11008] 42.5 -> 38.4).  From work 512 on, where the other
-//   kernel is near memory's rate, only where that one's strips and workgroups are filled badly ([5120, 28672] 32.5 -> 26.5, [6144, 24576] 29.1 -> 26.5).
+//   kernel is near memory's rate, only where that one's strips and workgroups are filled badly ([5120, 28672] 32.5 -> 26.5, [6144, 24576] 29.1 -> 26.5) or eight
+//   and more waves share four rows, or four of up to eleven groups ([9216, 16128] 30.1 -> 26.7, [11008, 14336] 30.5 -> 28.1; 1.03 times as fast on the mean of 229; the
+//   others of four waves and fewer 0.99).
 // * Else one vector is bound by the same instructions either way, and it takes the launch where the other's strips of 64 units and workgroups
 //   of 8 or 16 rows are filled badly: four-row steps of 16 units under 0.72 of what its busiest compute unit goes through ([4524, 16512] 18.2
 //   -> 14.6, [1024, 28672] 14.9 -> 8.4, [25471, 2240] 14.4 -> 11.8, [2675, 4672] 6.1 -> 5.6; 0.77 [6867, 3584] 6.7 -> 7.3), not in the
@@ -310,14 +313,15 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
             return kNo;
         }
         full = at_least(80);
-        if (bytes && ((each == 2 && steps == 4) || (full && !at_least(90) && (steps < 10 || steps >= 50)))) return kNo;
+        if (bytes && ((each == 2 && steps == 4) || (full && !at_least(90) && (steps < 10 || (steps >= 50 && (each < 8 || each >= 14)))))) return kNo;
     } else {
         const uint32_t group = static_cast<uint64_t>(units) * values >= 16384 ? 16 : 8, groups = rows / group + (rows % group != 0);
         const uint64_t stream = static_cast<uint64_t>((units + 63) / 64) * 64 * group * ((groups + kComputeUnits - 1) / kComputeUnits);
         const auto at_least = [&](uint32_t percent) { return work * 64 * 100 >= stream * percent; };  // ... of what the other goes through
         if (bytes) {
             const bool apart_by_2_18 = static_cast<uint64_t>(rows) * units % (1u << 22) == 0;  // 256 shares of units of 16 bytes
-            if (work < 64 || (work < 128 && each > 2 && each <= 6) || ((work >= 512 || apart_by_2_18) && at_least(85))) return kNo;
+            if (work < 64 || (work < 128 && each > 2 && each <= 6) || (at_least(85) && (apart_by_2_18 || (work < 512 && (each == 6 || each == 10))))) return kNo;
+            full = work >= 512 && at_least(85);
         } else if (fields4 && f16) {
             if (work <= 8 && (at_least(72) || (each == 1 && steps <= 4))) return kNo;
         } else {
@@ -330,7 +334,8 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const uint64_t slots = q.waves >> l, cost = (each + slots - 1) / slots * (4 * ((static_cast<uint64_t>(steps) + (1u << l) - 1) >> l) + 1);
         if (cost < least) q.shares_log2 = l, least = cost;
     }
-    if (vectors > 1 ? bytes && (q.shares_log2 == 0 || (q.shares_log2 == 1 && full)) : !bytes && !f16 && q.shares_log2 == 0 && (each == 5 || each == 9)) return kNo;
+    if (vectors > 1 ? bytes && (q.shares_log2 == 0 || (q.shares_log2 == 1 && full))
+                    : bytes ? full && q.shares_log2 < (each < 12 ? 2u : 3u) : !f16 && q.shares_log2 == 0 && (each == 5 || each == 9)) return kNo;
     const uint64_t lds = x_bytes + (each << q.shares_log2) * 64;
     if (lds > kMostLds) return kNo;
     q.lds = static_cast<uint32_t>(lds);

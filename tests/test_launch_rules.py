@@ -223,6 +223,8 @@ QUADS = {
     # ... of bytes: near memory's rate
     (2048, 1024, 4, 16, False, True, True): 0, (28672, 2048, 3, 16, False, True, True): 0, (28672, 4096, 3, 16, False, True, True): 16, (14336, 14336, 4, 16, False, False, True): 0,
     (28672, 11008, 2, 16, False, False, True): 16, (25344, 1664, 4, 16, False, False, True): 0, (6784, 7040, 3, 16, False, False, True): 0,
+    (9728, 23936, 2, 16, False, False, True): 16, (9216, 16128, 1, 16, False, False, True): 16, (11008, 14336, 1, 16, False, True, True): 16, (19712, 14336, 1, 16, False, False, True): 0,
+    (9856, 1664, 1, 16, False, False, True): 0, (6144, 6144, 1, 16, False, False, True): 0, (11008, 4096, 1, 16, False, True, True): 16,
     # one vector: eight waves with five groups
     (4708, 1152, 1, 16, False, False, False): 0, (4959, 3072, 1, 32, True, False, False): 0, (1024, 2048, 1, 32, True, True, False): 0, (1024, 4096, 1, 32, True, True, False): 8,
     # one vector of 4 bits of f16 in the smallest launches
