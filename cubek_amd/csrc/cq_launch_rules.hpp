@@ -248,10 +248,10 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 //   short rows of 8 bits in five groups of four rows for eight waves or pairs of waves ([5120, 1024] 2 vectors 4.33 -> 4.58, e4m3 3.98 -> 4.50,
 //   [4608, 3456] 3 6.85 -> 7.65; 8 bits [5120, 3072] 4 7.15 -> 6.68, e4m3 [4736, 5504] 3 8.94 -> 8.34).
 //   Rows of whole lines, which gemv_batch_kernel streams: 4 bits of bf16 and e2m1 bytes gain 1.05 times on the mean where others gain 1.15, and
-//   lose on two groups of up to eight steps (e2m1 bytes [2048, 4096] 4.80 -> 5.17), more of up to six ([5120, 2048] 3 4.87 -> 5.21, [19754, 1024] 6.51 -> 6.97), of fields
-//   on three groups of long rows and nine and more ([2863, 14080] 4 10.2 -> 11.3, [9435, 5120] 3 10.3 -> 11.0; six groups 1.04 times as fast), and from work 128 on
-//   where four-row groups fill rounds of sixteen waves badly, 14, 15, 18, 28 ([14336, 8192] 4 18.6 -> 19.9, [14336, 14336] 28.1 -> 30.1, [18326, 7168] 20.1 -> 22.5,
-//   [28672, 11008] 41.6 -> 43.9; [11008, 11008] 1.04 and [28672, 8192] 1.05 times as fast).
+//   lose with three and four vectors on two groups of four, six or eight steps (e2m1 bytes [2048, 4096] 4.80 -> 5.17; five and seven, and two vectors, 1.05 times as
+//   fast), on more of up to six ([5120, 2048] 3 4.87 -> 5.21, [19754, 1024] 6.51 -> 6.97), fields on nine and more of work 64 to 128, and on three of long rows with
+//   more than two vectors ([9435, 5120] 3 10.3 -> 11.0, [2863, 14080] 4 10.2 -> 11.3; six groups 1.04), and from work 128 on where they leave one or two of
+//   sixteen waves without a group, 14 and 15 (0.97 on the mean of 237, [14336, 8192] 4 18.6 -> 19.9, [14336, 14336] 28.1 -> 30.1; [11008, 11008] 1.04 and [28672, 8192] 1.05).
 //   e4m3 and e5m2, where the other is nearer to memory's rate: not in two groups of four steps ([2048, 1024] 3.53 -> 3.82), from 0.8 of the units on not for very short
 //   and very long rows ([28672, 2048] 12.3 -> 13.2, [14336, 14336] 34.8 -> 37.4; [28672, 4096] 1.15, [28672, 11008] 1.25 times as fast, long ones in eight to
 //   thirteen groups 1.09, [9728, 23936] 46.7 -> 39.8) nor where a wave or two have four rows
@@ -306,9 +306,9 @@ inline QuadsSplit quads_split(uint32_t rows, uint32_t units, uint32_t values, ui
         const auto at_least = [&](uint32_t percent) { return work * 64 * 100 >= busiest * percent; };  // ... of what the other goes through
         if (values == 32) {
             if (each > 1 && steps > 2 && work <= 8) return kNo;
-            if (lines && !(fields4 && f16) && (each == 2 ? steps <= 8 : each >= 5 && steps <= 6 && work < 64)) return kNo;
-            if (lines && fields4 && !f16 && work >= 64 && work < 128 && at_least(75) && (each >= 9 || (each == 3 && steps < 32))) return kNo;
-            if (lines && !(fields4 && f16) && work >= 128 && at_least(85) && (each == 14 || each == 15 || (at_least(89) && each > 15 && (each < 20 || each >= 28)))) return kNo;
+            if (lines && !(fields4 && f16) && (each == 2 ? vectors > 2 && steps > 2 && steps <= 8 && steps % 2 == 0 : each >= 5 && steps <= 6 && work < 64)) return kNo;
+            if (lines && fields4 && !f16 && work >= 64 && work < 128 && at_least(75) && (each >= 9 || (each == 3 && vectors > 2 && steps < 32))) return kNo;
+            if (lines && !(fields4 && f16) && work >= 128 && at_least(85) && (each == 14 || each == 15)) return kNo;
         } else if (each == 5 && work < (bytes ? 96 : 48)) {
             return kNo;
         }

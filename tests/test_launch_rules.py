@@ -218,7 +218,7 @@ QUADS = {
     # ... rows of whole lines: short ones, long ones in three groups, groups that fill rounds of sixteen waves badly
     (5120, 2048, 3, 32, True, False, False): 0, (5120, 2080, 3, 32, True, False, False): 8, (2048, 4096, 4, 32, False, True, False): 0, (19754, 1024, 3, 32, True, False, False): 0,
     (2863, 14080, 4, 32, True, False, False): 0, (2863, 14112, 4, 32, True, False, False): 16, (9435, 5120, 3, 32, True, False, False): 0, (14336, 8192, 2, 32, True, False, False): 0,
-    (14336, 8192, 2, 32, True, True, False): 16, (18326, 7168, 2, 32, True, False, False): 0, (28672, 11008, 3, 32, True, False, False): 0, (28672, 8192, 4, 32, True, False, False): 16,
+    (14336, 8192, 2, 32, True, True, False): 16, (28672, 5120, 3, 32, True, False, False): 16, (2048, 4096, 2, 32, True, False, False): 8, (28672, 8192, 4, 32, True, False, False): 16,
     (11008, 11008, 2, 32, True, False, False): 16,
     # ... of bytes: near memory's rate
     (2048, 1024, 4, 16, False, True, True): 0, (28672, 2048, 3, 16, False, True, True): 0, (28672, 4096, 3, 16, False, True, True): 16, (14336, 14336, 4, 16, False, False, True): 0,
