@@ -278,7 +278,7 @@ inline bool gemv_batch_streams(bool whole_lines, uint32_t groups, uint64_t row_b
 // Eight waves where there is little for sixteen to do: work 28 [7455, 2240] f16 5.7, 6.1 of 16; 64 [16115, 1920] 7.9, 7.3; 96 [4352, 24448]
 // 30, 22.8.  Shares of four rows are the fewest steps for the busiest wave, a quarter of one for each sum of its lanes.
 //
-// Over 2500 launches from [1024, 1024] to [28672, 28672] that it takes it is 1.17 times as fast as the others on the mean; 2 % are more than 2.5 % slower, e4m3 the
+// Over 3400 launches from [1024, 1024] to [28672, 28672] that it takes it is 1.18 times as fast as the others on the mean; 2 % are more than 2.5 % slower, e4m3 the
 // most ([13568, 9984] 4 vectors 24.8 -> 27.3, one [4224, 6656] 9.1 -> 10.0).
 struct QuadsSplit {
     uint32_t grid, waves, shares_log2, lds;  // grid 0: the other kernels
